@@ -100,6 +100,10 @@ struct DeviceProps {
 };
 int device_props(const DeviceProps** out);
 
+// Launches a kernel whose workgroups wait for each other: `grid` is at most what the device holds at once.  As an
+// ordinary launch while that is enough, as a cooperative one otherwise (see ftk_api.hip).
+int launch_resident(const void* fn, dim3 grid, dim3 block, void** args, size_t lds, hipStream_t s);
+
 // ---- vector types for MFMA operands ----------------------------------------
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef float v16f __attribute__((ext_vector_type(16)));

@@ -1,0 +1,929 @@
+// Stacked / dilated LSTM for stacks that wait: one launch for the whole (layer, time) grid, made for the time a
+// hidden state takes from the compute units that produce it to the compute units that need it next.
+//
+// What bounds such a stack is not its products but its chain of L + T - 1 dependent steps, so everything here is
+// about the length of one step.  A layer is spread over H / 16 workgroups of 4 waves (a team; with several row
+// slices a layer has several teams, each with batch rows of its own).  A workgroup owns 16 hidden units = 64 gate
+// columns and keeps its slice of [W;U] in registers for the whole launch.  An item is a block of 16 batch rows of one time
+// step (32 rows where a workgroup has several blocks to walk):
+//
+//   * Its four waves cut the CONTRACTION, not the columns: wave w multiplies quarter w of x_t and quarter w of h_{t-d}
+//     with all 64 columns.  A wave therefore loads exactly the activations it needs, from memory straight into the
+//     registers the matrix instruction reads (v_mfma_f32_16x16x32_f16, weights as the A operand, activations as B):
+//     no tile in LDS and nothing read twice by a compute unit.  The four partial sums of a column meet in LDS, one
+//     barrier per item.
+//   * The 16 columns of a matrix instruction are 4 units x {i, f, o, c~}, so a lane gets the four gates of one
+//     (row, unit) and the state update is one of its own values.
+//   * h is handed over as data, without flags.  The words of the exchange buffers hold a value no h can have (all
+//     ones: a NaN) until h is there, and whoever needs h loads the words until none of them is that value.  One trip of
+//     the data instead of data, acknowledgement, flag, look at the flag, data.
+//   * A team sits on one XCD (workgroups are dealt to the XCDs in turn, and the kernel compares the XCC ids it finds),
+//     so its members hand h over through the L2 they share: plain stores, agent-scope loads.  Measured between 8 / 16 /
+//     32 workgroups that exchange a whole tile: 0.49 / 0.76 / 0.98 us a step, against 0.81 / 1.24 / 1.71 us with
+//     write-through stores, which is what a team that does not sit together uses.
+//
+// A step of a single layer takes 1.1 us at H = 64, 1.3 at 128, 1.6 at 256 and 2.4 at 512 (fp32), where a hand-over of the
+// persistent kernel's serial schedule took 5 to 6 and a launch per step 20 and more: L 20 T 30 B 32 H 128 1004 -> 108 us,
+// L 8 T 100 B 64 H 512 7.3 -> 0.76 ms, L 1 T 16 B 64 H 256 100 -> 26 us of kernel time.
+//
+// The exchange buffers.  ring: the own layer's h for d = 1, four steps deep.  A workgroup that has all of h(t-1) knows
+// that every member of its team has read h(t-2) (it published h(t-1) behind a barrier that all its waves reached after
+// they had h(t-2)), so it sets its words of slot t-2 back to all ones, which are used again at t+2.  hand: every h of
+// every layer, for the layer above and for dilated recurrences; the producer itself sets the words of step t+2 to
+// all ones before it publishes step t+1, and a consumer looks at step t+2 only after it has seen step t+1.  The first
+// two steps, the ring and the input rows (in the same form) are written by the small kernel in front.
+//
+// Products.  fp32 data: an operand is an fp16 value and the fp16 of what that leaves, under a power-of-two scale of its
+// weight column or input row (h: 2^14); three fp16 matrix instructions per product, fp32 accumulation (see
+// lstm_persistent.hip).  A word of the exchange buffers is the pair.  fp16 data: one instruction per product, the
+// exchange buffers hold the fp16 h.
+//
+// Everything waits with a bound (spin_limit looks); when one runs out the status word is set and the launch drains.
+#include <stdlib.h>
+
+#include <algorithm>
+
+#include "ftk_common.h"
+
+namespace ftk {
+
+constexpr int kXLayers = 64;       // layers of one launch
+constexpr int kXBlocks = 128;      // row blocks a ragged batch may have
+constexpr int kXRing = 4;          // steps the own layer's ring holds
+constexpr int kXPlaces = 2048;     // workgroups of one launch
+constexpr int kXHandTop = 14;      // the scale of h: 2^14 (|h| < 1)
+constexpr unsigned kXSmallBits = (127u - 12u) << 23;   // h * 2^14 below 2^-12: see ftk_stacked_lstm_small_states
+
+struct ExchangeArgs {
+  const void* WU;
+  const float* bias;
+  void* hsss;
+  void* csss;
+  int* status;          // [0] error word, [1] small states
+  int* place;           // [groups]: 1 + the XCC id of every workgroup
+  unsigned char* ring;  // [L][nrb][kXRing] tiles
+  unsigned char* hand;  // [L + 1][T][nrb] tiles: the input rows, then every layer's h
+  const float* xratio;  // [T][row of a block] what the products of an input row are multiplied by to match h's (fp32 data)
+  int L, T, B, nrb;
+  int slices;           // row slices = teams per layer; slice s walks row blocks s, s + slices, ...
+  int units;            // L * slices teams
+  int per_xcd;          // > 0: teams per XCD, unit u on XCD u / per_xcd; 0: workgroups in order
+  int spin_limit;
+  int ragged;
+  int dil[kXLayers];
+  unsigned short steps_of[kXBlocks];   // ragged: steps row block rb takes part in
+};
+
+typedef unsigned long long u64;
+typedef unsigned short v2us __attribute__((ext_vector_type(2)));
+constexpr int kAgentScope = 16;      // sc1 in the cache-policy operand of a buffer load
+
+// A tile of the exchange buffers: the h of a row block.  fp32 data: [H / 4][rows][4 units] words (value, remainder); fp16
+// data: [H / 8][rows][8 units] halves.  What a wave stores is contiguous, what a lane loads is 16 bytes.
+constexpr int exchange_tile_bytes(int H, bool half, int rows) { return H * rows * (half ? 2 : 4); }
+
+// Hidden units of a workgroup.  Where the batch is large enough to keep workgroups busy (many) a workgroup takes as many
+// columns as its registers hold at one workgroup per compute unit: every column more is a use more of an activation that
+// has to come through L2 anyway.
+constexpr int exchange_units(int H, bool half, bool many) { return many && H * (half ? 1 : 2) == 512 ? 32 : 16; }
+// Workgroups a compute unit is to hold: the weights of 16 units take H / 2 registers of a lane (fp16 data: H / 4).
+constexpr int exchange_per_cu(int H, bool half, bool many) {
+  const int weights = H * exchange_units(H, half, many) / (half ? 64 : 32);
+  return weights >= 256 ? 1 : weights >= 128 || many ? 2 : 3;
+}
+
+// MANY == false: one row block of 16 rows per workgroup, where an item waits for the one before it and the wait is what is
+// being shortened.  MANY: row blocks of 32 rows (v_mfma_f32_32x32x16_f16: a fifth less time per product, half the
+// overhead per row), usually several per workgroup, so that the next item's h is there before this one is done.
+template <int H, bool HALF, bool MANY>
+__global__ __launch_bounds__(256, exchange_per_cu(H, HALF, MANY))
+void lstm_exchange_kernel(ExchangeArgs a) {
+  constexpr int UNITS = exchange_units(H, HALF, MANY);
+  constexpr int CT = UNITS / 16;
+  constexpr int W = H / UNITS;               // workgroups of a team
+  constexpr int RT = MANY ? 2 : 1;
+  constexpr int ROWS = 16 * RT;              // rows of a block
+  constexpr int KW = 32 / RT;                // k of a k step
+  constexpr int NT = 4 * CT / RT;            // tiles of 16 RT gate columns
+  constexpr int U = RT * CT;                 // units a lane updates
+  constexpr bool ROLES = H / 4 < KW;         // a quarter of H is half a k step: waves 0, 1 take x, waves 2, 3 take h
+  constexpr int XS = ROLES ? 1 : H / 4 / KW; // k steps per wave in the x half, and in the h half
+  constexpr int KS = ROLES ? 1 : 2 * XS;     // resident k steps
+  constexpr int NL = HALF ? XS : 2 * XS;     // 16-byte loads of a lane's share of a tile
+  constexpr int TILE = exchange_tile_bytes(H, HALF, ROWS);
+  constexpr int AR = 4 * RT * RT;            // accumulator registers of a tile
+  typedef float accum __attribute__((ext_vector_type(AR)));
+  typedef float sums __attribute__((ext_vector_type(4 * U)));   // the gates of a lane's units
+  __shared__ sums red[2][4][4][64];          // [parity][wave that takes them][wave that gives them][lane]
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int m = lane % ROWS;   // gate column of a weight fragment; batch row of everything else
+  const int kg = lane / ROWS;  // k group of a fragment; which of its wave's units a lane updates
+
+  int unit, pc;
+  if (a.per_xcd > 0) {
+    const int slot = blockIdx.x >> 3, n = slot / W;
+    unit = (int)(blockIdx.x & 7) * a.per_xcd + n;
+    pc = slot % W;
+    if (n >= a.per_xcd) return;
+  } else {
+    const int q = (int)(blockIdx.x & 7) * (int)(gridDim.x >> 3) + (int)(blockIdx.x >> 3);
+    unit = q / W;
+    pc = q % W;
+  }
+  if (unit >= a.units) return;
+  const int s = unit / a.L, l = unit % a.L;
+  const int d = a.dil[l];
+  const int T = a.T, B = a.B, nrb = a.nrb;
+
+  int xcc;
+  asm volatile("s_getreg_b32 %0, hwreg(HW_REG_XCC_ID)" : "=s"(xcc));
+  xcc = (xcc & 0xff) + 1;
+  if (tid == 0) __hip_atomic_store(a.place + unit * W + pc, xcc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+
+  // ---- resident weights: lane (m, kg) holds rows KW i + 8 kg .. +7 of column m of tile tt, for k step i.
+  // A column is a gate of a unit, ordered so that a lane gets the four gates of a unit next to each other in its
+  // accumulators (lane (m, kg) has rows 4 kg .. +3 of a 16-row result, and rows 8 q + 4 kg .. +3, q = 0 .. 3, of a
+  // 32-row one) and, with 32-row results, neighbouring units: two of the half tile its wave finishes, or four of a tile.
+  auto unit_of = [](int tt, int col) {
+    if (RT == 1) return 4 * tt + (col >> 2);
+    if (CT == 1) return 8 * tt + 4 * (col >> 4) + 2 * ((col >> 2) & 1) + ((col >> 3) & 1);
+    return 8 * tt + 4 * ((col >> 2) & 1) + (col >> 3);
+  };
+  v8h wt[KS][NT], wo[HALF ? 1 : KS][HALF ? 1 : NT];
+  constexpr float kLog2e = 1.4426950408889634f;
+  auto w_row = [&](int i) {      // first row of WU of resident k step i
+    if (ROLES) return 32 * wave;
+    return i < XS ? wave * (H / 4) + KW * i : H + wave * (H / 4) + KW * (i - XS);
+  };
+  const int my_unit = UNITS * pc + 4 * CT * wave + U * kg;   // the first of the units whose state this lane updates
+  float esc[HALF ? 1 : 4 * U], ebias[4 * U];                  // pre-activations: esc * sum + ebias, with -log2 e for the gates i, f, o
+  {
+    const size_t base = (size_t)l * 2 * H * 4 * H + (size_t)(m & 3) * H + UNITS * pc;
+    int uo[NT];
+#pragma unroll
+    for (int tt = 0; tt < NT; ++tt) uo[tt] = unit_of(tt, m);
+    if constexpr (HALF) {
+      const _Float16* wl = reinterpret_cast<const _Float16*>(a.WU) + base;
+#pragma unroll
+      for (int i = 0; i < KS; ++i) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+#pragma unroll
+          for (int tt = 0; tt < NT; ++tt) wt[i][tt][e] = wl[(size_t)(w_row(i) + 8 * kg + e) * 4 * H + uo[tt]];
+        if (i % (2 * RT) == 2 * RT - 1) asm volatile("" ::: "memory");   // 16-bit loads take a register each until they are packed
+      }
+    } else {
+      const float* wl = reinterpret_cast<const float*>(a.WU) + base;
+      float raw[KS][NT][8];
+#pragma unroll
+      for (int i = 0; i < KS; ++i)
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+#pragma unroll
+          for (int tt = 0; tt < NT; ++tt) raw[i][tt][e] = wl[(size_t)(w_row(i) + 8 * kg + e) * 4 * H + uo[tt]];
+      // the largest magnitude of each of the workgroup's columns, over the four waves
+      float* const cmaxs = reinterpret_cast<float*>(red);   // [4 waves][tile, column], then what undoes the scales
+#pragma unroll
+      for (int tt = 0; tt < NT; ++tt) {
+        float cmax = 0.0f;
+#pragma unroll
+        for (int i = 0; i < KS; ++i)
+#pragma unroll
+          for (int e = 0; e < 8; ++e) cmax = fmaxf(cmax, fabsf(raw[i][tt][e]));
+        cmax = fmaxf(cmax, __shfl_xor(cmax, 32));
+        if (RT == 1) cmax = fmaxf(cmax, __shfl_xor(cmax, 16));
+        cmaxs[wave * (64 * CT) + tt * ROWS + m] = cmax;
+      }
+      __syncthreads();
+#pragma unroll
+      for (int tt = 0; tt < NT; ++tt) {
+        float cmax = 0.0f;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) cmax = fmaxf(cmax, cmaxs[w * (64 * CT) + tt * ROWS + m]);
+        const int eb = min(max((int)((__float_as_uint(cmax) >> 23) & 0xff), 40), 230);
+        const float scale = __uint_as_float((unsigned)(127 + 14 + 127 - eb) << 23);   // column max -> [2^14, 2^15)
+        cmaxs[256 * CT + tt * ROWS + m] = __uint_as_float((unsigned)(eb - 14 - kXHandTop) << 23);
+#pragma unroll
+        for (int i = 0; i < KS; ++i)
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            const float w = raw[i][tt][e] * scale;
+            const _Float16 top = (_Float16)w;
+            wt[i][tt][e] = top;
+            wo[i][tt][e] = (_Float16)(w - (float)top);
+          }
+      }
+      __syncthreads();
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          // tile and column of gate g of unit my_unit + u
+          const int tt = RT == 1 || CT == 2 ? wave : wave >> 1;
+          const int col = RT == 1 ? 4 * kg + g : CT == 2 ? 8 * u + 4 * kg + g : 16 * (wave & 1) + 8 * u + 4 * kg + g;
+          esc[4 * u + g] = cmaxs[256 * CT + tt * ROWS + col] * (g == 3 ? 1.0f : -kLog2e);
+        }
+      __syncthreads();
+    }
+  }
+  // Where the weights take more than half of the register file, the matrix instructions read some of them from the
+  // accumulation registers, which nothing else can: left to itself the compiler keeps them there as spills and moves
+  // every one back in front of the instruction that uses it.
+  auto to_acc = [](v8h v) __attribute__((always_inline)) -> v8h {
+    const v4u u = __builtin_bit_cast(v4u, v);
+    unsigned a0, a1, a2, a3;
+    asm("v_accvgpr_write_b32 %0, %1" : "=a"(a0) : "v"(u[0]));
+    asm("v_accvgpr_write_b32 %0, %1" : "=a"(a1) : "v"(u[1]));
+    asm("v_accvgpr_write_b32 %0, %1" : "=a"(a2) : "v"(u[2]));
+    asm("v_accvgpr_write_b32 %0, %1" : "=a"(a3) : "v"(u[3]));
+    const v4u r = {a0, a1, a2, a3};
+    return __builtin_bit_cast(v8h, r);
+  };
+  if constexpr (H * CT * (HALF ? 1 : 2) >= 1024) {
+#pragma unroll
+    for (int i = 0; i < KS; ++i)
+#pragma unroll
+      for (int tt = 0; tt < NT; ++tt) {
+        if constexpr (HALF) {
+          if (i % 8 != 7 || !MANY) wt[i][tt] = to_acc(wt[i][tt]);
+        } else {
+          wo[i][tt] = to_acc(wo[i][tt]);
+          if (i % 4 < (MANY ? 3 : 2)) wt[i][tt] = to_acc(wt[i][tt]);
+        }
+      }
+  }
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+      ebias[4 * u + g] = a.bias ? a.bias[(size_t)l * 4 * H + g * H + my_unit + u] * (g == 3 ? 1.0f : -kLog2e) : 0.0f;
+
+  // ---- do the team, and the team above that reads from it, sit on this XCD?
+  bool alive = true;
+  auto look_at_places = [&](int u) -> bool {   // all of unit u's workgroups on this XCD
+    int v = xcc, n = 0;
+    for (int i0 = 0; i0 < W; i0 += 64) {
+      const int i = min(i0 + lane, W - 1);
+      int p = 0;
+      while (true) {
+        p = __hip_atomic_load(a.place + u * W + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (__builtin_amdgcn_ballot_w64(p == 0) == 0) break;
+        __builtin_amdgcn_s_sleep(2);
+        if (++n >= (1 << 20)) {
+          __hip_atomic_store(a.status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          alive = false;
+          return false;
+        }
+      }
+      if (p != xcc) v = 0;
+    }
+    return __builtin_amdgcn_ballot_w64(v != xcc) == 0;
+  };
+  const bool team_here = look_at_places(unit);
+  const bool has_upper = l + 1 < a.L;
+  const bool upper_here = has_upper && alive ? look_at_places(unit + 1) : true;
+  const bool own_by_ring = d == 1;
+  const bool uses_hand = has_upper || !own_by_ring;
+  // a dilated recurrence reads its own h from `hand` too
+  const bool hand_plain = upper_here && (own_by_ring || team_here);
+
+  const bool keep_c = d == 1 && s + a.slices >= nrb && !a.ragged;   // one row block: its c stays here
+  constexpr int ES = HALF ? 2 : 4;
+  constexpr int BLOCK = ROWS * H * ES;         // bytes of a row block of xs, hsss, csss
+  const int tiles_t = nrb * TILE;              // bytes of a time step of `hand`
+  const int rows_t = B * H * ES;               // bytes of a time step of xs, hsss, csss
+
+  // byte offsets of this lane within a tile
+  const unsigned put = HALF ? (my_unit / 8) * (ROWS * 16) + m * 16 + (my_unit % 8) * 2 : (my_unit / 4) * (ROWS * 16) + m * 16 + (my_unit % 4) * 4;
+  const int kq = ROLES ? 32 * (wave & 1) : wave * (H / 4);   // first k of this wave's share
+  const unsigned get = HALF ? (kq / 8 + kg) * (ROWS * 16) + m * 16 : (kq / 4 + 2 * kg) * (ROWS * 16) + m * 16;
+  const bool do_x = !ROLES || wave < 2, do_h = !ROLES || wave >= 2;
+
+  // All memory operations of the loop go through the buffer descriptors of this layer's arrays with a scalar offset that
+  // says where in the layer: no 64-bit addresses, and what must not happen (rows past the batch, nothing to store) is
+  // out of a descriptor's bounds instead of behind a branch.  Loads and stores complete in order on one
+  // counter; with the same number of operations on every path the compiler waits for exactly what it needs.
+  auto buffer = [](const void* p, size_t bytes) __attribute__((always_inline)) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (unsigned)bytes, 0x00020000);
+  };
+  const size_t hand_bytes = (size_t)T * tiles_t, out_bytes = (size_t)T * rows_t, ring_bytes = (size_t)nrb * kXRing * TILE;
+  const auto hand_l = buffer(a.hand + (l + 1) * hand_bytes, hand_bytes);
+  const auto below_l = buffer(a.hand + l * hand_bytes, hand_bytes);   // the layer below, or the input rows
+  const auto ratios = buffer(a.xratio, (size_t)T * nrb * ROWS * sizeof(float));
+  const auto own_l = own_by_ring ? buffer(a.ring + l * ring_bytes, ring_bytes) : hand_l;
+  const auto h_out = buffer(reinterpret_cast<unsigned char*>(a.hsss) + l * out_bytes, out_bytes);
+  const auto c_out = buffer(reinterpret_cast<unsigned char*>(a.csss) + l * out_bytes, out_bytes);
+  typedef decltype(buffer(nullptr, 0)) desc;
+
+  typedef v4u share[NL];
+  constexpr std::integral_constant<int, kAgentScope> fresh{};
+  constexpr std::integral_constant<int, 0> cached{};
+  // what k step i needs of a share; at: the tile's scalar offset, lane_at: this lane's offset in it (or out of bounds)
+  auto load_piece = [&](auto ic, desc rs, unsigned lane_at, int at, share& v, auto policy_c) __attribute__((always_inline)) {
+    constexpr int i = decltype(ic)::value, policy = decltype(policy_c)::value;
+    constexpr int step = KW / (HALF ? 8 : 4) * (ROWS * 16);   // bytes of a k step: 1024 or 2048
+    if constexpr (HALF) {
+      v[i] = __builtin_bit_cast(v4u, __builtin_amdgcn_raw_buffer_load_b128(rs, lane_at, at + i * step, policy));
+    } else {
+      v[2 * i] = __builtin_bit_cast(v4u, __builtin_amdgcn_raw_buffer_load_b128(rs, lane_at, at + i * step, policy));
+      v[2 * i + 1] = __builtin_bit_cast(v4u, __builtin_amdgcn_raw_buffer_load_b128(rs, lane_at + ROWS * 16, at + i * step, policy));
+    }
+  };
+  auto load_share = [&](desc rs, int at, share& v, auto policy_c) __attribute__((always_inline)) {
+    static_for<XS>([&](auto ic) __attribute__((always_inline)) { load_piece(ic, rs, get, at, v, policy_c); });
+  };
+  auto missing = [&](const share& v) __attribute__((always_inline)) -> bool {
+    if constexpr (HALF) {
+      v2us mx = {0, 0};
+#pragma unroll
+      for (int i = 0; i < NL; ++i)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          const unsigned w = v[i][c];
+          mx = __builtin_elementwise_max(mx, __builtin_bit_cast(v2us, w));
+        }
+      return __builtin_amdgcn_ballot_w64(mx[0] == 0xffff || mx[1] == 0xffff) != 0;
+    } else {
+      unsigned mx = 0;
+#pragma unroll
+      for (int i = 0; i < NL; ++i)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) mx = max(mx, v[i][c]);
+      return __builtin_amdgcn_ballot_w64(mx == ~0u) != 0;
+    }
+  };
+  auto wait_share = [&](desc rs, int at, share& v) __attribute__((always_inline)) {
+    if (!missing(v) || !alive) return;
+    int n = 0;
+    do {
+      if (++n >= a.spin_limit) {
+        __hip_atomic_store(a.status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        alive = false;
+        return;
+      }
+      if ((n & 1023) == 0 && __hip_atomic_load(a.status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) {
+        alive = false;
+        return;
+      }
+      asm volatile("" ::: "memory");   // the words change under us
+      load_share(rs, at, v, fresh);
+    } while (missing(v));
+  };
+
+  // The sums.  fp32 data, blocks of 16 rows: the products with a remainder have sums of their own (cross), added at the end;
+  // every addition rounds, and two thirds of them are of terms 2^-11 the size.  It also makes eight chains of the matrix
+  // instructions, which with four wait for each other (19.9 instead of 16 cycles each).
+  constexpr bool TWO = !HALF && !MANY;
+  accum acc[NT], cross[TWO ? NT : 1];
+  auto multiply = [](v8h w, v8h x, accum c) __attribute__((always_inline)) -> accum {
+    if constexpr (RT == 1) return __builtin_amdgcn_mfma_f32_16x16x32_f16(w, x, c, 0, 0, 0);
+    else return __builtin_amdgcn_mfma_f32_32x32x16_f16(w, x, c, 0, 0, 0);
+  };
+  // products of resident k step w with the fragment (top, rest); first: the sums start here
+  auto products = [&](auto wc, v8h top, v8h rest, auto first_c) __attribute__((always_inline)) {
+    constexpr int w = decltype(wc)::value;
+    constexpr bool first = decltype(first_c)::value;
+    accum zero;
+#pragma unroll
+    for (int r = 0; r < AR; ++r) zero[r] = 0.0f;
+    if constexpr (TWO) {
+#pragma unroll
+      for (int tt = 0; tt < NT; ++tt) {
+        acc[tt] = multiply(wt[w][tt], top, first ? zero : acc[tt]);
+        cross[tt] = multiply(wt[w][tt], rest, first ? zero : cross[tt]);
+      }
+#pragma unroll
+      for (int tt = 0; tt < NT; ++tt) cross[tt] = multiply(wo[w][tt], top, cross[tt]);
+    } else {
+#pragma unroll
+      for (int tt = 0; tt < NT; ++tt) acc[tt] = multiply(wt[w][tt], top, first ? zero : acc[tt]);
+      if constexpr (!HALF) {
+#pragma unroll
+        for (int tt = 0; tt < NT; ++tt) acc[tt] = multiply(wt[w][tt], rest, acc[tt]);
+#pragma unroll
+        for (int tt = 0; tt < NT; ++tt) acc[tt] = multiply(wo[w][tt], top, acc[tt]);
+      }
+    }
+  };
+  // all of a share of an exchange tile; base: the first resident k step.  each(i): called when v's part for k step i has
+  // been used, for memory operations that are due then
+  auto share_products = [&](share& v, auto base_c, auto first_c, auto each) __attribute__((always_inline)) {
+    constexpr int base = decltype(base_c)::value;
+    constexpr bool first = decltype(first_c)::value;
+    static_for<XS>([&](auto ic) __attribute__((always_inline)) {
+      constexpr int i = decltype(ic)::value;
+      constexpr std::integral_constant<bool, first && i == 0> start{};
+      if constexpr (HALF) {
+        products(std::integral_constant<int, base + i>{}, __builtin_bit_cast(v8h, v[i]), v8h{}, start);
+        each(ic);
+        __builtin_amdgcn_sched_barrier(0x6);   // vector and scalar instructions may pass, the loads stay between the products
+      } else {
+        const v4u p = v[2 * i], q = v[2 * i + 1];
+        v4u top, rest;
+        top[0] = __builtin_amdgcn_perm(p[1], p[0], 0x05040100);
+        top[1] = __builtin_amdgcn_perm(p[3], p[2], 0x05040100);
+        top[2] = __builtin_amdgcn_perm(q[1], q[0], 0x05040100);
+        top[3] = __builtin_amdgcn_perm(q[3], q[2], 0x05040100);
+        rest[0] = __builtin_amdgcn_perm(p[1], p[0], 0x07060302);
+        rest[1] = __builtin_amdgcn_perm(p[3], p[2], 0x07060302);
+        rest[2] = __builtin_amdgcn_perm(q[1], q[0], 0x07060302);
+        rest[3] = __builtin_amdgcn_perm(q[3], q[2], 0x07060302);
+        each(ic);
+        __builtin_amdgcn_sched_barrier(0x6);   // vector and scalar instructions may pass, the loads stay between the products
+        products(std::integral_constant<int, base + i>{}, __builtin_bit_cast(v8h, top), __builtin_bit_cast(v8h, rest), start);
+      }
+    });
+  };
+
+  // U words (fp16 data: halves) to a tile of the exchange buffers, as a plain or a write-through store: both are issued,
+  // one of them out of bounds (on == false: both)
+  constexpr int WORD_BYTES = U * (HALF ? 2 : 4);
+  auto store_bytes = [](auto policy_c, auto w, desc rs, unsigned off, int at) __attribute__((always_inline)) {
+    constexpr int policy = decltype(policy_c)::value;
+    if constexpr (sizeof(w) == 2) __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(unsigned short, w), rs, off, at, policy);
+    else if constexpr (sizeof(w) == 4) __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, w), rs, off, at, policy);
+    else if constexpr (sizeof(w) == 8) __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(v2u, w), rs, off, at, policy);
+    else __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4u, w), rs, off, at, policy);
+  };
+  struct words {
+    typename std::conditional<HALF, unsigned short, unsigned>::type v[U];
+  };
+  static_assert(sizeof(words) == WORD_BYTES, "a lane's words are stored at once");
+  words all_ones;
+#pragma unroll
+  for (int u = 0; u < U; ++u) all_ones.v[u] = (decltype(all_ones.v[0] + 0))~0u;
+  auto put_words = [&](desc rs, int at, words w, bool plain, bool on) __attribute__((always_inline)) {
+    store_bytes(cached, w, rs, on && plain ? put : ~0u, at);
+    store_bytes(fresh, w, rs, on && !plain ? put : ~0u, at);
+  };
+  // the lane's values of a row of hsss or csss
+  struct values {
+    typename std::conditional<HALF, _Float16, float>::type v[U];
+  };
+  auto put_row = [&](desc rs, unsigned off, int at, const float (&x)[U]) __attribute__((always_inline)) {
+    values w;
+#pragma unroll
+    for (int u = 0; u < U; ++u) w.v[u] = x[u];
+    store_bytes(cached, w, rs, off, at);
+  };
+  // h and c of an item, and the words of later steps it sets back: stored when the next item has asked for its h, so
+  // that nothing the chain waits for is behind them
+  struct Later {
+    int row = 0, hand = 0, ring = 0;   // scalar offsets
+    unsigned row_off = ~0u;
+    float hv[U] = {}, cv[U] = {};
+    bool on_hand = false, on_ring = false;
+  } later;
+  auto store_later = [&]() __attribute__((always_inline)) {
+    put_row(h_out, later.row_off, later.row, later.hv);
+    put_row(c_out, later.row_off, later.row, later.cv);
+    put_words(hand_l, later.hand, all_ones, hand_plain, later.on_hand);
+    put_words(own_l, later.ring, all_ones, team_here, later.on_ring);
+  };
+
+  // ---- items.  An item's place: time step, row block, and the byte offsets of its time step
+  struct Item {
+    int t, rb;
+    int tile, row;   // of time step t: in a layer of `hand`, in a layer of xs / hsss / csss
+  };
+  auto after = [&](Item it) __attribute__((always_inline)) -> Item {   // it.t == T: no further item
+    do {
+      it.rb += a.slices;
+      if (!MANY || it.rb >= nrb) {
+        it.rb = s;
+        ++it.t;
+        it.tile += tiles_t;
+        it.row += rows_t;
+      }
+    } while (a.ragged && it.t < T && it.t >= (int)a.steps_of[it.rb]);
+    return it;
+  };
+  auto h_at = [&](const Item& it) __attribute__((always_inline)) -> int {
+    return own_by_ring ? (it.rb * kXRing + ((it.t - 1) & (kXRing - 1))) * TILE : it.tile - d * tiles_t + it.rb * TILE;
+  };
+  auto row_off_of = [&](int rb) { return rb * ROWS + m < B ? (unsigned)((m * H + my_unit) * ES) : ~0u; };
+  float cp[U] = {};   // c of d steps before
+  float xr = 1.0f;
+  share v;
+  auto ask_c = [&](unsigned off, int at) __attribute__((always_inline)) {
+    values v;
+    if constexpr (sizeof(values) == 2) v = __builtin_bit_cast(values, __builtin_amdgcn_raw_buffer_load_b16(c_out, off, at, 0));
+    else if constexpr (sizeof(values) == 4) v = __builtin_bit_cast(values, __builtin_amdgcn_raw_buffer_load_b32(c_out, off, at, 0));
+    else if constexpr (sizeof(values) == 8) v = __builtin_bit_cast(values, __builtin_amdgcn_raw_buffer_load_b64(c_out, off, at, 0));
+    else v = __builtin_bit_cast(values, __builtin_amdgcn_raw_buffer_load_b128(c_out, off, at, 0));
+#pragma unroll
+    for (int u = 0; u < U; ++u) cp[u] = (float)v.v[u];
+  };
+
+  bool small_reported = false;
+  // four neighbouring units of a row that are all small and not all zero: those of lanes m, m + ROWS, ...
+  auto look_for_small = [&](const float (&h)[U]) __attribute__((always_inline)) {
+    if constexpr (!HALF) {
+      unsigned largest = 0;
+#pragma unroll
+      for (int u = 0; u < U; ++u) largest = max(largest, __float_as_uint(h[u] * (float)(1 << kXHandTop)) & 0x7fffffffu);
+      const u64 sm = __builtin_amdgcn_ballot_w64(largest < kXSmallBits);
+      if (__builtin_expect(sm != 0 && !small_reported && alive, 0)) {
+        u64 all = sm, any = __builtin_amdgcn_ballot_w64(largest != 0);
+        if (U < 4) {
+          all &= all >> 32;
+          any |= any >> 32;
+        }
+        if (U < 2) {
+          all &= all >> 16;
+          any |= any >> 16;
+        }
+        if (U < 4) all &= U == 1 ? 0xffffull : 0xffffffffull;
+        if ((all & any) != 0) {
+          small_reported = true;
+          if (lane == 0) __hip_atomic_store(a.status + 1, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+      }
+    }
+  };
+  // this wave's sums, to LDS; all four waves' sums of the units it updates, from LDS
+  auto give_sums = [&](int parity) __attribute__((always_inline)) {
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      constexpr int per = 4 * U;   // of a tile's registers: all, or (CT == 1 and 32 rows) the half of a wave
+      sums v;
+#pragma unroll
+      for (int r = 0; r < per; ++r) v[r] = TWO ? acc[w % NT][r % AR] + cross[w % (TWO ? NT : 1)][r % AR] : per == AR ? acc[w % NT][r] : acc[w / 2 % NT][(w % 2) * per % AR + r];
+      red[parity][w][wave][lane] = v;
+    }
+  };
+  auto take_sums = [&](int parity) __attribute__((always_inline)) -> sums {
+    sums pre = red[parity][wave][0][lane] + red[parity][wave][1][lane];
+    pre += red[parity][wave][2][lane] + red[parity][wave][3][lane];
+    return pre;
+  };
+  // the state update of this lane's units and their words of the exchange buffers
+  auto update = [&](sums pre, const float (&c_prev)[U], float (&c)[U], float (&h)[U]) __attribute__((always_inline)) -> words {
+    auto gate = [](float e) { return __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(e)); };
+    words w;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      float p[4];
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        if constexpr (HALF) p[g] = pre[4 * u + g] * (g == 3 ? 1.0f : -kLog2e) + ebias[4 * u + g];
+        else p[g] = pre[4 * u + g] * esc[4 * u + g] + ebias[4 * u + g];
+      }
+      c[u] = gate(p[1]) * c_prev[u] + gate(p[0]) * tanh_f(p[3]);
+      h[u] = gate(p[2]) * tanh_f(c[u]);
+      unsigned word;
+      if constexpr (HALF) {
+        c[u] = (float)(_Float16)c[u];
+        word = __builtin_bit_cast(unsigned short, (_Float16)h[u]);
+        if (word == 0xffffu) word = 0x7e00u;   // a NaN, but not the one that stands for "not there yet"
+      } else {
+        const float v = h[u] * (float)(1 << kXHandTop);
+        const _Float16 top = (_Float16)v;
+        const v2h pair = {top, (_Float16)(v - (float)top)};
+        word = __builtin_bit_cast(unsigned, pair);
+        if (word == ~0u) word = 0x7e007e00u;
+      }
+      w.v[u] = word;
+    }
+    return w;
+  };
+  auto ring_at = [&](int rb, int t) { return (rb * kXRing + (t & (kXRing - 1))) * TILE; };
+  auto later_of = [&](const Item& it, const float (&h)[U], const float (&c)[U]) __attribute__((always_inline)) {
+    later.row = it.row + it.rb * BLOCK;
+    later.row_off = alive ? row_off_of(it.rb) : ~0u;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      later.hv[u] = h[u];
+      later.cv[u] = c[u];
+    }
+    later.hand = it.tile + it.rb * TILE + 2 * tiles_t;
+    later.on_hand = alive && uses_hand && it.t + 2 < T;
+    later.ring = ring_at(it.rb, it.t - 2);
+    later.on_ring = alive && own_by_ring && it.t >= 2;
+  };
+  // x of an item: through the caches, because the team's other workgroups fetch the same tile into this XCD's L2.  (A
+  // line that was fetched too early holds all-ones words still; wait_share asks for it again past the caches.)
+  auto x_at = [&](const Item& it) { return it.tile + it.rb * TILE; };
+  auto ask_ratio = [&](const Item& it) __attribute__((always_inline)) {
+    xr = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(ratios, m * 4, (it.t * nrb + it.rb) * (ROWS * 4), 0));
+  };
+  auto scale_input = [&](float ratio) __attribute__((always_inline)) {
+#pragma unroll
+    for (int tt = 0; tt < NT; ++tt)
+#pragma unroll
+      for (int r = 0; r < AR; ++r) {
+        acc[tt][r] *= ratio;
+        if constexpr (TWO) cross[tt][r] *= ratio;
+      }
+  };
+  constexpr std::integral_constant<int, 0> x_steps{};
+  constexpr std::integral_constant<int, ROLES ? 0 : XS> h_steps{};
+
+  // The loop.  FIRST: the layer reads the input rows.  One set of registers takes turns: while the products of an item's h
+  // are formed, the pieces of the next item's x are asked for one by one into the registers that have been used (a burst
+  // of loads would hold up the wave: 64 bytes a cycle is what a compute unit gets), and while those of x are formed
+  // (which is after this item's h has been published) the pieces of the next h.
+  auto walk = [&](auto first_c) __attribute__((always_inline)) {
+    constexpr bool FIRST = decltype(first_c)::value;
+    constexpr unsigned kOut = 0x80000000u;   // a lane offset beyond every descriptor: the load returns zeros
+    // products of the x in v; the pieces of h (and c) of the same item take its place.  Where there is nothing (no step
+    // that far back, or the half of the contraction another wave has) v is zeros and the products are those of zeros.
+    auto take_x = [&](const Item& it) __attribute__((always_inline)) {
+      const bool has_prev = it.t >= d;
+      if constexpr (!FIRST) wait_share(below_l, x_at(it), v);
+      if (!keep_c) ask_c(has_prev ? row_off_of(it.rb) : ~0u, has_prev ? it.row - d * rows_t + it.rb * BLOCK : 0);
+      const unsigned lane_at = has_prev && do_h ? get : kOut;
+      const int at = has_prev ? h_at(it) : 0;
+      const float ratio = xr;
+      share_products(v, x_steps, std::true_type{}, [&](auto ic) __attribute__((always_inline)) {
+        load_piece(ic, own_l, lane_at, at, v, fresh);
+      });
+      if constexpr (FIRST && !HALF) scale_input(ratio);
+    };
+    int parity = 0;
+    bool follows = false;   // the item before is what this one takes its c from
+    Item it{0, s, 0, 0};
+    if (a.ragged && a.steps_of[s] == 0) it = after(it);
+    if (it.t >= T) return;
+    static_for<XS>([&](auto ic) __attribute__((always_inline)) { load_piece(ic, below_l, do_x ? get : kOut, x_at(it), v, cached); });
+    if constexpr (FIRST && !HALF) ask_ratio(it);
+    take_x(it);
+    while (true) {   // (a wave that has given up walks on without waiting, to every barrier the others wait at)
+      const bool has_prev = it.t >= d;
+      const Item next = after(it);
+      const bool more = next.t < T;
+      const int next_x = x_at(more ? next : it);   // there is always something to ask for: the same operations on every path
+      wait_share(own_l, has_prev ? h_at(it) : 0, v);
+      share_products(v, h_steps, std::false_type{}, [&](auto ic) __attribute__((always_inline)) {
+        load_piece(ic, below_l, do_x ? get : kOut, next_x, v, cached);
+      });
+      if constexpr (FIRST && !HALF) ask_ratio(more ? next : it);
+      float c_prev[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) c_prev[u] = !has_prev ? 0.0f : keep_c || follows ? later.cv[u] : cp[u];
+      follows = next.rb == it.rb && next.t == it.t + d;
+      give_sums(parity);
+      // what the item before stored is complete before anything of this one is published: only what was asked for since
+      // may be outstanding
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(NL + (FIRST && !HALF ? 1 : 0)) : "memory");
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+      const sums pre = take_sums(parity);
+      parity ^= 1;
+      float c[U], h[U];
+      const words word = update(pre, c_prev, c, h);
+      put_words(own_l, ring_at(it.rb, it.t), word, team_here, alive && own_by_ring);
+      put_words(hand_l, x_at(it), word, hand_plain, alive && uses_hand);
+      asm volatile("" ::: "memory");
+      later_of(it, h, c);
+      look_for_small(h);
+      if (more) take_x(next);
+      asm volatile("" ::: "memory");
+      store_later();
+      asm volatile("" ::: "memory");
+      if (!more) break;
+      it = next;
+    }
+  };
+  if (l == 0) walk(std::true_type{});
+  else walk(std::false_type{});
+}
+
+// In front of the kernel above: status block, places, the ring and the first two steps of `hand` (blockIdx.y < layers), and
+// the input rows as tiles (blockIdx.y == layers; one wave per row, rows past the batch are zeros).  fp32 rows are cut
+// under a power-of-two scale of their own.
+template <bool HALF>
+__global__ __launch_bounds__(256) void lstm_exchange_prepare_kernel(int* status, int first_word, int* place, int nplaces, v4u* ring,
+                                                                    size_t ring_per_layer, v4u* hand, size_t hand_per_layer,
+                                                                    size_t hand_first, const void* xs, float* xratio, int layers,
+                                                                    int T, int B, int nrb, int block, int H) {
+  const size_t at = (size_t)blockIdx.x * 256 + threadIdx.x, step = (size_t)gridDim.x * 256;
+  const int l = blockIdx.y;
+  if (l < layers) {
+    const v4u ones = {~0u, ~0u, ~0u, ~0u};
+    for (size_t i = at; i < ring_per_layer; i += step) ring[l * ring_per_layer + i] = ones;
+    for (size_t i = at; i < hand_first; i += step) hand[(l + 1) * hand_per_layer + i] = ones;
+    if (l == 0) {
+      for (size_t i = at; i < (size_t)nplaces; i += step) place[i] = 0;
+      if (at < kStatusBytes / sizeof(int) && (int)at >= first_word) status[at] = 0;
+    }
+    return;
+  }
+  const int lane = threadIdx.x & 63;
+  const int per_step = nrb * block, rows = T * per_step;   // block: rows of a row block
+  for (int r = blockIdx.x * 4 + (threadIdx.x >> 6); r < rows; r += gridDim.x * 4) {
+    const int t = r / per_step, b = r - t * per_step;
+    unsigned char* dst = reinterpret_cast<unsigned char*>(hand) + (size_t)(r / block) * exchange_tile_bytes(H, HALF, block) + (r % block) * 16;
+    const size_t src = ((size_t)t * B + b) * H;
+    if constexpr (HALF) {
+      for (int k = 8 * lane; k < H; k += 512) {
+        v4u v = {0, 0, 0, 0};
+        if (b < B) v = *reinterpret_cast<const v4u*>(reinterpret_cast<const _Float16*>(xs) + src + k);
+        *reinterpret_cast<v4u*>(dst + (k >> 3) * (block * 16)) = v;
+      }
+    } else {
+      v4f x[4];   // H <= 1024
+      float mx = 0.0f;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int k = 4 * lane + 256 * i;
+        x[i] = v4f{0.f, 0.f, 0.f, 0.f};
+        if (k < H && b < B) x[i] = *reinterpret_cast<const v4f*>(reinterpret_cast<const float*>(xs) + src + k);
+        mx = fmaxf(mx, fmaxf(fmaxf(fabsf(x[i][0]), fabsf(x[i][1])), fmaxf(fabsf(x[i][2]), fabsf(x[i][3]))));
+      }
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
+      const int eb = min(max((int)((__float_as_uint(mx) >> 23) & 0xff), 15), 254);
+      const float scale = __uint_as_float((unsigned)(127 + 14 + 127 - eb) << 23);   // the row's largest -> [2^14, 2^15)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int k = 4 * lane + 256 * i;
+        v4u w;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float v = x[i][e] * scale;
+          const _Float16 top = (_Float16)v;
+          const v2h pair = {top, (_Float16)(v - (float)top)};
+          w[e] = __builtin_bit_cast(unsigned, pair);
+        }
+        if (k < H) *reinterpret_cast<v4u*>(dst + (k >> 2) * (block * 16)) = w;
+      }
+      if (lane == 0) xratio[r] = __uint_as_float((unsigned)eb << 23);   // the products carry 2^(141 - eb), h's 2^14
+    }
+  }
+}
+
+namespace {
+
+struct ExchangeFlavour {
+  const void* one;    // row blocks of 16 rows, one per workgroup
+  const void* many;   // row blocks of 32 rows
+};
+
+template <int H, bool HALF>
+ExchangeFlavour exchange_flavour() {
+  return {(const void*)lstm_exchange_kernel<H, HALF, false>, (const void*)lstm_exchange_kernel<H, HALF, true>};
+}
+
+// The kernel for a hidden size and element type, or nulls.
+ExchangeFlavour exchange_flavour_of(int H, bool half) {
+  if (half) {
+    switch (H) {
+      case 256: return exchange_flavour<256, true>();
+      case 512: return exchange_flavour<512, true>();
+      case 1024: return exchange_flavour<1024, true>();
+      default: return {nullptr, nullptr};
+    }
+  }
+  switch (H) {
+    case 64: return exchange_flavour<64, false>();
+    case 128: return exchange_flavour<128, false>();
+    case 256: return exchange_flavour<256, false>();
+    case 512: return exchange_flavour<512, false>();
+    default: return {nullptr, nullptr};
+  }
+}
+
+// Workgroups the device holds at once (0 on any error).
+int exchange_slots(const void* fn) {
+  constexpr int kKept = 16, kDev = 16;
+  static std::atomic<const void*> fns[kKept];
+  static std::atomic<int> kept[kKept][kDev];
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kDev) return 0;
+  int at = 0;
+  for (; at < kKept; ++at) {
+    const void* f = fns[at].load(std::memory_order_acquire);
+    if (f == fn) break;
+    if (!f) {
+      const void* none = nullptr;
+      if (fns[at].compare_exchange_strong(none, fn) || none == fn) break;
+    }
+  }
+  if (at < kKept)
+    if (const int v = kept[at][dev].load(std::memory_order_acquire)) return v;
+  const DeviceProps* dp = nullptr;
+  int per_cu = 0;
+  if (device_props(&dp) != FTK_OK || hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, 256, 0) != hipSuccess) return 0;
+  const int slots = per_cu * dp->cus;
+  if (at < kKept) kept[at][dev].store(slots, std::memory_order_release);
+  return slots;
+}
+
+// How a stack of L layers (as many as one launch holds) is laid out on the chip.
+struct ExchangePlan {
+  int layers = 0;    // layers per launch, 0: the device cannot hold one
+  int slices = 0;    // row slices of a layer
+  int per_xcd = 0;   // teams per XCD, 0: workgroups in order
+};
+
+ExchangePlan exchange_plan(int L, int W, int nrb, int slots) {   // W: workgroups of a team
+  ExchangePlan p;
+  const int here = std::min(slots, kXPlaces);
+  const int room = here / 8 / W;   // teams an XCD holds
+  const int teams = room ? 8 * room : here / W;   // (a team may be larger than an XCD)
+  if (teams == 0) return p;
+  p.layers = std::min({L, teams, kXLayers});
+  p.slices = std::max(1, std::min(nrb, teams / p.layers));
+  const int blocks = (nrb + p.slices - 1) / p.slices;   // the fewest slices that walk no more blocks each
+  p.slices = (nrb + blocks - 1) / blocks;
+  if (room) p.per_xcd = (p.layers * p.slices + 7) / 8;
+  return p;
+}
+
+constexpr size_t align256(size_t v) { return (v + 255) / 256 * 256; }
+constexpr size_t exchange_xratio_at = align256(kStatusBytes + kXPlaces * sizeof(int));
+
+}  // namespace
+
+// Whether lstm_exchange runs this hidden size and type at all.
+bool exchange_takes(int H, bool half) { return exchange_flavour_of(H, half).one != nullptr; }
+
+// Bytes of workspace for L layers: [status block][places][xratio][ring][hand], with either kind of row block.
+size_t exchange_workspace_bytes(int L, int T, int B, int H, bool half) {
+  const size_t rows = (size_t)(B + 31) / 32 * 32;   // never less than with blocks of 16
+  return exchange_xratio_at + align256((size_t)T * rows * sizeof(float)) +
+         rows * H * (half ? 2 : 4) * ((size_t)L * kXRing + (size_t)(L + 1) * T);
+}
+
+// Whether a layer of a buffer stays below what a buffer descriptor and its offsets reach.
+bool exchange_fits(int T, int B, int H, bool half) { return (size_t)T * ((size_t)(B + 31) / 32 * 32) * H * (half ? 2 : 4) < (1ull << 31) - (1 << 20); }
+
+// Whether the whole batch of every layer fits the chip with one block of 16 rows per workgroup.
+bool exchange_one_block(int L, int B, int H, bool half) {
+  const ExchangeFlavour f = exchange_flavour_of(H, half);
+  if (!f.one) return false;
+  const int nrb = (B + 15) / 16;
+  const ExchangePlan p = exchange_plan(L, H / exchange_units(H, half, false), nrb, exchange_slots(f.one));
+  return p.layers == L && p.slices == nrb;
+}
+
+// Runs the stack; *handled is false when the device cannot hold a layer.  Deeper stacks than a launch holds run as
+// consecutive launches, each reading the hidden sequence of the layer below it like the first reads xs.
+int run_exchange(bool half, const void* xs, const void* WU, const float* bias, const int* dil, const int* active, void* hsss,
+                 void* csss, int L, int T, int B, int H, void* ws, size_t ws_bytes, hipStream_t s, bool* handled, int spin_limit) {
+  *handled = false;
+  const ExchangeFlavour f = exchange_flavour_of(H, half);
+  if (!f.one) return FTK_OK;
+  const bool many = !exchange_one_block(L, B, H, half);
+  const int slots = exchange_slots(many ? f.many : f.one), block = many ? 32 : 16, nrb = (B + block - 1) / block;
+  const int W = H / exchange_units(H, half, many);
+  const int most = exchange_plan(L, W, nrb, slots).layers;
+  if (most == 0) return FTK_OK;
+  const size_t esize = half ? 2 : 4, slab = (size_t)T * B * H, wlayer = (size_t)8 * H * H, tile = exchange_tile_bytes(H, half, block);
+  const size_t need = exchange_workspace_bytes(std::min(L, most), T, B, H, half);
+  if (!ws || ws_bytes < need) return fail(FTK_ERR_WORKSPACE, "stacked LSTM needs a %zu-byte workspace, got %zu", need, ws_bytes);
+  for (int l0 = 0; l0 < L; l0 += most) {
+    const int lc = std::min(most, L - l0);
+    const ExchangePlan p = exchange_plan(lc, W, nrb, slots);
+    ExchangeArgs a;
+    const void* x = l0 == 0 ? xs : (const char*)hsss + (size_t)(l0 - 1) * slab * esize;
+    a.WU = (const char*)WU + (size_t)l0 * wlayer * esize;
+    a.bias = bias ? bias + (size_t)l0 * 4 * H : nullptr;
+    a.hsss = (char*)hsss + (size_t)l0 * slab * esize;
+    a.csss = (char*)csss + (size_t)l0 * slab * esize;
+    a.status = (int*)ws;
+    a.place = (int*)((char*)ws + kStatusBytes);
+    float* xratio = (float*)((char*)ws + exchange_xratio_at);
+    a.xratio = xratio;
+    a.ring = (unsigned char*)ws + exchange_xratio_at + align256((size_t)T * nrb * block * sizeof(float));
+    a.hand = a.ring + (size_t)lc * nrb * kXRing * tile;
+    a.L = lc; a.T = T; a.B = B; a.nrb = nrb;
+    a.slices = p.slices;
+    a.units = lc * p.slices;
+    a.per_xcd = p.per_xcd;
+    a.spin_limit = spin_limit > 0 ? spin_limit : 1 << 22;
+    a.ragged = active && nrb <= kXBlocks ? 1 : 0;
+    for (int l = 0; l < kXLayers; ++l) a.dil[l] = l < lc && dil ? dil[l0 + l] : 1;
+    for (int rb = 0; rb < kXBlocks; ++rb) {
+      int steps = 0;
+      if (a.ragged)
+        while (steps < T && active[steps] > block * rb) ++steps;
+      a.steps_of[rb] = (unsigned short)steps;
+    }
+    const int groups = a.units * W;
+    const unsigned grid = p.per_xcd ? 8u * p.per_xcd * W : (unsigned)((groups + 7) / 8 * 8);
+    const size_t ring_per_layer = (size_t)nrb * kXRing * tile / 16, hand_per_layer = (size_t)T * nrb * tile / 16;
+    const size_t hand_first = (size_t)std::min(T, 2) * nrb * tile / 16;
+    const size_t px = std::max({(ring_per_layer + 1023) / 1024, (hand_first + 1023) / 1024, ((size_t)T * nrb * block + 3) / 4});
+    const dim3 pgrid((unsigned)std::min<size_t>(px, 1024), lc + 1);
+    if (half)
+      hipLaunchKernelGGL(lstm_exchange_prepare_kernel<true>, pgrid, dim3(256), 0, s, a.status, l0 > 0 ? 2 : 0, a.place, groups,
+                         (v4u*)a.ring, ring_per_layer, (v4u*)a.hand, hand_per_layer, hand_first, x, xratio, lc, T, B, nrb, block, H);
+    else
+      hipLaunchKernelGGL(lstm_exchange_prepare_kernel<false>, pgrid, dim3(256), 0, s, a.status, l0 > 0 ? 2 : 0, a.place, groups,
+                         (v4u*)a.ring, ring_per_layer, (v4u*)a.hand, hand_per_layer, hand_first, x, xratio, lc, T, B, nrb, block, H);
+    int rc = check_launch("lstm_exchange_prepare_kernel");
+    if (rc) return rc;
+    void* kargs[] = {&a};
+    rc = launch_resident(many ? f.many : f.one, dim3(grid), dim3(256), kargs, 0, s);
+    if (rc) return rc;
+  }
+  *handled = true;
+  return FTK_OK;
+}
+
+}  // namespace ftk

@@ -40,7 +40,7 @@
 // (comment above the loop): loads and stores share a counter, so a load result
 // is only known once nothing at all is outstanding.  Two barriers per item.
 //
-// All workgroups must be co-resident: the host launches cooperatively with at
+// All workgroups must be co-resident: the host launches (launch_resident) at
 // most one workgroup per compute unit (each uses the whole register file of
 // its CU).  Every wait is bounded by spin_limit polls; on expiry the kernel
 // records an error word and every workgroup drains.
@@ -62,6 +62,13 @@ int run_wavefront_f16(const void* xs, const void* WU, const float* bias, const i
 size_t split_stack_workspace_bytes(int L, int T, int B, int H);
 int run_wavefront_split(const float* xs, const float* WU, const float* bias, const int* dil, const int* active, float* hsss,
                         float* csss, int L, int T, int B, int H, void* ws, hipStream_t s);
+// lstm_exchange.hip: the kernel for stacks that are bound by their chain of dependent steps
+bool exchange_takes(int H, bool half);
+bool exchange_fits(int T, int B, int H, bool half);
+bool exchange_one_block(int L, int B, int H, bool half);
+size_t exchange_workspace_bytes(int L, int T, int B, int H, bool half);
+int run_exchange(bool half, const void* xs, const void* WU, const float* bias, const int* dil, const int* active, void* hsss,
+                 void* csss, int L, int T, int B, int H, void* ws, size_t ws_bytes, hipStream_t s, bool* handled, int spin_limit);
 
 constexpr int PH = 256;            // hidden size this kernel is specialised for
 constexpr int PK = 2 * PH;         // K of the gate GEMM
@@ -1501,20 +1508,6 @@ static int products_mode() {
   return g_products;
 }
 
-// Profiling hook: FTK_LSTM_PLAIN_LAUNCH=1 launches without the cooperative
-// co-residency check (counter collection tools that cannot follow cooperative
-// launches).  The grid never exceeds one workgroup per compute unit, so on an
-// otherwise idle device the workgroups are co-resident all the same; if they
-// are not, the bounded waits end the launch with the error word set.
-static bool plain_launch() {
-  static int v = -1;
-  if (v < 0) {
-    const char* e = getenv("FTK_LSTM_PLAIN_LAUNCH");
-    v = (e && atoi(e) != 0) ? 1 : 0;
-  }
-  return v == 1;
-}
-
 // Tuning hook: FTK_LSTM_TRACE=<logical workgroup> records that workgroup's per-item timeline.
 static int trace_workgroup() {
   static int v = -2;
@@ -1682,16 +1675,8 @@ static int run_persistent(int mode, const void* xs, const void* WU, const float*
   }
 
   void* kargs[] = {&a};
-  if (plain_launch()) {
-    if (mode == kHalfData) hipLaunchKernelGGL(lstm_persistent_kernel<kHalfData>, dim3(grid), dim3(256), lds, s, a);
-    else if (mode == kHalfData256) hipLaunchKernelGGL(lstm_persistent_kernel<kHalfData256>, dim3(grid), dim3(256), lds, s, a);
-    else if (split) hipLaunchKernelGGL(lstm_persistent_kernel<kProductsSplit>, dim3(grid), dim3(256), lds, s, a);
-    else hipLaunchKernelGGL(lstm_persistent_kernel<kProductsF32>, dim3(grid), dim3(256), lds, s, a);
-    rc = check_launch("lstm_persistent_kernel");
-    if (rc) return rc;
-  } else {
-    FTK_HIP(hipLaunchCooperativeKernel(fn, dim3(grid), dim3(256), kargs, (unsigned)lds, s));
-  }
+  rc = launch_resident(fn, dim3(grid), dim3(256), kargs, lds, s);
+  if (rc) return rc;
   *handled = true;
   return FTK_OK;
 }
@@ -1741,6 +1726,29 @@ static int check_stack_args(const char* who, const float* xs, const float* WU, f
   return FTK_OK;
 }
 
+// Which stacks go to the exchange kernel (lstm_exchange.hip): all it takes whose batch it spreads over the chip with one row
+// block per workgroup, because then the chain of dependent steps is the time (L 1 .. 8, T 32, B 64, H 256, fp32: 67 ..
+// 124 us against 198 .. 265; H 512, 8 layers, T 100: 0.92 ms against 7.3).  With more rows than that it walks several blocks per
+// workgroup, and there
+//   H = 256 has the paired schedule of the persistent kernel, which feeds the matrix pipe better: ahead from 16 layers x
+//     256 rows on (L 16 B 192: 536 against 575 us, L 16 B 256: 660 against 585, L 32 B 192: 998 against 937; fp16 data: L 16
+//     B 192 370 / 382, L 32 B 192 769 / 597), and for dilated stacks, whose chains are short (L 6 T 128 B 256: 1.22 / 0.83 ms);
+//   H = 1024 (fp16 data) holds four layers on the chip at a time, and deep stacks of large batches are better streamed
+//     (L 8 B 256 T 32: 1.87 against 2.31 ms, L 32 B 256 T 64: 14.7 against 12.3).
+// FTK_LSTM_EXCHANGE=1 / =0 in the environment forces the one or the other.
+static bool exchange_chosen(int L, int T, int B, int H, const int* dil, bool half) {
+  if (!exchange_takes(H, half) || !exchange_fits(T, B, H, half)) return false;
+  if (const char* e = getenv("FTK_LSTM_EXCHANGE")) return e[0] == '1';
+  if (exchange_one_block(L, B, H, half)) return true;
+  if (H == PH) {
+    for (int l = 0; dil && l < L; ++l)
+      if (dil[l] != 1) return false;
+    return L * ((B + 31) / 32) < 112;
+  }
+  if (H == 1024) return L < 12 || B <= 192;
+  return true;
+}
+
 static int run_stack(const char* who, const float* xs, const float* WU, const float* bias, const int* dil,
                      const int* active, float* hsss, float* csss, int L, int T, int B, int H, void* ws,
                      size_t ws_bytes, hipStream_t s, int products = FTK_LSTM_PRODUCTS_DEFAULT, int spin_limit = 0) {
@@ -1758,6 +1766,11 @@ static int run_stack(const char* who, const float* xs, const float* WU, const fl
         return fail(FTK_ERR_INVALID_ARGUMENT, "%s: active_rows must be non-increasing (rows sorted by length), but [%d]=%d > [%d]=%d",
                     who, t, active[t], t - 1, active[t - 1]);
     }
+  }
+  if (products == FTK_LSTM_PRODUCTS_F16X3 && exchange_chosen(L, T, B, H, dil, false) && ws && ws_bytes >= exchange_workspace_bytes(L, T, B, H, false)) {
+    bool handled = false;
+    rc = run_exchange(false, xs, WU, bias, dil, active, hsss, csss, L, T, B, H, ws, ws_bytes, s, &handled, spin_limit);
+    if (rc || handled) return rc;
   }
   if (H == PH) {
     // A stack deeper than the chip holds at eight workgroups a layer runs as consecutive persistent launches: a
@@ -1820,17 +1833,20 @@ extern "C" {
 
 size_t ftk_stacked_lstm_workspace_bytes(int L, int T, int B, int H) {
   if (L <= 0 || T <= 0 || B <= 0 || H <= 0) return 0;
-  if (H != ftk::PH && H % 32 == 0) return ftk::split_stack_workspace_bytes(L, T, B, H);  // planes, scales, re-laid weights
-  return ftk::workspace_need(L, T, B);
+  // what the call chooses depends on the device and the product mode: room for any of them
+  const size_t exchange = ftk::exchange_takes(H, false) ? ftk::exchange_workspace_bytes(L, T, B, H, false) : 0;
+  if (H != ftk::PH && H % 32 == 0) return std::max(exchange, ftk::split_stack_workspace_bytes(L, T, B, H));  // planes, scales, re-laid weights
+  return std::max(exchange, ftk::workspace_need(L, T, B));
 }
 
 size_t ftk_stacked_lstm_f16_workspace_bytes(int L, int T, int B, int H) {
   if (L <= 0 || T <= 0 || B <= 0 || H <= 0) return 0;
   // the status block and the re-laid weights of the streaming kernel
-  const size_t packed = ftk::kStatusBytes + (size_t)L * 2 * H * 4 * H * sizeof(_Float16);
+  const size_t packed = std::max(ftk::kStatusBytes + (size_t)L * 2 * H * 4 * H * sizeof(_Float16),
+                                 ftk::exchange_takes(H, true) ? ftk::exchange_workspace_bytes(L, T, B, H, true) : (size_t)0);
   if (!ftk::f16_fits_on_chip(B, H)) return packed;
   // which of the two runs is decided per call (a ragged batch stays with the persistent kernel): room for either
-  return std::max(ftk::xratio_offset_bytes(L, T, B), ftk::f16_streams(L, B, H, false) ? packed : (size_t)0);
+  return std::max(ftk::xratio_offset_bytes(L, T, B), packed);
 }
 
 int ftk_stacked_lstm_f16(const void* xs, const void* WU, const float* bias, const int* dilations,
@@ -1856,6 +1872,12 @@ int ftk_stacked_lstm_f16(const void* xs, const void* WU, const float* bias, cons
       if (t > 0 && active_rows[t] > active_rows[t - 1])
         return fail(FTK_ERR_INVALID_ARGUMENT, "%s: active_rows must be non-increasing (rows sorted by length)", who);
     }
+  if (exchange_chosen(L, T, B, H, dilations, true) && workspace && workspace_bytes >= exchange_workspace_bytes(L, T, B, H, true)) {
+    bool handled = false;
+    const int rcx = run_exchange(true, xs, WU, bias, dilations, active_rows, hsss, csss, L, T, B, H, workspace, workspace_bytes,
+                                 (hipStream_t)stream, &handled, 0);
+    if (rcx || handled) return rcx;
+  }
   // every other shape streams the weights, one launch per stage of independent cells (dead rows are computed too)
   // (the workspace takes the weights re-laid per unit block, so that a workgroup reads one contiguous run)
   if (!on_chip) {

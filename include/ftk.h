@@ -298,7 +298,8 @@ int ftk_stacked_lstm_small_states(const void* workspace, ftk_stream_t stream);
  * the reference.  The first call on a device does set-up that is no
  * allocation but is no stream work either (the scratch's address, a function
  * attribute, an occupancy query): make one call per device before any region
- * that must hold nothing but launches.  The launch is a cooperative one
+ * that must hold nothing but launches.  In a stream capture, and once a second
+ * stream has used the persistent kernels, the launch is a cooperative one
  * (hipLaunchCooperativeKernel); that a stream capture records it has not been
  * exercised here.  Same operands and results as ftk_stacked_lstm_opts_f32
  * with {FTK_LSTM_PRODUCTS_F32, 0} and no active_rows; H must be 256, and the

@@ -1374,3 +1374,52 @@ def test_windowed_attention_rejects_bad_arguments(core):
         core.windowed_attention(Q, Q, Q, 3, 1, torch.zeros((2, 8, 2), dtype=torch.int64, device='cuda'))
     with pytest.raises(ValueError):
         core.windowed_attention(Q, Q[:, :4], Q, 3)
+
+
+@pytest.mark.parametrize('half,H,L,T,B,dil', [
+    (False, 64, 3, 5, 17, None),           # half a k step per wave: x and h waves; the second row block holds one row
+    (False, 64, 32, 4, 130, None),         # several 32-row blocks per workgroup, the last of two rows
+    (False, 128, 2, 1, 15, None),          # a single step
+    (False, 128, 4, 11, 16, [1, 2, 4, 8]), # recurrences that read their own h from the layer-to-layer buffer
+    (False, 128, 20, 6, 100, None),        # slices of one and of two row blocks in one launch
+    (False, 256, 1, 9, 33, None),
+    (False, 512, 2, 7, 1, None),           # one row
+    (False, 512, 8, 5, 33, None),          # two 32-row blocks on one workgroup, every layer on an XCD of its own
+    (False, 512, 9, 3, 20, None),          # a layer more than the chip holds: two launches
+    (True, 256, 3, 7, 17, None),
+    (True, 512, 17, 3, 40, [1, 2] * 8 + [3]),
+    (True, 1024, 2, 6, 18, None),          # a layer larger than an XCD
+    (True, 1024, 5, 4, 65, None),          # the same, several row blocks, two launches
+])
+def test_stacked_lstm_exchange_kernel(core, half, H, L, T, B, dil):
+    """Shapes at the edges of the exchange kernel's row blocks, slices, launches and steps (rings of four steps, buffers
+    set back two steps ahead), dense and ragged, against the oracle; three launches on one workspace give the same bits."""
+    xs, WU, bs = lstm_inputs(77, L, T, B, H, 1.0 / np.sqrt(H))
+    xs[0] *= 8.0                            # input rows of different magnitude
+    rows = sorted({0, B // 2, B - 1})
+    if half:
+        xs, WU = xs.astype(np.float16), WU.astype(np.float16)
+        hr, cr = ko.stacked_lstm_f16(xs[:, rows], WU, bs, dil)
+    else:
+        hr, cr = ko.stacked_lstm(xs[:, rows], WU, bs, dilations=dil)
+    fn = core.stacked_lstm_f16 if half else core.stacked_lstm
+    nbytes = (core.lib.ftk_stacked_lstm_f16_workspace_bytes if half else core.stacked_lstm_workspace_bytes)(L, T, B, H)
+    ws = torch.full((nbytes,), 0x3c, dtype=torch.uint8, device='cuda')      # no value that stands for "not there yet"
+    lens = np.maximum(1, T - (np.arange(B) * T) // B)
+    for active in (None, [int((lens > t).sum()) for t in range(T)]):
+        first = None
+        for _ in range(3):
+            h, c = fn(dev(xs), dev(WU), dev(bs), dilations=dil, workspace=ws, active_rows=active)
+            assert core.persistent_status(ws) == 0, 'a wait gave up'
+            live = torch.ones((T, B), dtype=torch.bool) if active is None else torch.from_numpy(np.arange(T)[:, None] < lens[None, :])
+            got = [t.cpu()[:, live] for t in (h, c)]
+            assert first is None or all(torch.equal(a, b) for a, b in zip(first, got))
+            first = got
+        ref_live = live[:, rows].numpy()
+        for t, ref, what in ((h, hr, 'h'), (c, cr, 'c')):
+            t = t[:, :, rows].float().cpu().numpy()[:, ref_live]
+            if half:
+                # h and c carry an fp16 rounding, 2^-11 of themselves, through T steps and L layers that damp it
+                assert ko.max_rel_err(t, ref.astype(np.float32)[:, ref_live]) <= 1e-2, what
+            else:
+                assert_lstm_close(torch.from_numpy(t), ref[:, ref_live], what)
