@@ -1,8 +1,14 @@
 """ctypes binding of libftkernels.so, the C ABI declared in include/ftk.h.
 
 This is the only place the package touches native code.  The library is
-required: importing this module without a built libftkernels.so raises, and
-no function here has a CPU or PyTorch fallback.
+required: importing this module without a built libftkernels.so (and the
+module beside it, _fast) raises, and no function here has a CPU or PyTorch
+fallback.
+
+The fused entry points first hand their arguments to _fast, which checks,
+allocates and launches in one native call and returns None, with nothing done,
+for whatever is not plainly right; the code below it then says what is wrong
+(or handles the rarer options).
 """
 from __future__ import annotations
 
@@ -21,7 +27,7 @@ EXPORTS = (
     'ftk_lstm_cell_f32', 'ftk_lstm_cell_f16', 'ftk_lstm_layer_f32', 'ftk_lstm_layer_f16', 'ftk_lstm_elementwise_f32',
     'ftk_stacked_lstm_workspace_bytes', 'ftk_stacked_lstm_f32', 'ftk_dilated_lstm_f32',
     'ftk_stacked_lstm_wavefront_f32', 'ftk_stacked_lstm_ragged_f32', 'ftk_lstm_set_products', 'ftk_lstm_get_products',
-    'ftk_stacked_lstm_opts_f32', 'ftk_stacked_lstm_status', 'ftk_stacked_lstm_small_states', 'ftk_stacked_lstm_noalloc_f32',
+    'ftk_stacked_lstm_opts_f32', 'ftk_stacked_lstm_status', 'ftk_stacked_lstm_small_states', 'ftk_stacked_lstm_result', 'ftk_stacked_lstm_noalloc_f32',
     'ftk_stacked_lstm_f16_workspace_bytes', 'ftk_stacked_lstm_f16',
     'ftk_b2b_gemm_f16', 'ftk_b2b_gemm_f16_supported', 'ftk_b2b_gemm_rowmajor_f16', 'ftk_gemm_f16', 'ftk_batched_gemm_f16', 'ftk_flash_attn_f16', 'ftk_flash_attn_f16_workspace_bytes', 'ftk_flash_attn_ws_f16', 'ftk_flash_attn_f32_workspace_bytes', 'ftk_flash_attn_f32', 'ftk_online_softmax_f32', 'ftk_embedding_gather_f32',
     'ftk_grid_rnn_workspace_bytes', 'ftk_grid_rnn_f32', 'ftk_windowed_attn_f32',
@@ -124,6 +130,14 @@ launch_counts: dict = {}
 
 def _count(name: str) -> None:
     launch_counts[name] = launch_counts.get(name, 0) + 1
+
+
+try:
+    from . import _fast
+except ImportError as e:
+    raise ImportError(f'{_HERE}/_fast.so cannot be loaded ({e}): build it with `make -C fractaltensor_amd/csrc` '
+                      '(or __graft_entry__.build()); there is no fallback path') from e
+_fast.init(launch_counts, _check)
 
 
 def version() -> int:
@@ -250,6 +264,16 @@ def stacked_lstm(xs, WU, bias=None, dilations: Optional[Sequence[int]] = None, s
     the fixed scale of their fp16 planes were written (stacked_lstm_small_states), compute the stack again on fp32
     products, so that layers that fade towards zero are accurate relative to their own size as well.
     """
+    if schedule == 'auto' and active_rows is None and not spin_limit and (products is None or products in LSTM_PRODUCTS):
+        small = exact_small_states and products != 'f32'
+        done = _fast.stacked_lstm(False, xs, WU, bias, dilations, out, workspace, -1 if products is None else LSTM_PRODUCTS[products],
+                                  check, small)
+        if done is not None:
+            if not (small and done[2]):
+                return done[0], done[1]
+            _count('stacked_lstm_repeated_on_f32_products')
+            return stacked_lstm(xs, WU, bias, dilations=dilations, out=(done[0], done[1]), workspace=workspace, products='f32',
+                                check=workspace is None if check is None else check)
     f32 = torch.float32
     _req(xs, f32, 'xs'); _req(WU, f32, 'WU')
     T, B, H = xs.shape
@@ -366,6 +390,10 @@ def stacked_lstm_f16(xs, WU, bias=None, dilations: Optional[Sequence[int]] = Non
     """fp16 storage: xs [T,B,H], WU [L,2H,4H] fp16, bias [L,4H] fp32 or None -> hsss, csss [L,T,B,H] fp16.
     H a multiple of 32: H = 512, and H = 256 with an even batch, run in the persistent kernel, every other
     shape as one launch of the streaming cell kernel per stage of independent cells."""
+    if active_rows is None:
+        done = _fast.stacked_lstm(True, xs, WU, bias, dilations, out, workspace, -1, check, False)
+        if done is not None:
+            return done[0], done[1]
     f16 = torch.float16
     _req(xs, f16, 'xs'); _req(WU, f16, 'WU')
     T, B, H = xs.shape
@@ -436,6 +464,9 @@ def persistent_status(workspace: torch.Tensor) -> int:
 
 def b2b_gemm(A, B_nk, C_pn, out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """D = (A @ B) @ C.  A [G,M,K]; B_nk [G,N,K] (B stored column-major); C_pn [G,P,N]; D [G,M,P]; fp16."""
+    D = _fast.b2b_gemm(A, B_nk, C_pn, out)
+    if D is not None:
+        return D
     f16 = torch.float16
     _req(A, f16, 'A'); _req(B_nk, f16, 'B_nk'); _req(C_pn, f16, 'C_pn')
     squeeze = A.dim() == 2
@@ -515,6 +546,9 @@ def flash_attention(Q, K, V, scale: Optional[float] = None, out: Optional[torch.
     A grid that does not fill the chip (few queries, heads and samples) with many keys is split over the keys and
     merged (ftk_flash_attn_ws_f16); the workspace for that is allocated here unless one is given, split_keys=False
     keeps the single launch."""
+    O = _fast.flash_attention(True, Q, K, V, scale, out, workspace, split_keys)
+    if O is not None:
+        return O
     f16 = torch.float16
     _req(Q, f16, 'Q'); _req(K, f16, 'K'); _req(V, f16, 'V')
     B, Hd, Sq, D = Q.shape
@@ -545,6 +579,9 @@ def flash_attention_f32(Q, K, V, scale: Optional[float] = None, out: Optional[to
                         workspace: Optional[torch.Tensor] = None) -> torch.Tensor:
     """Non-causal attention with fp32 Q [B,Hd,Sq,D], K, V [B,Hd,Skv,D] -> O [B,Hd,Sq,D] fp32; D of 32, 64, 96 or 128.
     Every product as three fp16 MFMAs of split operands, fp32 accumulation and softmax state."""
+    O = _fast.flash_attention(False, Q, K, V, scale, out, workspace, False)
+    if O is not None:
+        return O
     f32 = torch.float32
     _req(Q, f32, 'Q'); _req(K, f32, 'K'); _req(V, f32, 'V')
     if Q.dim() != 4 or K.dim() != 4 or K.shape != V.shape or Q.shape[:2] != K.shape[:2] or Q.shape[3] != K.shape[3]:

@@ -45,8 +45,10 @@
 // its CU).  Every wait is bounded by spin_limit polls; on expiry the kernel
 // records an error word and every workgroup drains.
 #include <stdlib.h>
+#include <string.h>
 
 #include <algorithm>
+#include <chrono>
 #include <mutex>
 #include <type_traits>
 
@@ -1715,6 +1717,76 @@ static int scratch_of_current_device(const char* who, void** out, bool lookup) {
   return FTK_OK;
 }
 
+// The first two words of a workspace's status block, once the stream has come to them: a one-thread kernel writes them to
+// pinned host memory, where the host waits for them.  (A copy to pageable memory and a wait for the stream take 25 to 30
+// us of the host's time, this about 6.)  The host looks for two milliseconds, which covers the stacks for which that
+// matters, and leaves the rest of the wait to the runtime.  The sixteen slots are allocated once and kept; with all of
+// them in use by other threads the words are copied.
+struct StatusSlot {
+  int seq;       // written last: the words are those of this request
+  int words[2];
+  int pad[13];   // a cache line each
+};
+constexpr int kStatusSlots = 16;
+__global__ void report_status_kernel(const int* status, StatusSlot* slot, int seq) {
+  const int w0 = status[0], w1 = status[1];
+  __hip_atomic_store(&slot->words[0], w0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  __hip_atomic_store(&slot->words[1], w1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  __hip_atomic_store(&slot->seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+static int read_status_words(const void* workspace, int (&words)[2], hipStream_t s) {
+  static std::mutex mu;
+  static StatusSlot* slots = nullptr;
+  static unsigned in_use = 0;
+  static int next_seq = 0;
+  int at = -1, seq = 0;
+  {
+    std::lock_guard<std::mutex> lock(mu);
+    if (!slots) {
+      void* p = nullptr;
+      if (hipHostMalloc(&p, kStatusSlots * sizeof(StatusSlot), hipHostMallocPortable | hipHostMallocMapped) == hipSuccess) {
+        memset(p, 0, kStatusSlots * sizeof(StatusSlot));
+        slots = reinterpret_cast<StatusSlot*>(p);
+      } else {
+        (void)hipGetLastError();
+      }
+    }
+    for (int i = 0; slots && i < kStatusSlots && at < 0; ++i)
+      if (!(in_use >> i & 1)) at = i;
+    if (at >= 0) {
+      in_use |= 1u << at;
+      seq = next_seq = next_seq % 0x3fffffff + 1;
+    }
+  }
+  if (at < 0) {
+    FTK_HIP(hipMemcpyAsync(words, workspace, sizeof(words), hipMemcpyDeviceToHost, s));
+    FTK_HIP(hipStreamSynchronize(s));
+    return FTK_OK;
+  }
+  StatusSlot* slot = slots + at;
+  hipLaunchKernelGGL(report_status_kernel, dim3(1), dim3(1), 0, s, reinterpret_cast<const int*>(workspace), slot, seq);
+  int rc = check_launch("report_status_kernel");
+  if (rc == FTK_OK) {
+    const auto begin = std::chrono::steady_clock::now();
+    bool there = false;
+    for (unsigned n = 1; !(there = __atomic_load_n(&slot->seq, __ATOMIC_ACQUIRE) == seq); ++n) {
+      __builtin_ia32_pause();
+      if (n % 256 == 0 && std::chrono::steady_clock::now() - begin > std::chrono::milliseconds(2)) break;
+    }
+    if (!there) {
+      const hipError_t e = hipStreamSynchronize(s);
+      if (e != hipSuccess) rc = fail(FTK_ERR_LAUNCH, "hipStreamSynchronize: %s", hipGetErrorString(e));
+      else if (__atomic_load_n(&slot->seq, __ATOMIC_ACQUIRE) != seq) rc = fail(FTK_ERR_DEVICE, "stacked LSTM: the status words did not arrive");
+    }
+    words[0] = slot->words[0];
+    words[1] = slot->words[1];
+  }
+  std::lock_guard<std::mutex> lock(mu);
+  in_use &= ~(1u << at);
+  return rc;
+}
+
 static int check_stack_args(const char* who, const float* xs, const float* WU, float* hsss, float* csss, int L, int T,
                             int B, int H, const int* dil) {
   if (!xs || !WU || !hsss || !csss) return fail(FTK_ERR_INVALID_ARGUMENT, "%s: xs, WU, hsss, csss must be non-NULL", who);
@@ -1936,23 +2008,29 @@ int ftk_stacked_lstm_status(const void* workspace, ftk_stream_t stream) {
                   "ftk_stacked_lstm_status: workspace is NULL and ftk_stacked_lstm_noalloc_f32 has not run on the current device");
     workspace = ptr;
   }
-  int word = 0;
-  FTK_HIP(hipMemcpyAsync(&word, workspace, sizeof(int), hipMemcpyDeviceToHost, (hipStream_t)stream));
-  FTK_HIP(hipStreamSynchronize((hipStream_t)stream));
-  if (word != 0)
-    return fail(FTK_ERR_TIMEOUT,
-                "stacked LSTM: a bounded wait of the persistent launch ran out of polls (status word %d); the launch drained "
-                "early and hsss / csss are incomplete", word);
-  return FTK_OK;
+  return ftk_stacked_lstm_result(workspace, nullptr, stream);
 }
 
 int ftk_stacked_lstm_small_states(const void* workspace, ftk_stream_t stream) {
   using namespace ftk;
   if (!workspace) return fail(FTK_ERR_INVALID_ARGUMENT, "ftk_stacked_lstm_small_states: workspace is NULL");
-  int word = 0;
-  FTK_HIP(hipMemcpyAsync(&word, reinterpret_cast<const int*>(workspace) + 1, sizeof(int), hipMemcpyDeviceToHost, (hipStream_t)stream));
-  FTK_HIP(hipStreamSynchronize((hipStream_t)stream));
-  return word != 0 ? 1 : 0;
+  int words[2] = {0, 0};
+  const int rc = read_status_words(workspace, words, (hipStream_t)stream);
+  return rc ? rc : words[1] != 0 ? 1 : 0;
+}
+
+int ftk_stacked_lstm_result(const void* workspace, int* small_states, ftk_stream_t stream) {
+  using namespace ftk;
+  if (!workspace) return fail(FTK_ERR_INVALID_ARGUMENT, "ftk_stacked_lstm_result: workspace is NULL");
+  int words[2] = {0, 0};
+  const int rc = read_status_words(workspace, words, (hipStream_t)stream);
+  if (rc) return rc;
+  if (small_states) *small_states = words[1] != 0 ? 1 : 0;
+  if (words[0] != 0)
+    return fail(FTK_ERR_TIMEOUT,
+                "stacked LSTM: a bounded wait of the persistent launch ran out of polls (status word %d); the launch drained "
+                "early and hsss / csss are incomplete", words[0]);
+  return FTK_OK;
 }
 
 int ftk_stacked_lstm_noalloc_f32(const float* xs, const float* WU, const float* bias, const int* dilations, float* hsss,

@@ -11,6 +11,7 @@ memory (zero copy), and `from_dense()` wraps a dense tensor the other way.
 """
 from __future__ import annotations
 
+import math
 from collections.abc import Sequence
 from typing import List, Optional, Tuple, Union
 
@@ -94,8 +95,15 @@ class FractalTensor(Sequence):
         self._offsets = None
 
     @property
+    def has_indices(self) -> bool:
+        """Whether there is an index tree (a look that does not build the one of a regular FractalTensor)."""
+        return self._type._dims is not None or self._type._indices is not None
+
+    @property
     def numel(self) -> int:
         """Number of leaf tensors."""
+        if self._type._dims is not None:
+            return math.prod(self._type._dims)
         if self.indices is None:
             raise RuntimeError('numel is data dependent. No data is given.')
         return _count_leaves(self.indices)
@@ -140,6 +148,8 @@ class FractalTensor(Sequence):
     # ---- dense view ---------------------------------------------------------
     def dense_shape(self) -> Optional[Tuple[int, ...]]:
         """(n1, ..., nk) when every level has a uniform width, else None."""
+        if self._type._dims is not None:
+            return self._type._dims
         if self.indices is None:
             return None
         dims = []
@@ -173,14 +183,7 @@ class FractalTensor(Sequence):
         for _ in range(depth - 1):
             typ = FractalTensorStorage(typ)
         ft = FractalTensor(typ)
-
-        def build(level):
-            n = t.shape[level]
-            if level == depth - 1:
-                return list(range(n))
-            return [build(level + 1) for _ in range(n)]
-
-        ft.indices = build(0)
+        ft._type.set_regular(t.shape[:depth])
         ft._T = t.reshape(-1)
         return ft
 
@@ -195,20 +198,28 @@ class FractalTensor(Sequence):
         return self._offsets
 
     def index(self, idx: int):
-        if self._T is None or self.indices is None:
+        if self._T is None or not self.has_indices:
             raise RuntimeError('FractalTensor is not initialized.')
-        n = len(self.indices)
+        n = len(self)
         if idx < 0:
             idx += n
         if idx < 0 or idx >= n:
             raise IndexError('FractalTensor index out of range')
         es = self.element_size
-        offs = self._child_offsets()
-        lo, hi = offs[idx] * es, offs[idx + 1] * es
+        dims = self._type._dims
+        if dims is not None:
+            each = math.prod(dims[1:]) * es
+            lo, hi = idx * each, (idx + 1) * each
+        else:
+            offs = self._child_offsets()
+            lo, hi = offs[idx] * es, offs[idx + 1] * es
         if self.depth == 1:
             return Tensor.from_tensor(self._T[lo:hi].view(*self.element_shape))
         child = FractalTensor(self._type.dtype.dtype)
-        child.indices = _renumber(self.indices[idx])
+        if dims is not None:
+            child._type.set_regular(dims[1:])
+        else:
+            child.indices = _renumber(self.indices[idx])
         child._T = self._T[lo:hi]
         return child
 
@@ -243,6 +254,8 @@ class FractalTensor(Sequence):
         raise TypeError(f'unsupported index type {type(i)}')
 
     def __len__(self) -> int:
+        if self._type._dims is not None:
+            return self._type._dims[0]
         if self.indices is None:
             raise RuntimeError('FractalTensor is not initialized.')
         return len(self.indices)
@@ -328,18 +341,34 @@ class Iterative(Sequence):
     """The result of zip: a sequence of per-position field lists."""
 
     def __init__(self, *xs):
-        self._items = list(xs)
+        self._built = list(xs)
         self.sources = None   # set by zip: the sequences the items were taken from
+
+    @staticmethod
+    def over(sources, n: int) -> 'Iterative':
+        """What zip makes of `sources`, n items each: the field lists are taken from them when somebody looks (a fused
+        kernel takes the sources as they are)."""
+        out = Iterative()
+        out._built = None
+        out.sources = tuple(sources)
+        out._n = n
+        return out
+
+    @property
+    def _items(self):
+        if self._built is None:
+            self._built = [[x[i] for x in self.sources] for i in range(self._n)]
+        return self._built
 
     def __getitem__(self, i):
         return self._items[i]
 
     def __len__(self) -> int:
-        return len(self._items)
+        return self._n if self._built is None else len(self._built)
 
     @property
     def length(self) -> int:
-        return len(self._items)
+        return len(self)
 
     @staticmethod
     def make_iterative(*xs) -> 'Iterative':

@@ -106,7 +106,7 @@ def note_dilation(dilation: int) -> None:
 _SCALARS = (int, float, str, bool, bytes, type(None))
 
 
-def _code_names(code, seen=None):
+def _code_names(code):
     """Global names a code object reads, those of the lambdas and functions defined inside it included."""
     names = list(code.co_names)
     for c in code.co_consts:
@@ -115,7 +115,53 @@ def _code_names(code, seen=None):
     return names
 
 
-def _fingerprint(f, level: int = 0, seen=None):
+# Per (code object, module globals): what the code reaches through its globals, as one number.  An entry holds everything
+# that was looked at (_Seen); as long as all of it is the same objects the number stands, and a call of a routed program
+# pays a dozen identity checks for it.
+_reached: dict = {}
+_numbers: dict = {}
+_number_count = 0
+_MISSING = object()
+
+
+class _Seen:
+    """What a fingerprint looked at."""
+
+    def __init__(self):
+        self.names = []          # (globals, name, value)
+        self.functions = []      # (function, code, defaults, keyword defaults, closure contents)
+        self.stable = True       # nothing among it that can change in place (a list held as a default or in a closure)
+
+    def unchanged(self) -> bool:
+        for g, name, v in self.names:
+            if g.get(name, _MISSING) is not v:
+                return False
+        for f, code, defaults, kw, cells in self.functions:
+            if f.__code__ is not code or f.__defaults__ is not defaults or f.__kwdefaults__ is not kw:
+                return False
+            for cell, v in cells:
+                try:
+                    if cell.cell_contents is not v:
+                        return False
+                except ValueError:
+                    if v is not _MISSING:
+                        return False
+        return True
+
+
+def _number_of(parts):
+    global _number_count
+    if len(_numbers) >= 1024:
+        _numbers.clear()
+        _reached.clear()
+    n = _numbers.get(parts)
+    if n is None:
+        _number_count += 1           # never used twice: a verdict kept under an old number is only forgotten
+        n = _numbers[parts] = _number_count
+    return n
+
+
+def _fingerprint(f, level: int = 0, seen=None, looked=None):
     """What identifies a user function between calls (a lambda is a new object at every call of the program, its
     code object is not): its code, its default arguments, the scalars and functions it closes over, and the scalars
     and functions its code reaches through module globals -- so that a layer function, a cell or a scale that is
@@ -140,31 +186,61 @@ def _fingerprint(f, level: int = 0, seen=None):
         if isinstance(v, (Tensor, FractalTensor, Iterative, torch.Tensor)):
             return type(v).__name__
         if isinstance(v, (tuple, list)) and len(v) <= 16 and all(isinstance(e, _SCALARS) for e in v):
+            if looked is not None and isinstance(v, list):
+                looked.stable = False
             return tuple(v)
         if callable(v) and hasattr(v, '__code__'):
-            return _fingerprint(v, level + 1, seen)
+            return _fingerprint(v, level + 1, seen, looked)
         if isinstance(v, type(os)):                       # a module: its name (ops, torch, math ...)
             return ('module', v.__name__)
         if isinstance(v, type):
             return ('class', v.__module__, v.__qualname__)
+        if looked is not None:
+            looked.stable = False
         return ('id', type(v).__name__, id(v))
 
-    parts = [code]
-    for d in (getattr(f, '__defaults__', None) or ()):
+    parts = []
+    defaults, kw, closure = getattr(f, '__defaults__', None), getattr(f, '__kwdefaults__', None), getattr(f, '__closure__', None)
+    for d in (defaults or ()):
         parts.append(of_value(d))
-    for k, d in sorted((getattr(f, '__kwdefaults__', None) or {}).items()):
+    for k, d in sorted((kw or {}).items()):
         parts.append((k, of_value(d)))
-    for cell in (getattr(f, '__closure__', None) or ()):
+    cells = []
+    for cell in (closure or ()):
         try:
-            parts.append(of_value(cell.cell_contents))
+            v = cell.cell_contents
         except ValueError:
+            cells.append((cell, _MISSING))
             continue
+        cells.append((cell, v))
+        parts.append(of_value(v))
+    if looked is not None:
+        looked.functions.append((f, code, defaults, kw, cells))
+        if kw:
+            looked.stable = False
+
     g = getattr(f, '__globals__', None) or {}
-    for name in _code_names(code):
-        if name in g:
-            v = g[name]
-            if isinstance(v, _SCALARS) or (callable(v) and hasattr(v, '__code__')):
-                parts.append((name, of_value(v)))
+
+    def of_globals(record):
+        names = []
+        for name in _code_names(code):
+            v = g.get(name, _MISSING)
+            record.names.append((g, name, v))
+            if v is not _MISSING and (isinstance(v, _SCALARS) or (callable(v) and hasattr(v, '__code__'))):
+                names.append((name, v if isinstance(v, _SCALARS) else _fingerprint(v, level + 1, seen, record)))
+        return (code, tuple(names))
+
+    if looked is not None:               # reached from another function: part of that one's number
+        parts.append(of_globals(looked))
+        return tuple(parts)
+    entry = _reached.get((id(code), id(g), level))
+    if entry is None or not entry[0].unchanged():
+        record = _Seen()
+        n = _number_of(of_globals(record))
+        entry = (record, n, code, g)      # (code and g are kept alive: their ids stay theirs)
+        if record.stable:
+            _reached[(id(code), id(g), level)] = entry
+    parts.append(entry[1])
     return tuple(parts)
 
 
@@ -184,7 +260,7 @@ def _rel_err(got: torch.Tensor, ref: torch.Tensor) -> float:
 # ------------------------------------------------------------------ stacked / dilated LSTM behind fold, map and scan
 
 def _is_gate_params(p, shape) -> bool:
-    return (isinstance(p, FractalTensor) and p.depth == 1 and p.data is not None and _on_device(p.data) and p.indices is not None
+    return (isinstance(p, FractalTensor) and p.depth == 1 and p.data is not None and _on_device(p.data) and p.has_indices
             and len(p) == 4 and tuple(p.element_shape) == tuple(shape))
 
 
@@ -227,6 +303,22 @@ _fading_stacks: set = set()        # packed weights whose last launch on split p
 def clear_weight_cache() -> None:
     _weights.clear()
     _fading_stacks.clear()
+
+
+def _packed_sources(sources):
+    """The same for a stack whose layers are the items of three zipped FractalTensors [L][4]: Wss, Uss, bss."""
+    srcs = [p.data for p in sources]
+    key = tuple((t.data_ptr(), t._version, t.numel(), t.dtype) for t in srcs)
+    hit = _weights.get(key)
+    if hit is not None:
+        stats['weight_cache_hits'] += 1
+        return hit[0], hit[1]
+    from . import fused
+    WU, bias = fused.pack_lstm_weights(*sources)
+    if len(_weights) >= _MAX_WEIGHTS:
+        _weights.pop(next(iter(_weights)))
+    _weights[key] = (WU, bias, srcs)
+    return WU, bias
 
 
 def _packed_stack(layers):
@@ -388,15 +480,33 @@ def _match_fold(xs, H: int, dtype):
     return layers
 
 
+def _stack_sources(xs, H: int, dtype):
+    """(Wss, Uss, bss) if the fold items are those of three zipped regular [L][4] parameter FractalTensors of hidden size H
+    and type dtype on the GPU: what _match_fold finds item by item, seen at once.  None: look item by item."""
+    src = getattr(xs, 'sources', None)
+    if not isinstance(xs, Iterative) or src is None or len(src) != 3 or len(xs) == 0:
+        return None
+    for p, shape in ((src[0], (H, H)), (src[1], (H, H)), (src[2], (1, H))):
+        if not isinstance(p, FractalTensor) or p.depth != 2 or p.data is None or p.data.dtype != dtype or not _on_device(p.data):
+            return None
+        dims = p._type._dims
+        if dims is None or dims != (len(xs), 4) or p.element_shape != shape:
+            return None
+    return src
+
+
 def _fold_verdict(func: Callable, xs, layers, H: int, dtype, seq_depth: int):
-    """{'dilations': per layer, 'layout': ...} if func has been seen to compute an LSTM layer on every probed item, else None."""
-    indexed = layers[0][0] is not None
-    L = len(layers)
+    """{'dilations': per layer, 'layout': ...} if func has been seen to compute an LSTM layer on every probed item, else None.
+    layers: the fold items as _match_fold gives them, or None for three zipped sources (_stack_sources)."""
+    indexed = layers is not None and layers[0][0] is not None
+    L = len(xs)
     key = ('fold', _fingerprint(func), indexed, L if indexed else 0, H, dtype, seq_depth)
     if key not in _verdicts:
         stats['probes'] += 1
         verdict = None
         try:
+            if layers is None:
+                layers = _match_fold(xs, H, dtype)
             gen = torch.Generator().manual_seed(20240229)
             # without an index the function cannot tell the layers apart except through their parameters
             which = range(L) if indexed else range(1)
@@ -417,7 +527,7 @@ def _fold_verdict(func: Callable, xs, layers, H: int, dtype, seq_depth: int):
 
 def _sequence_operand(seq, depths=(1, 2)):
     """(H, dtype) of a GPU FractalTensor of [1, H] rows that the LSTM kernels take, else None."""
-    if not isinstance(seq, FractalTensor) or seq.depth not in depths or seq.data is None or not _on_device(seq.data) or seq.indices is None:
+    if not isinstance(seq, FractalTensor) or seq.depth not in depths or seq.data is None or not _on_device(seq.data) or not seq.has_indices:
         return None
     if len(seq.element_shape) != 2 or seq.element_shape[0] != 1:
         return None
@@ -478,9 +588,11 @@ def try_fold(func: Callable, xs, initializer, kwargs):
     if op is None:
         return NotImplemented
     H, dtype = op
-    layers = _match_fold(xs, H, dtype)
-    if layers is None:
+    sources = _stack_sources(xs, H, dtype)
+    layers = None if sources is not None else _match_fold(xs, H, dtype)
+    if sources is None and layers is None:
         return NotImplemented
+    packed = lambda: _packed_sources(sources) if sources is not None else _packed_stack(layers)
     cap = _capturing()
     if cap is not None:
         if seq.depth != 1:
@@ -499,7 +611,7 @@ def try_fold(func: Callable, xs, initializer, kwargs):
 
     from . import fused
     if seq.depth == 1:
-        WU, bias = _packed_stack(layers)
+        WU, bias = packed()
         T = len(seq)
         h = _run_lstm(seq.as_dense().reshape(T, 1, H), WU, bias, dilations)
         stats[name] += 1
@@ -508,7 +620,7 @@ def try_fold(func: Callable, xs, initializer, kwargs):
         lengths = [len(sample) for sample in seq.indices]
         if min(lengths) <= 0:
             return NotImplemented
-        WU, bias = _packed_stack(layers)
+        WU, bias = packed()
         h, launches = _run_batch_major(seq.data.view(-1, H), lengths, WU, bias, dilations)
         stats[name] += launches
         return _rows_to_batch_major(h, lengths)
@@ -518,7 +630,7 @@ def try_fold(func: Callable, xs, initializer, kwargs):
         dense, sizes = fused.pad_time_major(seq)
     except ValueError:
         return NotImplemented                   # ragged, but not a time-major batch of length-sorted sequences
-    WU, bias = _packed_stack(layers)
+    WU, bias = packed()
     h = _run_lstm(dense, WU, bias, dilations, sizes)
     stats[name] += 1
     return fused.unpad_time_major(h, sizes)

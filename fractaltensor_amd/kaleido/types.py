@@ -194,7 +194,9 @@ class FractalTensorStorage(Storage):
             raise TypeError('dtype should be a Number, TensorStorage or FractalTensorStorage.')
         self._dtype = dtype
         self._indices = None
+        self._dims = None     # (n1, ..., nk) while the index tree is the regular one of these widths (built when asked for)
         self._length = -1
+        self._depth = dtype._depth + 1 if isinstance(dtype, FractalTensorStorage) else 1
 
     @property
     def dtype(self):
@@ -202,11 +204,20 @@ class FractalTensorStorage(Storage):
 
     @property
     def depth(self) -> int:
-        d, t = 1, self._dtype
-        while isinstance(t, FractalTensorStorage):
-            d += 1
+        return self._depth
+
+    def set_regular(self, dims) -> None:
+        """The index tree of a regular nesting, dims[i] items at every node of level i: noted, and built when somebody
+        looks at it (a batch of a few thousand rows costs more to number than a fused kernel takes to run)."""
+        nest = next((i + 1 for i, n in enumerate(dims) if n == 0), len(dims))
+        if len(dims) != self._depth or nest != self._depth:
+            raise ValueError(f'indices nest {nest} deep but the type has depth {self._depth}.')
+        self._indices = None
+        self._dims = tuple(dims)
+        t = self
+        for n in dims:
+            t._length = n
             t = t._dtype
-        return d
 
     @property
     def length(self) -> int:
@@ -214,10 +225,22 @@ class FractalTensorStorage(Storage):
 
     @property
     def indices(self):
+        if self._indices is None and self._dims is not None:
+            dims = self._dims
+
+            def build(level):
+                if level == len(dims) - 1:
+                    return list(range(dims[level]))
+                return [build(level + 1) for _ in range(dims[level])]
+
+            self._indices = build(0)
+            self._dims = None     # from here on the tree itself says what it is
         return self._indices
 
     @indices.setter
     def indices(self, value):
+        self._dims = None
+
         def nesting(v):
             n = 0
             while isinstance(v, (list, tuple)):

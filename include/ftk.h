@@ -292,6 +292,13 @@ int ftk_stacked_lstm_status(const void* workspace, ftk_stream_t stream);
 int ftk_stacked_lstm_small_states(const void* workspace, ftk_stream_t stream);
 
 /*
+ * The two calls above in one wait: FTK_OK or FTK_ERR_TIMEOUT as
+ * ftk_stacked_lstm_status, and in *small_states (may be NULL) what
+ * ftk_stacked_lstm_small_states returns.
+ */
+int ftk_stacked_lstm_result(const void* workspace, int* small_states, ftk_stream_t stream);
+
+/*
  * ftk_stacked_lstm_opts_f32 with fp32 products for callers that cannot
  * allocate device memory or pass a workspace: tight serving loops, harnesses
  * that forbid hipMalloc, code that prepares a HIP graph.  No counterpart in
