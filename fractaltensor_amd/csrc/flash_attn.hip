@@ -50,6 +50,12 @@
 
 namespace ftk {
 
+// flash_decode.hip: at most kDecodeQueries queries a head
+constexpr int kDecodeQueries = 16;
+int decode_parts(long long bh, int Skv, int D, int cus, int* part_keys);
+int launch_decode(const void* Q, const void* K, const void* V, void* O, int BH, int Sq, int Skv, int D, float scale, int nparts,
+                  int part_keys, float* part_o, float* part_ml, hipStream_t s);
+
 constexpr float FA_TAU = 8.0f;     // slack (in powers of two) before the running maximum is moved
 constexpr float FA_PMAX = 32768.0f;  // phase-alternating kernel: a lane's sum of exponentials above this moves the reference
 constexpr int FA_TRACE_TILES = 256;
@@ -982,37 +988,93 @@ static int launch_fa(const void* Q, const void* K, const void* V, void* O, int B
 }
 
 // The parts of a row merged by the rule of an online softmax: m = max m_p, l = sum l_p 2^(m_p - m),
-// O = sum O_p 2^(m_p - m) / l.  One thread per (row, four columns).
+// O = sum O_p 2^(m_p - m) / l.  Bound by latency: a chain of loads a part long took 12 us for 32 parts of a single row.
+// So a row's parts are dealt over `slices` threads for each four columns, four parts to a thread (all asked for at
+// once), and the slices meet in LDS.
 template <int D>
 __global__ __launch_bounds__(256) void attn_merge_kernel(const float* __restrict__ part_o, const float* __restrict__ part_ml,
-                                                        _Float16* __restrict__ O, int nparts, int Sq, long long rows) {
+                                                        _Float16* __restrict__ O, int nparts, int slices, int Sq, long long rows) {
   constexpr int CPR = D / 4;
-  const long long idx = (long long)blockIdx.x * 256 + threadIdx.x;
-  if (idx >= rows * CPR) return;
-  const long long row = idx / CPR;
-  const int c = (int)(idx - row * CPR);
-  const long long bh = row / Sq;
-  const int r = (int)(row - bh * Sq);
-  float m = -INFINITY;
-  for (int p = 0; p < nparts; ++p) m = fmaxf(m, part_ml[2 * ((bh * nparts + p) * Sq + r)]);
-  float l = 0.0f;
-  float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
-  for (int p = 0; p < nparts; ++p) {
-    const long long at = (bh * nparts + p) * Sq + r;
-    const float w = __builtin_amdgcn_exp2f(part_ml[2 * at] - m);
-    l += w * part_ml[2 * at + 1];
-    const float4 o = *reinterpret_cast<const float4*>(part_o + at * D + 4 * c);
-    acc.x += w * o.x; acc.y += w * o.y; acc.z += w * o.z; acc.w += w * o.w;
+  __shared__ v4f so[256];
+  __shared__ float2 sml[256];
+  const int unit = threadIdx.x / CPR, c = threadIdx.x - unit * CPR;
+  const int rb = (256 / CPR) / slices;             // rows of a block
+  const int slice = unit % slices;
+  const long long row = (long long)blockIdx.x * rb + unit / slices;
+  const bool on = unit < rb * slices && row < rows;
+  float m = -INFINITY, l = 0.0f;
+  v4f acc = {0.f, 0.f, 0.f, 0.f};
+  if (on) {
+    const long long bh = row / Sq;
+    const int r = (int)(row - bh * Sq);
+    for (int p0 = slice; p0 < nparts; p0 += 4 * slices) {
+      float2 ml[4];
+      v4f o[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const long long at = (bh * nparts + min(p0 + i * slices, nparts - 1)) * Sq + r;
+        ml[i] = *reinterpret_cast<const float2*>(part_ml + 2 * at);
+        o[i] = *reinterpret_cast<const v4f*>(part_o + at * D + 4 * c);
+      }
+      const float before = m;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) m = fmaxf(m, ml[i].x);   // a part asked for twice changes no maximum
+      const float alpha = __builtin_amdgcn_exp2f(before - m);
+      l *= alpha;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) acc[k] *= alpha;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float w = p0 + i * slices < nparts ? __builtin_amdgcn_exp2f(ml[i].x - m) : 0.0f;
+        l += w * ml[i].y;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) acc[k] += w * o[i][k];
+      }
+    }
   }
+  if (slices > 1) {
+    so[threadIdx.x] = acc;
+    sml[threadIdx.x] = make_float2(m, l);
+    __syncthreads();
+    if (slice == 0 && on) {
+      const float mine = m;
+      for (int i = 1; i < slices; ++i) m = fmaxf(m, sml[threadIdx.x + i * CPR].x);
+      const float w0 = __builtin_amdgcn_exp2f(mine - m);
+      l *= w0;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) acc[k] *= w0;
+      for (int i = 1; i < slices; ++i) {
+        const float2 ml = sml[threadIdx.x + i * CPR];
+        const v4f o = so[threadIdx.x + i * CPR];
+        const float w = __builtin_amdgcn_exp2f(ml.x - m);
+        l += w * ml.y;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) acc[k] += w * o[k];
+      }
+    }
+  }
+  if (!on || slice) return;
   const float inv = 1.0f / l;
-  const v4h out = {(_Float16)(acc.x * inv), (_Float16)(acc.y * inv), (_Float16)(acc.z * inv), (_Float16)(acc.w * inv)};
+  const v4h out = {(_Float16)(acc[0] * inv), (_Float16)(acc[1] * inv), (_Float16)(acc[2] * inv), (_Float16)(acc[3] * inv)};
   *reinterpret_cast<v4h*>(O + row * D + 4 * c) = out;
+}
+
+template <int D>
+static int launch_merge(const float* part_o, const float* part_ml, void* O, int nparts, int Sq, long long rows, hipStream_t s) {
+  constexpr int units = 256 / (D / 4);
+  int slices = 1;
+  while (slices * 4 < nparts && slices * 2 <= units) slices *= 2;
+  const int rb = units / slices;
+  hipLaunchKernelGGL(attn_merge_kernel<D>, dim3((unsigned)((rows + rb - 1) / rb)), dim3(256), 0, s, part_o, part_ml, (_Float16*)O, nparts,
+                     slices, Sq, rows);
+  return check_launch("attn_merge_kernel");
 }
 
 // How many parts the keys are cut into (1: no split).  A grid of 128-row query blocks that fills less than half the
 // chip, with enough keys that every part keeps at least four tiles.
-static int fa_split_parts(long long bh, int Sq, int Skv, int cus, int* part_keys) {
+static int fa_split_parts(long long bh, int Sq, int Skv, int D, int cus, int* part_keys) {
   *part_keys = Skv;
+  if (Sq <= kDecodeQueries) return decode_parts(bh, Skv, D, cus, part_keys);
   const long long blocks = (long long)((Sq + 127) / 128) * bh;
   if (blocks * 2 > cus || Skv < 2048) return 1;
   long long want = std::min<long long>(std::min<long long>(cus / blocks, 64), Skv / (4 * FA_KT));
@@ -1029,6 +1091,14 @@ static size_t fa_split_bytes(long long bh, int Sq, int D, int nparts) {
 template <int D>
 static int launch_fa_split(const void* Q, const void* K, const void* V, void* O, int BH, int Sq, int Skv, float scale, int nparts,
                            int part_keys, float* ws, int lds_max, hipStream_t s) {
+  float* part_o = ws;
+  float* part_ml = ws + (size_t)nparts * BH * Sq * D;
+  const long long rows = (long long)BH * Sq;
+  if (Sq <= kDecodeQueries) {
+    const int rc = launch_decode(Q, K, V, O, BH, Sq, Skv, D, scale, nparts, part_keys, part_o, part_ml, s);
+    if (rc) return rc;
+    return launch_merge<D>(part_o, part_ml, O, nparts, Sq, rows, s);
+  }
   constexpr int WAVES = 4;
   const size_t lds = (size_t)3 * FaLayout<D>::KTB + (size_t)2 * FaLayout<D>::VTB;
   if ((int)lds > lds_max) return fail(FTK_ERR_UNSUPPORTED_SHAPE, "ftk_flash_attn_ws_f16: needs %zu bytes of LDS", lds);
@@ -1042,17 +1112,12 @@ static int launch_fa_split(const void* Q, const void* K, const void* V, void* O,
   const int nqb = (Sq + WAVES * 32 - 1) / (WAVES * 32);
   const long long total = (long long)nqb * BH * nparts;
   if (total > 0x7fffffffLL) return fail(FTK_ERR_UNSUPPORTED_SHAPE, "ftk_flash_attn_ws_f16: grid too large");
-  float* part_o = ws;
-  float* part_ml = ws + (size_t)nparts * BH * Sq * D;
   hipLaunchKernelGGL((flash_attn_kernel<D, 1, WAVES, 1, false, true, true>), dim3((unsigned)total), dim3(WAVES * 64), lds, s,
                      (const _Float16*)Q, (const _Float16*)K, (const _Float16*)V, (_Float16*)O, Sq, Skv, scale * 1.4426950408889634f, nqb,
                      (long long*)nullptr, 0, nparts, part_keys, part_o, part_ml);
   int rc = check_launch("flash_attn_kernel (key parts)");
   if (rc) return rc;
-  const long long rows = (long long)BH * Sq;
-  const long long threads = rows * (D / 4);
-  hipLaunchKernelGGL(attn_merge_kernel<D>, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, s, part_o, part_ml, (_Float16*)O, nparts, Sq, rows);
-  return check_launch("attn_merge_kernel");
+  return launch_merge<D>(part_o, part_ml, O, nparts, Sq, rows, s);
 }
 
 // Tuning hook: FTK_FA_VARIANT=1|3 pins the tiling variant (read once).
@@ -1087,7 +1152,7 @@ extern "C" size_t ftk_flash_attn_f16_workspace_bytes(int B, int Hd, int Sq, int 
   const DeviceProps* dp = nullptr;
   const int cus = device_props(&dp) == FTK_OK ? dp->cus : 256;   // without a device: the part this library is written for
   int keys = 0;
-  const int nparts = fa_split_parts((long long)B * Hd, Sq, Skv, cus, &keys);
+  const int nparts = fa_split_parts((long long)B * Hd, Sq, Skv, D, cus, &keys);
   return nparts > 1 ? fa_split_bytes((long long)B * Hd, Sq, D, nparts) : 0;
 }
 
@@ -1101,7 +1166,7 @@ extern "C" int ftk_flash_attn_ws_f16(const void* Q, const void* K, const void* V
     if (rc) return rc;
     int keys = 0;
     const long long bh = (long long)B * Hd;
-    const int nparts = fa_split_parts(bh, Sq, Skv, dp->cus, &keys);
+    const int nparts = fa_split_parts(bh, Sq, Skv, D, dp->cus, &keys);
     if (nparts > 1 && workspace_bytes >= fa_split_bytes(bh, Sq, D, nparts) && reinterpret_cast<uintptr_t>(workspace) % 16 == 0) {
       hipStream_t s = (hipStream_t)stream;
       float* ws = reinterpret_cast<float*>(workspace);
@@ -1130,6 +1195,7 @@ extern "C" int ftk_flash_attn_f16(const void* Q, const void* K, const void* V, v
   int rc = device_props(&dp);
   if (rc) return rc;
   hipStream_t s = (hipStream_t)stream;
+  if (Sq <= kDecodeQueries) return launch_decode(Q, K, V, O, (int)bh, Sq, Skv, D, scale, 1, Skv, nullptr, nullptr, s);
   // Variant: 0 = choose by problem size, 1 = 4 waves x 32 query rows (interleaved kernel), 3 = 8 waves x 32 query rows.
   // Eight waves (two per SIMD; K / V tiles shared by 256 rows) whenever 256-row blocks fill the chip, and also on
   // smaller grids once there are 512 keys or more: measured on MI355X at B2 H12 S2048 D64 33 against 49 us, B1 H16 S2048

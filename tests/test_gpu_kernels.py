@@ -1083,6 +1083,28 @@ def test_flash_attention_split_over_the_keys(core, B, Hd, Sq, Skv, D):
     assert int(core.lib.ftk_flash_attn_f16_workspace_bytes(8, 16, 2048, 2048, 128)) == 0
 
 
+@pytest.mark.parametrize('B,Hd,Sq,Skv,D', [
+    (1, 1, 1, 1, 32),              # three waves without a key
+    (1, 3, 16, 33, 64),            # the last row of queries; a tile and one key
+    (2, 2, 4, 31, 96),
+    (1, 2, 15, 128, 128),          # a tile for each wave
+    (1, 2, 3, 1153, 96),           # parts of unequal length, a wave with one key more than a tile
+    (3, 90, 1, 300, 64),           # more heads than the chip takes at once, no parts
+    (1, 1, 16, 9000, 128),         # as many parts as the merge takes
+    (1, 5, 2, 4097, 32),
+])
+def test_flash_attention_few_queries(core, B, Hd, Sq, Skv, D):
+    """At most 16 queries a head: the waves of a workgroup cut the keys.  Against float64; the weights are rounded to
+    fp16 before the second product (2^-11 of each), and so is O."""
+    rng = np.random.default_rng(29)
+    Q, K, V = (rng.standard_normal((B, Hd, s, D)).astype(np.float16) for s in (Sq, Skv, Skv))
+    K[..., Skv // 2:, :] *= 2                                            # the running maximum moves on the way
+    ref = ko.attention(Q, K, V, D ** -0.5)
+    for split in (True, False):
+        O = core.flash_attention(dev(Q), dev(K), dev(V), D ** -0.5, split_keys=split)
+        assert ko.max_rel_err(O.float().cpu().numpy(), ref) <= F16_TOL
+
+
 F32_ATTN_TOL = 1e-4      # the fp32 path's bound; the split products are expected two orders inside it
 
 
