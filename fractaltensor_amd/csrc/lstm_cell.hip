@@ -29,6 +29,7 @@
 #include <vector>
 
 #include "ftk_common.h"
+#include "tile_loop.h"
 
 namespace ftk {
 
@@ -570,6 +571,128 @@ __global__ __launch_bounds__(WAVES * 64, 8 / WAVES) void lstm_cell_f16_kernel(Ce
   }
 }
 
+// ------------------------------------------------ packed fp16 cells, whole tiles
+// Where tile_product finds the operands of a cell: A's row is x_t, then h_{t-d}, each H long (whole pairs of chunks); Bm is
+// a unit block's packed weights, a chunk 16 KB in a row.
+struct CellSource {
+  unsigned a_voff[8], b_voff[4];
+  unsigned a_back[2];                        // never used: the contraction has whole pairs
+  const char *a_next, *b_next, *h_first;     // h_first: this wave's first row of h
+  int nch, npairs, x_pairs, a_idx, b_idx;
+  template <typename Main>
+  __device__ __forceinline__ void a_advance(Main) {
+    if (Main::value || a_idx + 1 < npairs) {
+      ++a_idx;
+      a_next = a_idx == x_pairs ? h_first : a_next + 128;
+    }
+  }
+  template <typename Main>
+  __device__ __forceinline__ void b_advance(Main) {
+    if (Main::value || b_idx + 1 < nch) {
+      ++b_idx;
+      b_next += G_BST;
+    }
+  }
+  __device__ __forceinline__ void left_main_loop(int) {}
+  __device__ __forceinline__ bool a_is_half() const { return false; }
+};
+
+// The cells of lstm_cell_f16_kernel<packed> for I = H, a multiple of 64: 256 batch rows x 64 units of a cell on the loop
+// of the plain product, one wave per SIMD with 128 x 128 outputs.  Bound by the matrix pipe and the LDS reads that feed
+// it: with 128 x 64 outputs to a wave a k step read 12 KB of fragments for 16 MFMAs instead of 16 KB for 32, and two waves
+// per SIMD stood at the same barrier.  L 32 T 64 B 256 H 1024: 12.70 -> 11.63 ms for the stack.
+__global__ __launch_bounds__(256, 1) void lstm_cell_tile_kernel(CellListH list, int B, int H) {
+  const int nub = H / 64, nrb = (B + GT - 1) / GT;
+  const int slot = (int)(blockIdx.x >> 3), cell = (int)(blockIdx.x & 7) + 8 * (slot / (nub * nrb));   // a cell's tiles on one XCD
+  if (cell >= list.n) return;
+  const CellDescH cd = list.cells[cell];
+  const int Bc = cd.rows > 0 ? cd.rows : B;  // rows of this cell
+  const int ub = slot % nub, rb = (slot / nub) % nrb;
+  if (rb * GT >= Bc) return;  // a row block past the live rows of this step
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wr = wave >> 1, wc = wave & 1;
+  const int j = lane & 31, hh = lane >> 5;
+
+  CellSource src;
+  src.nch = (cd.h_prev ? 2 * H : H) / GK;
+  src.npairs = src.nch >> 1;
+  src.x_pairs = H / (2 * GK);
+  src.a_idx = src.b_idx = 0;
+  const int row0 = min(rb * GT + 64 * wave, Bc - 1);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {   // rows past the end of the batch repeat the last row; they are never stored
+    const int row = min(rb * GT + 64 * wave + 8 * i + (lane >> 3), Bc - 1);
+    src.a_voff[i] = (unsigned)(row - row0) * (unsigned)(2 * H) + (unsigned)(((lane & 7) ^ (4 * (i & 1) + (lane >> 4))) * 16);
+    asm volatile("" : "+v"(src.a_voff[i]));   // kept in registers, not formed again at every copy
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) src.b_voff[i] = 1024u * i + 16u * lane;   // the packed rows hold their chunks in the slots' order
+  src.a_back[0] = src.a_back[1] = 0;
+  src.a_next = reinterpret_cast<const char*>(cd.x + (size_t)row0 * H);
+  src.h_first = reinterpret_cast<const char*>(cd.h_prev + (size_t)row0 * H);   // (not looked at without an h)
+  src.b_next = reinterpret_cast<const char*>(cd.WU) + (size_t)ub * 2 * H * G_ROWB + wave * 4096;
+  v16f acc[4][4];
+  tile_product(src, src.nch, acc);
+
+  // Lane (row j, half hh) holds the four gates of units 4 hh .. + 3 of each of its unit groups.  h and c move 16 bytes at
+  // a time: of two neighbouring groups the lower lane moves the first's eight units, the upper lane the second's.
+  auto swap_halves = [](v2u& first, v2u& second) __attribute__((always_inline)) {
+#pragma unroll
+    for (int w = 0; w < 2; ++w)   // upper lanes' first <-> lower lanes' second
+      asm volatile("s_nop 1\n\tv_permlane32_swap_b32_e32 %0, %1\n\ts_nop 1" : "+v"(first[w]), "+v"(second[w]));
+  };
+  const _Float16* c_prev = reinterpret_cast<const _Float16*>(cd.c_prev);
+#pragma unroll
+  for (int np = 0; np < 2; ++np) {
+    const int u0 = ub * 64 + 64 / 2 * wc + 16 * np;   // the first unit of the two groups
+    v4f bias[2][4];
+#pragma unroll
+    for (int n = 0; n < 2; ++n)
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+        bias[n][g] = cd.bias ? *reinterpret_cast<const v4f*>(cd.bias + (size_t)g * H + u0 + 8 * n + 4 * hh) : v4f{0.f, 0.f, 0.f, 0.f};
+    v4u cw[4];
+#pragma unroll
+    for (int rt = 0; rt < 4; ++rt) {
+      const int row = min(rb * GT + 128 * wr + 32 * rt + j, Bc - 1);
+      cw[rt] = v4u{0, 0, 0, 0};
+      if (c_prev) cw[rt] = *reinterpret_cast<const v4u*>(c_prev + (size_t)row * H + u0 + 8 * hh);
+    }
+#pragma unroll
+    for (int rt = 0; rt < 4; ++rt) {
+      const int row = rb * GT + 128 * wr + 32 * rt + j;
+      v2u cp[2] = {v2u{cw[rt][0], cw[rt][1]}, v2u{cw[rt][2], cw[rt][3]}}, ho[2], co[2];
+      swap_halves(cp[0], cp[1]);
+#pragma unroll
+      for (int n = 0; n < 2; ++n) {
+        const v16f& s = acc[rt][2 * np + n];
+        const v4h c16 = __builtin_bit_cast(v4h, cp[n]);
+        v4h hv, cv;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const float ig = sigmoid_f(s[r] + bias[n][0][r]);
+          const float fg = sigmoid_f(s[4 + r] + bias[n][1][r]);
+          const float og = sigmoid_f(s[8 + r] + bias[n][2][r]);
+          const float cand = tanh_f(s[12 + r] + bias[n][3][r]);
+          const float c = fg * (float)c16[r] + ig * cand;
+          cv[r] = (_Float16)c;
+          hv[r] = (_Float16)(og * tanh_f(c));
+        }
+        co[n] = __builtin_bit_cast(v2u, cv);
+        ho[n] = __builtin_bit_cast(v2u, hv);
+      }
+      swap_halves(co[0], co[1]);
+      swap_halves(ho[0], ho[1]);
+      if (row < Bc) {
+        const size_t at = (size_t)row * H + u0 + 8 * hh;
+        *reinterpret_cast<v4u*>(reinterpret_cast<_Float16*>(cd.c) + at) = v4u{co[0][0], co[0][1], co[1][0], co[1][1]};
+        *reinterpret_cast<v4u*>(reinterpret_cast<_Float16*>(cd.h) + at) = v4u{ho[0][0], ho[0][1], ho[1][0], ho[1][1]};
+      }
+    }
+  }
+}
+
 // ------------------------------------------------ split flavour, four tiles per chunk
 // The split products of a chunk from one copy of each plane: a stage holds the four tiles [x value][x
 // remainder][w value][w remainder] of a 32-row chunk (64 KB at 64 hidden units per workgroup), and the three
@@ -835,8 +958,20 @@ static int launch_cells(const CellListH& list, int B, int I, int H, hipStream_t 
   if (list.packed == 2)  // split products, three chunks in a row
     return cell_unit_block(H) == 64 ? launch_cells_f16<true, 8, true>(list, B, I, H, s)
                                     : launch_cells_f16<true, 4, true>(list, B, I, H, s);
-  if (cell_unit_block(H) == 64)
-    return list.packed ? launch_cells_f16<true, 8, false>(list, B, I, H, s) : launch_cells_f16<false, 8, false>(list, B, I, H, s);
+  if (cell_unit_block(H) == 64) {
+    if (!list.packed) return launch_cells_f16<false, 8, false>(list, B, I, H, s);
+    if (I != H) return fail(FTK_ERR_UNSUPPORTED_SHAPE, "packed cells need I = H, got %d and %d", I, H);
+    static DeviceOnce attr_once;
+    unsigned attr_bit;
+    if (attr_once.pending(&attr_bit)) {
+      FTK_HIP(hipFuncSetAttribute((const void*)lstm_cell_tile_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, G_LDS));
+      attr_once.done(attr_bit);
+    }
+    const int groups = (list.n + 7) / 8;
+    dim3 grid(8 * groups * (H / 64) * ((B + GT - 1) / GT));
+    hipLaunchKernelGGL(lstm_cell_tile_kernel, grid, dim3(256), G_LDS, s, list, B, H);
+    return check_launch("lstm_cell_tile_kernel");
+  }
   return list.packed ? launch_cells_f16<true, 4, false>(list, B, I, H, s) : launch_cells_f16<false, 4, false>(list, B, I, H, s);
 }
 

@@ -1445,3 +1445,28 @@ def test_stacked_lstm_exchange_kernel(core, half, H, L, T, B, dil):
                 assert ko.max_rel_err(t, ref.astype(np.float32)[:, ref_live]) <= 1e-2, what
             else:
                 assert_lstm_close(torch.from_numpy(t), ref[:, ref_live], what)
+
+
+@pytest.mark.parametrize('H,L,T,B,dil', [
+    (64, 2, 3, 1, None),                   # one pair of chunks without an h, two with one
+    (64, 3, 4, 256, [1, 2, 3]),
+    (128, 1, 2, 257, None),                # a second row block of one row
+    (192, 2, 3, 63, None),
+    (320, 2, 3, 255, None),                # 10 and 20 chunks: the unrolled loop's boundary
+    (576, 1, 2, 40, None),                 # 18 and 36 chunks, the h rows start inside the unrolled loop
+    (704, 2, 2, 300, None),
+])
+def test_streamed_f16_cells_whole_tiles(core, H, L, T, B, dil):
+    """fp16 stacks whose cells stream their weights, 256 rows x 64 units to a workgroup: sizes around the loop's pairs of
+    chunks and the row blocks, dense and ragged, against the oracle (h and c carry an fp16 rounding a step)."""
+    xs, WU, bs = lstm_inputs(78, L, T, B, H, 1.0 / np.sqrt(H))
+    xs, WU = xs.astype(np.float16), WU.astype(np.float16)
+    rows = sorted({0, B // 2, B - 1})
+    hr, cr = ko.stacked_lstm_f16(xs[:, rows], WU, bs, dil)
+    lens = np.maximum(1, T - (np.arange(B) * T) // B)
+    for active in (None, [int((lens > t).sum()) for t in range(T)]):
+        h, c = core.stacked_lstm_f16(dev(xs), dev(WU), dev(bs), dilations=dil, active_rows=active)
+        live = np.ones((T, len(rows)), bool) if active is None else np.arange(T)[:, None] < lens[rows][None, :]
+        for t, ref, what in ((h, hr, 'h'), (c, cr, 'c')):
+            got = t[:, :, rows].float().cpu().numpy()
+            assert ko.max_rel_err(got[:, live], ref.astype(np.float32)[:, live]) <= 1e-2, what
