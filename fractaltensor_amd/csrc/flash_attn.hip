@@ -56,6 +56,14 @@ int decode_parts(long long bh, int Skv, int D, int cus, int* part_keys);
 int launch_decode(const void* Q, const void* K, const void* V, void* O, int BH, int Sq, int Skv, int D, float scale, int nparts,
                   int part_keys, float* part_o, float* part_ml, hipStream_t s);
 
+// LDS layout of a tile without padding, for head size 128 with two key groups (padded, their ten tiles take 186 KB): K
+// row r keeps 16-byte chunk c in slot c ^ (r & 15), V row r its 64-byte group g in g ^ (r & 3).
+template <int D>
+struct FaSwizzled {
+  static constexpr int KRS = 2 * D, VRS = 2 * D, KTB = FA_KT * KRS, VTB = FA_KT * VRS;
+};
+constexpr bool fa_swizzled(int D, int KG) { return D == 128 && KG == 2; }
+
 constexpr float FA_TAU = 8.0f;     // slack (in powers of two) before the running maximum is moved
 constexpr float FA_PMAX = 32768.0f;  // phase-alternating kernel: a lane's sum of exponentials above this moves the reference
 constexpr int FA_TRACE_TILES = 256;
@@ -73,8 +81,11 @@ __device__ long long fa_trace_buf[FA_TRACE_TILES * 6];
 // PART: the workgroup takes one contiguous range of the keys (part_keys of them, a multiple of the tile) and leaves
 // its unnormalised accumulators, reference maximum and sum of exponentials in part_o / part_ml for attn_merge_kernel:
 // small grids with many keys are split over the keys so that they fill the chip.
-template <int D, int QT, int WAVES, int MINB, bool TRACE, bool RAG, bool PART = false>
-__global__ __launch_bounds__(WAVES * 64, MINB) void flash_attn_kernel(const _Float16* __restrict__ Q,
+// KG == 2: the workgroup has two groups of WAVES waves for the same query rows.  Each walks half of the keys with tiles of
+// its own in LDS, and the first takes in the second's result at the end: two waves per SIMD where the grid of query
+// blocks does not fill the chip, each with half of the chain of tiles (see launch_fa's callers for where that pays).
+template <int D, int QT, int WAVES, int MINB, bool TRACE, bool RAG, bool PART = false, int KG = 1>
+__global__ __launch_bounds__(WAVES * KG * 64, MINB) void flash_attn_kernel(const _Float16* __restrict__ Q,
                                                          const _Float16* __restrict__ K,
                                                          const _Float16* __restrict__ V,
                                                          _Float16* __restrict__ O, int Sq, int Skv_all,
@@ -83,7 +94,9 @@ __global__ __launch_bounds__(WAVES * 64, MINB) void flash_attn_kernel(const _Flo
                                                          int nparts = 1, int part_keys = 0,
                                                          float* __restrict__ part_o = nullptr,
                                                          float* __restrict__ part_ml = nullptr) {
-  using L = FaLayout<D>;
+  constexpr bool SWZ = fa_swizzled(D, KG);
+  using L = typename std::conditional<SWZ, FaSwizzled<D>, FaLayout<D>>::type;
+  static_assert(KG == 1 || (KG == 2 && QT == 1), "two key groups, one query tile a wave");
   constexpr int DS = D / 16;  // k steps of S^T
   constexpr int DT = D / 32;  // d tiles of O^T
   constexpr int RB = 2 * D;   // bytes per K or V row in global memory
@@ -91,21 +104,21 @@ __global__ __launch_bounds__(WAVES * 64, MINB) void flash_attn_kernel(const _Flo
   constexpr int KCP = (KTB / 1024 + WAVES - 1) / WAVES;  // 1 KB copies per wave per K tile (upper bound)
   constexpr int VCP = (VTB / 1024 + WAVES - 1) / WAVES;
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
-  unsigned char* const Kb = smem;            // [3][KTB]
-  unsigned char* const Vb = smem + 3 * KTB;  // [2][VTB]
-
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  // wave index as a scalar, so that LDS copy destinations are provably wave-uniform
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // wave index (within its key group) as a scalar, so that LDS copy destinations are provably wave-uniform
+  const int wave = __builtin_amdgcn_readfirstlane((tid >> 6) % WAVES);
+  const int group = KG == 1 ? 0 : __builtin_amdgcn_readfirstlane((tid >> 6) / WAVES);
+  constexpr int GROUP_LDS = 3 * KTB + 2 * VTB;
+  unsigned char* const Kb = smem + group * GROUP_LDS;   // [3][KTB]
+  unsigned char* const Vb = Kb + 3 * KTB;               // [2][VTB]
+
   const int j = lane & 31;
   const int hh = lane >> 5;
   // One-dimensional grid of nqb query blocks x (batch*heads).  The hardware
   // deals workgroups round-robin over the 8 XCDs; remap so that the query
   // blocks of one head run on one XCD and share its L2 copy of K and V.
-  int id = blockIdx.x;
-  const int total = gridDim.x;
-  if ((total & 7) == 0) id = (blockIdx.x & 7) * (total >> 3) + (blockIdx.x >> 3);
+  int id = xcd_consecutive(blockIdx.x, gridDim.x);
   int part = 0;
   if constexpr (PART) {
     part = id % nparts;
@@ -114,8 +127,12 @@ __global__ __launch_bounds__(WAVES * 64, MINB) void flash_attn_kernel(const _Flo
   const int bh = id / nqb;
   const int qb = id - bh * nqb;
   const int q_base = qb * (WAVES * 32 * QT) + wave * (32 * QT);
-  const int key_first = PART ? part * part_keys : 0;
-  const int Skv = PART ? min(part_keys, Skv_all - key_first) : Skv_all;   // the keys this workgroup sees
+  const int key_wg = PART ? part * part_keys : 0;
+  const int Skv_wg = PART ? min(part_keys, Skv_all - key_wg) : Skv_all;   // the keys this workgroup sees
+  // the first group has the first half of the tiles, one more than the second when they are odd (never fewer than two in all)
+  const int first_tiles = ((Skv_wg + FA_KT - 1) / FA_KT + 1) / 2;
+  const int key_first = key_wg + group * first_tiles * FA_KT;
+  const int Skv = KG == 1 ? Skv_wg : group == 0 ? first_tiles * FA_KT : Skv_wg - first_tiles * FA_KT;   // the keys this group sees
 
   const _Float16* Qg = Q + (size_t)bh * Sq * D;
   const _Float16* Kg = K + ((size_t)bh * Skv_all + key_first) * D;
@@ -158,13 +175,15 @@ __global__ __launch_bounds__(WAVES * 64, MINB) void flash_attn_kernel(const _Flo
   for (int i = 0; i < KCP; ++i) {
     const int x = 1024 * (wave + WAVES * i) + 16 * lane;
     const int row = min(x / KRS, FA_KT - 1), col = x % KRS;
-    k_src[i] = row * RB + (col < RB ? col : 0);
+    if constexpr (SWZ) k_src[i] = row * RB + (col ^ (16 * (row & 15)));
+    else k_src[i] = row * RB + (col < RB ? col : 0);
   }
 #pragma unroll
   for (int i = 0; i < VCP; ++i) {
     const int x = 1024 * (wave + WAVES * i) + 16 * lane;
     const int row = min(x / VRS, FA_KT - 1), col = x % VRS;
-    v_src[i] = row * RB + (col < RB ? col : 0);
+    if constexpr (SWZ) v_src[i] = row * RB + (col ^ (64 * (row & 3)));
+    else v_src[i] = row * RB + (col < RB ? col : 0);
   }
   // copy i (of this wave's share) of K tile kt into the K buffer at dst; no-op past the wave's last copy
   auto copy_k = [&](unsigned char* dst, int kt, auto i_c) __attribute__((always_inline)) {
@@ -215,10 +234,19 @@ __global__ __launch_bounds__(WAVES * 64, MINB) void flash_attn_kernel(const _Flo
   // ---- fragment addresses: one lane-dependent base per tile kind, everything
   // else (half tile, contraction step, d tile) is an immediate offset.
   // K: lane (j, hh) reads row 32*k2 + j, bytes [32s + 16hh, +16)
-  const int k_lane = j * KRS + 16 * hh;
+  // (swizzled rows: the 16-byte chunks, and the 64-byte groups of V, change places by row, so there is an offset per
+  // step and d tile)
+  const int k_lane = j * KRS + (SWZ ? 0 : 16 * hh);
   // V: lane hands in (key a = (lane&15)>>2, column chunk b = lane&3) of the 16-column block
   // dhalf = (lane>>4)&1 of d tile dt, keys 4*hh + a (+ constant) of the step
   const int v_lane = (4 * hh + ((lane & 15) >> 2)) * VRS + 32 * ((lane >> 4) & 1) + 8 * (lane & 3);
+  unsigned k_swz[SWZ ? DS : 1], v_swz[SWZ ? DT : 1];
+  if constexpr (SWZ) {
+#pragma unroll
+    for (int s = 0; s < DS; ++s) k_swz[s] = (unsigned)(((2 * s + hh) ^ (j & 15)) * 16);
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) v_swz[dt] = (unsigned)((dt ^ ((lane & 15) >> 2)) * 64);
+  }
 
   const int ntiles = (Skv + FA_KT - 1) / FA_KT;
 
@@ -226,11 +254,14 @@ __global__ __launch_bounds__(WAVES * 64, MINB) void flash_attn_kernel(const _Flo
   typedef short v8s __attribute__((ext_vector_type(8)));
   // kbase / vbase: LDS address of the half tile plus the lane's base
   auto read_k = [&](const unsigned char* kbase, int s) __attribute__((always_inline)) {
-    return *reinterpret_cast<const v8h*>(kbase + 32 * s);
+    if constexpr (SWZ) return *reinterpret_cast<const v8h*>(kbase + k_swz[s]);
+    else return *reinterpret_cast<const v8h*>(kbase + 32 * s);
   };
   // A-operand of the PV product for (step s, d tile dt) of one half tile
   auto read_v = [&](const unsigned char* vbase, int s, int dt) __attribute__((always_inline)) {
-    const unsigned char* p0 = vbase + 16 * s * VRS + 64 * dt;
+    const unsigned char* p0 = vbase + 16 * s * VRS;
+    if constexpr (SWZ) p0 += v_swz[dt];
+    else p0 += 64 * dt;
     const v4s lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s*)(p0));
     const v4s hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s*)(p0 + 8 * VRS));
     const v8s both = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
@@ -433,6 +464,7 @@ __global__ __launch_bounds__(WAVES * 64, MINB) void flash_attn_kernel(const _Flo
 #pragma unroll
       for (int r = 1; r < 16; ++r) m = fmaxf(m, sa[qt][r]);
       m = max_with_other_half(m);
+      if (KG == 2 && m == -INFINITY) m = 0.0f;   // no score yet: the group's share must come out as nothing, not as a NaN
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         sa[qt][r] -= m;
@@ -454,7 +486,7 @@ __global__ __launch_bounds__(WAVES * 64, MINB) void flash_attn_kernel(const _Flo
     // A wave is held at issue while its copy instructions queue up in the memory pipeline.  With two waves
     // per SIMD the two take turns: the first issues its copies when the step begins, the second after the
     // first half tile, so that one of them always has MFMAs to issue.
-    const bool copy_first = WAVES < 8 || wave < WAVES / 2;
+    const bool copy_first = KG == 2 ? group == 0 : WAVES < 8 || wave < WAVES / 2;
     if (copy_first) {
       if (kt + 2 < ntiles) copy_k_all(Kb + kfree, kt + 2);
       if (kt + 1 < ntiles) copy_v_all(Vb + vnext, kt + 1);
@@ -491,6 +523,42 @@ __global__ __launch_bounds__(WAVES * 64, MINB) void flash_attn_kernel(const _Flo
   } else {
     if (ntiles > 1) step(ntiles - 2, std::true_type{}, std::false_type{});
     step(ntiles - 1, std::false_type{}, std::false_type{});
+  }
+
+  if constexpr (KG == 2) {
+    if (group == 1 && ntiles < first_tiles) __syncthreads();   // the first group's last tile
+    // the second group leaves its accumulators, reference and sum in its part of LDS, by lane; the first takes them in
+    // by the rule of an online softmax
+    unsigned char* const other = smem + GROUP_LDS;
+    v4f* const oo = reinterpret_cast<v4f*>(other) + wave * (DT * 4 * 64) + lane;
+    float2* const oml = reinterpret_cast<float2*>(other + WAVES * (DT * 4 * 64 * 16)) + wave * 64 + lane;
+    static_assert(WAVES * (DT * 4 * 64 * 16 + 64 * 8) <= GROUP_LDS, "the second group's result fits its tiles' place");
+    if (group == 1) {
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+          oo[(4 * dt + g) * 64] = v4f{oacc[0][dt][4 * g], oacc[0][dt][4 * g + 1], oacc[0][dt][4 * g + 2], oacc[0][dt][4 * g + 3]};
+      *oml = make_float2(-nref[0][0], l_run[0] + __shfl_xor(l_run[0], 32));
+    }
+    __syncthreads();
+    if (group == 1) return;
+    const float2 ml = *oml;
+    const float l_mine = l_run[0] + __shfl_xor(l_run[0], 32), m_mine = -nref[0][0];
+    const float m = !(ml.y > 0.0f) ? m_mine : !(l_mine > 0.0f) ? ml.x : fmaxf(m_mine, ml.x);
+    const float wm = l_mine == 0.0f ? 0.0f : __builtin_amdgcn_exp2f(m_mine - m);
+    const float wo = ml.y == 0.0f ? 0.0f : __builtin_amdgcn_exp2f(ml.x - m);
+    l_run[0] = hh == 0 ? wm * l_mine + wo * ml.y : 0.0f;   // (the lanes' shares are added up below)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) nref[0][r] = -m;
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const v4f o = oo[(4 * dt + g) * 64];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) oacc[0][dt][4 * g + k] = wm * oacc[0][dt][4 * g + k] + wo * o[k];
+      }
   }
 
   // ---- normalise and store.  A lane holds d = 32dt + 8g + 4*half + r of its row: 8-byte pieces scattered over
@@ -602,9 +670,7 @@ __global__ __launch_bounds__(512, 1) void flash_attn_pp_kernel(const _Float16* _
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int group = wave >> 2, cw = wave & 3;
   const int j = lane & 31, hh = lane >> 5;
-  int id = blockIdx.x;
-  const int total = gridDim.x;
-  if ((total & 7) == 0) id = (blockIdx.x & 7) * (total >> 3) + (blockIdx.x >> 3);
+  int id = xcd_consecutive(blockIdx.x, gridDim.x);
   const int bh = id / nqb;
   const int qb = id - bh * nqb;
   const int q_base = qb * 256 + wave * 32;
@@ -946,20 +1012,21 @@ static int launch_fa_pp(const void* Q, const void* K, const void* V, void* O, in
 }
 
 
-template <int D, int QT, int WAVES, int MINB>
+template <int D, int QT, int WAVES, int MINB, int KG = 1>
 static int launch_fa(const void* Q, const void* K, const void* V, void* O, int BH, int Sq, int Skv, float scale,
                      int lds_max, hipStream_t s) {
-  const size_t lds = (size_t)3 * FaLayout<D>::KTB + (size_t)2 * FaLayout<D>::VTB;  // three K tiles, two V tiles
+  using L = typename std::conditional<fa_swizzled(D, KG), FaSwizzled<D>, FaLayout<D>>::type;
+  const size_t lds = (size_t)KG * (3 * L::KTB + 2 * L::VTB);  // three K tiles, two V tiles
   if ((int)lds > lds_max) return fail(FTK_ERR_UNSUPPORTED_SHAPE, "ftk_flash_attn_f16: needs %zu bytes of LDS", lds);
   static DeviceOnce attr_once;
   unsigned attr_bit;
   if (attr_once.pending(&attr_bit)) {
-    FTK_HIP(hipFuncSetAttribute((const void*)flash_attn_kernel<D, QT, WAVES, MINB, false, false>,
+    FTK_HIP(hipFuncSetAttribute((const void*)flash_attn_kernel<D, QT, WAVES, MINB, false, false, false, KG>,
                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    FTK_HIP(hipFuncSetAttribute((const void*)flash_attn_kernel<D, QT, WAVES, MINB, false, true>,
+    FTK_HIP(hipFuncSetAttribute((const void*)flash_attn_kernel<D, QT, WAVES, MINB, false, true, false, KG>,
                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
 #ifdef FTK_DEBUG_TRACE
-    FTK_HIP(hipFuncSetAttribute((const void*)flash_attn_kernel<D, QT, WAVES, MINB, true, true>,
+    FTK_HIP(hipFuncSetAttribute((const void*)flash_attn_kernel<D, QT, WAVES, MINB, true, true, false, KG>,
                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
 #endif
     attr_once.done(attr_bit);
@@ -970,18 +1037,18 @@ static int launch_fa(const void* Q, const void* K, const void* V, void* O, int B
   if (total > 0x7fffffffLL) return fail(FTK_ERR_UNSUPPORTED_SHAPE, "ftk_flash_attn_f16: grid too large");
 #ifdef FTK_DEBUG_TRACE
   if (long long* trace = fa_trace_ptr()) {
-    hipLaunchKernelGGL((flash_attn_kernel<D, QT, WAVES, MINB, true, true>), dim3((unsigned)total), dim3(WAVES * 64), lds,
+    hipLaunchKernelGGL((flash_attn_kernel<D, QT, WAVES, MINB, true, true, false, KG>), dim3((unsigned)total), dim3(WAVES * KG * 64), lds,
                        s, (const _Float16*)Q, (const _Float16*)K, (const _Float16*)V, (_Float16*)O, Sq, Skv,
                        scale * 1.4426950408889634f, nqb, trace, fa_trace_wave());
     return check_launch("flash_attn_kernel");
   }
 #endif
   if (Skv % FA_KT)
-    hipLaunchKernelGGL((flash_attn_kernel<D, QT, WAVES, MINB, false, true>), dim3((unsigned)total), dim3(WAVES * 64), lds,
+    hipLaunchKernelGGL((flash_attn_kernel<D, QT, WAVES, MINB, false, true, false, KG>), dim3((unsigned)total), dim3(WAVES * KG * 64), lds,
                        s, (const _Float16*)Q, (const _Float16*)K, (const _Float16*)V, (_Float16*)O, Sq, Skv,
                        scale * 1.4426950408889634f, nqb, (long long*)nullptr, 0);
   else
-    hipLaunchKernelGGL((flash_attn_kernel<D, QT, WAVES, MINB, false, false>), dim3((unsigned)total), dim3(WAVES * 64), lds,
+    hipLaunchKernelGGL((flash_attn_kernel<D, QT, WAVES, MINB, false, false, false, KG>), dim3((unsigned)total), dim3(WAVES * KG * 64), lds,
                        s, (const _Float16*)Q, (const _Float16*)K, (const _Float16*)V, (_Float16*)O, Sq, Skv,
                        scale * 1.4426950408889634f, nqb, (long long*)nullptr, 0);
   return check_launch("flash_attn_kernel");
@@ -1070,16 +1137,30 @@ static int launch_merge(const float* part_o, const float* part_ml, void* O, int 
   return check_launch("attn_merge_kernel");
 }
 
-// How many parts the keys are cut into (1: no split).  A grid of 128-row query blocks that fills less than half the
-// chip, with enough keys that every part keeps at least four tiles.
+// How many parts the keys are cut into (1: no split): the number that makes the sum of both costs least, in microseconds.
+// A workgroup's chain is half of its tiles (two key groups) of about 0.4 + 0.0095 D each (16 tiles of each group: 15 at
+// D = 64, 26 at 128).  Parts cost the merge's launch and its trip through memory, what every part writes and the merge
+// reads at about 2.5 TB/s (8 heads of 64, 2048 queries and keys: 2 parts take 23.2, one 19.3; 128 queries, 4096 keys: 12.5
+// and 30.5).  At most as many workgroups as compute units, at least four tiles to a part.
 static int fa_split_parts(long long bh, int Sq, int Skv, int D, int cus, int* part_keys) {
   *part_keys = Skv;
   if (Sq <= kDecodeQueries) return decode_parts(bh, Skv, D, cus, part_keys);
   const long long blocks = (long long)((Sq + 127) / 128) * bh;
-  if (blocks * 2 > cus || Skv < 2048) return 1;
-  long long want = std::min<long long>(std::min<long long>(cus / blocks, 64), Skv / (4 * FA_KT));
+  const long long most = std::min<long long>(std::min<long long>(cus / blocks, 64), Skv / (4 * FA_KT));
+  const float chain = (float)Skv / (2 * FA_KT) * (0.4f + 0.0095f * (float)D);
+  const float part = (float)(bh * Sq) * (float)(D + 2) * (8.0f / 2.5e6f);
+  float least = chain;
+  int want = 1;
+  for (int p = 2; p <= most; ++p) {
+    const float cost = chain / (float)p + 6.0f + part * (float)p;
+    if (cost < least) {
+      least = cost;
+      want = p;
+    }
+  }
   if (want < 2) return 1;
-  const int keys = (int)(((Skv + want - 1) / want + FA_KT - 1) / FA_KT * FA_KT);
+  int keys = (int)(((Skv + want - 1) / want + FA_KT - 1) / FA_KT * FA_KT);
+  while ((Skv - 1) % keys < FA_KT) keys += FA_KT;   // the last part has more than a tile too: a key group walks at least one
   *part_keys = keys;
   return (Skv + keys - 1) / keys;
 }
@@ -1099,20 +1180,21 @@ static int launch_fa_split(const void* Q, const void* K, const void* V, void* O,
     if (rc) return rc;
     return launch_merge<D>(part_o, part_ml, O, nparts, Sq, rows, s);
   }
-  constexpr int WAVES = 4;
-  const size_t lds = (size_t)3 * FaLayout<D>::KTB + (size_t)2 * FaLayout<D>::VTB;
+  constexpr int WAVES = 4, KG = 2;
+  using L = typename std::conditional<fa_swizzled(D, KG), FaSwizzled<D>, FaLayout<D>>::type;
+  const size_t lds = (size_t)KG * (3 * L::KTB + 2 * L::VTB);
   if ((int)lds > lds_max) return fail(FTK_ERR_UNSUPPORTED_SHAPE, "ftk_flash_attn_ws_f16: needs %zu bytes of LDS", lds);
   static DeviceOnce attr_once;
   unsigned attr_bit;
   if (attr_once.pending(&attr_bit)) {
-    FTK_HIP(hipFuncSetAttribute((const void*)flash_attn_kernel<D, 1, WAVES, 1, false, true, true>,
+    FTK_HIP(hipFuncSetAttribute((const void*)flash_attn_kernel<D, 1, WAVES, 1, false, true, true, KG>,
                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     attr_once.done(attr_bit);
   }
   const int nqb = (Sq + WAVES * 32 - 1) / (WAVES * 32);
   const long long total = (long long)nqb * BH * nparts;
   if (total > 0x7fffffffLL) return fail(FTK_ERR_UNSUPPORTED_SHAPE, "ftk_flash_attn_ws_f16: grid too large");
-  hipLaunchKernelGGL((flash_attn_kernel<D, 1, WAVES, 1, false, true, true>), dim3((unsigned)total), dim3(WAVES * 64), lds, s,
+  hipLaunchKernelGGL((flash_attn_kernel<D, 1, WAVES, 1, false, true, true, KG>), dim3((unsigned)total), dim3(WAVES * KG * 64), lds, s,
                      (const _Float16*)Q, (const _Float16*)K, (const _Float16*)V, (_Float16*)O, Sq, Skv, scale * 1.4426950408889634f, nqb,
                      (long long*)nullptr, 0, nparts, part_keys, part_o, part_ml);
   int rc = check_launch("flash_attn_kernel (key parts)");
@@ -1126,7 +1208,7 @@ static int fa_variant_override() {
   if (v < 0) {
     const char* e = getenv("FTK_FA_VARIANT");
     v = e ? atoi(e) : 0;
-    if (v != 1 && v != 3) v = 0;
+    if (v < 1 || v > 3) v = 0;
   }
   return v;
 }
@@ -1196,13 +1278,17 @@ extern "C" int ftk_flash_attn_f16(const void* Q, const void* K, const void* V, v
   if (rc) return rc;
   hipStream_t s = (hipStream_t)stream;
   if (Sq <= kDecodeQueries) return launch_decode(Q, K, V, O, (int)bh, Sq, Skv, D, scale, 1, Skv, nullptr, nullptr, s);
-  // Variant: 0 = choose by problem size, 1 = 4 waves x 32 query rows (interleaved kernel), 3 = 8 waves x 32 query rows.
-  // Eight waves (two per SIMD; K / V tiles shared by 256 rows) whenever 256-row blocks fill the chip, and also on
-  // smaller grids once there are 512 keys or more: measured on MI355X at B2 H12 S2048 D64 33 against 49 us, B1 H16 S2048
-  // D128 44 against 50 us, B2 H8 S1024 D128 22.3 against 23.5 us (64 workgroups against 128), B4 H8 S1024 D32 14.6
-  // against 16.7 us; with few keys a launch is its own latency (9.5-10 us either way) and the 128-row blocks, which
-  // spread a short problem over more compute units, are kept (B1 H4 S300 D128: 10.7 against 12.2 us).
+  // Variant: 0 = choose by problem size, 1 = 4 waves x 32 query rows (interleaved kernel), 2 = the same with two key groups,
+  // 3 = 8 waves x 32 query rows.
+  // Two key groups where 128-row blocks are at most one to a compute unit: half of the chain of tiles to each wave, two
+  // waves per SIMD, and half the padding of 256-row blocks (us, against 8 waves and 4 waves: B3 H12 S777x1333 D64 18.6,
+  // 24.1, 27.0; B2 H12 S700 D96 12.4, 17.2, 16.6; B1 H12 S1536 D64 15.0, 21.3, 23.6; B1 H8 S512 D64 7.7, 9.7, 9.8; B1 H16 S2048
+  // D128, exactly one block each, 37, 38.5, 43).  Up to two tiles of keys nothing is gained (B8 H16 S64x100 D128 7.6, 8.0, 6.6).
+  // With more blocks than that, eight waves (two per SIMD; K / V tiles shared by 256 rows) whenever 256-row blocks fill
+  // the chip, and also on smaller grids once there are 512 keys or more (B2 H12 S2048 D64 33 against 49 us); with few
+  // keys a launch is its own latency and the 128-row blocks spread a short problem over more compute units.
   int variant = fa_variant_override();
+  if (variant == 0 && (long long)((Sq + 127) / 128) * bh <= dp->cus && Skv > 2 * FA_KT) variant = 2;
   if (variant == 0) variant = ((long long)((Sq + 255) / 256) * bh >= dp->cus || Skv >= 512) ? 3 : 1;
   const int lds = dp->lds_optin;
   // Grids with enough query blocks for eight waves take the kernel whose two waves per SIMD alternate between matrix
@@ -1210,18 +1296,22 @@ extern "C" int ftk_flash_attn_f16(const void* Q, const void* K, const void* V, v
   // 234 at D = 96, 165 against 180 at D = 64, 98 against 114 at D = 32); the interleaved kernel keeps the 128-row
   // blocks of small grids.
   if (D == 128) {
+    if (variant == 2) return launch_fa<128, 1, 4, 1, 2>(Q, K, V, O, (int)bh, Sq, Skv, scale, lds, s);
     if (variant == 1) return launch_fa<128, 1, 4, 1>(Q, K, V, O, (int)bh, Sq, Skv, scale, lds, s);
     return launch_fa_pp<128>(Q, K, V, O, (int)bh, Sq, Skv, scale, lds, s);
   }
   if (D == 96) {
+    if (variant == 2) return launch_fa<96, 1, 4, 1, 2>(Q, K, V, O, (int)bh, Sq, Skv, scale, lds, s);
     if (variant == 1) return launch_fa<96, 1, 4, 1>(Q, K, V, O, (int)bh, Sq, Skv, scale, lds, s);
     return launch_fa_pp<96>(Q, K, V, O, (int)bh, Sq, Skv, scale, lds, s);
   }
   if (D == 64) {
+    if (variant == 2) return launch_fa<64, 1, 4, 1, 2>(Q, K, V, O, (int)bh, Sq, Skv, scale, lds, s);
     if (variant == 1) return launch_fa<64, 1, 4, 1>(Q, K, V, O, (int)bh, Sq, Skv, scale, lds, s);
     return launch_fa_pp<64>(Q, K, V, O, (int)bh, Sq, Skv, scale, lds, s);
   }
   // D = 32: the head dimension of the reference's example program (examples/flash_attention/flash_attention.py:96-110)
+  if (variant == 2) return launch_fa<32, 1, 4, 1, 2>(Q, K, V, O, (int)bh, Sq, Skv, scale, lds, s);
   if (variant == 1) return launch_fa<32, 1, 4, 1>(Q, K, V, O, (int)bh, Sq, Skv, scale, lds, s);
   return launch_fa_pp<32>(Q, K, V, O, (int)bh, Sq, Skv, scale, lds, s);
 }

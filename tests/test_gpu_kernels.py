@@ -1470,3 +1470,26 @@ def test_streamed_f16_cells_whole_tiles(core, H, L, T, B, dil):
         for t, ref, what in ((h, hr, 'h'), (c, cr, 'c')):
             got = t[:, :, rows].float().cpu().numpy()
             assert ko.max_rel_err(got[:, live], ref.astype(np.float32)[:, live]) <= 1e-2, what
+
+
+@pytest.mark.parametrize('B,Hd,Sq,Skv,D', [
+    (1, 3, 17, 129, 32),           # the fewest keys: two tiles and one, the second group's a single key
+    (1, 2, 100, 192, 64),          # groups of two tiles and one
+    (2, 3, 129, 256, 128),         # a second block of one row; groups of equal length
+    (1, 5, 300, 321, 128),         # five tiles and one key
+    (3, 1, 77, 1000, 96),          # parts of the keys as well, the last one ragged
+    (1, 1, 33, 4097, 128),         # parts whose last would hold one key
+    (1, 2, 64, 2305, 64),
+])
+def test_flash_attention_two_key_groups(core, B, Hd, Sq, Skv, D):
+    """Small grids of query blocks: two groups of waves share a block's keys.  Against float64, weights and O rounded to fp16;
+    the largest scores sit in the second half of the keys, then in the first."""
+    rng = np.random.default_rng(31)
+    Q, K, V = (rng.standard_normal((B, Hd, s, D)).astype(np.float16) for s in (Sq, Skv, Skv))
+    for half in (slice(Skv // 2, None), slice(None, Skv // 2)):
+        K2 = K.copy()
+        K2[..., half, :] *= 3
+        ref = ko.attention(Q, K2, V, D ** -0.5)
+        for split in (True, False):
+            O = core.flash_attention(dev(Q), dev(K2), dev(V), D ** -0.5, split_keys=split)
+            assert ko.max_rel_err(O.float().cpu().numpy(), ref) <= F16_TOL
