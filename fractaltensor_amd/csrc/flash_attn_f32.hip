@@ -13,8 +13,8 @@
 // what a sum of products is accurate to anyway: 22 significant bits of its own are kept by every element within
 // 2^-17 of the largest.
 //
-// Three launches besides a clear: the largest |K| and |V| per (batch, head); the split of K and V into planes
-// [row][top D | rest D] in the workspace; the attention kernel, which splits its rows of Q (times scale * log2 e)
+// Launches: the largest |K| and |V| per (batch, head) and the split of K and V into planes [row][top D | rest D] in the
+// workspace, in one launch where heads are small, else in three; the attention kernel, which splits its rows of Q (times scale * log2 e)
 // itself, in registers.  A plane row is an fp16 row of 2 D
 // elements, so tiles, copies and fragment reads are those of the fp16 kernel at twice the head dimension
 // (fa_common.h), and the contractions are its transposed ones: S^T = K Q^T, O^T += V^T P^T, a lane owns one query
@@ -72,42 +72,85 @@ __global__ __launch_bounds__(256) void attn_f32_absmax_kernel(const float* K, co
   }
 }
 
-// One wave per row of D floats of K (blockIdx.y 0) or V (1): planes [top D | rest D] of the row under its (batch,
-// head)'s scale.
+// Eight neighbouring floats of a row into its planes [top D | rest D].
+template <int D>
+__device__ __forceinline__ void split_eight(const float* X, _Float16* planes, long long chunk, float scale) {
+  constexpr int CPR = D / 8;
+  const long long row = chunk / CPR;
+  const int c = (int)(chunk - row * CPR);
+  const float4 a = *reinterpret_cast<const float4*>(X + row * D + 8 * c), b = *reinterpret_cast<const float4*>(X + row * D + 8 * c + 4);
+  const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+  v8h top, rest;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const float s = v[e] * scale;
+    top[e] = (_Float16)s;
+    rest[e] = (_Float16)(s - (float)top[e]);
+  }
+  _Float16* const dst = planes + row * (2 * D) + 8 * c;
+  *reinterpret_cast<v8h*>(dst) = top;
+  *reinterpret_cast<v8h*>(dst + D) = rest;
+}
+
+// Planes of K (blockIdx.y 0) and V (1) under each (batch, head)'s scale, eight floats to a thread.
 template <int D>
 __global__ __launch_bounds__(256) void attn_f32_split_kernel(const float* K, const float* V, _Float16* kplanes, _Float16* vplanes,
                                                             const unsigned* group_bits, int rows_per_bh, long long rows, int BH) {
-  constexpr int PER = D / 32;   // floats per lane: 1, 2, 3 or 4
-  const int lane = threadIdx.x & 63;
-  const long long row = (long long)blockIdx.x * 4 + (threadIdx.x >> 6);
+  const long long chunk = (long long)blockIdx.x * 256 + threadIdx.x, row = chunk / (D / 8);
   if (row >= rows) return;
-  const float* X = blockIdx.y ? V : K;
-  _Float16* planes = blockIdx.y ? vplanes : kplanes;
-  constexpr int LANES = D / PER > 64 ? 64 : D / PER;   // 32 lanes x PER floats cover a row
   float scale, inv;
   split_scale(group_bits[blockIdx.y * BH + row / rows_per_bh], &scale, &inv);
-  if (lane < LANES) {
-    _Float16* dst = planes + row * (2 * D) + lane * PER;
-#pragma unroll
-    for (int e = 0; e < PER; ++e) {
-      const float s = X[row * D + lane * PER + e] * scale;
-      const _Float16 top = (_Float16)s;
-      dst[e] = top;
-      dst[D + e] = (_Float16)(s - (float)top);
-    }
-  }
+  split_eight<D>(blockIdx.y ? V : K, blockIdx.y ? vplanes : kplanes, chunk, scale);
 }
 
-// 4 waves x 32 query rows per workgroup, one workgroup per compute unit (the accumulators of O, both planes of Q
-// and the scores take more than 256 registers at D = 128).  K and V tiles of 64 keys, both double buffered.  A wave
+// Largest magnitude and planes in one launch, for heads that a compute unit reads in a microsecond or two: each of a
+// head's `parts` workgroups finds the head's largest magnitude for itself (the others find the rows in their XCD's L2) and
+// writes its share of the planes.  The three launches of the other way (clear, largest, split) take 11 us whatever the size
+// (B 2, 8 heads, 1024 keys of 32).
+constexpr int kPlanesThreads = 512;
+template <int D>
+__global__ __launch_bounds__(kPlanesThreads) void attn_f32_planes_kernel(const float* K, const float* V, _Float16* kplanes, _Float16* vplanes,
+                                                                         unsigned* bits, int Skv, int BH, int parts) {
+  __shared__ unsigned wave_max[kPlanesThreads / 64];
+  const int id = xcd_consecutive(blockIdx.x, gridDim.x);
+  const int group = id / parts, part = id - group * parts;   // group: (batch, head) of K, then of V
+  const bool is_v = group >= BH;
+  const size_t head = (size_t)(is_v ? group - BH : group) * Skv * D;
+  const float* const X = (is_v ? V : K) + head;
+  _Float16* const planes = (is_v ? vplanes : kplanes) + 2 * head;
+  const int quads = Skv * (D / 4);
+  unsigned m = 0;
+#pragma unroll 8
+  for (int i = threadIdx.x; i < quads; i += kPlanesThreads) {
+    const float4 v = *reinterpret_cast<const float4*>(X + 4 * (size_t)i);
+    m = max(max(m, __float_as_uint(fabsf(v.x))), max(__float_as_uint(fabsf(v.y)), max(__float_as_uint(fabsf(v.z)), __float_as_uint(fabsf(v.w)))));
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) m = max(m, (unsigned)__shfl_xor((int)m, o));
+  if ((threadIdx.x & 63) == 0) wave_max[threadIdx.x >> 6] = m;
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < kPlanesThreads / 64; ++w) m = max(m, wave_max[w]);
+  if (part == 0 && threadIdx.x == 0) bits[group] = m;
+  float scale, inv;
+  split_scale(m, &scale, &inv);
+  const int chunks = Skv * (D / 8);
+  for (int i = part * kPlanesThreads + threadIdx.x; i < chunks; i += parts * kPlanesThreads) split_eight<D>(X, planes, i, scale);
+}
+
+// 4 waves x 32 query rows per workgroup.  Two workgroups to a compute unit at head sizes up to 64 (B 4, 16 heads, 1024 keys of 64: 88
+// -> 77 us with a bound of 256 registers, of which the compiler had taken a few more), one above: the accumulators of O,
+// both planes of Q and the scores take some 400 registers at D = 128.  K and V tiles of 64 keys, both double buffered.  A wave
 // works through the tiles in halves of 32 keys, and with one wave per SIMD the softmax of a half has no other
 // wave's MFMAs to run beside: it is cut in two, the maxima under the P V MFMAs of the half before and the weights
 // under the score MFMAs of the half after (the comments in the kernel give the order).
-template <int D>
-__global__ __launch_bounds__(256, 1) void flash_attn_f32_kernel(const float* __restrict__ Q, const _Float16* __restrict__ Kp,
+// KG == 2 (head sizes up to 64, whose registers allow two waves per SIMD): two groups of four waves share the query rows,
+// each walks half of the keys with tiles of its own in LDS, and the first takes in the second's result at the end.
+template <int D, int KG>
+__global__ __launch_bounds__(KG * 256, KG == 1 && D <= 64 ? 2 : 1) void flash_attn_f32_kernel(const float* __restrict__ Q, const _Float16* __restrict__ Kp,
                                                                 const _Float16* __restrict__ Vp, float q_mul,
                                                                 const unsigned* __restrict__ kv_bits, float* __restrict__ O,
-                                                                int Sq, int Skv, int nqb, int BH) {
+                                                                int Sq, int Skv_all, int nqb, int BH) {
   using L = FaLayout<2 * D>;          // a plane row is an fp16 row of 2 D elements
   constexpr int DS = D / 16;          // k steps of S^T
   constexpr int DT = D / 32;          // d tiles of O^T
@@ -116,23 +159,26 @@ __global__ __launch_bounds__(256, 1) void flash_attn_f32_kernel(const float* __r
   constexpr int WAVES = 4;
   constexpr int KCP = (KTB / 1024 + WAVES - 1) / WAVES, VCP = (VTB / 1024 + WAVES - 1) / WAVES;
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
-  unsigned char* const Kb = smem;            // [2][KTB]
-  unsigned char* const Vb = smem + 2 * KTB;  // [2][VTB]
-
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wave = __builtin_amdgcn_readfirstlane((tid >> 6) & 3);   // within its key group
+  const int group = KG == 1 ? 0 : __builtin_amdgcn_readfirstlane(tid >> 8);
+  constexpr int GROUP_LDS = 2 * (KTB + VTB);
+  unsigned char* const Kb = smem + group * GROUP_LDS;   // [2][KTB]
+  unsigned char* const Vb = Kb + 2 * KTB;               // [2][VTB]
   const int j = lane & 31;
   const int hh = lane >> 5;
-  int id = blockIdx.x;
-  const int total = gridDim.x;
-  if ((total & 7) == 0) id = (blockIdx.x & 7) * (total >> 3) + (blockIdx.x >> 3);   // a head's query blocks share an XCD
+  const int id = xcd_consecutive(blockIdx.x, gridDim.x);   // a head's query blocks share an XCD
   const int bh = id / nqb;
   const int qb = id - bh * nqb;
   const int q_base = qb * (WAVES * 32) + wave * 32;
 
-  const _Float16* Kg = Kp + (size_t)bh * Skv * (2 * D);
-  const _Float16* Vg = Vp + (size_t)bh * Skv * (2 * D);
+  // the first group has the first half of the tiles, one more than the second when they are odd (never fewer than two in all)
+  const int first_tiles = ((Skv_all + FA_KT - 1) / FA_KT + 1) / 2;
+  const int key_first = group * first_tiles * FA_KT;
+  const int Skv = KG == 1 ? Skv_all : group == 0 ? first_tiles * FA_KT : Skv_all - key_first;   // the keys this group sees
+  const _Float16* Kg = Kp + ((size_t)bh * Skv_all + key_first) * (2 * D);
+  const _Float16* Vg = Vp + ((size_t)bh * Skv_all + key_first) * (2 * D);
   float* Og = O + (size_t)bh * Sq * D;
 
   // The lane's query row: the fp32 row is read, multiplied by q_mul (scale * log2 e: a score leaves the matrix unit in
@@ -491,14 +537,47 @@ __global__ __launch_bounds__(256, 1) void flash_attn_f32_kernel(const float* __r
     const v16f none = zero16;
     pv_and_maxima(std::false_type{}, std::false_type{}, std::false_type{}, pend_v, nullptr, none, 0);
   }
+  if (KG == 2 && group == 1 && ntiles < first_tiles) {   // the first group's last tile
+    __syncthreads();
+    __syncthreads();
+  }
   __syncthreads();   // LDS is reused below
+  float l = l_run + __shfl_xor(l_run, 32);
+  if constexpr (KG == 2) {
+    // the second group leaves its accumulators, reference and sum in its part of LDS, by lane; the first takes them in by
+    // the rule of an online softmax
+    unsigned char* const other = smem + GROUP_LDS;
+    v4f* const oo = reinterpret_cast<v4f*>(other) + wave * (DT * 4 * 64) + lane;
+    float2* const oml = reinterpret_cast<float2*>(other + WAVES * (DT * 4 * 64 * 16)) + wave * 64 + lane;
+    static_assert(WAVES * (DT * 4 * 64 * 16 + 64 * 8) <= GROUP_LDS, "the second group's result fits its tiles' place");
+    if (group == 1) {
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) oo[(4 * dt + g) * 64] = v4f{om[dt][4 * g], om[dt][4 * g + 1], om[dt][4 * g + 2], om[dt][4 * g + 3]};
+      *oml = make_float2(m_ref, l);
+    }
+    __syncthreads();
+    if (group == 1) return;
+    const float2 ml = *oml;
+    const float m = fmaxf(m_ref, ml.x);
+    const float wm = __builtin_amdgcn_exp2f(m_ref - m), wo = __builtin_amdgcn_exp2f(ml.x - m);
+    l = wm * l + wo * ml.y;
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const v4f o = oo[(4 * dt + g) * 64];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) om[dt][4 * g + k] = wm * om[dt][4 * g + k] + wo * o[k];
+      }
+  }
 
   // ---- normalise and store: the wave turns its 32 x D tile round through the LDS nobody reads any more (the
   // barrier above ended the last tile), so that whole rows leave as consecutive bytes
   constexpr int ORS = 4 * D + 16;
   constexpr int LPR = D / 4;   // 16-byte chunks per row
   unsigned char* const ot = smem + wave * (32 * ORS);
-  const float l = l_run + __shfl_xor(l_run, 32);
   const float fin = v_inv / l;   // l in the scale of the weights' planes, as O's accumulators
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt)
@@ -534,39 +613,64 @@ static F32Layout f32_layout(long long bh, int Skv, int D) {
   return w;
 }
 
-template <int D>
-static int launch_fa_f32(const float* Q, const float* K, const float* V, float* O, int BH, int Sq, int Skv, float scale, char* ws,
-                         const F32Layout& w, int lds_max, hipStream_t s) {
+template <int D, int KG>
+static int launch_fa_f32_blocks(const float* Q, const _Float16* kp, const _Float16* vp, const unsigned* bits, float* O, int BH, int Sq, int Skv,
+                                float scale, int lds_max, hipStream_t s) {
   using L = FaLayout<2 * D>;
-  const size_t lds = std::max((size_t)2 * (L::KTB + L::VTB), (size_t)4 * 32 * (4 * D + 16));
+  const size_t lds = std::max((size_t)KG * 2 * (L::KTB + L::VTB), (size_t)4 * 32 * (4 * D + 16));
   if ((int)lds > lds_max) return fail(FTK_ERR_DEVICE, "ftk_flash_attn_f32: D=%d needs %zu bytes of LDS, the device offers %d", D, lds, lds_max);
-  unsigned* bits = reinterpret_cast<unsigned*>(ws + w.bits);
-  _Float16* kp = reinterpret_cast<_Float16*>(ws + w.kp);
-  _Float16* vp = reinterpret_cast<_Float16*>(ws + w.vp);
-  hipLaunchKernelGGL(attn_f32_clear_kernel, dim3((2 * BH + 255) / 256), dim3(256), 0, s, bits, 2 * BH);
-  int rc = check_launch("attn_f32_clear_kernel");
-  if (rc) return rc;
-  const size_t per_bh = (size_t)Skv * D;
-  const int chunks = (int)std::min<size_t>(std::max(1, 4096 / (2 * BH)), (per_bh + 4095) / 4096);   // some 4096 workgroups in all
-  hipLaunchKernelGGL(attn_f32_absmax_kernel, dim3(chunks, BH, 2), dim3(256), 0, s, K, V, bits, per_bh, BH);
-  rc = check_launch("attn_f32_absmax_kernel");
-  if (rc) return rc;
-  const long long krows = (long long)BH * Skv;
-  hipLaunchKernelGGL(attn_f32_split_kernel<D>, dim3((unsigned)((krows + 3) / 4), 2), dim3(256), 0, s, K, V, kp, vp, (const unsigned*)bits, Skv, krows,
-                     BH);
-  rc = check_launch("attn_f32_split_kernel");
-  if (rc) return rc;
   const int nqb = (Sq + 127) / 128;
   const long long blocks = (long long)nqb * BH;
   if (blocks > 0x7fffffffLL) return fail(FTK_ERR_UNSUPPORTED_SHAPE, "ftk_flash_attn_f32: grid too large");
   static DeviceOnce attr_once;
   unsigned attr_bit;
   if (attr_once.pending(&attr_bit)) {
-    FTK_HIP(hipFuncSetAttribute((const void*)flash_attn_f32_kernel<D>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    FTK_HIP(hipFuncSetAttribute((const void*)flash_attn_f32_kernel<D, KG>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     attr_once.done(attr_bit);
   }
-  hipLaunchKernelGGL(flash_attn_f32_kernel<D>, dim3((unsigned)blocks), dim3(256), lds, s, Q, kp, vp, scale * 1.4426950408889634f, bits, O, Sq, Skv, nqb, BH);
+  hipLaunchKernelGGL((flash_attn_f32_kernel<D, KG>), dim3((unsigned)blocks), dim3(KG * 256), lds, s, Q, kp, vp, scale * 1.4426950408889634f, bits, O, Sq,
+                     Skv, nqb, BH);
   return check_launch("flash_attn_f32_kernel");
+}
+
+template <int D>
+static int launch_fa_f32(const float* Q, const float* K, const float* V, float* O, int BH, int Sq, int Skv, float scale, char* ws,
+                         const F32Layout& w, const DeviceProps& dp, hipStream_t s) {
+  unsigned* bits = reinterpret_cast<unsigned*>(ws + w.bits);
+  _Float16* kp = reinterpret_cast<_Float16*>(ws + w.kp);
+  _Float16* vp = reinterpret_cast<_Float16*>(ws + w.vp);
+  const size_t per_bh = (size_t)Skv * D, head_bytes = per_bh * sizeof(float);
+  // One launch while heads are small and what all its workgroups read for the largest magnitudes stays below 96 MB (a few
+  // microseconds of L2); up to two workgroups to a compute unit (B 4, 16 heads, 1024 keys of 64: four parts each, 134 MB, were slower
+  // than three launches).
+  const size_t all_heads = 2 * (size_t)BH * head_bytes, most_read = (size_t)96 << 20;
+  const int parts = (int)std::max<size_t>(1, std::min({512 / (2 * (size_t)BH), per_bh / (8 * kPlanesThreads), most_read / all_heads}));
+  int rc;
+  if (head_bytes <= 512 * 1024 && all_heads * parts <= most_read) {
+    hipLaunchKernelGGL(attn_f32_planes_kernel<D>, dim3((unsigned)(2 * BH * parts)), dim3(kPlanesThreads), 0, s, K, V, kp, vp, bits, Skv, BH, parts);
+    rc = check_launch("attn_f32_planes_kernel");
+    if (rc) return rc;
+  } else {
+    hipLaunchKernelGGL(attn_f32_clear_kernel, dim3((2 * BH + 255) / 256), dim3(256), 0, s, bits, 2 * BH);
+    rc = check_launch("attn_f32_clear_kernel");
+    if (rc) return rc;
+    const int chunks = (int)std::min<size_t>(std::max(1, 4096 / (2 * BH)), (per_bh + 4095) / 4096);   // some 4096 workgroups in all
+    hipLaunchKernelGGL(attn_f32_absmax_kernel, dim3(chunks, BH, 2), dim3(256), 0, s, K, V, bits, per_bh, BH);
+    rc = check_launch("attn_f32_absmax_kernel");
+    if (rc) return rc;
+    const long long krows = (long long)BH * Skv;
+    hipLaunchKernelGGL(attn_f32_split_kernel<D>, dim3((unsigned)((krows * (D / 8) + 255) / 256), 2), dim3(256), 0, s, K, V, kp, vp, (const unsigned*)bits,
+                       Skv, krows, BH);
+    rc = check_launch("attn_f32_split_kernel");
+    if (rc) return rc;
+  }
+  // Two key groups while there is at most one block of query rows to a compute unit and more than two tiles of keys (us, the
+  // whole call without and with: B2 H8 S1024 D32 37.4, 25.9; B2 H12 S512 D64 32, 24; B1 H8 S2048 D64 80, 57; B1 H16 S2048 D32 67, 50).
+  if constexpr (D <= 64) {
+    if ((long long)((Sq + 127) / 128) * BH <= dp.cus && Skv > 2 * FA_KT)
+      return launch_fa_f32_blocks<D, 2>(Q, kp, vp, bits, O, BH, Sq, Skv, scale, dp.lds_optin, s);
+  }
+  return launch_fa_f32_blocks<D, 1>(Q, kp, vp, bits, O, BH, Sq, Skv, scale, dp.lds_optin, s);
 }
 
 }  // namespace ftk
@@ -599,9 +703,9 @@ extern "C" int ftk_flash_attn_f32(const float* Q, const float* K, const float* V
   hipStream_t s = (hipStream_t)stream;
   char* ws = reinterpret_cast<char*>(workspace);
   switch (D) {
-    case 32: return launch_fa_f32<32>(Q, K, V, O, (int)bh, Sq, Skv, scale, ws, w, dp->lds_optin, s);
-    case 64: return launch_fa_f32<64>(Q, K, V, O, (int)bh, Sq, Skv, scale, ws, w, dp->lds_optin, s);
-    case 96: return launch_fa_f32<96>(Q, K, V, O, (int)bh, Sq, Skv, scale, ws, w, dp->lds_optin, s);
-    default: return launch_fa_f32<128>(Q, K, V, O, (int)bh, Sq, Skv, scale, ws, w, dp->lds_optin, s);
+    case 32: return launch_fa_f32<32>(Q, K, V, O, (int)bh, Sq, Skv, scale, ws, w, *dp, s);
+    case 64: return launch_fa_f32<64>(Q, K, V, O, (int)bh, Sq, Skv, scale, ws, w, *dp, s);
+    case 96: return launch_fa_f32<96>(Q, K, V, O, (int)bh, Sq, Skv, scale, ws, w, *dp, s);
+    default: return launch_fa_f32<128>(Q, K, V, O, (int)bh, Sq, Skv, scale, ws, w, *dp, s);
   }
 }

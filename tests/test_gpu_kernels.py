@@ -1493,3 +1493,28 @@ def test_flash_attention_two_key_groups(core, B, Hd, Sq, Skv, D):
         for split in (True, False):
             O = core.flash_attention(dev(Q), dev(K2), dev(V), D ** -0.5, split_keys=split)
             assert ko.max_rel_err(O.float().cpu().numpy(), ref) <= F16_TOL
+
+
+@pytest.mark.parametrize('B,Hd,Sq,Skv,D', [
+    (1, 2, 100, 129, 32),          # key groups of two tiles and a single key
+    (2, 3, 129, 192, 64),          # two tiles and one
+    (1, 5, 300, 321, 64),          # the second group a tile shorter, and ragged
+    (3, 2, 64, 1024, 32),          # equal groups
+    (1, 1, 16, 5, 32),             # planes of less than a workgroup's share
+    (1, 1, 32, 4100, 32),          # a head just above what one launch makes the planes of
+    (2, 2, 40, 1000, 128),         # head sizes without key groups
+    (1, 3, 33, 77, 96),
+])
+def test_flash_attention_f32_key_groups_and_planes(core, B, Hd, Sq, Skv, D):
+    """Small grids and small heads in fp32, heads of different magnitude, the largest scores in one half of the keys and then
+    in the other, against float64."""
+    rng = np.random.default_rng(37)
+    Q, K, V = (rng.standard_normal((B, Hd, s, D)).astype(np.float32) for s in (Sq, Skv, Skv))
+    V *= 10.0 ** np.arange(Hd, dtype=np.float32)[None, :, None, None]
+    for half in (slice(Skv // 2, None), slice(None, Skv // 2)):
+        K2 = K.copy()
+        K2[..., half, :] *= 3
+        ref = ko.attention(Q.astype(np.float64), K2.astype(np.float64), V.astype(np.float64), D ** -0.5)
+        O = core.flash_attention_f32(dev(Q), dev(K2), dev(V), D ** -0.5).cpu().numpy()
+        for h in range(Hd):                                  # each head on its own: a sum of weights times fp32 values
+            assert ko.max_rel_err(O[:, h], ref[:, h]) <= 1e-5
