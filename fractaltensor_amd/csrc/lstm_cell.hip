@@ -34,6 +34,7 @@
 namespace ftk {
 
 constexpr int kMaxCellsPerLaunch = 40;
+constexpr int kFlowLayers = 64;   // layers of a stack that runs as one launch (lstm_cell_flow_kernel)
 
 struct CellDesc {
   const float* x;       // [B, I]
@@ -601,14 +602,11 @@ struct CellSource {
 // of the plain product, one wave per SIMD with 128 x 128 outputs.  Bound by the matrix pipe and the LDS reads that feed
 // it: with 128 x 64 outputs to a wave a k step read 12 KB of fragments for 16 MFMAs instead of 16 KB for 32, and two waves
 // per SIMD stood at the same barrier.  L 32 T 64 B 256 H 1024: 12.70 -> 11.63 ms for the stack.
-__global__ __launch_bounds__(256, 1) void lstm_cell_tile_kernel(CellListH list, int B, int H) {
-  const int nub = H / 64, nrb = (B + GT - 1) / GT;
-  const int slot = (int)(blockIdx.x >> 3), cell = (int)(blockIdx.x & 7) + 8 * (slot / (nub * nrb));   // a cell's tiles on one XCD
-  if (cell >= list.n) return;
-  const CellDescH cd = list.cells[cell];
-  const int Bc = cd.rows > 0 ? cd.rows : B;  // rows of this cell
-  const int ub = slot % nub, rb = (slot / nub) % nrb;
-  if (rb * GT >= Bc) return;  // a row block past the live rows of this step
+// A tile of a cell: rows 256 rb .. of the batch, units 64 ub .. .  SHARED: h and c are read by workgroups of this launch, on
+// any XCD, so they are written through to memory.
+constexpr int kThrough = 16;   // sc1 in the cache-policy operand of a buffer store
+template <bool SHARED>
+__device__ __forceinline__ void cell_tile(const CellDescH& cd, int Bc, int H, int rb, int ub) {
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wr = wave >> 1, wc = wave & 1;
@@ -642,6 +640,8 @@ __global__ __launch_bounds__(256, 1) void lstm_cell_tile_kernel(CellListH list, 
     for (int w = 0; w < 2; ++w)   // upper lanes' first <-> lower lanes' second
       asm volatile("s_nop 1\n\tv_permlane32_swap_b32_e32 %0, %1\n\ts_nop 1" : "+v"(first[w]), "+v"(second[w]));
   };
+  [[maybe_unused]] const auto h_out = __builtin_amdgcn_make_buffer_rsrc(cd.h, 0, (unsigned)(2 * Bc * H), 0x00020000);
+  [[maybe_unused]] const auto c_out = __builtin_amdgcn_make_buffer_rsrc(cd.c, 0, (unsigned)(2 * Bc * H), 0x00020000);
   const _Float16* c_prev = reinterpret_cast<const _Float16*>(cd.c_prev);
 #pragma unroll
   for (int np = 0; np < 2; ++np) {
@@ -675,7 +675,7 @@ __global__ __launch_bounds__(256, 1) void lstm_cell_tile_kernel(CellListH list, 
           const float fg = sigmoid_f(s[4 + r] + bias[n][1][r]);
           const float og = sigmoid_f(s[8 + r] + bias[n][2][r]);
           const float cand = tanh_f(s[12 + r] + bias[n][3][r]);
-          const float c = fg * (float)c16[r] + ig * cand;
+          const float c = fmaf(fg, (float)c16[r], ig * cand);
           cv[r] = (_Float16)c;
           hv[r] = (_Float16)(og * tanh_f(c));
         }
@@ -684,12 +684,138 @@ __global__ __launch_bounds__(256, 1) void lstm_cell_tile_kernel(CellListH list, 
       }
       swap_halves(co[0], co[1]);
       swap_halves(ho[0], ho[1]);
-      if (row < Bc) {
+      const v4u cs = {co[0][0], co[0][1], co[1][0], co[1][1]}, hs = {ho[0][0], ho[0][1], ho[1][0], ho[1][1]};
+      if constexpr (SHARED) {
+        const unsigned at = row < Bc ? (unsigned)(row * H + u0 + 8 * hh) * 2u : ~0u;   // past the batch: out of bounds
+        __builtin_amdgcn_raw_buffer_store_b128(cs, c_out, at, 0, kThrough);
+        __builtin_amdgcn_raw_buffer_store_b128(hs, h_out, at, 0, kThrough);
+      } else if (row < Bc) {
         const size_t at = (size_t)row * H + u0 + 8 * hh;
-        *reinterpret_cast<v4u*>(reinterpret_cast<_Float16*>(cd.c) + at) = v4u{co[0][0], co[0][1], co[1][0], co[1][1]};
-        *reinterpret_cast<v4u*>(reinterpret_cast<_Float16*>(cd.h) + at) = v4u{ho[0][0], ho[0][1], ho[1][0], ho[1][1]};
+        *reinterpret_cast<v4u*>(reinterpret_cast<_Float16*>(cd.c) + at) = cs;
+        *reinterpret_cast<v4u*>(reinterpret_cast<_Float16*>(cd.h) + at) = hs;
       }
     }
+  }
+}
+
+__global__ __launch_bounds__(256, 1) void lstm_cell_tile_kernel(CellListH list, int B, int H) {
+  const int nub = H / 64, nrb = (B + GT - 1) / GT;
+  const int slot = (int)(blockIdx.x >> 3), cell = (int)(blockIdx.x & 7) + 8 * (slot / (nub * nrb));   // a cell's tiles on one XCD
+  if (cell >= list.n) return;
+  const CellDescH cd = list.cells[cell];
+  const int Bc = cd.rows > 0 ? cd.rows : B;  // rows of this cell
+  const int ub = slot % nub, rb = (slot / nub) % nrb;
+  if (rb * GT >= Bc) return;  // a row block past the live rows of this step
+  cell_tile<false>(cd, Bc, H, rb, ub);
+}
+
+// A whole dense stack in one launch.  With a launch per stage of independent cells, a stage whose tiles are no multiple of
+// the compute units leaves some idle: 158 rounds of tiles instead of 128 at L 32 T 64 B 256 H 1024, and 95 gaps between
+// launches (11.2 -> 10.5 ms; L 20 T 64 B 230 8.8 -> 6.8).  What is left is a tile of 73 us where a compute unit with the
+// chip to itself takes 46: every tile has 1 MB of weights of its own to fetch, 3.5 TB/s with all of them at it.  Here a workgroup takes one tile after another, of the cells in the order of their stages (l + t), waits until
+// the cells below and before it are complete (done counts a cell's finished tiles), and publishes its own.
+//
+// Eight queues, cell k in queue k % 8, a workgroup takes from the queue of its place among the XCDs: a cell's tiles share
+// an L2 copy of its activations.  A workgroup holds one ticket, taken in order, and waits only for cells earlier in the
+// order: the earliest unfinished tile is always being worked on or about to be taken, whatever part of the grid is
+// resident, so ordinary launches do, next to anything else.  The wait is bounded all the same (status word).
+//
+// h and c are written through to memory, and complete before the tile is counted.  They are read through the caches:
+// nothing of a cell is read before it is complete, and a cell starts at a cache line (the host looks), so no cache holds
+// an older line of it.
+struct FlowArgs {
+  const _Float16* xs;
+  const _Float16* WU;   // packed
+  const float* bias;
+  _Float16* hsss;
+  _Float16* csss;
+  int* status;
+  int* tickets;   // [8], 64 bytes apart
+  int* done;      // [L][T]
+  int L, T, B, H, spin_limit;
+  int dil[kFlowLayers];
+};
+// Cell k of a stack of L layers and T steps in the order of the stages l + t, low layers first: its layer and step.
+__host__ __device__ inline void flow_cell(int k, int L, int T, int* l, int* t) {
+  const int m = L < T ? L : T, ramp = m * (m - 1) / 2;   // the first m - 1 stages have 1, 2, .. m - 1 cells, the last as many
+  const bool tail = k >= L * T - ramp;
+  const int i = tail ? L * T - 1 - k : k;
+  int stage, pos, low;
+  if (i < ramp) {
+    stage = (int)((sqrtf(8.0f * (float)i + 1.0f) - 1.0f) * 0.5f);
+    while (stage * (stage + 1) / 2 > i) --stage;
+    while ((stage + 1) * (stage + 2) / 2 <= i) ++stage;
+    pos = i - stage * (stage + 1) / 2;
+    if (tail) {
+      pos = stage - pos;
+      stage = L + T - 2 - stage;
+    }
+  } else {
+    stage = m - 1 + (i - ramp) / m;
+    pos = (i - ramp) % m;
+  }
+  low = stage - T + 1 > 0 ? stage - T + 1 : 0;
+  *l = low + pos;
+  *t = stage - *l;
+}
+__global__ __launch_bounds__(256, 1) void lstm_cell_flow_kernel(FlowArgs) {
+  extern __shared__ __attribute__((aligned(1024))) unsigned char tile_smem[];
+  int* const word = reinterpret_cast<int*>(tile_smem);   // the next tile: layer (-1: none), step, tile of the cell
+  while (true) {
+    // read again for every tile: kept over the product, whose loop takes all registers, the arguments would be spilled
+    auto* args = (const __attribute__((address_space(4))) FlowArgs*)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(args));
+    const auto& a = *args;
+    const int L = a.L, T = a.T, B = a.B, H = a.H;
+    const int nub = H / 64, tiles = nub * ((B + GT - 1) / GT);
+    const int q = (int)(blockIdx.x & 7), mine = (L * T - q + 7) / 8 * tiles;
+    const size_t cell = (size_t)B * H;
+    if (threadIdx.x < 64) {
+      int l = -1, t = 0, tile = 0;
+      if (threadIdx.x == 0) {
+        const int ticket = __hip_atomic_fetch_add(a.tickets + 16 * q, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (ticket < mine) {
+          tile = ticket % tiles;
+          flow_cell(q + 8 * (ticket / tiles), L, T, &l, &t);
+          const int d = a.dil[l];
+          const int* const below = l > 0 ? a.done + (l - 1) * T + t : nullptr;
+          const int* const before = t >= d ? a.done + l * T + t - d : nullptr;
+          for (int n = 1;; ++n) {
+            const bool there = (!below || __hip_atomic_load(below, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == tiles) &&
+                               (!before || __hip_atomic_load(before, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == tiles);
+            if (there) break;
+            if (n >= a.spin_limit || ((n & 255) == 0 && __hip_atomic_load(a.status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0)) {
+              __hip_atomic_store(a.status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+              l = -1;
+              break;
+            }
+            __builtin_amdgcn_s_sleep(4);
+          }
+        }
+        word[0] = l;
+        word[1] = t;
+        word[2] = tile;
+      }
+    }
+    __syncthreads();
+    const int l = __builtin_amdgcn_readfirstlane(word[0]), t = __builtin_amdgcn_readfirstlane(word[1]);
+    const int tile = __builtin_amdgcn_readfirstlane(word[2]);
+    __syncthreads();   // the words are read: the tile's copies may take their place
+    if (l < 0) return;
+    const int d = a.dil[l];
+    CellDescH cd;
+    cd.x = l == 0 ? a.xs + (size_t)t * cell : a.hsss + ((size_t)(l - 1) * T + t) * cell;
+    cd.h_prev = t >= d ? a.hsss + ((size_t)l * T + t - d) * cell : nullptr;
+    cd.c_prev = t >= d ? a.csss + ((size_t)l * T + t - d) * cell : nullptr;
+    cd.WU = a.WU + (size_t)l * 8 * H * H;
+    cd.bias = a.bias ? a.bias + (size_t)l * 4 * H : nullptr;
+    cd.h = a.hsss + ((size_t)l * T + t) * cell;
+    cd.c = a.csss + ((size_t)l * T + t) * cell;
+    int* const done = a.done + l * T + t;
+    cell_tile<true>(cd, B, H, tile / nub, tile % nub);
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");   // h and c of this wave are in memory
+    __syncthreads();
+    if (threadIdx.x == 0) __hip_atomic_fetch_add(done, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
 }
 
@@ -895,11 +1021,12 @@ static int launch_cells(const CellList& list, int B, int I, int H, hipStream_t s
 
 // WU [n_layers, K2, 4H] -> per layer and block ub of UB hidden units the [K2][4*UB] tile the cell kernel keeps
 // in LDS: row k holds chunks of 8 columns, chunk 4*ug + q = gate q of units UB*ub + 8*ug .. +8, stored in slot
-// chunk ^ ((k & 3) << 2).  One thread per 16-byte chunk.
+// chunk ^ ((k & 3) << 2).  One thread per 16-byte chunk.  Clears nclear words on the way, for the launch behind it.
 __global__ __launch_bounds__(256) void lstm_pack_weights_f16_kernel(const _Float16* __restrict__ WU,
                                                                     _Float16* __restrict__ packed, size_t chunks,
-                                                                    int K2, int H, int UB) {
+                                                                    int K2, int H, int UB, int* clear, int nclear) {
   const size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x;
+  for (size_t i = idx; i < (size_t)nclear; i += (size_t)gridDim.x * 256) clear[i] = 0;
   if (idx >= chunks) return;
   const int per_row = H / 2;  // 4H / 8
   const int n8 = (int)(idx % per_row);
@@ -917,10 +1044,10 @@ __global__ __launch_bounds__(256) void lstm_pack_weights_f16_kernel(const _Float
 // Hidden units per workgroup of the streaming kernel at hidden size H.
 static int cell_unit_block(int H) { return H % 64 == 0 ? 64 : 32; }
 
-int pack_weights_f16(const void* WU, void* packed, int layers, int K2, int H, hipStream_t s) {
+static int pack_weights_f16(const void* WU, void* packed, int layers, int K2, int H, int* clear, int nclear, hipStream_t s) {
   const size_t chunks = (size_t)layers * K2 * (H / 2);
   hipLaunchKernelGGL(lstm_pack_weights_f16_kernel, dim3((unsigned)((chunks + 255) / 256)), dim3(256), 0, s,
-                     (const _Float16*)WU, (_Float16*)packed, chunks, K2, H, cell_unit_block(H));
+                     (const _Float16*)WU, (_Float16*)packed, chunks, K2, H, cell_unit_block(H), clear, nclear);
   return check_launch("lstm_pack_weights_f16_kernel");
 }
 
@@ -1043,16 +1170,56 @@ int run_wavefront(const float* xs, const float* WU, const float* bias, const int
   return run_wavefront_of<float, CellList>(xs, WU, bias, dil, hsss, csss, L, T, B, H, s);
 }
 
-// The same schedule over fp16 arrays (H a multiple of 32).  packed: a buffer of the size of WU, into which the
-// weights are first re-laid per unit block, or nullptr to read WU as it is.
+constexpr size_t kFlowTicketBytes = 8 * 64;
+static size_t packed_f16_bytes(int L, int H) { return (size_t)L * 2 * H * 4 * H * sizeof(_Float16); }
+size_t wavefront_f16_workspace_bytes(int L, int T, int H) {
+  return kStatusBytes + packed_f16_bytes(L, H) + kFlowTicketBytes + (size_t)L * T * sizeof(int);
+}
+
+// The same schedule over fp16 arrays (H a multiple of 32).  ws: status block (cleared by the caller), the weights re-laid
+// per unit block, the tickets and counters of the single launch.
 int run_wavefront_f16(const void* xs, const void* WU, const float* bias, const int* dil, const int* active, void* hsss,
-                      void* csss, int L, int T, int B, int H, void* packed, hipStream_t s) {
-  if (packed) {
-    int rc = pack_weights_f16(WU, packed, L, 2 * H, H, s);
-    if (rc) return rc;
+                      void* csss, int L, int T, int B, int H, void* ws, hipStream_t s) {
+  char* const packed = reinterpret_cast<char*>(ws) + kStatusBytes;
+  int* const tickets = reinterpret_cast<int*>(packed + packed_f16_bytes(L, H));
+  const DeviceProps* dp = nullptr;
+  int rc = device_props(&dp);
+  if (rc) return rc;
+  // One launch where the tile kernel runs and the cells of h and c start at cache lines (H a multiple of 64, and the
+  // arrays' starts); a ragged batch stays with the launches, which leave out the row blocks that have ended.  A stage with less than half
+  // a chip of tiles is bound by its chain, and there a launch per stage hands over sooner than tickets and counters do
+  // (H 1024, B 256, us, launches and one launch: L 4 T 32 1698, 1767; L 8 T 32 1885, 1969; L 10 T 64 4372, 3999; L 12 T 64 4582,
+  // 4489; L 20 T 64 8986, 6693; L 32 T 64 11.2 ms, 10.5 ms).  FTK_LSTM_F16_FLOW=1 / =0 forces the one or the other.
+  const long long stage_tiles = (long long)std::min(L, T) * (H / 64) * ((B + GT - 1) / GT);
+  const char* e = getenv("FTK_LSTM_F16_FLOW");
+  const bool flow = cell_unit_block(H) == 64 && !active && L <= kFlowLayers && stage_tiles * std::max(L, T) < (1ll << 30) &&
+                    (reinterpret_cast<uintptr_t>(hsss) | reinterpret_cast<uintptr_t>(csss)) % 128 == 0 &&
+                    (e ? e[0] == '1' : 2 * stage_tiles > dp->cus);
+  rc = pack_weights_f16(WU, packed, L, 2 * H, H, tickets, flow ? (int)(kFlowTicketBytes / sizeof(int)) + L * T : 0, s);
+  if (rc) return rc;
+  if (!flow)
+    return run_wavefront_of<_Float16, CellListH>((const _Float16*)xs, (const _Float16*)packed, bias, dil, (_Float16*)hsss, (_Float16*)csss, L, T, B,
+                                                 H, s, true, active);
+  static DeviceOnce attr_once;
+  unsigned attr_bit;
+  if (attr_once.pending(&attr_bit)) {
+    FTK_HIP(hipFuncSetAttribute((const void*)lstm_cell_flow_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, G_LDS));
+    attr_once.done(attr_bit);
   }
-  return run_wavefront_of<_Float16, CellListH>((const _Float16*)xs, (const _Float16*)(packed ? packed : WU), bias, dil,
-                                               (_Float16*)hsss, (_Float16*)csss, L, T, B, H, s, packed != nullptr, active);
+  FlowArgs a;
+  a.xs = (const _Float16*)xs;
+  a.WU = (const _Float16*)packed;
+  a.bias = bias;
+  a.hsss = (_Float16*)hsss;
+  a.csss = (_Float16*)csss;
+  a.status = (int*)ws;
+  a.tickets = tickets;
+  a.done = tickets + kFlowTicketBytes / sizeof(int);
+  a.L = L; a.T = T; a.B = B; a.H = H;
+  a.spin_limit = 1 << 22;
+  for (int l = 0; l < kFlowLayers; ++l) a.dil[l] = l < L && dil ? dil[l] : 1;
+  hipLaunchKernelGGL(lstm_cell_flow_kernel, dim3(dp->cus), dim3(256), G_LDS, s, a);
+  return check_launch("lstm_cell_flow_kernel");
 }
 
 // ------------------------------------------------- fp32 stack on split products

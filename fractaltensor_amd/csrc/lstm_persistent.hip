@@ -60,7 +60,8 @@ namespace ftk {
 int run_wavefront(const float* xs, const float* WU, const float* bias, const int* dil, float* hsss, float* csss,
                   int L, int T, int B, int H, hipStream_t s);
 int run_wavefront_f16(const void* xs, const void* WU, const float* bias, const int* dil, const int* active, void* hsss,
-                      void* csss, int L, int T, int B, int H, void* packed, hipStream_t s);
+                      void* csss, int L, int T, int B, int H, void* ws, hipStream_t s);
+size_t wavefront_f16_workspace_bytes(int L, int T, int H);
 size_t split_stack_workspace_bytes(int L, int T, int B, int H);
 int run_wavefront_split(const float* xs, const float* WU, const float* bias, const int* dil, const int* active, float* hsss,
                         float* csss, int L, int T, int B, int H, void* ws, hipStream_t s);
@@ -1805,10 +1806,13 @@ static int check_stack_args(const char* who, const float* xs, const float* WU, f
 //   H = 256 has the paired schedule of the persistent kernel, which feeds the matrix pipe better: ahead from 16 layers x
 //     256 rows on (L 16 B 192: 536 against 575 us, L 16 B 256: 660 against 585, L 32 B 192: 998 against 937; fp16 data: L 16
 //     B 192 370 / 382, L 32 B 192 769 / 597), and for dilated stacks, whose chains are short (L 6 T 128 B 256: 1.22 / 0.83 ms);
-//   H = 1024 (fp16 data) holds four layers on the chip at a time, and deep stacks of large batches are better streamed
-//     (L 8 B 256 T 32: 1.87 against 2.31 ms, L 32 B 256 T 64: 14.7 against 12.3).
+//   H = 1024 (fp16 data) holds four layers on the chip at a time, a pass over them takes some 3.6 us a step and block of 32 rows,
+//     and the streamed cells 5 us a step and layer per 256 rows, not below 12 layers' (T 64, ms, exchange and streamed: L 9
+//     B 256 4.21, 3.86; L 12 B 256 5.47, 4.49; L 16 B 192 5.58, 5.22, B 160 4.67, 5.09; L 20 B 192 7.01, 6.69, B 160 5.85,
+//     6.58; L 32 B 256 14.8, 10.5, B 192 11.2, 10.3, B 160 9.33, 10.17; T 32 L 8 B 256 1.85, 1.89).  Ragged batches run a launch per
+//     stage there, without the layers of the next stage to fill it.
 // FTK_LSTM_EXCHANGE=1 / =0 in the environment forces the one or the other.
-static bool exchange_chosen(int L, int T, int B, int H, const int* dil, bool half) {
+static bool exchange_chosen(int L, int T, int B, int H, const int* dil, bool half, bool ragged) {
   if (!exchange_takes(H, half) || !exchange_fits(T, B, H, half)) return false;
   if (const char* e = getenv("FTK_LSTM_EXCHANGE")) return e[0] == '1';
   if (exchange_one_block(L, B, H, half)) return true;
@@ -1817,7 +1821,7 @@ static bool exchange_chosen(int L, int T, int B, int H, const int* dil, bool hal
       if (dil[l] != 1) return false;
     return L * ((B + 31) / 32) < 112;
   }
-  if (H == 1024) return L < 12 || B <= 192;
+  if (H == 1024) return ragged ? L < 12 || B <= 192 : 7ll * ((L + 3) / 4) * ((B + 31) / 32) <= 10ll * std::max(L, 12) * ((B + 255) / 256);
   return true;
 }
 
@@ -1839,7 +1843,7 @@ static int run_stack(const char* who, const float* xs, const float* WU, const fl
                     who, t, active[t], t - 1, active[t - 1]);
     }
   }
-  if (products == FTK_LSTM_PRODUCTS_F16X3 && exchange_chosen(L, T, B, H, dil, false) && ws && ws_bytes >= exchange_workspace_bytes(L, T, B, H, false)) {
+  if (products == FTK_LSTM_PRODUCTS_F16X3 && exchange_chosen(L, T, B, H, dil, false, active != nullptr) && ws && ws_bytes >= exchange_workspace_bytes(L, T, B, H, false)) {
     bool handled = false;
     rc = run_exchange(false, xs, WU, bias, dil, active, hsss, csss, L, T, B, H, ws, ws_bytes, s, &handled, spin_limit);
     if (rc || handled) return rc;
@@ -1913,8 +1917,8 @@ size_t ftk_stacked_lstm_workspace_bytes(int L, int T, int B, int H) {
 
 size_t ftk_stacked_lstm_f16_workspace_bytes(int L, int T, int B, int H) {
   if (L <= 0 || T <= 0 || B <= 0 || H <= 0) return 0;
-  // the status block and the re-laid weights of the streaming kernel
-  const size_t packed = std::max(ftk::kStatusBytes + (size_t)L * 2 * H * 4 * H * sizeof(_Float16),
+  // the status block, the re-laid weights and the counters of the streaming kernel
+  const size_t packed = std::max(ftk::wavefront_f16_workspace_bytes(L, T, H),
                                  ftk::exchange_takes(H, true) ? ftk::exchange_workspace_bytes(L, T, B, H, true) : (size_t)0);
   if (!ftk::f16_fits_on_chip(B, H)) return packed;
   // which of the two runs is decided per call (a ragged batch stays with the persistent kernel): room for either
@@ -1944,13 +1948,13 @@ int ftk_stacked_lstm_f16(const void* xs, const void* WU, const float* bias, cons
       if (t > 0 && active_rows[t] > active_rows[t - 1])
         return fail(FTK_ERR_INVALID_ARGUMENT, "%s: active_rows must be non-increasing (rows sorted by length)", who);
     }
-  if (exchange_chosen(L, T, B, H, dilations, true) && workspace && workspace_bytes >= exchange_workspace_bytes(L, T, B, H, true)) {
+  if (exchange_chosen(L, T, B, H, dilations, true, active_rows != nullptr) && workspace && workspace_bytes >= exchange_workspace_bytes(L, T, B, H, true)) {
     bool handled = false;
     const int rcx = run_exchange(true, xs, WU, bias, dilations, active_rows, hsss, csss, L, T, B, H, workspace, workspace_bytes,
                                  (hipStream_t)stream, &handled, 0);
     if (rcx || handled) return rcx;
   }
-  // every other shape streams the weights, one launch per stage of independent cells (dead rows are computed too)
+  // every other shape streams the weights, in one launch or one per stage of independent cells (lstm_cell.hip)
   // (the workspace takes the weights re-laid per unit block, so that a workgroup reads one contiguous run)
   if (!on_chip) {
     const size_t need = ftk_stacked_lstm_f16_workspace_bytes(L, T, B, H);
@@ -1960,8 +1964,7 @@ int ftk_stacked_lstm_f16(const void* xs, const void* WU, const float* bias, cons
                        (size_t)(kStatusBytes / sizeof(int)));  // nothing below waits: the status word is zero
     int rcz = check_launch("fill_zero_kernel");
     if (rcz) return rcz;
-    return run_wavefront_f16(xs, WU, bias, dilations, active_rows, hsss, csss, L, T, B, H,
-                             reinterpret_cast<char*>(workspace) + kStatusBytes, (hipStream_t)stream);
+    return run_wavefront_f16(xs, WU, bias, dilations, active_rows, hsss, csss, L, T, B, H, workspace, (hipStream_t)stream);
   }
   const void* fn = nullptr;
   int slots = 0;

@@ -1518,3 +1518,32 @@ def test_flash_attention_f32_key_groups_and_planes(core, B, Hd, Sq, Skv, D):
         O = core.flash_attention_f32(dev(Q), dev(K2), dev(V), D ** -0.5).cpu().numpy()
         for h in range(Hd):                                  # each head on its own: a sum of weights times fp32 values
             assert ko.max_rel_err(O[:, h], ref[:, h]) <= 1e-5
+
+
+@pytest.mark.parametrize('H,L,T,B,dil', [
+    (64, 1, 1, 1, None),                   # a single tile
+    (64, 3, 40, 5, None),                  # fewer layers than queues, a long chain
+    (128, 40, 3, 257, None),               # more layers than steps; two row blocks
+    (192, 5, 9, 70, [1, 3, 2, 20, 1]),     # a dilation beyond the last step
+    (320, 9, 9, 300, None),                # as many layers as steps
+    (1024, 10, 4, 200, None),
+])
+def test_streamed_f16_stack_in_one_launch(core, monkeypatch, H, L, T, B, dil):
+    """The fp16 stack whose tiles wait for each other in one launch has the bits of a launch per stage of cells, three times on
+    one workspace and the same outputs; an output that does not start at a cache line takes the launches."""
+    monkeypatch.setenv('FTK_LSTM_EXCHANGE', '0')
+    monkeypatch.setenv('FTK_LSTM_F16_STREAM', '1')
+    xs, WU, bs = (dev(a) for a in lstm_inputs(79, L, T, B, H, 1.0 / np.sqrt(H)))
+    xs, WU = xs.half(), WU.half()
+    ws = torch.full((int(core.lib.ftk_stacked_lstm_f16_workspace_bytes(L, T, B, H)),), 0x5a, dtype=torch.uint8, device='cuda')
+    monkeypatch.setenv('FTK_LSTM_F16_FLOW', '0')
+    ref = core.stacked_lstm_f16(xs, WU, bs, dilations=dil)
+    assert all(torch.isfinite(r).all() for r in ref)
+    monkeypatch.setenv('FTK_LSTM_F16_FLOW', '1')
+    n = L * T * B * H
+    for shift in (0, 0, 0, 8):
+        flat = [torch.full((n + 8,), float('nan'), dtype=torch.float16, device='cuda') for _ in range(2)]
+        out = tuple(f[shift:shift + n].view(L, T, B, H) for f in flat)
+        core.stacked_lstm_f16(xs, WU, bs, dilations=dil, out=out, workspace=ws)
+        assert core.persistent_status(ws) == 0
+        assert all(torch.equal(a, b) for a, b in zip(out, ref))
