@@ -68,8 +68,7 @@ __global__ __launch_bounds__(256) void b2b_gemm_kernel(const _Float16* __restric
   const int hh = lane >> 5;
 
   // consecutive logical ids land on one XCD (hardware deals workgroups round-robin over 8 XCDs)
-  int id = blockIdx.x;
-  if ((gr.total & 7) == 0) id = (blockIdx.x & 7) * (gr.total >> 3) + (blockIdx.x >> 3);
+  const int id = xcd_consecutive(blockIdx.x, gr.total);
   const int part = id % gr.per_problem;
   const int pt_idx = (id / gr.per_problem) % gr.ptiles;
   const int g = id / (gr.per_problem * gr.ptiles);
@@ -303,8 +302,7 @@ __global__ __launch_bounds__(512) void b2b_gemm8_kernel(const _Float16* __restri
   const int j = lane & 31;
   const int hh = lane >> 5;
 
-  int id = blockIdx.x;
-  if ((gr.total & 7) == 0) id = (blockIdx.x & 7) * (gr.total >> 3) + (blockIdx.x >> 3);
+  const int id = xcd_consecutive(blockIdx.x, gr.total);
   const int part = id % gr.per_problem;
   const int pt_idx = (id / gr.per_problem) % gr.ptiles;
   const int g = id / (gr.per_problem * gr.ptiles);

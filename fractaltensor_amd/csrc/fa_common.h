@@ -10,13 +10,6 @@ constexpr int FA_KT = 64;          // keys per tile
 
 typedef short v4s __attribute__((ext_vector_type(4)));
 
-// Workgroups are dealt to the 8 XCDs in turn; the index that makes those of one XCD neighbours, for any grid (XCD x has the
-// x-th share of the indexes, the first `total` % 8 shares one more than the others).
-__device__ __forceinline__ int xcd_consecutive(int block, int total) {
-  const int x = block & 7;
-  return x * (total >> 3) + min(x, total & 7) + (block >> 3);
-}
-
 // 16 bytes per lane from global memory (wave-uniform base + per-lane byte
 // offset) straight into LDS at lds_base + 16*lane (lds_base wave-uniform).
 // Issued as opaque assembly on purpose: the compiler would otherwise wait for

@@ -73,8 +73,13 @@ int launch_resident(const void* fn, dim3 grid, dim3 block, void** args, size_t l
       if (capture != hipStreamCaptureStatusNone) d.cooperative = true;
     }
     if (!d.cooperative && d.used && d.stream != s) {
-      const hipError_t e = hipStreamQuery(d.stream);
-      if (e == hipErrorNotReady) {
+      // (a stream under capture must not be asked: that would end its capture; nothing can be put behind it either)
+      if (hipStreamIsCapturing(d.stream, &capture) != hipSuccess) (void)hipGetLastError();
+      const bool capturing = capture != hipStreamCaptureStatusNone;
+      const hipError_t e = capturing ? hipSuccess : hipStreamQuery(d.stream);
+      if (capturing) {
+        d.cooperative = true;
+      } else if (e == hipErrorNotReady) {
         (void)hipGetLastError();
         hipEvent_t behind;
         FTK_HIP(hipEventCreateWithFlags(&behind, hipEventDisableTiming));

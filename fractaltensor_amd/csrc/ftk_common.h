@@ -124,6 +124,14 @@ __device__ __forceinline__ void static_for(F&& f) {
   }
 }
 
+// ---- placement
+// Workgroups are dealt to the 8 XCDs in turn; the index that makes those of one XCD neighbours, for any grid (XCD x has the
+// x-th share of the indexes, the first `total` % 8 shares one more than the others).
+__device__ __forceinline__ int xcd_consecutive(int block, int total) {
+  const int x = block & 7;
+  return x * (total >> 3) + min(x, total & 7) + (block >> 3);
+}
+
 // ---- device math ------------------------------------------------------------
 // exp through the hardware base-2 exponential (about 1 ulp), reciprocal through
 // v_rcp_f32 (1 ulp).  sigmoid is accurate to a few 1e-7 relative everywhere.
