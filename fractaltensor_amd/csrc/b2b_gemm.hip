@@ -553,7 +553,7 @@ static int launch_b2b8(const void* A, const void* B, const void* C, void* D, int
   return check_launch("b2b_gemm8_kernel");
 }
 
-// Wide-N form (N = 256 or 512, K and P 64 or 128), built for the shapes of the reference's own benchmark, [M, 64] x [64, 256 | 512] x [., 64]
+// Wide-N form (N = 256 or 512, K 64 or 128, P 64 or a multiple of 128), built for the shapes of the reference's own benchmark, [M, 64] x [64, 256 | 512] x [., 64]
 // (benchmarks/fused_two_hgemms/fractaltensor/fused_two_hgemms.cu:152-175): one problem, few bytes (2 to 4.5 MB that
 // stay in the caches), so what counts is the length of the dependency chain and how many cache lines a workgroup
 // touches.  The WAVES waves of a workgroup split N: wave w forms the 32*NTW columns [n0, n0 + 32 NTW) of P for a
@@ -568,7 +568,7 @@ template <int KS, int PT, int NTW, int WAVES>
 __global__ __launch_bounds__(WAVES * 64) void b2b_wide_kernel(const _Float16* __restrict__ A,
                                                               const _Float16* __restrict__ Bm,
                                                               const _Float16* __restrict__ Cm, _Float16* __restrict__ D,
-                                                              int M, int units, int per) {
+                                                              int M, int units, int per, int P_all) {
   constexpr int K = 16 * KS;
   constexpr int N = 32 * NTW * WAVES;
   constexpr int P = 32 * PT;
@@ -588,14 +588,14 @@ __global__ __launch_bounds__(WAVES * 64) void b2b_wide_kernel(const _Float16* __
   const int wave = tid >> 6;
   const int j = lane & 31;
   const int hh = lane >> 5;
-  const int g = blockIdx.x / per;
-  const int part = blockIdx.x - g * per;
+  const int id = xcd_consecutive(blockIdx.x, gridDim.x), ptiles = P_all / P;
+  const int part = id % per, p0 = id / per % ptiles * P, g = id / (per * ptiles);
   const int n0 = wave * 32 * NTW;
 
   const _Float16* Ag = A + (size_t)g * M * K;
   const _Float16* Bg = Bm + (size_t)g * N * K;
-  const _Float16* Cg = Cm + (size_t)g * P * N;
-  _Float16* Dg = D + (size_t)g * M * P;
+  const _Float16* Cg = Cm + ((size_t)g * P_all + p0) * N;
+  _Float16* Dg = D + (size_t)g * M * P_all + p0;
 
   // ---- B, C and the first A unit: every load requested before the first is used
   constexpr int nb = N * CPR, nc = P * (N / 8);
@@ -720,7 +720,7 @@ __global__ __launch_bounds__(WAVES * 64) void b2b_wide_kernel(const _Float16* __
       }
       if (r0 + r < M) {
         const v4h o = {(_Float16)sum[0], (_Float16)sum[1], (_Float16)sum[2], (_Float16)sum[3]};
-        __builtin_nontemporal_store(o, reinterpret_cast<v4h*>(Dg + (size_t)(r0 + r) * P + 4 * c4));
+        __builtin_nontemporal_store(o, reinterpret_cast<v4h*>(Dg + (size_t)(r0 + r) * P_all + 4 * c4));
       }
     }
     if (next < units) park_a(buf ^ 1);
@@ -730,16 +730,17 @@ __global__ __launch_bounds__(WAVES * 64) void b2b_wide_kernel(const _Float16* __
 }
 
 template <int KS, int PT, int NTW, int WAVES>
-static int launch_b2b_wide(const void* A, const void* B, const void* C, void* D, int G, int M, int cus, int lds_max,
+static int launch_b2b_wide(const void* A, const void* B, const void* C, void* D, int G, int M, int P_all, int cus, int lds_max,
                            bool* handled, hipStream_t s) {
   constexpr int K = 16 * KS, N = 32 * NTW * WAVES, P = 32 * PT;
   const size_t loop_bytes = (size_t)2 * 32 * (K + 8) * 2 + (size_t)WAVES * 32 * (P + 4) * sizeof(float);
   const size_t stage_bytes = std::max((size_t)N * (K + 8) * 2, (size_t)P * (N + 4) * 2);
   const size_t lds = std::max(loop_bytes, stage_bytes);
   const long long units = (M + 31) / 32;
+  const long long pieces = (long long)G * (P_all / P);
   // enough workgroups to fill the chip once; each walks its share of the units with B and C fragments in registers
-  const long long per = std::max(1LL, std::min(units, (long long)cus / std::max(1, G)));
-  *handled = (int)lds <= lds_max && per * G <= 0x7fffffffLL;
+  const long long per = std::max(1LL, std::min(units, (long long)cus / std::max(1LL, pieces)));
+  *handled = (int)lds <= lds_max && per * pieces <= 0x7fffffffLL;
   if (!*handled) return FTK_OK;
   static DeviceOnce attr_once;
   unsigned attr_bit;
@@ -747,8 +748,8 @@ static int launch_b2b_wide(const void* A, const void* B, const void* C, void* D,
     FTK_HIP(hipFuncSetAttribute((const void*)b2b_wide_kernel<KS, PT, NTW, WAVES>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     attr_once.done(attr_bit);
   }
-  hipLaunchKernelGGL((b2b_wide_kernel<KS, PT, NTW, WAVES>), dim3((unsigned)(per * G)), dim3(WAVES * 64), lds, s,
-                     (const _Float16*)A, (const _Float16*)B, (const _Float16*)C, (_Float16*)D, M, (int)units, (int)per);
+  hipLaunchKernelGGL((b2b_wide_kernel<KS, PT, NTW, WAVES>), dim3((unsigned)(per * pieces)), dim3(WAVES * 64), lds, s,
+                     (const _Float16*)A, (const _Float16*)B, (const _Float16*)C, (_Float16*)D, M, (int)units, (int)per, P_all);
   return check_launch("b2b_wide_kernel");
 }
 
@@ -942,27 +943,28 @@ extern "C" int ftk_b2b_gemm_f16(const void* A, const void* B, const void* C, voi
   int rc = device_props(&dp);
   if (rc) return rc;
   hipStream_t s = (hipStream_t)stream;
-  const bool fast = b2b_fits_fused(N, K, P, dp->lds_optin);
-  if (!fast) return launch_b2b_stream(A, B, C, D, G, M, N, K, P, dp->lds_optin, s);
-  // wide N with few columns of D (the reference benchmark's shapes): N split over the waves of a workgroup.
-  // FTK_B2B_WIDE=0 keeps them on the general kernel.
+  // wide N (the reference benchmark's shapes among them): N split over the waves of a workgroup, whose registers hold B and
+  // 64 or 128 rows of C; every 128 columns of D are formed by workgroups of their own, which repeat the first product.  Against the
+  // kernel that keeps B and C in LDS 1 x [16384,128,256,256] 30.9 -> 10.7 us, 19 x [2222,64,256,256] 33 -> 22; against the general one,
+  // which takes what LDS does not hold (N = 512), 3 x [16384,128,512,256] 98 -> 36 us, 1 x [600,128,512,128] 13 -> 7.  FTK_B2B_WIDE=0 keeps them there.
   static const bool allow_wide = !(getenv("FTK_B2B_WIDE") && atoi(getenv("FTK_B2B_WIDE")) == 0);
-  if (allow_wide && (K == 64 || K == 128) && (P == 64 || P == 128) && (N == 256 || N == 512)) {
+  if (allow_wide && (K == 64 || K == 128) && (P == 64 || P % 128 == 0) && (N == 256 || N == 512)) {
     bool handled = false;
     const int cus = dp->cus, lds = dp->lds_optin;
-    const int sel = (K == 128) * 4 + (P == 128) * 2 + (N == 512);
+    const int sel = (K == 128) * 4 + (P != 64) * 2 + (N == 512);
     switch (sel) {
-      case 0: rc = launch_b2b_wide<4, 2, 1, 8>(A, B, C, D, G, M, cus, lds, &handled, s); break;
-      case 1: rc = launch_b2b_wide<4, 2, 2, 8>(A, B, C, D, G, M, cus, lds, &handled, s); break;
-      case 2: rc = launch_b2b_wide<4, 4, 1, 8>(A, B, C, D, G, M, cus, lds, &handled, s); break;
-      case 3: rc = launch_b2b_wide<4, 4, 2, 8>(A, B, C, D, G, M, cus, lds, &handled, s); break;
-      case 4: rc = launch_b2b_wide<8, 2, 1, 8>(A, B, C, D, G, M, cus, lds, &handled, s); break;
-      case 5: rc = launch_b2b_wide<8, 2, 2, 8>(A, B, C, D, G, M, cus, lds, &handled, s); break;
-      case 6: rc = launch_b2b_wide<8, 4, 1, 8>(A, B, C, D, G, M, cus, lds, &handled, s); break;
-      default: rc = launch_b2b_wide<8, 4, 2, 8>(A, B, C, D, G, M, cus, lds, &handled, s); break;
+      case 0: rc = launch_b2b_wide<4, 2, 1, 8>(A, B, C, D, G, M, P, cus, lds, &handled, s); break;
+      case 1: rc = launch_b2b_wide<4, 2, 2, 8>(A, B, C, D, G, M, P, cus, lds, &handled, s); break;
+      case 2: rc = launch_b2b_wide<4, 4, 1, 8>(A, B, C, D, G, M, P, cus, lds, &handled, s); break;
+      case 3: rc = launch_b2b_wide<4, 4, 2, 8>(A, B, C, D, G, M, P, cus, lds, &handled, s); break;
+      case 4: rc = launch_b2b_wide<8, 2, 1, 8>(A, B, C, D, G, M, P, cus, lds, &handled, s); break;
+      case 5: rc = launch_b2b_wide<8, 2, 2, 8>(A, B, C, D, G, M, P, cus, lds, &handled, s); break;
+      case 6: rc = launch_b2b_wide<8, 4, 1, 8>(A, B, C, D, G, M, P, cus, lds, &handled, s); break;
+      default: rc = launch_b2b_wide<8, 4, 2, 8>(A, B, C, D, G, M, P, cus, lds, &handled, s); break;
     }
     if (rc || handled) return rc;
   }
+  if (!b2b_fits_fused(N, K, P, dp->lds_optin)) return launch_b2b_stream(A, B, C, D, G, M, N, K, P, dp->lds_optin, s);
   switch (K) {
     case 32: return launch_b2b<2>(A, B, C, D, G, M, N, P, dp->cus, dp->lds_optin, s);
     case 64: return launch_b2b<4>(A, B, C, D, G, M, N, P, dp->cus, dp->lds_optin, s);

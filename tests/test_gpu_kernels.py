@@ -1547,3 +1547,16 @@ def test_streamed_f16_stack_in_one_launch(core, monkeypatch, H, L, T, B, dil):
         core.stacked_lstm_f16(xs, WU, bs, dilations=dil, out=out, workspace=ws)
         assert core.persistent_status(ws) == 0
         assert all(torch.equal(a, b) for a, b in zip(out, ref))
+
+
+@pytest.mark.parametrize('G,M,N,K,P', [(1, 1, 256, 64, 256), (3, 33, 512, 128, 256), (2, 700, 256, 128, 384), (5, 65, 512, 64, 128), (300, 40, 256, 64, 256)])
+def test_b2b_gemm_wide_with_several_column_tiles(core, G, M, N, K, P):
+    """N split over the waves of a workgroup, D in tiles of 128 columns: one row, rows beyond a unit of 32, more pieces than
+    compute units.  Against float64 with the intermediate rounded to fp16."""
+    rng = np.random.default_rng(41)
+    A = (rng.standard_normal((G, M, K)) / np.sqrt(K)).astype(np.float16)
+    B, C = rng.standard_normal((G, N, K)).astype(np.float16), (rng.standard_normal((G, P, N)) / np.sqrt(N)).astype(np.float16)
+    D = core.b2b_gemm(dev(A), dev(B), dev(C)).float().cpu().numpy()
+    ref = np.matmul(np.matmul(A.astype(np.float64), B.astype(np.float64).transpose(0, 2, 1)).astype(np.float16).astype(np.float64),
+                    C.astype(np.float64).transpose(0, 2, 1))
+    assert ko.max_rel_err(D, ref) <= F16_TOL
