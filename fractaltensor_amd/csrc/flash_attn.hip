@@ -670,7 +670,9 @@ __global__ __launch_bounds__(512, 1) void flash_attn_pp_kernel(const _Float16* _
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int group = wave >> 2, cw = wave & 3;
   const int j = lane & 31, hh = lane >> 5;
-  int id = xcd_consecutive(blockIdx.x, gridDim.x);
+  int id = blockIdx.x;
+  const int total = gridDim.x;
+  if ((total & 7) == 0) id = (blockIdx.x & 7) * (total >> 3) + (blockIdx.x >> 3);
   const int bh = id / nqb;
   const int qb = id - bh * nqb;
   const int q_base = qb * 256 + wave * 32;
@@ -1202,7 +1204,7 @@ static int launch_fa_split(const void* Q, const void* K, const void* V, void* O,
   return launch_merge<D>(part_o, part_ml, O, nparts, Sq, rows, s);
 }
 
-// Tuning hook: FTK_FA_VARIANT=1|3 pins the tiling variant (read once).
+// Tuning hook: FTK_FA_VARIANT=1|2|3 pins the tiling variant (read once).
 static int fa_variant_override() {
   static int v = -1;
   if (v < 0) {
@@ -1288,6 +1290,7 @@ extern "C" int ftk_flash_attn_f16(const void* Q, const void* K, const void* V, v
   // the chip, and also on smaller grids once there are 512 keys or more (B2 H12 S2048 D64 33 against 49 us); with few
   // keys a launch is its own latency and the 128-row blocks spread a short problem over more compute units.
   int variant = fa_variant_override();
+  if (variant == 2 && Skv <= FA_KT) variant = 1;   // a key group walks at least one tile
   if (variant == 0 && (long long)((Sq + 127) / 128) * bh <= dp->cus && Skv > 2 * FA_KT) variant = 2;
   if (variant == 0) variant = ((long long)((Sq + 255) / 256) * bh >= dp->cus || Skv >= 512) ? 3 : 1;
   const int lds = dp->lds_optin;
