@@ -34,7 +34,7 @@
 namespace ftk {
 
 constexpr int kMaxCellsPerLaunch = 40;
-constexpr int kFlowLayers = 64;   // layers of a stack that runs as one launch (lstm_cell_flow_kernel)
+constexpr int kFlowLayers = 48;   // layers of a stack that runs as one launch (lstm_cell_flow_kernel): counters in the status block
 
 struct CellDesc {
   const float* x;       // [B, I]
@@ -713,7 +713,8 @@ __global__ __launch_bounds__(256, 1) void lstm_cell_tile_kernel(CellListH list, 
 // the compute units leaves some idle: 158 rounds of tiles instead of 128 at L 32 T 64 B 256 H 1024, and 95 gaps between
 // launches (11.2 -> 10.5 ms; L 20 T 64 B 230 8.8 -> 6.8).  What is left is a tile of 73 us where a compute unit with the
 // chip to itself takes 46: every tile has 1 MB of weights of its own to fetch, 3.5 TB/s with all of them at it.  Here a workgroup takes one tile after another, of the cells in the order of their stages (l + t), waits until
-// the cells below and before it are complete (done counts a cell's finished tiles), and publishes its own.
+// the cells below and before it are complete, and publishes its own.  A counter per layer is enough: a layer's cells follow
+// each other (d = 1), so cell t is complete when (t + 1) cells' tiles are counted.
 //
 // Eight queues, cell k in queue k % 8, a workgroup takes from the queue of its place among the XCDs: a cell's tiles share
 // an L2 copy of its activations.  A workgroup holds one ticket, taken in order, and waits only for cells earlier in the
@@ -730,10 +731,9 @@ struct FlowArgs {
   _Float16* hsss;
   _Float16* csss;
   int* status;
-  int* tickets;   // [8], 64 bytes apart
-  int* done;      // [L][T]
+  int* tickets;   // [8]
+  int* done;      // [L]: finished tiles of the layer
   int L, T, B, H, spin_limit;
-  int dil[kFlowLayers];
 };
 // Cell k of a stack of L layers and T steps in the order of the stages l + t, low layers first: its layer and step.
 __host__ __device__ inline void flow_cell(int k, int L, int T, int* l, int* t) {
@@ -773,16 +773,16 @@ __global__ __launch_bounds__(256, 1) void lstm_cell_flow_kernel(FlowArgs) {
     if (threadIdx.x < 64) {
       int l = -1, t = 0, tile = 0;
       if (threadIdx.x == 0) {
-        const int ticket = __hip_atomic_fetch_add(a.tickets + 16 * q, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const int ticket = __hip_atomic_fetch_add(a.tickets + q, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         if (ticket < mine) {
           tile = ticket % tiles;
           flow_cell(q + 8 * (ticket / tiles), L, T, &l, &t);
-          const int d = a.dil[l];
-          const int* const below = l > 0 ? a.done + (l - 1) * T + t : nullptr;
-          const int* const before = t >= d ? a.done + l * T + t - d : nullptr;
+          const int* const below = a.done + max(l - 1, 0);
+          const int* const before = a.done + l;
+          const int of_below = l > 0 ? (t + 1) * tiles : 0, of_before = t * tiles;
           for (int n = 1;; ++n) {
-            const bool there = (!below || __hip_atomic_load(below, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == tiles) &&
-                               (!before || __hip_atomic_load(before, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == tiles);
+            const bool there = __hip_atomic_load(below, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= of_below &&
+                               __hip_atomic_load(before, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= of_before;
             if (there) break;
             if (n >= a.spin_limit || ((n & 255) == 0 && __hip_atomic_load(a.status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0)) {
               __hip_atomic_store(a.status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -802,16 +802,15 @@ __global__ __launch_bounds__(256, 1) void lstm_cell_flow_kernel(FlowArgs) {
     const int tile = __builtin_amdgcn_readfirstlane(word[2]);
     __syncthreads();   // the words are read: the tile's copies may take their place
     if (l < 0) return;
-    const int d = a.dil[l];
     CellDescH cd;
     cd.x = l == 0 ? a.xs + (size_t)t * cell : a.hsss + ((size_t)(l - 1) * T + t) * cell;
-    cd.h_prev = t >= d ? a.hsss + ((size_t)l * T + t - d) * cell : nullptr;
-    cd.c_prev = t >= d ? a.csss + ((size_t)l * T + t - d) * cell : nullptr;
+    cd.h_prev = t > 0 ? a.hsss + ((size_t)l * T + t - 1) * cell : nullptr;
+    cd.c_prev = t > 0 ? a.csss + ((size_t)l * T + t - 1) * cell : nullptr;
     cd.WU = a.WU + (size_t)l * 8 * H * H;
     cd.bias = a.bias ? a.bias + (size_t)l * 4 * H : nullptr;
     cd.h = a.hsss + ((size_t)l * T + t) * cell;
     cd.c = a.csss + ((size_t)l * T + t) * cell;
-    int* const done = a.done + l * T + t;
+    int* const done = a.done + l;
     cell_tile<true>(cd, B, H, tile / nub, tile % nub);
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");   // h and c of this wave are in memory
     __syncthreads();
@@ -1021,12 +1020,11 @@ static int launch_cells(const CellList& list, int B, int I, int H, hipStream_t s
 
 // WU [n_layers, K2, 4H] -> per layer and block ub of UB hidden units the [K2][4*UB] tile the cell kernel keeps
 // in LDS: row k holds chunks of 8 columns, chunk 4*ug + q = gate q of units UB*ub + 8*ug .. +8, stored in slot
-// chunk ^ ((k & 3) << 2).  One thread per 16-byte chunk.  Clears nclear words on the way, for the launch behind it.
+// chunk ^ ((k & 3) << 2).  One thread per 16-byte chunk.
 __global__ __launch_bounds__(256) void lstm_pack_weights_f16_kernel(const _Float16* __restrict__ WU,
                                                                     _Float16* __restrict__ packed, size_t chunks,
-                                                                    int K2, int H, int UB, int* clear, int nclear) {
+                                                                    int K2, int H, int UB) {
   const size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x;
-  for (size_t i = idx; i < (size_t)nclear; i += (size_t)gridDim.x * 256) clear[i] = 0;
   if (idx >= chunks) return;
   const int per_row = H / 2;  // 4H / 8
   const int n8 = (int)(idx % per_row);
@@ -1044,10 +1042,10 @@ __global__ __launch_bounds__(256) void lstm_pack_weights_f16_kernel(const _Float
 // Hidden units per workgroup of the streaming kernel at hidden size H.
 static int cell_unit_block(int H) { return H % 64 == 0 ? 64 : 32; }
 
-static int pack_weights_f16(const void* WU, void* packed, int layers, int K2, int H, int* clear, int nclear, hipStream_t s) {
+static int pack_weights_f16(const void* WU, void* packed, int layers, int K2, int H, hipStream_t s) {
   const size_t chunks = (size_t)layers * K2 * (H / 2);
   hipLaunchKernelGGL(lstm_pack_weights_f16_kernel, dim3((unsigned)((chunks + 255) / 256)), dim3(256), 0, s,
-                     (const _Float16*)WU, (_Float16*)packed, chunks, K2, H, cell_unit_block(H), clear, nclear);
+                     (const _Float16*)WU, (_Float16*)packed, chunks, K2, H, cell_unit_block(H));
   return check_launch("lstm_pack_weights_f16_kernel");
 }
 
@@ -1170,34 +1168,40 @@ int run_wavefront(const float* xs, const float* WU, const float* bias, const int
   return run_wavefront_of<float, CellList>(xs, WU, bias, dil, hsss, csss, L, T, B, H, s);
 }
 
-constexpr size_t kFlowTicketBytes = 8 * 64;
-static size_t packed_f16_bytes(int L, int H) { return (size_t)L * 2 * H * 4 * H * sizeof(_Float16); }
-size_t wavefront_f16_workspace_bytes(int L, int T, int H) {
-  return kStatusBytes + packed_f16_bytes(L, H) + kFlowTicketBytes + (size_t)L * T * sizeof(int);
-}
-
-// The same schedule over fp16 arrays (H a multiple of 32).  ws: status block (cleared by the caller), the weights re-laid
-// per unit block, the tickets and counters of the single launch.
+// The same schedule over fp16 arrays (H a multiple of 32).  ws: status block (cleared by the caller; words 8 .. 15 are the
+// tickets of the single launch, words 16 .. its counters), then the weights re-laid per unit block.
+constexpr int kFlowTicketsAt = 8, kFlowDoneAt = 16;
+static_assert((kFlowDoneAt + kFlowLayers) * sizeof(int) <= kStatusBytes, "tickets and counters fit the status block");
 int run_wavefront_f16(const void* xs, const void* WU, const float* bias, const int* dil, const int* active, void* hsss,
                       void* csss, int L, int T, int B, int H, void* ws, hipStream_t s) {
   char* const packed = reinterpret_cast<char*>(ws) + kStatusBytes;
-  int* const tickets = reinterpret_cast<int*>(packed + packed_f16_bytes(L, H));
   const DeviceProps* dp = nullptr;
   int rc = device_props(&dp);
   if (rc) return rc;
-  // One launch where the tile kernel runs and the cells of h and c start at cache lines (H a multiple of 64, and the
-  // arrays' starts); a ragged batch stays with the launches, which leave out the row blocks that have ended.  A stage with less than half
-  // a chip of tiles is bound by its chain, and there a launch per stage hands over sooner than tickets and counters do
-  // (H 1024, B 256, us, launches and one launch: L 4 T 32 1698, 1767; L 8 T 32 1885, 1969; L 10 T 64 4372, 3999; L 12 T 64 4582,
-  // 4489; L 20 T 64 8986, 6693; L 32 T 64 11.2 ms, 10.5 ms).  FTK_LSTM_F16_FLOW=1 / =0 forces the one or the other.
-  const long long stage_tiles = (long long)std::min(L, T) * (H / 64) * ((B + GT - 1) / GT);
-  const char* e = getenv("FTK_LSTM_F16_FLOW");
-  const bool flow = cell_unit_block(H) == 64 && !active && L <= kFlowLayers && stage_tiles * std::max(L, T) < (1ll << 30) &&
-                    (reinterpret_cast<uintptr_t>(hsss) | reinterpret_cast<uintptr_t>(csss)) % 128 == 0 &&
-                    (e ? e[0] == '1' : 2 * stage_tiles > dp->cus);
-  rc = pack_weights_f16(WU, packed, L, 2 * H, H, tickets, flow ? (int)(kFlowTicketBytes / sizeof(int)) + L * T : 0, s);
+  // One launch where the tile kernel runs, the cells of h and c start at cache lines (H a multiple of 64, and the arrays'
+  // starts) and a layer's cells follow each other (no dilation); a ragged batch stays with the launches, which leave out the
+  // row blocks that have ended.  It saves the rounds of tiles that stages leave partly filled, and a tile of it takes some
+  // 5 % longer (the hand-over): chosen where a twelfth of the launches' rounds is saved (H 1024, B 256, T 64, ms, launches and one
+  // launch: L 9 3.79, 4.08; L 12 4.40, 4.53; L 16 B 192, whole rounds, 4.86, 5.29; L 20 B 192 7.43, 6.58; L 24 B 160 8.15,
+  // 7.61; L 32 10.4 .. 11.2, 10.1 .. 10.5).  FTK_LSTM_F16_FLOW=1 / =0 forces the one or the other.
+  const int cell_tiles = (H / 64) * ((B + GT - 1) / GT);
+  bool one_launch = cell_unit_block(H) == 64 && !active && L <= kFlowLayers && (long long)L * T * cell_tiles < (1ll << 30) &&
+                    (reinterpret_cast<uintptr_t>(hsss) | reinterpret_cast<uintptr_t>(csss)) % 128 == 0;
+  for (int l = 0; dil && l < L; ++l) one_launch = one_launch && dil[l] == 1;
+  if (const char* e = getenv("FTK_LSTM_F16_FLOW")) {
+    one_launch = one_launch && e[0] == '1';
+  } else if (one_launch) {
+    double rounds = 0, filled = 0;
+    for (int stage = 0; stage < L + T - 1; ++stage) {
+      const long long tiles = (long long)(std::min(stage, L - 1) - std::max(0, stage - T + 1) + 1) * cell_tiles;
+      rounds += (double)((tiles + dp->cus - 1) / dp->cus);
+      filled += std::max(1.0, (double)tiles / dp->cus);
+    }
+    one_launch = filled * 12 < rounds * 11;
+  }
+  rc = pack_weights_f16(WU, packed, L, 2 * H, H, s);
   if (rc) return rc;
-  if (!flow)
+  if (!one_launch)
     return run_wavefront_of<_Float16, CellListH>((const _Float16*)xs, (const _Float16*)packed, bias, dil, (_Float16*)hsss, (_Float16*)csss, L, T, B,
                                                  H, s, true, active);
   static DeviceOnce attr_once;
@@ -1213,11 +1217,10 @@ int run_wavefront_f16(const void* xs, const void* WU, const float* bias, const i
   a.hsss = (_Float16*)hsss;
   a.csss = (_Float16*)csss;
   a.status = (int*)ws;
-  a.tickets = tickets;
-  a.done = tickets + kFlowTicketBytes / sizeof(int);
+  a.tickets = (int*)ws + kFlowTicketsAt;
+  a.done = (int*)ws + kFlowDoneAt;
   a.L = L; a.T = T; a.B = B; a.H = H;
   a.spin_limit = 1 << 22;
-  for (int l = 0; l < kFlowLayers; ++l) a.dil[l] = l < L && dil ? dil[l] : 1;
   hipLaunchKernelGGL(lstm_cell_flow_kernel, dim3(dp->cus), dim3(256), G_LDS, s, a);
   return check_launch("lstm_cell_flow_kernel");
 }

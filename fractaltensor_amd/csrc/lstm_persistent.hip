@@ -61,7 +61,6 @@ int run_wavefront(const float* xs, const float* WU, const float* bias, const int
                   int L, int T, int B, int H, hipStream_t s);
 int run_wavefront_f16(const void* xs, const void* WU, const float* bias, const int* dil, const int* active, void* hsss,
                       void* csss, int L, int T, int B, int H, void* ws, hipStream_t s);
-size_t wavefront_f16_workspace_bytes(int L, int T, int H);
 size_t split_stack_workspace_bytes(int L, int T, int B, int H);
 int run_wavefront_split(const float* xs, const float* WU, const float* bias, const int* dil, const int* active, float* hsss,
                         float* csss, int L, int T, int B, int H, void* ws, hipStream_t s);
@@ -1917,8 +1916,8 @@ size_t ftk_stacked_lstm_workspace_bytes(int L, int T, int B, int H) {
 
 size_t ftk_stacked_lstm_f16_workspace_bytes(int L, int T, int B, int H) {
   if (L <= 0 || T <= 0 || B <= 0 || H <= 0) return 0;
-  // the status block, the re-laid weights and the counters of the streaming kernel
-  const size_t packed = std::max(ftk::wavefront_f16_workspace_bytes(L, T, H),
+  // the status block and the re-laid weights of the streaming kernel
+  const size_t packed = std::max(ftk::kStatusBytes + (size_t)L * 2 * H * 4 * H * sizeof(_Float16),
                                  ftk::exchange_takes(H, true) ? ftk::exchange_workspace_bytes(L, T, B, H, true) : (size_t)0);
   if (!ftk::f16_fits_on_chip(B, H)) return packed;
   // which of the two runs is decided per call (a ragged batch stays with the persistent kernel): room for either

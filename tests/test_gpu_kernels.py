@@ -1523,8 +1523,10 @@ def test_flash_attention_f32_key_groups_and_planes(core, B, Hd, Sq, Skv, D):
 @pytest.mark.parametrize('H,L,T,B,dil', [
     (64, 1, 1, 1, None),                   # a single tile
     (64, 3, 40, 5, None),                  # fewer layers than queues, a long chain
-    (128, 40, 3, 257, None),               # more layers than steps; two row blocks
-    (192, 5, 9, 70, [1, 3, 2, 20, 1]),     # a dilation beyond the last step
+    (128, 48, 3, 257, None),               # more layers than steps, as many as there are counters; two row blocks
+    (64, 49, 2, 3, None),                  # a layer more: the launches
+    (192, 5, 9, 70, None),                 # fewer tiles in a stage than a queue has takers
+    (192, 3, 9, 70, [1, 3, 20]),           # dilated: the launches
     (320, 9, 9, 300, None),                # as many layers as steps
     (1024, 10, 4, 200, None),
 ])
