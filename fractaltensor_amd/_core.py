@@ -388,8 +388,9 @@ def stacked_lstm_f16(xs, WU, bias=None, dilations: Optional[Sequence[int]] = Non
                      active_rows: Optional[Sequence[int]] = None, check: Optional[bool] = None
                      ) -> Tuple[torch.Tensor, torch.Tensor]:
     """fp16 storage: xs [T,B,H], WU [L,2H,4H] fp16, bias [L,4H] fp32 or None -> hsss, csss [L,T,B,H] fp16.
-    H a multiple of 32: H = 512, and H = 256 with an even batch, run in the persistent kernel, every other
-    shape as one launch of the streaming cell kernel per stage of independent cells."""
+    H a multiple of 32.  H = 256, 512 and 1024 run in one launch per group of layers whose weights the chip holds,
+    where that is faster; every other shape streams its weights through the cell kernels, in one launch or one per stage
+    of independent cells."""
     if active_rows is None:
         done = _fast.stacked_lstm(True, xs, WU, bias, dilations, out, workspace, -1, check, False)
         if done is not None:

@@ -185,17 +185,14 @@ int ftk_stacked_lstm_ragged_f32(const float* xs, const float* WU,
  * The stack with fp16 storage, the numeric form of the reference's CuTe LSTM:
  * xs [T,B,H], WU [L,2H,4H], hsss, csss [L,T,B,H] all fp16 (h and c are rounded
  * to fp16 when written, and read back rounded), bias [L,4H] fp32 or NULL, gate
- * sums accumulated in fp32.  H%32==0.  H = 512 and H = 256 with even B, the
- * first two hidden sizes of the reference's sweep, run in the persistent
- * kernel: fp16 weights of H = 512 take the registers the fp32 weights of
- * H = 256 take; stacks deeper than the chip holds at once (16 layers of
- * H = 512, 32 of H = 256 on 256 compute units) run as consecutive launches.
- * Every other shape (H = 1024, the third size of the sweep, among them) does
- * not fit on chip: its weights are streamed, one launch of the fp16 cell
- * kernel per stage of independent cells, on the rows that live at the cell's
- * step (which is also the faster way for H = 512 stacks of more than 16
- * layers, unless active_rows is given; FTK_LSTM_F16_STREAM=1 / 0 forces
- * either); the
+ * sums accumulated in fp32.  H%32==0.  H = 256, 512 and 1024, the hidden sizes
+ * of the reference's sweep, keep the fp16 weights of as many layers on the
+ * chip as it holds and run deeper stacks as consecutive launches, where that
+ * is the faster way.  Every other shape streams its weights through the fp16
+ * cell kernels, in one launch or in one per stage of independent cells, on the
+ * rows that live at the cell's step (H = 512 stacks of more than 16 layers and
+ * deep H = 1024 stacks of large batches among them;
+ * FTK_LSTM_F16_STREAM=1 / 0 forces either where both can run); the
  * workspace then takes a re-laid copy of WU (ftk_stacked_lstm_f16_workspace_bytes
  * says how much for a shape).
  * dilations, active_rows: host arrays or NULL, as above.
@@ -468,9 +465,10 @@ int ftk_flash_attn_f16(const void* Q, const void* K, const void* V, void* O,
                        ftk_stream_t stream);
 
 /*
- * The same call with a workspace, for grids that do not fill the chip: when
- * batch x heads x (query blocks of 128 rows) covers less than half of the
- * compute units and there are at least 2048 keys, the keys are cut into up to
+ * The same call with a workspace, for grids that do not fill the chip: where
+ * batch x heads x (query blocks of 128 rows; for at most 16 queries: heads
+ * alone) leaves compute units idle and the chain of keys is long enough to pay
+ * for a merge, the keys are cut into up to
  * 64 contiguous parts, every part runs as a workgroup of its own and leaves
  * (reference maximum, sum of exponentials, unnormalised O) in the workspace,
  * and a second launch merges the parts by the rule of an online softmax
