@@ -167,8 +167,12 @@ def _fingerprint(f, level: int = 0, seen=None, looked=None):
     and functions its code reaches through module globals -- so that a layer function, a cell or a scale that is
     redefined at module level under an unchanged caller is a different key.  Other callables (functools.partial,
     callable objects) are keyed on the object itself, which the key then keeps alive; data (tensors) only by kind:
-    operand structure is checked on every call."""
-    seen = set() if seen is None else seen
+    operand structure is checked on every call.
+
+    seen: the functions met so far in this traversal, each with the place it was met at.  One met again stands as that
+    place.  What is kept between calls (of_globals) starts a traversal of its own: a place in a call's traversal may be
+    another function in the next call."""
+    seen = {} if seen is None else seen
     code = getattr(f, '__code__', None)
     if code is None:
         try:
@@ -176,9 +180,13 @@ def _fingerprint(f, level: int = 0, seen=None, looked=None):
         except TypeError:
             return ('unhashable', type(f).__name__, id(f))
         return ('object', f)
-    if id(f) in seen or level > 6:
-        return ('seen', code)
-    seen.add(id(f))
+    if id(f) in seen:
+        return ('seen', seen[id(f)])
+    if level > 6:
+        if looked is not None:
+            looked.functions.append((f, code, getattr(f, '__defaults__', None), getattr(f, '__kwdefaults__', None), []))
+        return ('deep', code)
+    seen[id(f)] = len(seen)
 
     def of_value(v):
         if isinstance(v, _SCALARS):
@@ -221,7 +229,7 @@ def _fingerprint(f, level: int = 0, seen=None, looked=None):
 
     g = getattr(f, '__globals__', None) or {}
 
-    def of_globals(record):
+    def of_globals(record, seen):
         names = []
         for name in _code_names(code):
             v = g.get(name, _MISSING)
@@ -231,12 +239,12 @@ def _fingerprint(f, level: int = 0, seen=None, looked=None):
         return (code, tuple(names))
 
     if looked is not None:               # reached from another function: part of that one's number
-        parts.append(of_globals(looked))
+        parts.append(of_globals(looked, seen))
         return tuple(parts)
     entry = _reached.get((id(code), id(g), level))
     if entry is None or not entry[0].unchanged():
         record = _Seen()
-        n = _number_of(of_globals(record))
+        n = _number_of(of_globals(record, {}))
         entry = (record, n, code, g)      # (code and g are kept alive: their ids stay theirs)
         if record.stable:
             _reached[(id(code), id(g), level)] = entry

@@ -92,6 +92,45 @@ def test_function_fingerprint_follows_module_globals_and_defaults():
     assert dispatch._fingerprint(part) == ('object', part) and dispatch._fingerprint(part) != dispatch._fingerprint(functools.partial(_global_layer))
 
 
+def _reads_global_scale(x):
+    return x * _GLOBAL_SCALE
+
+
+def _calls_helper(x):
+    return _reads_global_scale(x)
+
+
+def test_function_fingerprint_of_a_helper_met_through_a_closure_first():
+    """What a program reaches through module globals is remembered between calls.  A helper that one call met through its
+    closure first must be followed all the same when another call's closure holds another function; and a function met
+    twice is that function, not any other of the same code."""
+    from kaleido.operations import dispatch
+    dispatch.reset()
+
+    def program(inner):
+        return lambda x: inner(_calls_helper(x))
+
+    other = lambda x: x
+    g = globals()
+    saved = g['_GLOBAL_SCALE']
+    try:
+        for first in (_reads_global_scale, _calls_helper):
+            g['_GLOBAL_SCALE'] = saved
+            dispatch._fingerprint(program(first))
+            before = dispatch._fingerprint(program(other))
+            g['_GLOBAL_SCALE'] = saved + 1.0
+            assert dispatch._fingerprint(program(other)) != before
+    finally:
+        g['_GLOBAL_SCALE'] = saved
+
+    scaled = lambda s: (lambda x: x * s)
+    then = lambda f: (lambda x: f(x))
+    pair = lambda a, b, c: (lambda x: a(x) + b(x) + c(x))
+    half, double = scaled(0.5), scaled(2.0)
+    assert dispatch._fingerprint(pair(half, double, then(half))) == dispatch._fingerprint(pair(half, double, then(half)))
+    assert dispatch._fingerprint(pair(half, double, then(half))) != dispatch._fingerprint(pair(half, double, then(double)))
+
+
 def test_kaleido_core_is_the_c_abi_binding():
     """`kaleido._core`, the module name of the reference's native binding (kaleido/__init__.py:20-26), is
     fractaltensor_amd._core."""
