@@ -71,7 +71,7 @@ struct ExchangeArgs {
   int spin_limit;
   int ragged;
   int dil[kXLayers];
-  unsigned short steps_of[kXBlocks];   // ragged: steps row block rb takes part in
+  int steps_of[kXBlocks];   // ragged: steps row block rb takes part in (T reaches 262143 at H = 64)
 };
 
 typedef unsigned long long u64;
@@ -498,7 +498,7 @@ void lstm_exchange_kernel(ExchangeArgs a) {
         it.tile += tiles_t;
         it.row += rows_t;
       }
-    } while (a.ragged && it.t < T && it.t >= (int)a.steps_of[it.rb]);
+    } while (a.ragged && it.t < T && it.t >= a.steps_of[it.rb]);
     return it;
   };
   auto h_at = [&](const Item& it) __attribute__((always_inline)) -> int {
@@ -902,7 +902,7 @@ int run_exchange(bool half, const void* xs, const void* WU, const float* bias, c
       int steps = 0;
       if (a.ragged)
         while (steps < T && active[steps] > block * rb) ++steps;
-      a.steps_of[rb] = (unsigned short)steps;
+      a.steps_of[rb] = steps;
     }
     const int groups = a.units * W;
     const unsigned grid = p.per_xcd ? 8u * p.per_xcd * W : (unsigned)((groups + 7) / 8 * 8);
