@@ -1071,7 +1071,7 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(const float* __restrict
   const int slice = unit % slices;
   const long long row = (long long)blockIdx.x * rb + unit / slices;
   const bool on = unit < rb * slices && row < rows;
-  float m = -INFINITY, l = 0.0f;
+  float m = -3.402823466e38f, l = 0.0f;   // finite: parts without a score (reference -inf) weigh nothing, however many in a row
   v4f acc = {0.f, 0.f, 0.f, 0.f};
   if (on) {
     const long long bh = row / Sq;

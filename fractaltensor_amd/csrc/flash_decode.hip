@@ -25,6 +25,9 @@ namespace ftk {
 
 constexpr int kDecKeys = 32;     // keys of a tile
 constexpr int kDecWaves = 4;
+// The reference before any score: finite, so that a tile whose scores are all -inf weighs nothing (-inf - -inf is a NaN).
+// Every finite score is above it or equal to it, and 2^(kNoRef - score) is zero.
+constexpr float kNoRef = -3.402823466e38f;
 
 // LDS slots of a row's 16-byte chunks: chunk c of row r sits in slot c ^ decode_swizzle(r).  The 16 lanes that an LDS
 // read of 16 bytes serves together hold one chunk of 16 rows; these are then 16 different places of the 256-byte bank line.
@@ -94,7 +97,7 @@ __global__ __launch_bounds__(kDecWaves * 64) void flash_decode_kernel(const _Flo
   v4f o[DT];
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt) o[dt] = v4f{0.f, 0.f, 0.f, 0.f};
-  float ref = -INFINITY, l = 0.0f;
+  float ref = kNoRef, l = 0.0f;
 
   // this wave's tiles: wave, wave + 4, ...
   const int mine = ntiles > wave ? (ntiles - wave + kDecWaves - 1) / kDecWaves : 0;
@@ -193,7 +196,7 @@ __global__ __launch_bounds__(kDecWaves * 64) void flash_decode_kernel(const _Flo
   __syncthreads();
   const int q = tid & 15;
   if (q >= Sq) return;
-  float top = -INFINITY, sum = 0.0f, w[kDecWaves];
+  float top = kNoRef, sum = 0.0f, w[kDecWaves];
 #pragma unroll
   for (int i = 0; i < kDecWaves; ++i) top = fmaxf(top, sml[(i * 16 + q) * 2]);
 #pragma unroll

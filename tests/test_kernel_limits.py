@@ -1,4 +1,4 @@
-"""Kernels at the far ends of what their entry points accept: sequences longer than 16 bits count."""
+"""Kernels at the far ends of what their entry points accept: sequences longer than 16 bits count, scores of -inf."""
 import pytest
 import torch
 
@@ -29,3 +29,36 @@ def test_ragged_stack_longer_than_65535_steps(core, half, H, L):
         assert torch.equal(got[:, :ends], ref[:, :ends])
         assert torch.equal(got[:, ends:, :2], ref[:, ends:, :2])
     assert float(h[:, ends - 1].abs().max()) > 0
+
+
+def _masked_heads(Sq, Skv, D, spans, seed):
+    """One head per span: the keys of the span (start, end) score -inf, through a channel that is 1 in every query and -inf in
+    those keys."""
+    gen = torch.Generator().manual_seed(seed)
+    n = len(spans)
+    q, k, v = (torch.randn((1, n, s, D), generator=gen).half() for s in (Sq, Skv, Skv))
+    q[..., 0] = 1
+    k[..., 0] = 0
+    for i, (a, b) in enumerate(spans):
+        k[0, i, a:b, 0] = float('-inf')
+    scores = q.double() @ k.double().transpose(-1, -2) * D ** -0.5
+    return q.cuda(), k.cuda(), v.cuda(), torch.softmax(scores, -1) @ v.double()
+
+
+@pytest.mark.parametrize('Sq,Skv,D', [
+    (1, 300, 64),          # no parts: tiles of 32 keys dealt to four waves
+    (16, 161, 32),         # the last wave's only tile holds one key
+    (1, 9000, 128),        # many parts, merged several at a time
+    (5, 4097, 96),
+])
+def test_attention_of_few_queries_with_scores_of_minus_infinity(core, Sq, Skv, D):
+    """Keys that score -inf have weight zero wherever they lie: a wave's first tiles, whole parts, all but one key; a row
+    without any finite score is NaN, as a softmax of it is.  Weights and O are rounded to fp16 (2^-11 each)."""
+    spans = [(0, 32), (0, 128), (32, 64), (Skv // 3, Skv), (0, Skv - 1), (1, Skv), (0, 8 * Skv // 9), (0, 0), (0, Skv)]
+    q, k, v, ref = _masked_heads(Sq, Skv, D, spans, 5)
+    for split in (True, False):
+        o = core.flash_attention(q, k, v, split_keys=split).double().cpu()
+        assert bool(torch.isnan(o[:, -1]).all())
+        for i in range(len(spans) - 1):
+            err = float((o[:, i] - ref[:, i]).abs().max() / ref[:, i].abs().max())
+            assert err <= 1e-2, (split, spans[i], err)
