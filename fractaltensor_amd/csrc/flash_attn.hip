@@ -65,6 +65,10 @@ struct FaSwizzled {
 constexpr bool fa_swizzled(int D, int KG) { return D == 128 && KG == 2; }
 
 constexpr float FA_TAU = 8.0f;     // slack (in powers of two) before the running maximum is moved
+// The reference of a key group that has met no finite score: so low that the first one moves it (a reference of 0 would
+// leave scores far below 0 without weight), so small that 24 bits hold score + 1024 to 2^-14, an eighth of what rounding
+// the weights to fp16 costs.
+constexpr float FA_NO_REF = -1024.0f;
 constexpr float FA_PMAX = 32768.0f;  // phase-alternating kernel: a lane's sum of exponentials above this moves the reference
 constexpr int FA_TRACE_TILES = 256;
 
@@ -464,7 +468,7 @@ __global__ __launch_bounds__(WAVES * KG * 64, MINB) void flash_attn_kernel(const
 #pragma unroll
       for (int r = 1; r < 16; ++r) m = fmaxf(m, sa[qt][r]);
       m = max_with_other_half(m);
-      if (KG == 2 && m == -INFINITY) m = 0.0f;   // no score yet: the group's share must come out as nothing, not as a NaN
+      if (KG == 2 && m == -INFINITY) m = FA_NO_REF;   // no score yet: the group's share must come out as nothing, not as a NaN
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         sa[qt][r] -= m;

@@ -31,14 +31,14 @@ def test_ragged_stack_longer_than_65535_steps(core, half, H, L):
     assert float(h[:, ends - 1].abs().max()) > 0
 
 
-def _masked_heads(Sq, Skv, D, spans, seed):
+def _masked_heads(Sq, Skv, D, spans, seed, shift=0.0):
     """One head per span: the keys of the span (start, end) score -inf, through a channel that is 1 in every query and -inf in
-    those keys."""
+    those keys.  All other scores are shifted by about `shift`."""
     gen = torch.Generator().manual_seed(seed)
     n = len(spans)
     q, k, v = (torch.randn((1, n, s, D), generator=gen).half() for s in (Sq, Skv, Skv))
     q[..., 0] = 1
-    k[..., 0] = 0
+    k[..., 0] = shift * D ** 0.5
     for i, (a, b) in enumerate(spans):
         k[0, i, a:b, 0] = float('-inf')
     scores = q.double() @ k.double().transpose(-1, -2) * D ** -0.5
@@ -56,6 +56,26 @@ def test_attention_of_few_queries_with_scores_of_minus_infinity(core, Sq, Skv, D
     without any finite score is NaN, as a softmax of it is.  Weights and O are rounded to fp16 (2^-11 each)."""
     spans = [(0, 32), (0, 128), (32, 64), (Skv // 3, Skv), (0, Skv - 1), (1, Skv), (0, 8 * Skv // 9), (0, 0), (0, Skv)]
     q, k, v, ref = _masked_heads(Sq, Skv, D, spans, 5)
+    for split in (True, False):
+        o = core.flash_attention(q, k, v, split_keys=split).double().cpu()
+        assert bool(torch.isnan(o[:, -1]).all())
+        for i in range(len(spans) - 1):
+            err = float((o[:, i] - ref[:, i]).abs().max() / ref[:, i].abs().max())
+            assert err <= 1e-2, (split, spans[i], err)
+
+
+@pytest.mark.parametrize('shift', [0.0, -40.0])
+@pytest.mark.parametrize('Sq,Skv,D', [
+    (100, 192, 64),        # two key groups of two tiles and one
+    (17, 129, 128),        # the second group's single key
+    (77, 1000, 96),
+    (33, 4097, 128),       # parts of the keys as well
+])
+def test_key_groups_with_scores_of_minus_infinity(core, Sq, Skv, D, shift):
+    """A key group whose first 32 keys score -inf: its other keys count in full also where all scores are far below 0."""
+    half = ((Skv + 63) // 64 + 1) // 2 * 64                  # the first group's keys, where the keys are not cut into parts
+    spans = [(0, 32), (0, 64), (0, half), (half, Skv), (0, Skv - 1), (half, min(half + 32, Skv)), (0, 0), (0, Skv)]
+    q, k, v, ref = _masked_heads(Sq, Skv, D, spans, 6, shift)
     for split in (True, False):
         o = core.flash_attention(q, k, v, split_keys=split).double().cpu()
         assert bool(torch.isnan(o[:, -1]).all())
