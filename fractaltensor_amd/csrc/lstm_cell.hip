@@ -718,8 +718,11 @@ __global__ __launch_bounds__(256, 1) void lstm_cell_tile_kernel(CellListH list, 
 //
 // Eight queues, cell k in queue k % 8, a workgroup takes from the queue of its place among the XCDs: a cell's tiles share
 // an L2 copy of its activations.  A workgroup holds one ticket, taken in order, and waits only for cells earlier in the
-// order: the earliest unfinished tile is always being worked on or about to be taken, whatever part of the grid is
-// resident, so ordinary launches do, next to anything else.  The wait is bounded all the same (status word).
+// order.  One that has waited for long looks whether another queue's next tile is of an earlier cell and due, and computes
+// it first, keeping its ticket: so the earliest unfinished tile is being worked on or about to be taken as long as any
+// workgroup is resident, whatever queue that one takes from (beside another launch that fills an XCD, all workgroups of a
+// queue may have no place yet), and ordinary launches do, next to anything else.  The wait is bounded all the same (status
+// word).
 //
 // h and c are written through to memory, and complete before the tile is counted.  They are read through the caches:
 // nothing of a cell is read before it is complete, and a cell starts at a cache line (the host looks), so no cache holds
@@ -734,6 +737,7 @@ struct FlowArgs {
   int* tickets;   // [8]
   int* done;      // [L]: finished tiles of the layer
   int L, T, B, H, spin_limit;
+  int patience;   // polls between two looks at the other queues, a power of two less 1
 };
 // Cell k of a stack of L layers and T steps in the order of the stages l + t, low layers first: its layer and step.
 __host__ __device__ inline void flow_cell(int k, int L, int T, int* l, int* t) {
@@ -760,7 +764,8 @@ __host__ __device__ inline void flow_cell(int k, int L, int T, int* l, int* t) {
 }
 __global__ __launch_bounds__(256, 1) void lstm_cell_flow_kernel(FlowArgs) {
   extern __shared__ __attribute__((aligned(1024))) unsigned char tile_smem[];
-  int* const word = reinterpret_cast<int*>(tile_smem);   // the next tile: layer (-1: none), step, tile of the cell
+  int* const word = reinterpret_cast<int*>(tile_smem);   // the next tile: layer (-1: none), step, tile of the cell; the ticket kept
+  int held = -1;   // this workgroup's ticket while it computes another queue's tile
   while (true) {
     // read again for every tile: kept over the product, whose loop takes all registers, the arguments would be spilled
     auto* args = (const __attribute__((address_space(4))) FlowArgs*)__builtin_amdgcn_kernarg_segment_ptr();
@@ -771,23 +776,40 @@ __global__ __launch_bounds__(256, 1) void lstm_cell_flow_kernel(FlowArgs) {
     const int q = (int)(blockIdx.x & 7), mine = (L * T - q + 7) / 8 * tiles;
     const size_t cell = (size_t)B * H;
     if (threadIdx.x < 64) {
-      int l = -1, t = 0, tile = 0;
+      int l = -1, t = 0, tile = 0, keep = -1;
       if (threadIdx.x == 0) {
-        const int ticket = __hip_atomic_fetch_add(a.tickets + q, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const int ticket = held >= 0 ? held : __hip_atomic_fetch_add(a.tickets + q, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         if (ticket < mine) {
+          // the cells below and before cell (l, t) are complete
+          auto due = [&](int l, int t) {
+            return __hip_atomic_load(a.done + max(l - 1, 0), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= (l > 0 ? (t + 1) * tiles : 0) &&
+                   __hip_atomic_load(a.done + l, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= t * tiles;
+          };
+          const int k = q + 8 * (ticket / tiles);
           tile = ticket % tiles;
-          flow_cell(q + 8 * (ticket / tiles), L, T, &l, &t);
-          const int* const below = a.done + max(l - 1, 0);
-          const int* const before = a.done + l;
-          const int of_below = l > 0 ? (t + 1) * tiles : 0, of_before = t * tiles;
-          for (int n = 1;; ++n) {
-            const bool there = __hip_atomic_load(below, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= of_below &&
-                               __hip_atomic_load(before, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= of_before;
-            if (there) break;
+          flow_cell(k, L, T, &l, &t);
+          for (int n = held >= 0 ? a.patience : 1; !due(l, t); ++n) {
             if (n >= a.spin_limit || ((n & 255) == 0 && __hip_atomic_load(a.status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0)) {
               __hip_atomic_store(a.status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
               l = -1;
               break;
+            }
+            if ((n & a.patience) == 0) {
+              for (int j = 0; j < 8 && keep < 0; ++j) {
+                int next = __hip_atomic_load(a.tickets + j, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                const int kj = j + 8 * (next / tiles);
+                int lj, tj;
+                if (kj >= k) continue;   // not before this one's cell, or nothing left
+                flow_cell(kj, L, T, &lj, &tj);
+                if (due(lj, tj) && __hip_atomic_compare_exchange_strong(a.tickets + j, &next, next + 1, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                                                        __HIP_MEMORY_SCOPE_AGENT)) {
+                  keep = ticket;
+                  tile = next % tiles;
+                  l = lj;
+                  t = tj;
+                }
+              }
+              if (keep >= 0) break;
             }
             __builtin_amdgcn_s_sleep(4);
           }
@@ -795,11 +817,13 @@ __global__ __launch_bounds__(256, 1) void lstm_cell_flow_kernel(FlowArgs) {
         word[0] = l;
         word[1] = t;
         word[2] = tile;
+        word[3] = keep;
       }
     }
     __syncthreads();
     const int l = __builtin_amdgcn_readfirstlane(word[0]), t = __builtin_amdgcn_readfirstlane(word[1]);
     const int tile = __builtin_amdgcn_readfirstlane(word[2]);
+    held = __builtin_amdgcn_readfirstlane(word[3]);
     __syncthreads();   // the words are read: the tile's copies may take their place
     if (l < 0) return;
     CellDescH cd;
@@ -1221,6 +1245,13 @@ int run_wavefront_f16(const void* xs, const void* WU, const float* bias, const i
   a.done = (int*)ws + kFlowDoneAt;
   a.L = L; a.T = T; a.B = B; a.H = H;
   a.spin_limit = 1 << 22;
+  // Looked at 0.2 to 1 ms apart: a tile takes up to 0.1, and the first cells of a queue start up to four tiles after the
+  // launch.  FTK_LSTM_F16_FLOW_PATIENCE (polls, a power of two) is for tests of the other queues' tiles.
+  a.patience = 1024 - 1;
+  if (const char* e = getenv("FTK_LSTM_F16_FLOW_PATIENCE")) {
+    const int polls = atoi(e);
+    if (polls > 0 && polls <= (1 << 20) && (polls & (polls - 1)) == 0) a.patience = polls - 1;
+  }
   hipLaunchKernelGGL(lstm_cell_flow_kernel, dim3(dp->cus), dim3(256), G_LDS, s, a);
   return check_launch("lstm_cell_flow_kernel");
 }

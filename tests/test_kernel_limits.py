@@ -82,3 +82,60 @@ def test_key_groups_with_scores_of_minus_infinity(core, Sq, Skv, D, shift):
         for i in range(len(spans) - 1):
             err = float((o[:, i] - ref[:, i]).abs().max() / ref[:, i].abs().max())
             assert err <= 1e-2, (split, spans[i], err)
+
+
+def _f16_stack(L, T, B, H, seed):
+    gen = torch.Generator(device='cuda').manual_seed(seed)
+    xs = torch.randn((T, B, H), generator=gen, device='cuda').half()
+    WU = ((torch.rand((L, 2 * H, 4 * H), generator=gen, device='cuda') * 2 - 1) * H ** -0.5).half()
+    return xs, WU
+
+
+@pytest.mark.parametrize('polls', ['1', '64'])
+@pytest.mark.parametrize('L,T,B,H', [(3, 40, 5, 64), (20, 3, 257, 128), (9, 9, 300, 320)])
+def test_one_launch_stack_computes_other_queues_tiles(core, monkeypatch, L, T, B, H, polls):
+    """The fp16 stack in one launch, where a workgroup that waits takes the due tiles of other queues at (nearly) every look:
+    the bits are those of a launch per stage."""
+    monkeypatch.setenv('FTK_LSTM_EXCHANGE', '0')
+    monkeypatch.setenv('FTK_LSTM_F16_STREAM', '1')
+    xs, WU = _f16_stack(L, T, B, H, 11)
+    monkeypatch.setenv('FTK_LSTM_F16_FLOW', '0')
+    ref = core.stacked_lstm_f16(xs, WU)
+    monkeypatch.setenv('FTK_LSTM_F16_FLOW', '1')
+    monkeypatch.setenv('FTK_LSTM_F16_FLOW_PATIENCE', polls)
+    for _ in range(3):
+        out = tuple(torch.full_like(r, float('nan')) for r in ref)
+        core.stacked_lstm_f16(xs, WU, out=out, check=True)
+        assert all(torch.equal(a, b) for a, b in zip(out, ref))
+
+
+def test_one_launch_stacks_beside_other_waiting_kernels(core, monkeypatch):
+    """Two streams with the fp16 stack in one launch and a third with the kernel whose workgroups exchange states: each fills
+    the chip, so parts of each are resident while the others run, and all end with their own results."""
+    monkeypatch.setenv('FTK_LSTM_F16_STREAM', '1')
+    stacks = [_f16_stack(9, 9, 300, 320, 12), _f16_stack(12, 6, 256, 512, 13)]
+    xs, WU = (t.float() for t in _f16_stack(8, 24, 64, 512, 14))
+    monkeypatch.setenv('FTK_LSTM_EXCHANGE', '0')
+    monkeypatch.setenv('FTK_LSTM_F16_FLOW', '0')
+    refs = [core.stacked_lstm_f16(*s) for s in stacks]
+    monkeypatch.setenv('FTK_LSTM_EXCHANGE', '1')
+    refs.append(core.stacked_lstm(xs, WU))
+    monkeypatch.setenv('FTK_LSTM_F16_FLOW', '1')
+    half_bytes = [int(core.lib.ftk_stacked_lstm_f16_workspace_bytes(s[1].shape[0], *s[0].shape)) for s in stacks]
+    spaces = [torch.empty(n, dtype=torch.uint8, device='cuda') for n in half_bytes + [core.stacked_lstm_workspace_bytes(8, 24, 64, 512)]]
+    outs = [tuple(torch.full_like(r, float('nan')) for r in ref) for ref in refs]
+    streams = [torch.cuda.Stream() for _ in refs]
+    torch.cuda.synchronize()
+    for round_ in range(4):
+        print(f'three streams, launch {round_}', flush=True)
+        for i in (0, 2, 1):
+            with torch.cuda.stream(streams[i]):
+                monkeypatch.setenv('FTK_LSTM_EXCHANGE', '1' if i == 2 else '0')
+                if i == 2:
+                    core.stacked_lstm(xs, WU, out=outs[i], workspace=spaces[i])
+                else:
+                    core.stacked_lstm_f16(*stacks[i], out=outs[i], workspace=spaces[i])
+    torch.cuda.synchronize()
+    for out, ref, space in zip(outs, refs, spaces):
+        assert core.persistent_status(space) == 0
+        assert all(torch.equal(a, b) for a, b in zip(out, ref))
