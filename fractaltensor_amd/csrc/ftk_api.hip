@@ -5,6 +5,7 @@
 #include <mutex>
 
 #include "ftk_common.h"
+#include "launch_order.h"
 
 namespace ftk {
 
@@ -46,16 +47,47 @@ int device_props(const DeviceProps** out) {
 // resident in part and wait for the rest.  Launches on one stream follow each other anyway, so a process that uses one
 // stream gets ordinary launches.  When a second stream turns up while a launch of the first may still run, the new launch
 // is put behind the first stream's work, and from then on the device gets cooperative launches only; so it does from
-// the first stream capture on, whose graph may be replayed on any stream.  Kernels that merely occupy compute
-// units end by themselves and need no care.  FTK_COOPERATIVE_LAUNCH=1: cooperative launches always (for processes that share a
-// device).
+// the first stream capture on, whose graph may be replayed on any stream, and the first launch after it that is no
+// recording is put behind the ordinary ones (launch_order.h).  A replay is not seen here: a program
+// lets the launches it made before a capture end before it replays.  Kernels that merely occupy compute units end by themselves and need no care.
+// FTK_COOPERATIVE_LAUNCH=1: cooperative launches always (for processes that share a device).
+namespace {
+struct HipStreams {
+  bool capturing(hipStream_t s) {
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &capture) != hipSuccess) (void)hipGetLastError();
+    return capture != hipStreamCaptureStatusNone;
+  }
+  StreamState state(hipStream_t s) {
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    const hipError_t c = hipStreamIsCapturing(s, &capture);
+    if (c != hipSuccess) (void)hipGetLastError();
+    // (the default stream must not be asked either while a stream that waits for it records)
+    if (c == hipErrorStreamCaptureImplicit || capture != hipStreamCaptureStatusNone) return StreamState::kCapturing;
+    const hipError_t e = hipStreamQuery(s);
+    if (e == hipSuccess) return StreamState::kIdle;
+    (void)hipGetLastError();
+    return e == hipErrorNotReady ? StreamState::kBusy : StreamState::kGone;
+  }
+  int put_behind(hipStream_t s, hipStream_t of) {
+    hipEvent_t behind;
+    FTK_HIP(hipEventCreateWithFlags(&behind, hipEventDisableTiming));
+    hipError_t r = hipEventRecord(behind, of);
+    if (r == hipSuccess) r = hipStreamWaitEvent(s, behind, 0);
+    (void)hipEventDestroy(behind);
+    if (r != hipSuccess) return fail(FTK_ERR_LAUNCH, "launch behind another stream: %s", hipGetErrorString(r));
+    return FTK_OK;
+  }
+  int wait_for_device() {
+    FTK_HIP(hipDeviceSynchronize());
+    return FTK_OK;
+  }
+};
+}  // namespace
+
 int launch_resident(const void* fn, dim3 grid, dim3 block, void** args, size_t lds, hipStream_t s) {
   constexpr int kDev = 16;
-  struct Device {
-    bool used = false, cooperative = false;
-    hipStream_t stream = nullptr;   // of the ordinary launches so far
-  };
-  static Device devices[kDev];
+  static LaunchOrder<hipStream_t> devices[kDev];
   static std::mutex mu;
   static const bool always = [] {
     const char* e = getenv("FTK_COOPERATIVE_LAUNCH");
@@ -64,40 +96,10 @@ int launch_resident(const void* fn, dim3 grid, dim3 block, void** args, size_t l
   int dev = 0;
   FTK_HIP(hipGetDevice(&dev));
   std::lock_guard<std::mutex> lock(mu);   // held over the launch: the streams have them in the order decided here
-  bool cooperative = always || dev < 0 || dev >= kDev || s == hipStreamPerThread;   // (one handle, a stream per thread)
-  if (!cooperative) {
-    Device& d = devices[dev];
-    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-    if (!d.cooperative) {
-      if (hipStreamIsCapturing(s, &capture) != hipSuccess) (void)hipGetLastError();
-      if (capture != hipStreamCaptureStatusNone) d.cooperative = true;
-    }
-    if (!d.cooperative && d.used && d.stream != s) {
-      // (a stream under capture must not be asked: that would end its capture; nothing can be put behind it either)
-      if (hipStreamIsCapturing(d.stream, &capture) != hipSuccess) (void)hipGetLastError();
-      const bool capturing = capture != hipStreamCaptureStatusNone;
-      const hipError_t e = capturing ? hipSuccess : hipStreamQuery(d.stream);
-      if (capturing) {
-        d.cooperative = true;
-      } else if (e == hipErrorNotReady) {
-        (void)hipGetLastError();
-        hipEvent_t behind;
-        FTK_HIP(hipEventCreateWithFlags(&behind, hipEventDisableTiming));
-        hipError_t r = hipEventRecord(behind, d.stream);
-        if (r == hipSuccess) r = hipStreamWaitEvent(s, behind, 0);
-        (void)hipEventDestroy(behind);
-        if (r != hipSuccess) return fail(FTK_ERR_LAUNCH, "launch behind another stream: %s", hipGetErrorString(r));
-        d.cooperative = true;
-      } else if (e != hipSuccess) {   // the stream is gone; its work may not be
-        (void)hipGetLastError();
-        FTK_HIP(hipDeviceSynchronize());
-      }
-    }
-    if (!d.cooperative) {
-      d.used = true;
-      d.stream = s;
-    }
-    cooperative = d.cooperative;
+  bool cooperative = true;
+  if (!always && dev >= 0 && dev < kDev) {
+    const int rc = devices[dev].next(HipStreams(), s, s == hipStreamPerThread, &cooperative);
+    if (rc) return rc;
   }
   if (cooperative) FTK_HIP(hipLaunchCooperativeKernel(fn, grid, block, args, (unsigned)lds, s));
   else FTK_HIP(hipLaunchKernel(fn, grid, block, args, lds, s));
