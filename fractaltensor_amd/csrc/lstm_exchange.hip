@@ -861,6 +861,23 @@ bool exchange_one_block(int L, int B, int H, bool half) {
   return p.layers == L && p.slices == nrb;
 }
 
+namespace {
+// Layers of one launch (0: the device cannot hold one), and the kind of row block.
+int exchange_layers(int L, int B, int H, bool half, bool* many) {
+  const ExchangeFlavour f = exchange_flavour_of(H, half);
+  *many = !exchange_one_block(L, B, H, half);
+  const int block = *many ? 32 : 16;
+  return exchange_plan(L, H / exchange_units(H, half, *many), (B + block - 1) / block, exchange_slots(*many ? f.many : f.one)).layers;
+}
+}  // namespace
+
+// Bytes of workspace that run_exchange uses on the current device; without a device, what it could at most.
+size_t exchange_need(int L, int T, int B, int H, bool half) {
+  bool many;
+  const int most = exchange_layers(L, B, H, half, &many);
+  return exchange_workspace_bytes(most ? std::min(L, most) : L, T, B, H, half);
+}
+
 // Runs the stack; *handled is false when the device cannot hold a layer.  Deeper stacks than a launch holds run as
 // consecutive launches, each reading the hidden sequence of the layer below it like the first reads xs.
 int run_exchange(bool half, const void* xs, const void* WU, const float* bias, const int* dil, const int* active, void* hsss,
@@ -868,13 +885,13 @@ int run_exchange(bool half, const void* xs, const void* WU, const float* bias, c
   *handled = false;
   const ExchangeFlavour f = exchange_flavour_of(H, half);
   if (!f.one) return FTK_OK;
-  const bool many = !exchange_one_block(L, B, H, half);
+  bool many;
+  const int most = exchange_layers(L, B, H, half, &many);
+  if (most == 0) return FTK_OK;
   const int slots = exchange_slots(many ? f.many : f.one), block = many ? 32 : 16, nrb = (B + block - 1) / block;
   const int W = H / exchange_units(H, half, many);
-  const int most = exchange_plan(L, W, nrb, slots).layers;
-  if (most == 0) return FTK_OK;
   const size_t esize = half ? 2 : 4, slab = (size_t)T * B * H, wlayer = (size_t)8 * H * H, tile = exchange_tile_bytes(H, half, block);
-  const size_t need = exchange_workspace_bytes(std::min(L, most), T, B, H, half);
+  const size_t need = exchange_need(L, T, B, H, half);
   if (!ws || ws_bytes < need) return fail(FTK_ERR_WORKSPACE, "stacked LSTM needs a %zu-byte workspace, got %zu", need, ws_bytes);
   for (int l0 = 0; l0 < L; l0 += most) {
     const int lc = std::min(most, L - l0);

@@ -69,6 +69,7 @@ bool exchange_takes(int H, bool half);
 bool exchange_fits(int T, int B, int H, bool half);
 bool exchange_one_block(int L, int B, int H, bool half);
 size_t exchange_workspace_bytes(int L, int T, int B, int H, bool half);
+size_t exchange_need(int L, int T, int B, int H, bool half);
 int run_exchange(bool half, const void* xs, const void* WU, const float* bias, const int* dil, const int* active, void* hsss,
                  void* csss, int L, int T, int B, int H, void* ws, size_t ws_bytes, hipStream_t s, bool* handled, int spin_limit);
 
@@ -1842,7 +1843,7 @@ static int run_stack(const char* who, const float* xs, const float* WU, const fl
                     who, t, active[t], t - 1, active[t - 1]);
     }
   }
-  if (products == FTK_LSTM_PRODUCTS_F16X3 && exchange_chosen(L, T, B, H, dil, false, active != nullptr) && ws && ws_bytes >= exchange_workspace_bytes(L, T, B, H, false)) {
+  if (products == FTK_LSTM_PRODUCTS_F16X3 && exchange_chosen(L, T, B, H, dil, false, active != nullptr) && ws && ws_bytes >= exchange_need(L, T, B, H, false)) {
     bool handled = false;
     rc = run_exchange(false, xs, WU, bias, dil, active, hsss, csss, L, T, B, H, ws, ws_bytes, s, &handled, spin_limit);
     if (rc || handled) return rc;
@@ -1902,6 +1903,9 @@ static bool f16_streams(int L, int B, int H, bool ragged) {
   return H == 2 * PH && L > 16 && !ragged;
 }
 
+// Workspace of the streaming kernels: the status block and the re-laid weights.
+static size_t f16_stream_bytes(int L, int H) { return kStatusBytes + (size_t)L * 2 * H * 4 * H * sizeof(_Float16); }
+
 }  // namespace ftk
 
 extern "C" {
@@ -1916,12 +1920,12 @@ size_t ftk_stacked_lstm_workspace_bytes(int L, int T, int B, int H) {
 
 size_t ftk_stacked_lstm_f16_workspace_bytes(int L, int T, int B, int H) {
   if (L <= 0 || T <= 0 || B <= 0 || H <= 0) return 0;
-  // the status block and the re-laid weights of the streaming kernel
-  const size_t packed = std::max(ftk::kStatusBytes + (size_t)L * 2 * H * 4 * H * sizeof(_Float16),
-                                 ftk::exchange_takes(H, true) ? ftk::exchange_workspace_bytes(L, T, B, H, true) : (size_t)0);
-  if (!ftk::f16_fits_on_chip(B, H)) return packed;
-  // which of the two runs is decided per call (a ragged batch stays with the persistent kernel): room for either
-  return std::max(ftk::xratio_offset_bytes(L, T, B), packed);
+  // which kernel runs is decided per call (dilations, a ragged batch): room for any that the shape may go to
+  size_t need = ftk::f16_fits_on_chip(B, H) ? ftk::xratio_offset_bytes(L, T, B) : 0;
+  if (ftk::f16_streams(L, B, H, false)) need = std::max(need, ftk::f16_stream_bytes(L, H));
+  if (ftk::exchange_chosen(L, T, B, H, nullptr, true, false) || ftk::exchange_chosen(L, T, B, H, nullptr, true, true))
+    need = std::max(need, ftk::exchange_need(L, T, B, H, true));
+  return need;
 }
 
 int ftk_stacked_lstm_f16(const void* xs, const void* WU, const float* bias, const int* dilations,
@@ -1947,7 +1951,7 @@ int ftk_stacked_lstm_f16(const void* xs, const void* WU, const float* bias, cons
       if (t > 0 && active_rows[t] > active_rows[t - 1])
         return fail(FTK_ERR_INVALID_ARGUMENT, "%s: active_rows must be non-increasing (rows sorted by length)", who);
     }
-  if (exchange_chosen(L, T, B, H, dilations, true, active_rows != nullptr) && workspace && workspace_bytes >= exchange_workspace_bytes(L, T, B, H, true)) {
+  if (exchange_chosen(L, T, B, H, dilations, true, active_rows != nullptr) && workspace && workspace_bytes >= exchange_need(L, T, B, H, true)) {
     bool handled = false;
     const int rcx = run_exchange(true, xs, WU, bias, dilations, active_rows, hsss, csss, L, T, B, H, workspace, workspace_bytes,
                                  (hipStream_t)stream, &handled, 0);
@@ -1956,7 +1960,7 @@ int ftk_stacked_lstm_f16(const void* xs, const void* WU, const float* bias, cons
   // every other shape streams the weights, in one launch or one per stage of independent cells (lstm_cell.hip)
   // (the workspace takes the weights re-laid per unit block, so that a workgroup reads one contiguous run)
   if (!on_chip) {
-    const size_t need = ftk_stacked_lstm_f16_workspace_bytes(L, T, B, H);
+    const size_t need = f16_stream_bytes(L, H);
     if (!workspace || workspace_bytes < need)
       return fail(FTK_ERR_WORKSPACE, "%s: workspace of %zu bytes needed, %zu given", who, need, workspace ? workspace_bytes : (size_t)0);
     hipLaunchKernelGGL(fill_zero_kernel, dim3(1), dim3(64), 0, (hipStream_t)stream, reinterpret_cast<int*>(workspace),

@@ -126,3 +126,12 @@ def test_wrappers_refuse_cpu_tensors():
         core.lstm_cell(x, None, None, torch.zeros((64, 128)))
     with pytest.raises(RuntimeError, match='no CPU path'):
         core.online_softmax(x)
+
+
+def test_f16_stack_workspace_is_that_of_the_kernels_the_shape_goes_to():
+    """L 32 T 64 B 256: the streamed cells at H 1024 (status block and re-laid weights), the persistent kernel at H 256 (flags
+    only); neither asks for the state buffers of the exchange kernel."""
+    import fractaltensor_amd._core as core
+    size = core.lib.ftk_stacked_lstm_f16_workspace_bytes
+    assert size(32, 64, 256, 1024) == 256 + 32 * 2048 * 4096 * 2
+    assert 0 < size(32, 64, 256, 256) < 4 << 20

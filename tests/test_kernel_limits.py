@@ -139,3 +139,27 @@ def test_one_launch_stacks_beside_other_waiting_kernels(core, monkeypatch):
     for out, ref, space in zip(outs, refs, spaces):
         assert core.persistent_status(space) == 0
         assert all(torch.equal(a, b) for a, b in zip(out, ref))
+
+
+def test_f16_stack_takes_the_workspace_of_the_kernel_it_runs(core, monkeypatch):
+    """What the size query asks for is enough for every form of the call; with room for the re-laid weights only, less than
+    the exchange kernel would use, the weights are streamed."""
+    L, T, B, H = 1, 64, 256, 1024
+    xs, WU = _f16_stack(L, T, B, H, 15)
+    asked = int(core.lib.ftk_stacked_lstm_f16_workspace_bytes(L, T, B, H))
+    packed = 256 + L * 2 * H * 4 * H * 2
+    assert asked > packed
+    monkeypatch.setenv('FTK_LSTM_EXCHANGE', '0')
+    ref = core.stacked_lstm_f16(xs, WU)
+    monkeypatch.delenv('FTK_LSTM_EXCHANGE')
+    got = core.stacked_lstm_f16(xs, WU, workspace=torch.empty(packed, dtype=torch.uint8, device='cuda'), check=True)
+    assert all(torch.equal(a, b) for a, b in zip(got, ref))
+    with pytest.raises(core.FtkError):
+        core.stacked_lstm_f16(xs, WU, workspace=torch.empty(packed - 16, dtype=torch.uint8, device='cuda'))
+    # deep: no more than the layers that one launch of the exchange kernel holds
+    for L, T, B, H in [(20, 16, 160, 1024), (6, 8, 40, 512), (5, 7, 33, 256), (3, 4, 31, 96)]:
+        xs, WU = _f16_stack(L, T, B, H, 16)
+        ws = torch.empty(int(core.lib.ftk_stacked_lstm_f16_workspace_bytes(L, T, B, H)), dtype=torch.uint8, device='cuda')
+        for dil, active in ((None, None), ([1 + l % 2 for l in range(L)], None), (None, [B] * (T - 1) + [B // 2])):
+            h, _ = core.stacked_lstm_f16(xs, WU, dilations=dil, active_rows=active, workspace=ws, check=True)
+            assert bool(torch.isfinite(h[:, :, :B // 2]).all())
