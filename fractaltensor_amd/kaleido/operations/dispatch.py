@@ -42,6 +42,7 @@ from __future__ import annotations
 import math
 import os
 import threading
+import weakref
 from typing import Callable, Optional
 
 import torch
@@ -67,6 +68,8 @@ _local = threading.local()
 def reset() -> None:
     """Forget every verdict and zero the counters."""
     _verdicts.clear()
+    _reached.clear()
+    _numbers.clear()
     clear_weight_cache()
     for k in stats:
         stats[k] = 0
@@ -115,36 +118,82 @@ def _code_names(code):
     return names
 
 
-# Per (code object, module globals): what the code reaches through its globals, as one number.  An entry holds everything
+# Per (code object, module globals): what the code reaches through its globals, as one number.  An entry knows everything
 # that was looked at (_Seen); as long as all of it is the same objects the number stands, and a call of a routed program
-# pays a dozen identity checks for it.
+# pays a dozen identity checks for it.  Entries keep none of those objects alive (a program's tensors are among them).
 _reached: dict = {}
+_MAX_REACHED = 1024
 _numbers: dict = {}
 _number_count = 0
 _MISSING = object()
+
+
+def _mark(v):
+    """What tells later whether a name, a default or a cell still has the value v: the value itself if it is a scalar or a
+    tuple of scalars, a weak reference to it, or (what cannot be referred to weakly: containers, objects with slots, of
+    which a fingerprint takes nothing) one to its type."""
+    if v is _MISSING or isinstance(v, _SCALARS) or (type(v) is tuple and len(v) <= 16 and all(isinstance(e, _SCALARS) for e in v)):
+        return v, None, None
+    try:
+        return None, weakref.ref(v), None
+    except TypeError:
+        return None, None, weakref.ref(type(v))
+
+
+def _same(mark, v) -> bool:
+    value, ref, kind = mark
+    if ref is not None:
+        return ref() is v
+    return value is v if kind is None else type(v) is kind()
+
+
+def _content(cell):
+    try:
+        return cell.cell_contents
+    except ValueError:
+        return _MISSING
 
 
 class _Seen:
     """What a fingerprint looked at."""
 
     def __init__(self):
-        self.names = []          # (globals, name, value)
-        self.functions = []      # (function, code, defaults, keyword defaults, closure contents)
+        self.names = []          # (name, mark) in the globals that the entry is for
+        self.functions = []      # (weak function, code, marks of the defaults, of the closure, [(name, mark)] in its globals)
         self.stable = True       # nothing among it that can change in place (a list held as a default or in a closure)
 
-    def unchanged(self) -> bool:
-        for g, name, v in self.names:
-            if g.get(name, _MISSING) is not v:
+    def function(self, f, code, defaults, kw, cells):
+        """Notes a function, and returns the list its names go to."""
+        names = []
+        try:
+            self.functions.append((weakref.ref(f), code, [_mark(d) for d in defaults or ()], [_mark(v) for v in cells], names))
+        except TypeError:
+            self.stable = False
+        if kw:
+            self.stable = False
+        return names
+
+    def unchanged(self, g) -> bool:
+        for name, mark in self.names:
+            if not _same(mark, g.get(name, _MISSING)):
                 return False
-        for f, code, defaults, kw, cells in self.functions:
-            if f.__code__ is not code or f.__defaults__ is not defaults or f.__kwdefaults__ is not kw:
+        for ref, code, defaults, cells, names in self.functions:
+            f = ref()
+            if f is None or f.__code__ is not code:
                 return False
-            for cell, v in cells:
-                try:
-                    if cell.cell_contents is not v:
-                        return False
-                except ValueError:
-                    if v is not _MISSING:
+            now = getattr(f, '__defaults__', None) or ()
+            if len(now) != len(defaults) or getattr(f, '__kwdefaults__', None):
+                return False
+            for mark, v in zip(defaults, now):
+                if not _same(mark, v):
+                    return False
+            for mark, cell in zip(cells, getattr(f, '__closure__', None) or ()):
+                if not _same(mark, _content(cell)):
+                    return False
+            if names:
+                of = getattr(f, '__globals__', None) or {}
+                for name, mark in names:
+                    if not _same(mark, of.get(name, _MISSING)):
                         return False
         return True
 
@@ -184,7 +233,7 @@ def _fingerprint(f, level: int = 0, seen=None, looked=None):
         return ('seen', seen[id(f)])
     if level > 6:
         if looked is not None:
-            looked.functions.append((f, code, getattr(f, '__defaults__', None), getattr(f, '__kwdefaults__', None), []))
+            looked.function(f, code, getattr(f, '__defaults__', None), getattr(f, '__kwdefaults__', None), ())
         return ('deep', code)
     seen[id(f)] = len(seen)
 
@@ -213,40 +262,32 @@ def _fingerprint(f, level: int = 0, seen=None, looked=None):
         parts.append(of_value(d))
     for k, d in sorted((kw or {}).items()):
         parts.append((k, of_value(d)))
-    cells = []
-    for cell in (closure or ()):
-        try:
-            v = cell.cell_contents
-        except ValueError:
-            cells.append((cell, _MISSING))
-            continue
-        cells.append((cell, v))
-        parts.append(of_value(v))
-    if looked is not None:
-        looked.functions.append((f, code, defaults, kw, cells))
-        if kw:
-            looked.stable = False
-
+    cells = [_content(cell) for cell in (closure or ())]
+    for v in cells:
+        if v is not _MISSING:
+            parts.append(of_value(v))
     g = getattr(f, '__globals__', None) or {}
 
-    def of_globals(record, seen):
+    def of_globals(record, seen, to):
         names = []
         for name in _code_names(code):
             v = g.get(name, _MISSING)
-            record.names.append((g, name, v))
+            to.append((name, _mark(v)))
             if v is not _MISSING and (isinstance(v, _SCALARS) or (callable(v) and hasattr(v, '__code__'))):
                 names.append((name, v if isinstance(v, _SCALARS) else _fingerprint(v, level + 1, seen, record)))
         return (code, tuple(names))
 
     if looked is not None:               # reached from another function: part of that one's number
-        parts.append(of_globals(looked, seen))
+        parts.append(of_globals(looked, seen, looked.function(f, code, defaults, kw, cells)))
         return tuple(parts)
     entry = _reached.get((id(code), id(g), level))
-    if entry is None or not entry[0].unchanged():
+    if entry is None or not entry[0].unchanged(g):
         record = _Seen()
-        n = _number_of(of_globals(record, {}))
-        entry = (record, n, code, g)      # (code and g are kept alive: their ids stay theirs)
-        if record.stable:
+        n = _number_of(of_globals(record, {}, record.names))
+        entry = (record, n, code)         # the code is kept alive: its id stays its own.  Other globals at the id of these
+        if record.stable:                 # would be looked at name by name like these
+            if len(_reached) >= _MAX_REACHED:
+                _reached.clear()
             _reached[(id(code), id(g), level)] = entry
     parts.append(entry[1])
     return tuple(parts)

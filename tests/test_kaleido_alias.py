@@ -131,6 +131,47 @@ def test_function_fingerprint_of_a_helper_met_through_a_closure_first():
     assert dispatch._fingerprint(pair(half, double, then(half))) != dispatch._fingerprint(pair(half, double, then(double)))
 
 
+def test_remembered_fingerprints_keep_no_data_alive():
+    """Tensors and functions that a program reached through its globals, through a closure or a default are free once the
+    program lets go of them; a value of the same name that means something else is seen."""
+    import gc
+    import weakref
+    import torch
+    from kaleido.operations import dispatch
+    dispatch.reset()
+    source = ('def helper(x, d=data, t=(1, 2)):\n    return x + data + inner(x)\n'
+              'def layer(x):\n    return helper(x) * scale\n')
+
+    def closes_over(t):
+        return lambda x: x + t
+
+    def space(t):
+        g = {'data': t, 'inner': closes_over(t), 'scale': 2.0, 'many': [t]}
+        exec(source, g)
+        return g
+
+    g = space(torch.zeros(3))
+    first = dispatch._fingerprint(g['layer'])
+    assert dispatch._fingerprint(g['layer']) == first and dispatch._reached
+    held = [weakref.ref(g['data']), weakref.ref(g['helper']), weakref.ref(g['inner'])]
+    g['inner'] = lambda x: x
+    assert dispatch._fingerprint(g['layer']) != first
+    g['data'] = 3.0                                       # read as a scalar now
+    changed = dispatch._fingerprint(g['layer'])
+    g['data'] = 4.0
+    assert dispatch._fingerprint(g['layer']) != changed
+    g['helper'].__defaults__ = (1.0, (1, 2))
+    assert dispatch._fingerprint(g['layer']) != changed
+    entries = len(dispatch._reached)
+    del g
+    gc.collect()
+    assert [r() for r in held] == [None] * 3 and len(dispatch._reached) == entries
+
+    for i in range(3 * dispatch._MAX_REACHED):            # bounded, whatever programs come by
+        dispatch._fingerprint(space(None)['layer'])
+    assert len(dispatch._reached) <= dispatch._MAX_REACHED
+
+
 def test_kaleido_core_is_the_c_abi_binding():
     """`kaleido._core`, the module name of the reference's native binding (kaleido/__init__.py:20-26), is
     fractaltensor_amd._core."""
