@@ -154,17 +154,50 @@ def _content(cell):
         return _MISSING
 
 
+class _Names:
+    """Marks of the names that a code object reads in its globals, sorted by kind: a call of a routed program looks at all of
+    them."""
+    __slots__ = ('missing', 'values', 'refs', 'kinds')
+
+    def __init__(self):
+        self.missing, self.values, self.refs, self.kinds = set(), [], [], []
+
+    def add(self, name, v):
+        value, ref, kind = _mark(v)
+        if ref is not None:
+            self.refs.append((name, ref))
+        elif kind is not None:
+            self.kinds.append((name, kind))
+        elif value is _MISSING:
+            self.missing.add(name)
+        else:
+            self.values.append((name, value))
+
+    def unchanged(self, g) -> bool:
+        for name, ref in self.refs:
+            v = ref()
+            if v is None or g.get(name) is not v:
+                return False
+        for name, value in self.values:
+            if g.get(name, _MISSING) is not value:
+                return False
+        for name, kind in self.kinds:
+            if type(g.get(name, _MISSING)) is not kind():
+                return False
+        return g.keys().isdisjoint(self.missing)
+
+
 class _Seen:
     """What a fingerprint looked at."""
 
     def __init__(self):
-        self.names = []          # (name, mark) in the globals that the entry is for
-        self.functions = []      # (weak function, code, marks of the defaults, of the closure, [(name, mark)] in its globals)
+        self.names = _Names()    # in the globals that the entry is for
+        self.functions = []      # (weak function, code, marks of the defaults, of the closure, _Names in its globals)
         self.stable = True       # nothing among it that can change in place (a list held as a default or in a closure)
 
     def function(self, f, code, defaults, kw, cells):
-        """Notes a function, and returns the list its names go to."""
-        names = []
+        """Notes a function, and returns where its names go."""
+        names = _Names()
         try:
             self.functions.append((weakref.ref(f), code, [_mark(d) for d in defaults or ()], [_mark(v) for v in cells], names))
         except TypeError:
@@ -174,9 +207,8 @@ class _Seen:
         return names
 
     def unchanged(self, g) -> bool:
-        for name, mark in self.names:
-            if not _same(mark, g.get(name, _MISSING)):
-                return False
+        if not self.names.unchanged(g):
+            return False
         for ref, code, defaults, cells, names in self.functions:
             f = ref()
             if f is None or f.__code__ is not code:
@@ -184,17 +216,12 @@ class _Seen:
             now = getattr(f, '__defaults__', None) or ()
             if len(now) != len(defaults) or getattr(f, '__kwdefaults__', None):
                 return False
-            for mark, v in zip(defaults, now):
-                if not _same(mark, v):
-                    return False
-            for mark, cell in zip(cells, getattr(f, '__closure__', None) or ()):
-                if not _same(mark, _content(cell)):
-                    return False
-            if names:
-                of = getattr(f, '__globals__', None) or {}
-                for name, mark in names:
-                    if not _same(mark, of.get(name, _MISSING)):
-                        return False
+            if defaults and not all(map(_same, defaults, now)):
+                return False
+            if cells and not all(map(_same, cells, map(_content, f.__closure__))):
+                return False
+            if not names.unchanged(getattr(f, '__globals__', None) or {}):
+                return False
         return True
 
 
@@ -272,7 +299,7 @@ def _fingerprint(f, level: int = 0, seen=None, looked=None):
         names = []
         for name in _code_names(code):
             v = g.get(name, _MISSING)
-            to.append((name, _mark(v)))
+            to.add(name, v)
             if v is not _MISSING and (isinstance(v, _SCALARS) or (callable(v) and hasattr(v, '__code__'))):
                 names.append((name, v if isinstance(v, _SCALARS) else _fingerprint(v, level + 1, seen, record)))
         return (code, tuple(names))
