@@ -155,33 +155,32 @@ def _content(cell):
 
 
 class _Names:
-    """Marks of the names that a code object reads in its globals, sorted by kind: a call of a routed program looks at all of
-    them."""
+    """Marks of names in one module's globals, by kind: a call of a routed program looks at all of them."""
     __slots__ = ('missing', 'values', 'refs', 'kinds')
 
     def __init__(self):
-        self.missing, self.values, self.refs, self.kinds = set(), [], [], []
+        self.missing, self.values, self.refs, self.kinds = set(), {}, {}, {}
 
     def add(self, name, v):
         value, ref, kind = _mark(v)
         if ref is not None:
-            self.refs.append((name, ref))
+            self.refs[name] = ref
         elif kind is not None:
-            self.kinds.append((name, kind))
+            self.kinds[name] = kind
         elif value is _MISSING:
             self.missing.add(name)
         else:
-            self.values.append((name, value))
+            self.values[name] = value
 
     def unchanged(self, g) -> bool:
-        for name, ref in self.refs:
+        for name, ref in self.refs.items():
             v = ref()
             if v is None or g.get(name) is not v:
                 return False
-        for name, value in self.values:
+        for name, value in self.values.items():
             if g.get(name, _MISSING) is not value:
                 return False
-        for name, kind in self.kinds:
+        for name, kind in self.kinds.items():
             if type(g.get(name, _MISSING)) is not kind():
                 return False
         return g.keys().isdisjoint(self.missing)
@@ -190,39 +189,39 @@ class _Names:
 class _Seen:
     """What a fingerprint looked at."""
 
-    def __init__(self):
-        self.names = _Names()    # in the globals that the entry is for
-        self.functions = []      # (weak function, code, marks of the defaults, of the closure, _Names in its globals)
+    def __init__(self, g):
+        self.at = id(g)          # the globals that the entry is for
+        self.names = _Names()    # in them
+        self.functions = []      # (weak function, code, marks of the defaults, of the closure, _Names in its globals if others)
         self.stable = True       # nothing among it that can change in place (a list held as a default or in a closure)
 
     def function(self, f, code, defaults, kw, cells):
-        """Notes a function, and returns where its names go."""
-        names = _Names()
+        """Notes a function, and returns where its names go.  One that is alive keeps its globals alive, and they their id:
+        a function's names go to the entry's own if its globals are."""
+        own = id(getattr(f, '__globals__', None)) == self.at
+        names = None if own else _Names()
         try:
             self.functions.append((weakref.ref(f), code, [_mark(d) for d in defaults or ()], [_mark(v) for v in cells], names))
         except TypeError:
             self.stable = False
-        if kw:
+        if kw or not hasattr(f, '__defaults__'):
             self.stable = False
-        return names
+        return self.names if own else names
 
     def unchanged(self, g) -> bool:
-        if not self.names.unchanged(g):
-            return False
         for ref, code, defaults, cells, names in self.functions:
             f = ref()
-            if f is None or f.__code__ is not code:
+            if f is None or f.__code__ is not code or f.__kwdefaults__:
                 return False
-            now = getattr(f, '__defaults__', None) or ()
-            if len(now) != len(defaults) or getattr(f, '__kwdefaults__', None):
-                return False
-            if defaults and not all(map(_same, defaults, now)):
-                return False
+            now = f.__defaults__
+            if now or defaults:
+                if not now or len(now) != len(defaults) or not all(map(_same, defaults, now)):
+                    return False
             if cells and not all(map(_same, cells, map(_content, f.__closure__))):
                 return False
-            if not names.unchanged(getattr(f, '__globals__', None) or {}):
+            if names is not None and not names.unchanged(getattr(f, '__globals__', None) or {}):
                 return False
-        return True
+        return self.names.unchanged(g)
 
 
 def _number_of(parts):
@@ -309,7 +308,7 @@ def _fingerprint(f, level: int = 0, seen=None, looked=None):
         return tuple(parts)
     entry = _reached.get((id(code), id(g), level))
     if entry is None or not entry[0].unchanged(g):
-        record = _Seen()
+        record = _Seen(g)
         n = _number_of(of_globals(record, {}, record.names))
         entry = (record, n, code)         # the code is kept alive: its id stays its own.  Other globals at the id of these
         if record.stable:                 # would be looked at name by name like these
