@@ -1843,7 +1843,7 @@ static int run_stack(const char* who, const float* xs, const float* WU, const fl
                     who, t, active[t], t - 1, active[t - 1]);
     }
   }
-  if (products == FTK_LSTM_PRODUCTS_F16X3 && exchange_chosen(L, T, B, H, dil, false, active != nullptr) && ws && ws_bytes >= exchange_need(L, T, B, H, false)) {
+  if (products == FTK_LSTM_PRODUCTS_F16X3 && exchange_chosen(L, T, B, H, dil, false, active != nullptr)) {
     bool handled = false;
     rc = run_exchange(false, xs, WU, bias, dil, active, hsss, csss, L, T, B, H, ws, ws_bytes, s, &handled, spin_limit);
     if (rc || handled) return rc;
@@ -1951,7 +1951,7 @@ int ftk_stacked_lstm_f16(const void* xs, const void* WU, const float* bias, cons
       if (t > 0 && active_rows[t] > active_rows[t - 1])
         return fail(FTK_ERR_INVALID_ARGUMENT, "%s: active_rows must be non-increasing (rows sorted by length)", who);
     }
-  if (exchange_chosen(L, T, B, H, dilations, true, active_rows != nullptr) && workspace && workspace_bytes >= exchange_need(L, T, B, H, true)) {
+  if (exchange_chosen(L, T, B, H, dilations, true, active_rows != nullptr)) {
     bool handled = false;
     const int rcx = run_exchange(true, xs, WU, bias, dilations, active_rows, hsss, csss, L, T, B, H, workspace, workspace_bytes,
                                  (hipStream_t)stream, &handled, 0);
