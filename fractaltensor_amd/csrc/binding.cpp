@@ -68,6 +68,18 @@ PyObject* guarded(F&& f) {
   }
 }
 
+// Other Python threads run while one is in the library: a launch may wait for the lock that orders launches of several streams,
+// or for the device.
+struct WithoutGil {
+  PyThreadState* state = PyEval_SaveThread();
+  ~WithoutGil() { PyEval_RestoreThread(state); }
+};
+template <typename F>
+int in_library(F&& f) {
+  WithoutGil released;
+  return f();
+}
+
 PyObject* init(PyObject*, PyObject* const* args, Py_ssize_t n) {
   if (n != 2 || !PyDict_Check(args[0]) || !PyCallable_Check(args[1])) {
     PyErr_SetString(PyExc_TypeError, "init(counts, raise)");
@@ -100,7 +112,8 @@ PyObject* b2b_gemm(PyObject*, PyObject* const* a, Py_ssize_t n) {
       if (D.dim() != 3 || dim(D, 0) != G || dim(D, 1) != M || dim(D, 2) != P) Py_RETURN_NONE;
     }
     if (!count("b2b_gemm")) return nullptr;
-    const int rc = ftk_b2b_gemm_f16(A.data_ptr(), B.data_ptr(), C.data_ptr(), D.data_ptr(), G, M, N, K, P, stream());
+    void *const ap = A.data_ptr(), *const bp = B.data_ptr(), *const cp = C.data_ptr(), *const dp = D.data_ptr(), *const s = stream();
+    const int rc = in_library([&] { return ftk_b2b_gemm_f16(ap, bp, cp, dp, G, M, N, K, P, s); });
     return rc ? raise(rc) : THPVariable_Wrap(std::move(D));
   });
 }
@@ -140,21 +153,15 @@ PyObject* flash_attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
       ws = empty({(int64_t)need}, at::kByte, Q);
     }
     const size_t bytes = ws.defined() ? ws.nbytes() : 0;
-    int rc;
-    if (!half) {
-      if (!count("flash_attention_f32")) return nullptr;
-      rc = ftk_flash_attn_f32(Q.data_ptr<float>(), K.data_ptr<float>(), V.data_ptr<float>(), O.data_ptr<float>(), B, Hd, Sq, Skv, D,
-                              (float)scale, ws.defined() ? ws.data_ptr() : nullptr, bytes, stream());
-    } else {
-      if (!count("flash_attention")) return nullptr;
-      if (need) {
-        if (!count("flash_attention_split_keys")) return nullptr;
-        rc = ftk_flash_attn_ws_f16(Q.data_ptr(), K.data_ptr(), V.data_ptr(), O.data_ptr(), B, Hd, Sq, Skv, D, (float)scale,
-                                   ws.data_ptr(), bytes, stream());
-      } else {
-        rc = ftk_flash_attn_f16(Q.data_ptr(), K.data_ptr(), V.data_ptr(), O.data_ptr(), B, Hd, Sq, Skv, D, (float)scale, stream());
-      }
-    }
+    if (!count(half ? "flash_attention" : "flash_attention_f32")) return nullptr;
+    if (half && need && !count("flash_attention_split_keys")) return nullptr;
+    void *const qp = Q.data_ptr(), *const kp = K.data_ptr(), *const vp = V.data_ptr(), *const op = O.data_ptr();
+    void *const wp = ws.defined() ? ws.data_ptr() : nullptr, *const s = stream();
+    const int rc = in_library([&] {
+      if (!half) return ftk_flash_attn_f32((const float*)qp, (const float*)kp, (const float*)vp, (float*)op, B, Hd, Sq, Skv, D, (float)scale, wp, bytes, s);
+      if (need) return ftk_flash_attn_ws_f16(qp, kp, vp, op, B, Hd, Sq, Skv, D, (float)scale, wp, bytes, s);
+      return ftk_flash_attn_f16(qp, kp, vp, op, B, Hd, Sq, Skv, D, (float)scale, s);
+    });
     return rc ? raise(rc) : THPVariable_Wrap(std::move(O));
   });
 }
@@ -217,25 +224,22 @@ PyObject* stacked_lstm(PyObject*, PyObject* const* a, Py_ssize_t n) {
       ws = tensor_of(a[6]);
     }
     if (!count(half ? "stacked_lstm_f16" : "stacked_lstm")) return nullptr;
-    void* s = stream();
     const int* dp = dil.empty() ? nullptr : dil.data();
-    int rc;
-    if (half) {
-      rc = ftk_stacked_lstm_f16(xs.data_ptr(), WU.data_ptr(), bias, dp, nullptr, h.data_ptr(), c.data_ptr(), L, T, B, H, ws.data_ptr(),
-                                ws.nbytes(), s);
-    } else {
-      ftk_lstm_options options = {(int)PyLong_AsLong(a[7]), 0};
-      rc = ftk_stacked_lstm_opts_f32(xs.data_ptr<float>(), WU.data_ptr<float>(), bias, dp, nullptr, h.data_ptr<float>(),
-                                     c.data_ptr<float>(), L, T, B, H, &options, ws.data_ptr(), ws.nbytes(), s);
-    }
-    if (rc) return raise(rc);
+    const ftk_lstm_options options = {(int)PyLong_AsLong(a[7]), 0};
+    void *const xp = xs.data_ptr(), *const up = WU.data_ptr(), *const hp = h.data_ptr(), *const cp = c.data_ptr(), *const wp = ws.data_ptr();
+    void* const s = stream();
+    const size_t bytes = ws.nbytes();
+    const bool small_asked = a[9] == Py_True;
     int small = 0;
-    if (check || a[9] == Py_True) {
-      Py_BEGIN_ALLOW_THREADS
-      rc = ftk_stacked_lstm_result(ws.data_ptr(), &small, s);
-      Py_END_ALLOW_THREADS
-      if (rc && (check || rc != FTK_ERR_TIMEOUT)) return raise(rc);
-    }
+    const int rc = in_library([&] {
+      const int rc = half ? ftk_stacked_lstm_f16(xp, up, bias, dp, nullptr, hp, cp, L, T, B, H, wp, bytes, s)
+                          : ftk_stacked_lstm_opts_f32((const float*)xp, (const float*)up, bias, dp, nullptr, (float*)hp, (float*)cp, L, T, B, H,
+                                                      &options, wp, bytes, s);
+      if (rc || !(check || small_asked)) return rc;
+      const int waited = ftk_stacked_lstm_result(wp, &small, s);
+      return waited == FTK_ERR_TIMEOUT && !check ? FTK_OK : waited;
+    });
+    if (rc) return raise(rc);
     PyObject* out = PyTuple_New(3);
     if (!out) return nullptr;
     PyTuple_SET_ITEM(out, 0, THPVariable_Wrap(std::move(h)));
