@@ -1722,7 +1722,8 @@ static int scratch_of_current_device(const char* who, void** out, bool lookup) {
 // pinned host memory, where the host waits for them.  (A copy to pageable memory and a wait for the stream take 25 to 30
 // us of the host's time, this about 6.)  The host looks for two milliseconds, which covers the stacks for which that
 // matters, and leaves the rest of the wait to the runtime.  The sixteen slots are allocated once and kept; with all of
-// them in use by other threads the words are copied.
+// them in use by other threads the words are copied, and so are those of the built-in scratch (slot_wanted == false): its
+// callers do without allocations.
 struct StatusSlot {
   int seq;       // written last: the words are those of this request
   int words[2];
@@ -1736,13 +1737,13 @@ __global__ void report_status_kernel(const int* status, StatusSlot* slot, int se
   __hip_atomic_store(&slot->seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-static int read_status_words(const void* workspace, int (&words)[2], hipStream_t s) {
+static int read_status_words(const void* workspace, int (&words)[2], hipStream_t s, bool slot_wanted) {
   static std::mutex mu;
   static StatusSlot* slots = nullptr;
   static unsigned in_use = 0;
   static int next_seq = 0;
   int at = -1, seq = 0;
-  {
+  if (slot_wanted) {
     std::lock_guard<std::mutex> lock(mu);
     if (!slots) {
       void* p = nullptr;
@@ -2005,31 +2006,10 @@ int ftk_stacked_lstm_opts_f32(const float* xs, const float* WU, const float* bia
                         workspace, workspace_bytes, (hipStream_t)stream, products, spin_limit);
 }
 
-int ftk_stacked_lstm_status(const void* workspace, ftk_stream_t stream) {
+static int stack_result(const void* workspace, int* small_states, hipStream_t stream, bool slot_wanted) {
   using namespace ftk;
-  if (!workspace) {  // the built-in scratch of ftk_stacked_lstm_noalloc_f32 on the current device
-    void* ptr = nullptr;
-    if (scratch_of_current_device("ftk_stacked_lstm_status", &ptr, false) != FTK_OK || !ptr)
-      return fail(FTK_ERR_INVALID_ARGUMENT,
-                  "ftk_stacked_lstm_status: workspace is NULL and ftk_stacked_lstm_noalloc_f32 has not run on the current device");
-    workspace = ptr;
-  }
-  return ftk_stacked_lstm_result(workspace, nullptr, stream);
-}
-
-int ftk_stacked_lstm_small_states(const void* workspace, ftk_stream_t stream) {
-  using namespace ftk;
-  if (!workspace) return fail(FTK_ERR_INVALID_ARGUMENT, "ftk_stacked_lstm_small_states: workspace is NULL");
   int words[2] = {0, 0};
-  const int rc = read_status_words(workspace, words, (hipStream_t)stream);
-  return rc ? rc : words[1] != 0 ? 1 : 0;
-}
-
-int ftk_stacked_lstm_result(const void* workspace, int* small_states, ftk_stream_t stream) {
-  using namespace ftk;
-  if (!workspace) return fail(FTK_ERR_INVALID_ARGUMENT, "ftk_stacked_lstm_result: workspace is NULL");
-  int words[2] = {0, 0};
-  const int rc = read_status_words(workspace, words, (hipStream_t)stream);
+  const int rc = read_status_words(workspace, words, stream, slot_wanted);
   if (rc) return rc;
   if (small_states) *small_states = words[1] != 0 ? 1 : 0;
   if (words[0] != 0)
@@ -2037,6 +2017,32 @@ int ftk_stacked_lstm_result(const void* workspace, int* small_states, ftk_stream
                 "stacked LSTM: a bounded wait of the persistent launch ran out of polls (status word %d); the launch drained "
                 "early and hsss / csss are incomplete", words[0]);
   return FTK_OK;
+}
+
+int ftk_stacked_lstm_status(const void* workspace, ftk_stream_t stream) {
+  using namespace ftk;
+  if (!workspace) {  // the built-in scratch of ftk_stacked_lstm_noalloc_f32 on the current device
+    void* ptr = nullptr;
+    if (scratch_of_current_device("ftk_stacked_lstm_status", &ptr, false) != FTK_OK || !ptr)
+      return fail(FTK_ERR_INVALID_ARGUMENT,
+                  "ftk_stacked_lstm_status: workspace is NULL and ftk_stacked_lstm_noalloc_f32 has not run on the current device");
+    return stack_result(ptr, nullptr, (hipStream_t)stream, false);
+  }
+  return stack_result(workspace, nullptr, (hipStream_t)stream, true);
+}
+
+int ftk_stacked_lstm_small_states(const void* workspace, ftk_stream_t stream) {
+  using namespace ftk;
+  if (!workspace) return fail(FTK_ERR_INVALID_ARGUMENT, "ftk_stacked_lstm_small_states: workspace is NULL");
+  int words[2] = {0, 0};
+  const int rc = read_status_words(workspace, words, (hipStream_t)stream, true);
+  return rc ? rc : words[1] != 0 ? 1 : 0;
+}
+
+int ftk_stacked_lstm_result(const void* workspace, int* small_states, ftk_stream_t stream) {
+  using namespace ftk;
+  if (!workspace) return fail(FTK_ERR_INVALID_ARGUMENT, "ftk_stacked_lstm_result: workspace is NULL");
+  return stack_result(workspace, small_states, (hipStream_t)stream, true);
 }
 
 int ftk_stacked_lstm_noalloc_f32(const float* xs, const float* WU, const float* bias, const int* dilations, float* hsss,

@@ -265,6 +265,8 @@ int ftk_stacked_lstm_opts_f32(const float* xs, const float* WU, const float* bia
  * outputs of ftk_stacked_lstm_f32 / _dilated_ / _ragged_ / _opts_ / _f16.
  * workspace == NULL: the built-in scratch of ftk_stacked_lstm_noalloc_f32 on
  * the current device (FTK_ERR_INVALID_ARGUMENT if that has never run there).
+ * With a workspace, the first such call of a process allocates 1 KB of pinned
+ * host memory, which it keeps and waits on; with NULL nothing is allocated.
  * No counterpart in the reference, whose launches do not wait for each other.
  */
 int ftk_stacked_lstm_status(const void* workspace, ftk_stream_t stream);

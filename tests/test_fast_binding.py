@@ -1,4 +1,5 @@
-"""The native module over the library: Python's lock is not held inside the library, whose launches may wait."""
+"""The native module over the library, and what the library allocates: Python's lock is not held inside the library, whose launches may
+wait, and the callers that do without allocations get none."""
 import os
 import shutil
 import subprocess
@@ -42,3 +43,33 @@ def test_python_lock_is_released_in_the_library(tmp_path):
     shutil.copy(os.path.join(HERE, '..', 'fractaltensor_amd', '_fast.so'), tmp_path / '_fast.so')
     done = subprocess.run([sys.executable, '-c', PROGRAM, str(tmp_path / '_fast.so')], capture_output=True, text=True, timeout=100)
     assert done.returncode == 0 and 'released in' in done.stdout, done.stdout + done.stderr
+
+
+COUNTED = """
+import ctypes, sys
+counter = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
+import torch
+import fractaltensor_amd._core as core
+L, T, B, H = 1, 2, 32, 256
+xs, WU = torch.zeros((T, B, H), device='cuda'), torch.zeros((L, 2 * H, 4 * H), device='cuda')
+out = torch.empty((L, T, B, H), device='cuda'), torch.empty((L, T, B, H), device='cuda')
+core.stacked_lstm_noalloc(xs, WU, None, out)
+before = counter.host_allocations()
+core.stacked_lstm_check(None)
+core.stacked_lstm_check(None)
+print('without a workspace', counter.host_allocations() - before)
+ws = torch.empty(core.stacked_lstm_workspace_bytes(L, T, B, H), dtype=torch.uint8, device='cuda')
+core.stacked_lstm(xs, WU, workspace=ws)
+core.stacked_lstm_check(ws)
+core.stacked_lstm_check(ws)
+print('with one', counter.host_allocations() - before)
+"""
+
+
+def test_status_of_the_built_in_scratch_allocates_nothing(tmp_path):
+    """The callers of the entry point that allocates nothing read its status without an allocation too; with a workspace the
+    first status call keeps one block of pinned host memory."""
+    lib = str(tmp_path / 'count_host_alloc.so')
+    subprocess.run(['g++', '-shared', '-fPIC', '-O1', os.path.join(HERE, 'count_host_alloc.cpp'), '-o', lib, '-ldl'], check=True)
+    done = subprocess.run([sys.executable, '-c', COUNTED, lib], capture_output=True, text=True, timeout=100, cwd=os.path.dirname(HERE))
+    assert done.returncode == 0 and 'without a workspace 0' in done.stdout and 'with one 1' in done.stdout, done.stdout + done.stderr
