@@ -24,7 +24,8 @@
 //
 // A step of a single layer takes 1.1 us at H = 64, 1.3 at 128, 1.6 at 256 and 2.4 at 512 (fp32), where a hand-over of the
 // persistent kernel's serial schedule took 5 to 6 and a launch per step 20 and more: L 20 T 30 B 32 H 128 1004 -> 108 us,
-// L 8 T 100 B 64 H 512 7.3 -> 0.76 ms, L 1 T 16 B 64 H 256 100 -> 26 us of kernel time.
+// L 8 T 100 B 64 H 512 7.3 -> 0.76 .. 0.79 ms, L 1 T 16 B 64 H 256 100 -> 38 us for both kernels
+// (34 and 4).
 //
 // The exchange buffers.  ring: the own layer's h for d = 1, four steps deep.  A workgroup that has all of h(t-1) knows
 // that every member of its team has read h(t-2) (it published h(t-1) behind a barrier that all its waves reached after

@@ -1802,7 +1802,7 @@ static int check_stack_args(const char* who, const float* xs, const float* WU, f
 
 // Which stacks go to the exchange kernel (lstm_exchange.hip): all it takes whose batch it spreads over the chip with one row
 // block per workgroup, because then the chain of dependent steps is the time (L 1 .. 8, T 32, B 64, H 256, fp32: 67 ..
-// 124 us against 198 .. 265; H 512, 8 layers, T 100: 0.92 ms against 7.3).  With more rows than that it walks several blocks per
+// 124 us against 198 .. 265; H 512, 8 layers, T 100: 0.76 .. 0.79 ms against 7.3).  With more rows than that it walks several blocks per
 // workgroup, and there
 //   H = 256 has the paired schedule of the persistent kernel, which feeds the matrix pipe better: ahead from 16 layers x
 //     256 rows on (L 16 B 192: 536 against 575 us, L 16 B 256: 660 against 585, L 32 B 192: 998 against 937; fp16 data: L 16
@@ -1965,7 +1965,7 @@ int ftk_stacked_lstm_f16(const void* xs, const void* WU, const float* bias, cons
     if (!workspace || workspace_bytes < need)
       return fail(FTK_ERR_WORKSPACE, "%s: workspace of %zu bytes needed, %zu given", who, need, workspace ? workspace_bytes : (size_t)0);
     hipLaunchKernelGGL(fill_zero_kernel, dim3(1), dim3(64), 0, (hipStream_t)stream, reinterpret_cast<int*>(workspace),
-                       (size_t)(kStatusBytes / sizeof(int)));  // nothing below waits: the status word is zero
+                       (size_t)(kStatusBytes / sizeof(int)));  // status word, and the one launch's tickets and counters
     int rcz = check_launch("fill_zero_kernel");
     if (rcz) return rcz;
     return run_wavefront_f16(xs, WU, bias, dilations, active_rows, hsss, csss, L, T, B, H, workspace, (hipStream_t)stream);

@@ -190,11 +190,11 @@ int ftk_stacked_lstm_ragged_f32(const float* xs, const float* WU,
  * chip as it holds and run deeper stacks as consecutive launches, where that
  * is the faster way.  Every other shape streams its weights through the fp16
  * cell kernels, in one launch or in one per stage of independent cells, on the
- * rows that live at the cell's step (H = 512 stacks of more than 16 layers and
- * deep H = 1024 stacks of large batches among them;
- * FTK_LSTM_F16_STREAM=1 / 0 forces either where both can run); the
- * workspace then takes a re-laid copy of WU (ftk_stacked_lstm_f16_workspace_bytes
- * says how much for a shape).
+ * rows that live at the cell's step (deep H = 1024 stacks of large batches
+ * among them); the workspace then takes a re-laid copy of WU.
+ * ftk_stacked_lstm_f16_workspace_bytes says how much the kernels take that a
+ * shape may go to on the current device; with less the call runs on one that
+ * has room, if there is one (FTK_ERR_WORKSPACE otherwise).
  * dilations, active_rows: host arrays or NULL, as above.
  * Replaces StackedLstmRegion1/2/3 with Element = half as instantiated by
  * benchmarks/rnn/fractaltensor/cute_stacked_lstm/stacked_lstm.cu:16-19,59-155
@@ -313,8 +313,10 @@ int ftk_stacked_lstm_result(const void* workspace, int* small_states, ftk_stream
  * 64*T*ceil(B/32) + 256 bytes) must fit the library's built-in scratch of
  * 2 MiB per device (config 4, L32 T64 B256: 1.03 MiB), else
  * FTK_ERR_UNSUPPORTED_SHAPE; likewise when L layers do not fit the device in
- * one persistent launch.  The call allocates nothing, frees nothing and waits
- * for nothing.  Every call on a device shares that device's scratch: calls
+ * one persistent launch.  The call allocates no memory, frees nothing and
+ * waits for nothing, as long as the stream of the device's stacked-LSTM launch
+ * before it still exists (else it waits for the device; another stream's
+ * launch that still runs is followed through an event).  Every call on a device shares that device's scratch: calls
  * that overlap on one device (two streams, two threads) race; calls on one
  * stream are safe.  ftk_stacked_lstm_status(NULL, stream) reads the status
  * word of the current device's scratch.
