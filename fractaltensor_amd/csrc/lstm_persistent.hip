@@ -1800,6 +1800,21 @@ static int check_stack_args(const char* who, const float* xs, const float* WU, f
   return FTK_OK;
 }
 
+// The persistent kernel holds the fp16 weights of H = 512, and of H = 256 with two batch rows per tile row (even B).
+static bool f16_fits_on_chip(int B, int H) { return H == 2 * PH || (H == PH && !(B & 1)); }
+
+// Whether an fp16 stack that the exchange kernel does not run goes through the streaming cell kernels.  Always where the
+// weights do not fit on chip; at H = 512 also when the stack is deeper than the 16 layers that 256 compute units
+// hold at once: the persistent kernel then runs twice and fills its wavefront twice (5.5 ms at L = 32, T = 64,
+// B = 256), while the streamed cells find the 134 MB of weights in the last-level cache (3.75 ms).  A ragged
+// batch stays with the persistent kernel, which skips the row blocks that have ended.
+// FTK_LSTM_F16_STREAM=1 / =0 in the environment forces the one or the other where both can run.
+static bool f16_streams(int L, int B, int H, bool ragged) {
+  if (!f16_fits_on_chip(B, H)) return true;
+  if (const char* e = getenv("FTK_LSTM_F16_STREAM")) return e[0] == '1';
+  return H == 2 * PH && L > 16 && !ragged;
+}
+
 // Which stacks go to the exchange kernel (lstm_exchange.hip): all it takes whose batch it spreads over the chip with one row
 // block per workgroup, because then the chain of dependent steps is the time (L 1 .. 8, T 32, B 64, H 256, fp32: 67 ..
 // 124 us against 198 .. 265; H 512, 8 layers, T 100: 0.76 .. 0.79 ms against 7.3).  With more rows than that it walks several blocks per
@@ -1812,6 +1827,11 @@ static int check_stack_args(const char* who, const float* xs, const float* WU, f
 //     B 256 4.21, 3.86; L 12 B 256 5.47, 4.49; L 16 B 192 5.58, 5.22, B 160 4.67, 5.09; L 20 B 192 7.01, 6.69, B 160 5.85,
 //     6.58; L 32 B 256 14.8, 10.5, B 192 11.2, 10.3, B 160 9.33, 10.17; T 32 L 8 B 256 1.85, 1.89).  Ragged batches run a launch per
 //     stage there, without the layers of the next stage to fill it.
+//   H = 512, fp16 data, takes 0.25 us per cell and block of 32 rows, and the streamed cells some 31 us a stage (as long as its
+//     tiles fill the chip once) whatever the batch (T 64, ms, exchange and streamed: L 20 B 256 2.63, 2.65, L 24 B 176 2.46, 2.69,
+//     B 224 2.92, 2.77, L 32 B 128 2.31, 3.11, B 192 3.23, 3.22, B 256 4.16, 3.35; T 16 L 32 B 256 1.23, 1.48; T 32 1.97, 2.03 at B
+//     224, 2.19, 2.10 at B 256; T 128 L 20 B 224 4.58, 4.60).  Up to 16 layers and for ragged batches the choice is between this
+//     and the persistent kernel, which is behind throughout (L 16 B 256: 2.06, 2.24).
 // FTK_LSTM_EXCHANGE=1 / =0 in the environment forces the one or the other.
 static bool exchange_chosen(int L, int T, int B, int H, const int* dil, bool half, bool ragged) {
   if (!exchange_takes(H, half) || !exchange_fits(T, B, H, half)) return false;
@@ -1823,6 +1843,10 @@ static bool exchange_chosen(int L, int T, int B, int H, const int* dil, bool hal
     return L * ((B + 31) / 32) < 112;
   }
   if (H == 1024) return ragged ? L < 12 || B <= 192 : 7ll * ((L + 3) / 4) * ((B + 31) / 32) <= 10ll * std::max(L, 12) * ((B + 255) / 256);
+  if (half && f16_streams(L, B, H, ragged)) {   // H = 512
+    const long long tiles = (long long)std::min(L, T) * ((B + 255) / 256) * (H / 64);   // of the streamed cells, in a full stage
+    return 256ll * L * T * ((B + 31) / 32) <= 117ll * (L + T - 1) * std::max(256ll, tiles);
+  }
   return true;
 }
 
@@ -1888,21 +1912,6 @@ static int run_stack(const char* who, const float* xs, const float* WU, const fl
 }  // namespace ftk
 
 namespace ftk {
-
-// The persistent kernel holds the fp16 weights of H = 512, and of H = 256 with two batch rows per tile row (even B).
-static bool f16_fits_on_chip(int B, int H) { return H == 2 * PH || (H == PH && !(B & 1)); }
-
-// Whether the fp16 stack goes through the streaming cell kernel, one launch per stage of cells.  Always where the
-// weights do not fit on chip; at H = 512 also when the stack is deeper than the 16 layers that 256 compute units
-// hold at once: the persistent kernel then runs twice and fills its wavefront twice (5.5 ms at L = 32, T = 64,
-// B = 256), while the streamed cells find the 134 MB of weights in the last-level cache (3.75 ms).  A ragged
-// batch stays with the persistent kernel, which skips the row blocks that have ended.
-// FTK_LSTM_F16_STREAM=1 / =0 in the environment forces the one or the other where both can run.
-static bool f16_streams(int L, int B, int H, bool ragged) {
-  if (!f16_fits_on_chip(B, H)) return true;
-  if (const char* e = getenv("FTK_LSTM_F16_STREAM")) return e[0] == '1';
-  return H == 2 * PH && L > 16 && !ragged;
-}
 
 // Workspace of the streaming kernels: the status block and the re-laid weights.
 static size_t f16_stream_bytes(int L, int H) { return kStatusBytes + (size_t)L * 2 * H * 4 * H * sizeof(_Float16); }

@@ -163,3 +163,16 @@ def test_f16_stack_takes_the_workspace_of_the_kernel_it_runs(core, monkeypatch):
         for dil, active in ((None, None), ([1 + l % 2 for l in range(L)], None), (None, [B] * (T - 1) + [B // 2])):
             h, _ = core.stacked_lstm_f16(xs, WU, dilations=dil, active_rows=active, workspace=ws, check=True)
             assert bool(torch.isfinite(h[:, :, :B // 2]).all())
+
+
+@pytest.mark.parametrize('L,T,B,way', [(32, 64, 256, '0'), (24, 64, 224, '0'), (24, 64, 176, '1'), (32, 16, 256, '1'), (16, 128, 256, '1')])
+def test_deep_f16_stacks_at_512_units_take_the_faster_kernel(core, monkeypatch, L, T, B, way):
+    """Both sides of the line between the exchange kernel ('1') and the streamed cells ('0'), whose bits differ."""
+    xs, WU = _f16_stack(L, T, B, 512, 17)
+    default = core.stacked_lstm_f16(xs, WU)
+    for e in '01':
+        monkeypatch.setenv('FTK_LSTM_EXCHANGE', e)
+        if L <= 16 and e == '0':
+            continue                                          # the persistent kernel
+        h, _ = core.stacked_lstm_f16(xs, WU)
+        assert torch.equal(h, default[0]) == (e == way)
