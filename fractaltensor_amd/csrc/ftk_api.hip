@@ -47,8 +47,9 @@ int device_props(const DeviceProps** out) {
 // resident in part and wait for the rest.  Launches on one stream follow each other anyway, so a process that uses one
 // stream gets ordinary launches.  When a second stream turns up while a launch of the first may still run, the new launch
 // is put behind the first stream's work, and from then on the device gets cooperative launches only; so it does from
-// the first stream capture on, whose graph may be replayed on any stream, and the first launch after it that is no
-// recording is put behind the ordinary ones (launch_order.h).  A replay is not seen here: a program
+// the first stream capture on, whose graph may be replayed on any stream (the first launch after it that is no
+// recording is put behind the ordinary ones), and from the first launch on the per-thread handle, which is another stream in
+// every thread (launch_order.h).  A replay is not seen here: a program
 // lets the launches it made before a capture end before it replays.  Kernels that merely occupy compute units end by themselves and need no care.
 // FTK_COOPERATIVE_LAUNCH=1: cooperative launches always (for processes that share a device).
 namespace {
