@@ -22,10 +22,9 @@
 //     32 workgroups that exchange a whole tile: 0.49 / 0.76 / 0.98 us a step, against 0.81 / 1.24 / 1.71 us with
 //     write-through stores, which is what a team that does not sit together uses.
 //
-// A step of a single layer takes 1.1 us at H = 64, 1.3 at 128, 1.6 at 256 and 2.4 at 512 (fp32), where a hand-over of the
-// persistent kernel's serial schedule took 5 to 6 and a launch per step 20 and more: L 20 T 30 B 32 H 128 1004 -> 108 us,
-// L 8 T 100 B 64 H 512 7.3 -> 0.76 .. 0.79 ms, L 1 T 16 B 64 H 256 100 -> 38 us for both kernels
-// (34 and 4).
+// A step of a single layer takes 0.85 us at H = 64, 0.9 at 128, 1.2 at 256 and 1.9 at 512 (fp32), where a hand-over of the
+// persistent kernel's serial schedule took 5 to 6 and a launch per step 20 and more: L 20 T 30 B 32 H 128 1004 -> 82 us,
+// L 8 T 100 B 64 H 512 7.3 -> 0.76 .. 0.79 ms, L 1 T 16 B 64 H 256 100 -> 31 us for both kernels (27 and 4).
 //
 // The exchange buffers.  ring: the own layer's h for d = 1, four steps deep.  A workgroup that has all of h(t-1) knows
 // that every member of its team has read h(t-2) (it published h(t-1) behind a barrier that all its waves reached after
@@ -53,7 +52,7 @@ constexpr int kXBlocks = 128;      // row blocks a ragged batch may have
 constexpr int kXRing = 4;          // steps the own layer's ring holds
 constexpr int kXPlaces = 2048;     // workgroups of one launch
 constexpr int kXHandTop = 14;      // the scale of h: 2^14 (|h| < 1)
-constexpr unsigned kXSmallBits = (127u - 12u) << 23;   // h * 2^14 below 2^-12: see ftk_stacked_lstm_small_states
+constexpr unsigned kXSmallBits = (127u - 12u - kXHandTop) << 23;   // h * 2^14 below 2^-12: see ftk_stacked_lstm_small_states
 
 struct ExchangeArgs {
   const void* WU;
@@ -77,6 +76,9 @@ struct ExchangeArgs {
 
 typedef unsigned long long u64;
 typedef unsigned short v2us __attribute__((ext_vector_type(2)));
+// four weights at any place a caller's array may begin
+typedef float weights4f __attribute__((ext_vector_type(4), aligned(4)));
+typedef _Float16 weights4h __attribute__((ext_vector_type(4), aligned(2)));
 constexpr int kAgentScope = 16;      // sc1 in the cache-policy operand of a buffer load
 
 // A tile of the exchange buffers: the h of a row block.  fp32 data: [H / 4][rows][4 units] words (value, remainder); fp16
@@ -116,6 +118,10 @@ void lstm_exchange_kernel(ExchangeArgs a) {
   typedef float accum __attribute__((ext_vector_type(AR)));
   typedef float sums __attribute__((ext_vector_type(4 * U)));   // the gates of a lane's units
   __shared__ sums red[2][4][4][64];          // [parity][wave that takes them][wave that gives them][lane]
+  // h and c of an item, for the wave that stores them; a row's 16 units and some more: all lanes on different banks
+  using Value = typename std::conditional<HALF, _Float16, float>::type;
+  constexpr int OUT_ROW = HALF ? 24 : 20;
+  __shared__ __attribute__((aligned(16))) Value outs[MANY ? 1 : 2][MANY ? 1 : 2][MANY ? 1 : 16 * OUT_ROW];
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -148,8 +154,10 @@ void lstm_exchange_kernel(ExchangeArgs a) {
   // A column is a gate of a unit, ordered so that a lane gets the four gates of a unit next to each other in its
   // accumulators (lane (m, kg) has rows 4 kg .. +3 of a 16-row result, and rows 8 q + 4 kg .. +3, q = 0 .. 3, of a
   // 32-row one) and, with 32-row results, neighbouring units: two of the half tile its wave finishes, or four of a tile.
+  // With 16-row results the four tiles hold a lane four neighbouring units of a gate, which is what one load brings: with
+  // a load for each weight H 512 took 16 us to begin.
   auto unit_of = [](int tt, int col) {
-    if (RT == 1) return 4 * tt + (col >> 2);
+    if (RT == 1) return 4 * (col >> 2) + tt;
     if (CT == 1) return 8 * tt + 4 * (col >> 4) + 2 * ((col >> 2) & 1) + ((col >> 3) & 1);
     return 8 * tt + 4 * ((col >> 2) & 1) + (col >> 3);
   };
@@ -171,9 +179,17 @@ void lstm_exchange_kernel(ExchangeArgs a) {
 #pragma unroll
       for (int i = 0; i < KS; ++i) {
 #pragma unroll
-        for (int e = 0; e < 8; ++e)
+        for (int e = 0; e < 8; ++e) {
+          const _Float16* row = wl + (size_t)(w_row(i) + 8 * kg + e) * 4 * H;
+          if constexpr (RT == 1) {
+            const v4h w = *reinterpret_cast<const weights4h*>(row + uo[0]);
 #pragma unroll
-          for (int tt = 0; tt < NT; ++tt) wt[i][tt][e] = wl[(size_t)(w_row(i) + 8 * kg + e) * 4 * H + uo[tt]];
+            for (int tt = 0; tt < NT; ++tt) wt[i][tt][e] = w[tt];
+          } else {
+#pragma unroll
+            for (int tt = 0; tt < NT; ++tt) wt[i][tt][e] = row[uo[tt]];
+          }
+        }
         if (i % (2 * RT) == 2 * RT - 1) asm volatile("" ::: "memory");   // 16-bit loads take a register each until they are packed
       }
     } else {
@@ -182,9 +198,17 @@ void lstm_exchange_kernel(ExchangeArgs a) {
 #pragma unroll
       for (int i = 0; i < KS; ++i)
 #pragma unroll
-        for (int e = 0; e < 8; ++e)
+        for (int e = 0; e < 8; ++e) {
+          const float* row = wl + (size_t)(w_row(i) + 8 * kg + e) * 4 * H;
+          if constexpr (RT == 1) {
+            const v4f w = *reinterpret_cast<const weights4f*>(row + uo[0]);
 #pragma unroll
-          for (int tt = 0; tt < NT; ++tt) raw[i][tt][e] = wl[(size_t)(w_row(i) + 8 * kg + e) * 4 * H + uo[tt]];
+            for (int tt = 0; tt < NT; ++tt) raw[i][tt][e] = w[tt];
+          } else {
+#pragma unroll
+            for (int tt = 0; tt < NT; ++tt) raw[i][tt][e] = row[uo[tt]];
+          }
+        }
       // the largest magnitude of each of the workgroup's columns, over the four waves
       float* const cmaxs = reinterpret_cast<float*>(red);   // [4 waves][tile, column], then what undoes the scales
 #pragma unroll
@@ -223,8 +247,8 @@ void lstm_exchange_kernel(ExchangeArgs a) {
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
           // tile and column of gate g of unit my_unit + u
-          const int tt = RT == 1 || CT == 2 ? wave : wave >> 1;
-          const int col = RT == 1 ? 4 * kg + g : CT == 2 ? 8 * u + 4 * kg + g : 16 * (wave & 1) + 8 * u + 4 * kg + g;
+          const int tt = RT == 1 ? kg : CT == 2 ? wave : wave >> 1;
+          const int col = RT == 1 ? 4 * wave + g : CT == 2 ? 8 * u + 4 * kg + g : 16 * (wave & 1) + 8 * u + 4 * kg + g;
           esc[4 * u + g] = cmaxs[256 * CT + tt * ROWS + col] * (g == 3 ? 1.0f : -kLog2e);
         }
       __syncthreads();
@@ -286,12 +310,14 @@ void lstm_exchange_kernel(ExchangeArgs a) {
   const bool team_here = look_at_places(unit);
   const bool has_upper = l + 1 < a.L;
   const bool upper_here = has_upper && alive ? look_at_places(unit + 1) : true;
+  const bool keep_c = d == 1 && s + a.slices >= nrb && !a.ragged;   // one row block: its c stays here
+  // Teams that wait for one row block each have a loop with as few stores as their place allows (`lean`): every store
+  // instruction of a wave is time on its way round.
+  const bool lean = !MANY && keep_c && team_here;
+  // a dilated recurrence reads its own h from `hand` too
   const bool own_by_ring = d == 1;
   const bool uses_hand = has_upper || !own_by_ring;
-  // a dilated recurrence reads its own h from `hand` too
-  const bool hand_plain = upper_here && (own_by_ring || team_here);
-
-  const bool keep_c = d == 1 && s + a.slices >= nrb && !a.ragged;   // one row block: its c stays here
+  const bool hand_plain = __builtin_amdgcn_readfirstlane(upper_here && (own_by_ring || team_here)) != 0;
   constexpr int ES = HALF ? 2 : 4;
   constexpr int BLOCK = ROWS * H * ES;         // bytes of a row block of xs, hsss, csss
   const int tiles_t = nrb * TILE;              // bytes of a time step of `hand`
@@ -333,8 +359,8 @@ void lstm_exchange_kernel(ExchangeArgs a) {
       v[2 * i + 1] = __builtin_bit_cast(v4u, __builtin_amdgcn_raw_buffer_load_b128(rs, lane_at + ROWS * 16, at + i * step, policy));
     }
   };
-  auto load_share = [&](desc rs, int at, share& v, auto policy_c) __attribute__((always_inline)) {
-    static_for<XS>([&](auto ic) __attribute__((always_inline)) { load_piece(ic, rs, get, at, v, policy_c); });
+  auto load_share = [&](desc rs, unsigned lane_at, int at, share& v, auto policy_c) __attribute__((always_inline)) {
+    static_for<XS>([&](auto ic) __attribute__((always_inline)) { load_piece(ic, rs, lane_at, at, v, policy_c); });
   };
   auto missing = [&](const share& v) __attribute__((always_inline)) -> bool {
     if constexpr (HALF) {
@@ -370,7 +396,7 @@ void lstm_exchange_kernel(ExchangeArgs a) {
         return;
       }
       asm volatile("" ::: "memory");   // the words change under us
-      load_share(rs, at, v, fresh);
+      load_share(rs, get, at, v, fresh);
     } while (missing(v));
   };
 
@@ -462,7 +488,7 @@ void lstm_exchange_kernel(ExchangeArgs a) {
   };
   // the lane's values of a row of hsss or csss
   struct values {
-    typename std::conditional<HALF, _Float16, float>::type v[U];
+    Value v[U];
   };
   auto put_row = [&](desc rs, unsigned off, int at, const float (&x)[U]) __attribute__((always_inline)) {
     values w;
@@ -506,17 +532,14 @@ void lstm_exchange_kernel(ExchangeArgs a) {
     return own_by_ring ? (it.rb * kXRing + ((it.t - 1) & (kXRing - 1))) * TILE : it.tile - d * tiles_t + it.rb * TILE;
   };
   auto row_off_of = [&](int rb) { return rb * ROWS + m < B ? (unsigned)((m * H + my_unit) * ES) : ~0u; };
-  float cp[U] = {};   // c of d steps before
+  values cp = {};     // c of d steps before
   float xr = 1.0f;
   share v;
   auto ask_c = [&](unsigned off, int at) __attribute__((always_inline)) {
-    values v;
-    if constexpr (sizeof(values) == 2) v = __builtin_bit_cast(values, __builtin_amdgcn_raw_buffer_load_b16(c_out, off, at, 0));
-    else if constexpr (sizeof(values) == 4) v = __builtin_bit_cast(values, __builtin_amdgcn_raw_buffer_load_b32(c_out, off, at, 0));
-    else if constexpr (sizeof(values) == 8) v = __builtin_bit_cast(values, __builtin_amdgcn_raw_buffer_load_b64(c_out, off, at, 0));
-    else v = __builtin_bit_cast(values, __builtin_amdgcn_raw_buffer_load_b128(c_out, off, at, 0));
-#pragma unroll
-    for (int u = 0; u < U; ++u) cp[u] = (float)v.v[u];
+    if constexpr (sizeof(values) == 2) cp = __builtin_bit_cast(values, __builtin_amdgcn_raw_buffer_load_b16(c_out, off, at, 0));
+    else if constexpr (sizeof(values) == 4) cp = __builtin_bit_cast(values, __builtin_amdgcn_raw_buffer_load_b32(c_out, off, at, 0));
+    else if constexpr (sizeof(values) == 8) cp = __builtin_bit_cast(values, __builtin_amdgcn_raw_buffer_load_b64(c_out, off, at, 0));
+    else cp = __builtin_bit_cast(values, __builtin_amdgcn_raw_buffer_load_b128(c_out, off, at, 0));
   };
 
   bool small_reported = false;
@@ -525,7 +548,7 @@ void lstm_exchange_kernel(ExchangeArgs a) {
     if constexpr (!HALF) {
       unsigned largest = 0;
 #pragma unroll
-      for (int u = 0; u < U; ++u) largest = max(largest, __float_as_uint(h[u] * (float)(1 << kXHandTop)) & 0x7fffffffu);
+      for (int u = 0; u < U; ++u) largest = max(largest, __float_as_uint(h[u]) & 0x7fffffffu);
       const u64 sm = __builtin_amdgcn_ballot_w64(largest < kXSmallBits);
       if (__builtin_expect(sm != 0 && !small_reported && alive, 0)) {
         u64 all = sm, any = __builtin_amdgcn_ballot_w64(largest != 0);
@@ -557,8 +580,10 @@ void lstm_exchange_kernel(ExchangeArgs a) {
     }
   };
   auto take_sums = [&](int parity) __attribute__((always_inline)) -> sums {
-    sums pre = red[parity][wave][0][lane] + red[parity][wave][1][lane];
-    pre += red[parity][wave][2][lane] + red[parity][wave][3][lane];
+    // (16-row results: unit 4 wave + kg is in tile kg, at the lanes of k group `wave`)
+    const int tile = RT == 1 ? kg : wave, at = RT == 1 ? 16 * wave + m : lane;
+    sums pre = red[parity][tile][0][at] + red[parity][tile][1][at];
+    pre += red[parity][tile][2][at] + red[parity][tile][3][at];
     return pre;
   };
   // the state update of this lane's units and their words of the exchange buffers
@@ -573,8 +598,11 @@ void lstm_exchange_kernel(ExchangeArgs a) {
         if constexpr (HALF) p[g] = pre[4 * u + g] * (g == 3 ? 1.0f : -kLog2e) + ebias[4 * u + g];
         else p[g] = pre[4 * u + g] * esc[4 * u + g] + ebias[4 * u + g];
       }
-      c[u] = gate(p[1]) * c_prev[u] + gate(p[0]) * tanh_f(p[3]);
+      c[u] = __builtin_fmaf(gate(p[1]), c_prev[u], gate(p[0]) * tanh_f(p[3]));
       h[u] = gate(p[2]) * tanh_f(c[u]);
+      // rounded to 32 bits before 16 in every loop: one instruction may do both, with another last bit now and then, and
+      // a ragged batch, which takes another loop than a dense one, gives the same bits
+      if constexpr (HALF) asm("" : "+v"(c[u]), "+v"(h[u]));
       unsigned word;
       if constexpr (HALF) {
         c[u] = (float)(_Float16)c[u];
@@ -635,7 +663,7 @@ void lstm_exchange_kernel(ExchangeArgs a) {
     auto take_x = [&](const Item& it) __attribute__((always_inline)) {
       const bool has_prev = it.t >= d;
       if constexpr (!FIRST) wait_share(below_l, x_at(it), v);
-      if (!keep_c) ask_c(has_prev ? row_off_of(it.rb) : ~0u, has_prev ? it.row - d * rows_t + it.rb * BLOCK : 0);
+      ask_c(has_prev && !keep_c ? row_off_of(it.rb) : ~0u, has_prev && !keep_c ? it.row - d * rows_t + it.rb * BLOCK : 0);
       const unsigned lane_at = has_prev && do_h ? get : kOut;
       const int at = has_prev ? h_at(it) : 0;
       const float ratio = xr;
@@ -649,9 +677,12 @@ void lstm_exchange_kernel(ExchangeArgs a) {
     Item it{0, s, 0, 0};
     if (a.ragged && a.steps_of[s] == 0) it = after(it);
     if (it.t >= T) return;
-    static_for<XS>([&](auto ic) __attribute__((always_inline)) { load_piece(ic, below_l, do_x ? get : kOut, x_at(it), v, cached); });
+    load_share(below_l, do_x ? get : kOut, x_at(it), v, cached);
     if constexpr (FIRST && !HALF) ask_ratio(it);
     take_x(it);
+    // nothing yet, but as many stores behind the loads of h as on the way round the loop: the compiler waits for the loads
+    // by their number, and on the way round would wait for the stores of the item before with them
+    store_later();
     while (true) {   // (a wave that has given up walks on without waiting, to every barrier the others wait at)
       const bool has_prev = it.t >= d;
       const Item next = after(it);
@@ -664,7 +695,7 @@ void lstm_exchange_kernel(ExchangeArgs a) {
       if constexpr (FIRST && !HALF) ask_ratio(more ? next : it);
       float c_prev[U];
 #pragma unroll
-      for (int u = 0; u < U; ++u) c_prev[u] = !has_prev ? 0.0f : keep_c || follows ? later.cv[u] : cp[u];
+      for (int u = 0; u < U; ++u) c_prev[u] = !has_prev ? 0.0f : keep_c || follows ? later.cv[u] : (float)cp.v[u];
       follows = next.rb == it.rb && next.t == it.t + d;
       give_sums(parity);
       // what the item before stored is complete before anything of this one is published: only what was asked for since
@@ -681,14 +712,148 @@ void lstm_exchange_kernel(ExchangeArgs a) {
       asm volatile("" ::: "memory");
       later_of(it, h, c);
       look_for_small(h);
-      if (more) take_x(next);
+      if (!more) break;
+      take_x(next);
       asm volatile("" ::: "memory");
       store_later();
       asm volatile("" ::: "memory");
-      if (!more) break;
       it = next;
     }
+    store_later();
   };
+  // The loop of a team that has one row block, whose h every step waits for: a wave issues an instruction in four or five
+  // cycles at best, so what is not needed is left out of it (the loop above has ten stores an item and forty instructions
+  // more for the places of items).  The words go to the ring and to `hand`, and instead of store_later's every wave makes
+  // one store of 16 bytes a lane: wave 0 the h of the item before, wave 1 its c (both from LDS, where they are since the
+  // last barrier), wave 2 sets back the words of this workgroup's units in the ring, wave 3 those in `hand`.  (With `hand`
+  // for the own layer too, and no ring, a step took 0.1 us more: its lines are new to L2.)
+  // T 64 B 16 in us, the loop above -> this one, one layer / eight: fp32 H 64 79 -> 62 / 107 -> 94, 128 83 -> 65 / 113 -> 99,
+  // 256 103 -> 87 / 135 -> 116, 512 160 -> 142 / 196 -> 175; fp16 H 256 79 -> 58 / 105 -> 100, 512 106 -> 78 / 141 -> 118.
+  // PLAIN: the layer above is on this XCD, or there is none.
+  auto walk_lean = [&](auto first_c, auto plain_c) __attribute__((always_inline)) {
+    constexpr bool FIRST = decltype(first_c)::value, PLAIN = decltype(plain_c)::value;
+    constexpr std::integral_constant<int, PLAIN ? 0 : kAgentScope> up_policy{};
+    constexpr int step = TILE, wrap = kXRing * TILE - 1;
+    const int words_at = s * kXRing * TILE;
+    int words = 0;           // of this item in the ring: words_at + words
+    int x_at = s * TILE;     // this item's place in `hand` and in the layer below
+    // this wave's store: the next one goes to share_base + share_at, which moves on by share_step within share_wrap
+    const desc share_l = wave == 0 ? h_out : wave == 1 ? c_out : wave == 2 ? own_l : hand_l;
+    const int share_base = wave == 2 ? words_at : 0;
+    const int share_step = wave < 2 ? rows_t : wave == 2 ? step : tiles_t, share_wrap = wave == 2 ? wrap : ~0;
+    int share_at = wave < 2 ? s * BLOCK - rows_t : wave == 2 ? 2 * step : 2 * tiles_t + s * TILE;
+    const int share_row = HALF ? lane >> 1 : lane >> 2, share_part = HALF ? lane & 1 : lane & 3;   // 16 bytes of a row of 16 units
+    unsigned share_put = ~0u;
+    if (wave < 2 ? share_row < 16 && s * 16 + share_row < B : (wave == 2 || has_upper) && (!HALF || lane < 32))
+      share_put = wave < 2 ? (unsigned)((share_row * H + UNITS * pc) * ES + share_part * 16) : (unsigned)(UNITS * pc * 16 * ES + lane * 16);
+    unsigned share_next = ~0u;   // where the next one goes
+    unsigned my_put = put, up_put = has_upper ? put : ~0u;
+    const Value* const share_from = &outs[0][wave & 1][(share_row & 15) * OUT_ROW + share_part * (HALF ? 8 : 4)];
+    Value* const share_to = &outs[0][0][m * OUT_ROW + 4 * wave + kg];
+    constexpr int OUT_BUF = 2 * 16 * OUT_ROW;
+    auto store_share = [&](int parity) __attribute__((always_inline)) {
+      v4u w = {~0u, ~0u, ~0u, ~0u};
+      if (wave < 2) w = *reinterpret_cast<const v4u*>(share_from + parity * OUT_BUF);
+      store_bytes(cached, w, share_l, PLAIN || wave < 3 ? share_next : ~0u, share_base + share_at);
+      if constexpr (!PLAIN) store_bytes(fresh, w, share_l, wave < 3 ? ~0u : share_next, share_base + share_at);
+      share_at = (share_at + share_step) & share_wrap;
+      share_next = share_put;
+    };
+    auto wait_for = [&](desc rs, int at, share& v) __attribute__((always_inline)) {
+      if (__builtin_expect(missing(v), 0)) {
+        wait_share(rs, at, v);
+        if (!alive) my_put = up_put = share_put = share_next = ~0u;
+      }
+    };
+    load_share(below_l, do_x ? get : 0x80000000u, x_at, v, cached);
+    if constexpr (FIRST && !HALF) xr = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(ratios, m * 4, s * (ROWS * 4), 0));
+    // h is asked for in front of the products of x, where registers and its way leave time for it, and behind them: what comes
+    // too early is not there yet, and to ask again only then costs the whole way once more.  (L 1 T 64 B 16: H 128
+    // 69 us when asked for behind x only, 65 with both; L 20 T 30 B 32 H 128 83 and 81.6; fp16 H 512 88 and 78.)
+    constexpr bool TWICE = HALF ? H <= 512 : H <= 128;
+    share vh;
+    float c[U] = {}, h[U];
+    const unsigned x_get = do_x ? get : 0x80000000u, h_get = do_h ? get : 0x80000000u;   // out of bounds: zeros
+    int parity = 0;
+    // Nothing to store yet, but as many stores behind the loads of x as on the way round the loop: the compiler waits for
+    // the loads by their number, and on the way round would wait for the stores with them.
+    asm volatile("" ::: "memory");
+    static_for<PLAIN ? 3 : 4>([&](auto ic) __attribute__((always_inline)) {   // (two that are the same would become one)
+      store_bytes(cached, all_ones, own_l, ~0u, 64 * decltype(ic)::value);
+    });
+    if (wave >= 2) share_next = share_put;   // waves 0 and 1 have nothing at their first turn: there is no item before
+    for (int t = 0;; ++t) {
+      const bool more = t + 1 < T;
+      const int next_x = more ? x_at + tiles_t : x_at, before = words_at + ((words - step) & wrap);
+      const unsigned h_get_t = t > 0 ? h_get : 0x80000000u;
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (TWICE) {
+        if (HALF || !FIRST || has_upper) __builtin_amdgcn_s_sleep(2);   // 128 cycles
+        load_share(own_l, h_get_t, before, vh, fresh);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (!FIRST) wait_for(below_l, x_at, v);
+      share_products(v, x_steps, std::true_type{}, [](auto) __attribute__((always_inline)) {});
+      if constexpr (FIRST && !HALF) scale_input(xr);
+#pragma unroll
+      for (int tt = 0; tt < NT; ++tt) {   // (left to itself the compiler moves the scaling behind the wait for h)
+        asm volatile("" : "+v"(acc[tt]));
+        if constexpr (TWO) asm volatile("" : "+v"(cross[tt]));
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      load_share(own_l, h_get_t, before, v, fresh);
+      __builtin_amdgcn_sched_barrier(0);
+      share& h_words = TWICE ? vh : v;
+      if constexpr (TWICE) {
+        if (__builtin_expect(missing(vh), 0)) {
+          wait_for(own_l, before, v);
+#pragma unroll
+          for (int i = 0; i < NL; ++i) vh[i] = v[i];
+        }
+      } else {
+        wait_for(own_l, before, v);
+      }
+      share_products(h_words, h_steps, std::false_type{}, [&](auto ic) __attribute__((always_inline)) {
+        load_piece(ic, below_l, x_get, next_x, v, cached);
+      });
+      if constexpr (FIRST && !HALF)
+        xr = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(ratios, m * 4, ((more ? t + 1 : t) * nrb + s) * (ROWS * 4), 0));
+      give_sums(parity);
+      // what was set back after the item before is complete before anything of this one is published
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(NL + (FIRST && !HALF ? 1 : 0)) : "memory");
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+      const sums pre = take_sums(parity);
+      float c_prev[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) c_prev[u] = c[u];
+      const struct words word = update(pre, c_prev, c, h);
+      store_bytes(cached, word, own_l, my_put, words_at + words);
+      store_bytes(up_policy, word, hand_l, up_put, x_at);
+      share_to[parity * OUT_BUF] = (Value)h[0];
+      share_to[parity * OUT_BUF + 16 * OUT_ROW] = (Value)c[0];
+      asm volatile("" ::: "memory");
+      look_for_small(h);
+      parity ^= 1;
+      if (t + 2 >= T && wave == 3) share_put = share_next = ~0u;
+      store_share(parity);
+      if (!more) break;
+      asm volatile("" ::: "memory");
+      x_at = next_x;
+      words = (words + step) & wrap;
+    }
+    __syncthreads();   // h and c of the last item
+    if (wave < 2) store_share(parity ^ 1);
+  };
+  if constexpr (!MANY) {
+    if (lean) {
+      if (l == 0 && hand_plain) walk_lean(std::true_type{}, std::true_type{});
+      else if (l == 0) walk_lean(std::true_type{}, std::false_type{});
+      else if (hand_plain) walk_lean(std::false_type{}, std::true_type{});
+      else walk_lean(std::false_type{}, std::false_type{});
+      return;
+    }
+  }
   if (l == 0) walk(std::true_type{});
   else walk(std::false_type{});
 }
