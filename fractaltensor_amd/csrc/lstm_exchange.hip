@@ -75,6 +75,10 @@ struct ExchangeArgs {
 };
 
 typedef unsigned long long u64;
+
+// How words leave a workgroup that is not in a hurry: to `hand` as plain stores (the layer above, if any, on this XCD) or
+// write-through, to the ring as plain ones; or (teams over several XCDs) as either, by two stores of which one is out of bounds.
+enum { kAnyWay, kPlain, kThrough };
 typedef unsigned short v2us __attribute__((ext_vector_type(2)));
 // four weights at any place a caller's array may begin
 typedef float weights4f __attribute__((ext_vector_type(4), aligned(4)));
@@ -482,9 +486,10 @@ void lstm_exchange_kernel(ExchangeArgs a) {
   words all_ones;
 #pragma unroll
   for (int u = 0; u < U; ++u) all_ones.v[u] = (decltype(all_ones.v[0] + 0))~0u;
-  auto put_words = [&](desc rs, int at, words w, bool plain, bool on) __attribute__((always_inline)) {
-    store_bytes(cached, w, rs, on && plain ? put : ~0u, at);
-    store_bytes(fresh, w, rs, on && !plain ? put : ~0u, at);
+  auto put_words = [&](auto way_c, desc rs, int at, words w, bool plain, bool on) __attribute__((always_inline)) {
+    constexpr int WAY = decltype(way_c)::value;
+    if constexpr (WAY != kThrough) store_bytes(cached, w, rs, on && (WAY == kPlain || plain) ? put : ~0u, at);
+    if constexpr (WAY != kPlain) store_bytes(fresh, w, rs, on && (WAY == kThrough || !plain) ? put : ~0u, at);
   };
   // the lane's values of a row of hsss or csss
   struct values {
@@ -504,11 +509,11 @@ void lstm_exchange_kernel(ExchangeArgs a) {
     float hv[U] = {}, cv[U] = {};
     bool on_hand = false, on_ring = false;
   } later;
-  auto store_later = [&]() __attribute__((always_inline)) {
+  auto store_later = [&](auto way_c) __attribute__((always_inline)) {
     put_row(h_out, later.row_off, later.row, later.hv);
     put_row(c_out, later.row_off, later.row, later.cv);
-    put_words(hand_l, later.hand, all_ones, hand_plain, later.on_hand);
-    put_words(own_l, later.ring, all_ones, team_here, later.on_ring);
+    put_words(way_c, hand_l, later.hand, all_ones, hand_plain, later.on_hand);
+    put_words(std::integral_constant<int, decltype(way_c)::value == kAnyWay ? kAnyWay : kPlain>{}, own_l, later.ring, all_ones, team_here, later.on_ring);
   };
 
   // ---- items.  An item's place: time step, row block, and the byte offsets of its time step
@@ -532,14 +537,21 @@ void lstm_exchange_kernel(ExchangeArgs a) {
     return own_by_ring ? (it.rb * kXRing + ((it.t - 1) & (kXRing - 1))) * TILE : it.tile - d * tiles_t + it.rb * TILE;
   };
   auto row_off_of = [&](int rb) { return rb * ROWS + m < B ? (unsigned)((m * H + my_unit) * ES) : ~0u; };
-  values cp = {};     // c of d steps before
+  float cp[U] = {};   // c of d steps before
+  values raw_cp = {};  // the same as it was loaded: converted at once it would have to be there at once
   float xr = 1.0f;
   share v;
   auto ask_c = [&](unsigned off, int at) __attribute__((always_inline)) {
-    if constexpr (sizeof(values) == 2) cp = __builtin_bit_cast(values, __builtin_amdgcn_raw_buffer_load_b16(c_out, off, at, 0));
-    else if constexpr (sizeof(values) == 4) cp = __builtin_bit_cast(values, __builtin_amdgcn_raw_buffer_load_b32(c_out, off, at, 0));
-    else if constexpr (sizeof(values) == 8) cp = __builtin_bit_cast(values, __builtin_amdgcn_raw_buffer_load_b64(c_out, off, at, 0));
-    else cp = __builtin_bit_cast(values, __builtin_amdgcn_raw_buffer_load_b128(c_out, off, at, 0));
+    values v;
+    if constexpr (sizeof(values) == 2) v = __builtin_bit_cast(values, __builtin_amdgcn_raw_buffer_load_b16(c_out, off, at, 0));
+    else if constexpr (sizeof(values) == 4) v = __builtin_bit_cast(values, __builtin_amdgcn_raw_buffer_load_b32(c_out, off, at, 0));
+    else if constexpr (sizeof(values) == 8) v = __builtin_bit_cast(values, __builtin_amdgcn_raw_buffer_load_b64(c_out, off, at, 0));
+    else v = __builtin_bit_cast(values, __builtin_amdgcn_raw_buffer_load_b128(c_out, off, at, 0));
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if constexpr (HALF) raw_cp.v[u] = v.v[u];
+      else cp[u] = v.v[u];
+    }
   };
 
   bool small_reported = false;
@@ -655,8 +667,9 @@ void lstm_exchange_kernel(ExchangeArgs a) {
   // are formed, the pieces of the next item's x are asked for one by one into the registers that have been used (a burst
   // of loads would hold up the wave: 64 bytes a cycle is what a compute unit gets), and while those of x are formed
   // (which is after this item's h has been published) the pieces of the next h.
-  auto walk = [&](auto first_c) __attribute__((always_inline)) {
+  auto walk = [&](auto first_c, auto way_c) __attribute__((always_inline)) {
     constexpr bool FIRST = decltype(first_c)::value;
+    constexpr std::integral_constant<int, decltype(way_c)::value == kAnyWay ? kAnyWay : kPlain> own_way{};
     constexpr unsigned kOut = 0x80000000u;   // a lane offset beyond every descriptor: the load returns zeros
     // products of the x in v; the pieces of h (and c) of the same item take its place.  Where there is nothing (no step
     // that far back, or the half of the contraction another wave has) v is zeros and the products are those of zeros.
@@ -682,7 +695,7 @@ void lstm_exchange_kernel(ExchangeArgs a) {
     take_x(it);
     // nothing yet, but as many stores behind the loads of h as on the way round the loop: the compiler waits for the loads
     // by their number, and on the way round would wait for the stores of the item before with them
-    store_later();
+    if constexpr (MANY) store_later(way_c);
     while (true) {   // (a wave that has given up walks on without waiting, to every barrier the others wait at)
       const bool has_prev = it.t >= d;
       const Item next = after(it);
@@ -695,7 +708,7 @@ void lstm_exchange_kernel(ExchangeArgs a) {
       if constexpr (FIRST && !HALF) ask_ratio(more ? next : it);
       float c_prev[U];
 #pragma unroll
-      for (int u = 0; u < U; ++u) c_prev[u] = !has_prev ? 0.0f : keep_c || follows ? later.cv[u] : (float)cp.v[u];
+      for (int u = 0; u < U; ++u) c_prev[u] = !has_prev ? 0.0f : keep_c || follows ? later.cv[u] : (HALF ? (float)raw_cp.v[u] : cp[u]);
       follows = next.rb == it.rb && next.t == it.t + d;
       give_sums(parity);
       // what the item before stored is complete before anything of this one is published: only what was asked for since
@@ -707,19 +720,23 @@ void lstm_exchange_kernel(ExchangeArgs a) {
       parity ^= 1;
       float c[U], h[U];
       const words word = update(pre, c_prev, c, h);
-      put_words(own_l, ring_at(it.rb, it.t), word, team_here, alive && own_by_ring);
-      put_words(hand_l, x_at(it), word, hand_plain, alive && uses_hand);
+      put_words(own_way, own_l, ring_at(it.rb, it.t), word, team_here, alive && own_by_ring);
+      put_words(way_c, hand_l, x_at(it), word, hand_plain, alive && uses_hand);
       asm volatile("" ::: "memory");
       later_of(it, h, c);
       look_for_small(h);
       if (!more) break;
+      // With one row block the next h is what is waited for, and asking for it too early costs more than the stores in front
+      // (fp16 H 1024 L 4 T 64 B 16 238 -> 184 us); with several it is there, and the stores are in its way.
+      if constexpr (!MANY) store_later(way_c);
+      asm volatile("" ::: "memory");
       take_x(next);
       asm volatile("" ::: "memory");
-      store_later();
+      if constexpr (MANY) store_later(way_c);
       asm volatile("" ::: "memory");
       it = next;
     }
-    store_later();
+    store_later(way_c);
   };
   // The loop of a team that has one row block, whose h every step waits for: a wave issues an instruction in four or five
   // cycles at best, so what is not needed is left out of it (the loop above has ten stores an item and forty instructions
@@ -854,8 +871,17 @@ void lstm_exchange_kernel(ExchangeArgs a) {
       return;
     }
   }
-  if (l == 0) walk(std::true_type{});
-  else walk(std::false_type{});
+  auto walk_layer = [&](auto way_c) __attribute__((always_inline)) {
+    if (l == 0) walk(std::true_type{}, way_c);
+    else walk(std::false_type{}, way_c);
+  };
+  // One store instead of two wherever a team sits on one XCD (L 8 T 100 B 64 H 512 755 -> 730 us; fp32 at H 256 has no
+  // register left: with three copies of the loop it spills in the loop, 1070 -> 1190 us at L 16 T 114 B 104).
+  if constexpr (MANY && (HALF || CT == 1)) {
+    if (team_here && hand_plain) return walk_layer(std::integral_constant<int, kPlain>{});
+    if (team_here && own_by_ring) return walk_layer(std::integral_constant<int, kThrough>{});
+  }
+  walk_layer(std::integral_constant<int, kAnyWay>{});
 }
 
 // In front of the kernel above: status block, places, the ring and the first two steps of `hand` (blockIdx.y < layers), and
@@ -986,11 +1012,17 @@ struct ExchangePlan {
   int per_xcd = 0;   // teams per XCD, 0: workgroups in order
 };
 
-ExchangePlan exchange_plan(int L, int W, int nrb, int slots) {   // W: workgroups of a team
-  ExchangePlan p;
+// Teams of W workgroups that are on the chip at once.
+int exchange_teams(int W, int slots) {
   const int here = std::min(slots, kXPlaces);
   const int room = here / 8 / W;   // teams an XCD holds
-  const int teams = room ? 8 * room : here / W;   // (a team may be larger than an XCD)
+  return room ? 8 * room : here / W;   // (a team may be larger than an XCD)
+}
+
+ExchangePlan exchange_plan(int L, int W, int nrb, int slots) {   // W: workgroups of a team
+  ExchangePlan p;
+  const int teams = exchange_teams(W, slots);
+  const bool room = teams >= 8;
   if (teams == 0) return p;
   p.layers = std::min({L, teams, kXLayers});
   p.slices = std::max(1, std::min(nrb, teams / p.layers));
@@ -1018,24 +1050,31 @@ size_t exchange_workspace_bytes(int L, int T, int B, int H, bool half) {
 // Whether a layer of a buffer stays below what a buffer descriptor and its offsets reach.
 bool exchange_fits(int T, int B, int H, bool half) { return (size_t)T * ((size_t)(B + 31) / 32 * 32) * H * (half ? 2 : 4) < (1ull << 31) - (1 << 20); }
 
-// Whether the whole batch of every layer fits the chip with one block of 16 rows per workgroup.
-bool exchange_one_block(int L, int B, int H, bool half) {
+namespace {
+
+// Layers of one launch with one block of 16 rows per workgroup (0: the device holds none).
+int exchange_one_block_layers(int L, int B, int H, bool half) {
   const ExchangeFlavour f = exchange_flavour_of(H, half);
-  if (!f.one) return false;
-  const int nrb = (B + 15) / 16;
-  const ExchangePlan p = exchange_plan(L, H / exchange_units(H, half, false), nrb, exchange_slots(f.one));
-  return p.layers == L && p.slices == nrb;
+  if (!f.one) return 0;
+  return std::min({L, kXLayers, exchange_teams(H / exchange_units(H, half, false), exchange_slots(f.one)) / ((B + 15) / 16)});
 }
 
-namespace {
-// Layers of one launch (0: the device cannot hold one), and the kind of row block.
+// Layers of one launch (0: the device cannot hold one), and the kind of row block: 16 rows and one block per workgroup,
+// whose step is the shorter one, wherever that takes no more launches.  (L 23 T 67 B 10 fp32 H 512, three launches of
+// either kind: 831 us with blocks of 32, 540 with blocks of 16; at L 27 T 48 B 17, seven launches against four, they are level.)
 int exchange_layers(int L, int B, int H, bool half, bool* many) {
   const ExchangeFlavour f = exchange_flavour_of(H, half);
-  *many = !exchange_one_block(L, B, H, half);
-  const int block = *many ? 32 : 16;
-  return exchange_plan(L, H / exchange_units(H, half, *many), (B + block - 1) / block, exchange_slots(*many ? f.many : f.one)).layers;
+  *many = false;
+  if (!f.one) return 0;
+  const int one = exchange_one_block_layers(L, B, H, half);
+  const int more = one == L ? 0 : exchange_plan(L, H / exchange_units(H, half, true), (B + 31) / 32, exchange_slots(f.many)).layers;
+  *many = one == 0 || (one < L && more > 0 && (L + one - 1) / one > (L + more - 1) / more);
+  return *many ? more : one;
 }
 }  // namespace
+
+// Whether the whole batch of every layer fits the chip with one block of 16 rows per workgroup.
+bool exchange_one_block(int L, int B, int H, bool half) { return exchange_one_block_layers(L, B, H, half) == L; }
 
 // Bytes of workspace that run_exchange uses on the current device; without a device, what it could at most.
 size_t exchange_need(int L, int T, int B, int H, bool half) {

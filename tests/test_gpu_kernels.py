@@ -1398,6 +1398,27 @@ def test_windowed_attention_rejects_bad_arguments(core):
         core.windowed_attention(Q, Q[:, :4], Q, 3)
 
 
+@pytest.mark.parametrize('half,H,L,B', [
+    (False, 64, 1, 1), (False, 128, 9, 17), (False, 128, 20, 33), (False, 256, 2, 16), (False, 512, 2, 15),
+    (True, 256, 3, 18), (True, 512, 4, 16), (True, 1024, 2, 17),
+])
+@pytest.mark.parametrize('T', [1, 2, 3, 4, 9])
+def test_exchange_loops_give_the_same_bits(core, half, H, L, B, T):
+    """A dense batch takes the loop of teams that wait for one row block, a ragged one the general loop: rows that live to
+    the end have the same h and c bit for bit, and in every launch (the first and last items of a loop, stores an item late,
+    words set back or not, layers with and without another one above, on the same XCD and on another)."""
+    gen = torch.Generator(device='cuda').manual_seed(11)
+    dtype = torch.float16 if half else torch.float32
+    xs = torch.randn((T, B, H), generator=gen, device='cuda').to(dtype)
+    WU = ((torch.rand((L, 2 * H, 4 * H), generator=gen, device='cuda') * 2 - 1) * H ** -0.5).to(dtype)
+    bias = torch.rand((L, 4 * H), generator=gen, device='cuda')
+    fn = core.stacked_lstm_f16 if half else core.stacked_lstm
+    general = fn(xs, WU, bias, active_rows=[B] * T, check=True)
+    for _ in range(3):
+        dense = fn(xs, WU, bias, check=True)
+        assert all(torch.equal(a, b) for a, b in zip(dense, general))
+
+
 @pytest.mark.parametrize('half,H,L,T,B,dil', [
     (False, 64, 3, 5, 17, None),           # half a k step per wave: x and h waves; the second row block holds one row
     (False, 64, 32, 4, 130, None),         # several 32-row blocks per workgroup, the last of two rows
@@ -1408,6 +1429,7 @@ def test_windowed_attention_rejects_bad_arguments(core):
     (False, 512, 2, 7, 1, None),           # one row
     (False, 512, 8, 5, 33, None),          # two 32-row blocks on one workgroup, every layer on an XCD of its own
     (False, 512, 9, 3, 20, None),          # a layer more than the chip holds: two launches
+    (False, 512, 9, 4, 16, None),          # a layer more than the chip holds, blocks of 16 rows in both launches
     (True, 256, 3, 7, 17, None),
     (True, 512, 17, 3, 40, [1, 2] * 8 + [3]),
     (True, 1024, 2, 6, 18, None),          # a layer larger than an XCD
