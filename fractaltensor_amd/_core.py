@@ -337,6 +337,29 @@ def stacked_lstm(xs, WU, bias=None, dilations: Optional[Sequence[int]] = None, s
     return hsss, csss
 
 
+def stacked_lstm_launch(xs, WU, bias, dilations: Optional[Sequence[int]] = None, products: Optional[str] = None):
+    """The launch of stacked_lstm(..., exact_small_states=True) without its wait, so that a caller can do something meanwhile:
+    (hsss, csss, what stacked_lstm_finish takes), or None for operands that stacked_lstm has to look at more closely."""
+    if products is not None and products not in LSTM_PRODUCTS or xs.dim() != 3 or WU.dim() != 3 or not xs.is_cuda:
+        return None
+    workspace = _fast.stacked_lstm_workspace(False, xs, WU)
+    done = _fast.stacked_lstm(False, xs, WU, bias, dilations, None, workspace, -1 if products is None else LSTM_PRODUCTS[products],
+                              False, False)
+    return None if done is None else (done[0], done[1], (xs, WU, bias, dilations, products, workspace))
+
+
+def stacked_lstm_finish(launched) -> bool:
+    """Waits for a stacked_lstm_launch, raises FtkError if it gave up a wait, and repeats it on fp32 products, into the same
+    outputs, if it met states too small for split ones; says whether it did."""
+    hsss, csss, (xs, WU, bias, dilations, products, workspace) = launched
+    small = _fast.stacked_lstm_result(workspace)
+    if not small or products == 'f32':
+        return False
+    _count('stacked_lstm_repeated_on_f32_products')
+    stacked_lstm(xs, WU, bias, dilations=dilations, out=(hsss, csss), workspace=workspace, products='f32', check=True)
+    return True
+
+
 def stacked_lstm_noalloc(xs, WU, bias, out: Tuple[torch.Tensor, torch.Tensor], dilations: Optional[Sequence[int]] = None) -> None:
     """ftk_stacked_lstm_noalloc_f32: the fp32-product persistent stack (H = 256) into caller-supplied hsss, csss
     [L,T,B,H], with the launch's flags in the library's built-in per-device scratch.  Nothing is allocated, here or in

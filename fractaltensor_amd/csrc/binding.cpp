@@ -249,6 +249,36 @@ PyObject* stacked_lstm(PyObject*, PyObject* const* a, Py_ssize_t n) {
   });
 }
 
+// stacked_lstm_result(workspace): waits for the current stream, raises if the last stack on this workspace gave up a wait, and
+// says whether it met small states.
+PyObject* stacked_lstm_result(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  return guarded([&]() -> PyObject* {
+    if (n != 1 || !is_tensor(a[0]) || !tensor_of(a[0]).is_cuda()) {
+      PyErr_SetString(PyExc_TypeError, "stacked_lstm_result(workspace on the GPU)");
+      return nullptr;
+    }
+    const at::Tensor& ws = tensor_of(a[0]);
+    void *const wp = ws.data_ptr(), *const s = stream();
+    int small = 0;
+    const int rc = in_library([&] { return ftk_stacked_lstm_result(wp, &small, s); });
+    return rc ? raise(rc) : PyBool_FromLong(small);
+  });
+}
+
+// stacked_lstm_workspace(half, xs [T,B,H], WU [L,2H,4H]): the workspace of their stack.
+PyObject* stacked_lstm_workspace(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  return guarded([&]() -> PyObject* {
+    if (n != 3 || !is_tensor(a[1]) || !is_tensor(a[2]) || tensor_of(a[1]).dim() != 3 || tensor_of(a[2]).dim() != 3) {
+      PyErr_SetString(PyExc_TypeError, "stacked_lstm_workspace(half, xs [T,B,H], WU [L,2H,4H])");
+      return nullptr;
+    }
+    const at::Tensor& xs = tensor_of(a[1]);
+    const int L = dim(tensor_of(a[2]), 0), T = dim(xs, 0), B = dim(xs, 1), H = dim(xs, 2);
+    const size_t need = a[0] == Py_True ? ftk_stacked_lstm_f16_workspace_bytes(L, T, B, H) : ftk_stacked_lstm_workspace_bytes(L, T, B, H);
+    return THPVariable_Wrap(empty({(int64_t)need}, at::kByte, xs));
+  });
+}
+
 PyMethodDef methods[] = {
     {"init", (PyCFunction)(void*)init, METH_FASTCALL, "init(counts, raise)"},
     {"b2b_gemm", (PyCFunction)(void*)b2b_gemm, METH_FASTCALL, "b2b_gemm(A, B_nk, C_pn, out)"},
@@ -256,6 +286,8 @@ PyMethodDef methods[] = {
      "flash_attention(half, Q, K, V, scale, out, workspace, split_keys)"},
     {"stacked_lstm", (PyCFunction)(void*)stacked_lstm, METH_FASTCALL,
      "stacked_lstm(half, xs, WU, bias, dilations, out, workspace, products, check, small)"},
+    {"stacked_lstm_result", (PyCFunction)(void*)stacked_lstm_result, METH_FASTCALL, "stacked_lstm_result(workspace)"},
+    {"stacked_lstm_workspace", (PyCFunction)(void*)stacked_lstm_workspace, METH_FASTCALL, "stacked_lstm_workspace(half, xs, WU)"},
     {nullptr, nullptr, 0, nullptr}};
 
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_fast", "the fused entry points on torch tensors", -1, methods, nullptr, nullptr, nullptr, nullptr};

@@ -66,7 +66,8 @@ class FractalTensor(Sequence):
 
     @property
     def element_shape(self) -> Tuple[int, ...]:
-        return tuple(self.element_type.shape)
+        t = self._type._leaf
+        return tuple(t._shape) if isinstance(t, TensorStorage) else (1,)
 
     @property
     def element_size(self) -> int:
@@ -177,14 +178,18 @@ class FractalTensor(Sequence):
         """Wrap a dense tensor: its first `depth` dimensions become list levels."""
         if depth < 1 or depth >= t.dim() + 1:
             raise ValueError('depth must be between 1 and the rank of the tensor')
-        t = t.contiguous()
-        elem = TensorStorage(tuple(t.shape[depth:]) or (1,), torch_type_to_internal_type(t.dtype), device=t.device.type)
-        typ = elem
-        for _ in range(depth - 1):
+        shape = tuple(t.shape)
+        return FractalTensor._regular(t.contiguous().view(-1), shape[:depth], shape[depth:] or (1,))
+
+    @staticmethod
+    def _regular(flat: torch.Tensor, dims: Tuple[int, ...], element_shape: Tuple[int, ...]) -> 'FractalTensor':
+        """A regular FractalTensor of these widths over a contiguous one-dimensional buffer."""
+        typ = TensorStorage(element_shape, torch_type_to_internal_type(flat.dtype), device='cuda' if flat.is_cuda else flat.device.type)
+        for _ in range(len(dims) - 1):
             typ = FractalTensorStorage(typ)
         ft = FractalTensor(typ)
-        ft._type.set_regular(t.shape[:depth])
-        ft._T = t.reshape(-1)
+        ft._type.set_regular(dims)
+        ft._T = flat
         return ft
 
     # ---- element access -------------------------------------------------------

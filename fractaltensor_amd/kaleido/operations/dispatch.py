@@ -75,9 +75,15 @@ def reset() -> None:
         stats[k] = 0
 
 
+_core_module = None
+
+
 def _core():
-    from ... import _core
-    return _core
+    global _core_module
+    if _core_module is None:             # an import statement that finds its module takes a microsecond
+        from ... import _core as module
+        _core_module = module
+    return _core_module
 
 
 def _probing() -> bool:
@@ -286,7 +292,7 @@ def _fingerprint(f, level: int = 0, seen=None, looked=None):
     defaults, kw, closure = getattr(f, '__defaults__', None), getattr(f, '__kwdefaults__', None), getattr(f, '__closure__', None)
     for d in (defaults or ()):
         parts.append(of_value(d))
-    for k, d in sorted((kw or {}).items()):
+    for k, d in sorted(kw.items()) if kw else ():
         parts.append((k, of_value(d)))
     cells = [_content(cell) for cell in (closure or ())]
     for v in cells:
@@ -382,8 +388,8 @@ def clear_weight_cache() -> None:
 
 def _packed_sources(sources):
     """The same for a stack whose layers are the items of three zipped FractalTensors [L][4]: Wss, Uss, bss."""
-    srcs = [p.data for p in sources]
-    key = tuple((t.data_ptr(), t._version, t.numel(), t.dtype) for t in srcs)
+    srcs = [p._T for p in sources]
+    key = tuple([(t.data_ptr(), t._version, t.numel(), t.dtype) for t in srcs])
     hit = _weights.get(key)
     if hit is not None:
         stats['weight_cache_hits'] += 1
@@ -439,6 +445,21 @@ def _run_lstm(xs: torch.Tensor, WU: torch.Tensor, bias: torch.Tensor, dilations,
             _fading_stacks.add(key)
             stats['repeated_on_f32_products'] += 1
     return (hsss[-1], csss[-1]) if both else hsss[-1]
+
+
+def _launch_lstm(xs: torch.Tensor, WU: torch.Tensor, bias: torch.Tensor, dilations):
+    """The first half of _run_lstm for fp32 [T, B, H], up to the wait for the launch; None: take _run_lstm."""
+    return _core().stacked_lstm_launch(xs, WU, bias, dilations, 'f32' if _fading_stacks and (WU.data_ptr(), WU._version) in _fading_stacks else None)
+
+
+def _finish_lstm(launched) -> None:
+    """The second half: waits, with what _run_lstm does for a stack that fades."""
+    if _core().stacked_lstm_finish(launched):
+        WU = launched[2][1]
+        if len(_fading_stacks) >= 64:
+            _fading_stacks.clear()
+        _fading_stacks.add((WU.data_ptr(), WU._version))
+        stats['repeated_on_f32_products'] += 1
 
 
 def _run_batch_major(flat: torch.Tensor, lengths, WU, bias, dilations, both: bool = False):
@@ -561,11 +582,12 @@ def _stack_sources(xs, H: int, dtype):
     src = getattr(xs, 'sources', None)
     if not isinstance(xs, Iterative) or src is None or len(src) != 3 or len(xs) == 0:
         return None
-    for p, shape in ((src[0], (H, H)), (src[1], (H, H)), (src[2], (1, H))):
-        if not isinstance(p, FractalTensor) or p.depth != 2 or p.data is None or p.data.dtype != dtype or not _on_device(p.data):
+    widths, square = (len(xs), 4), (H, H)
+    for p, shape in ((src[0], square), (src[1], square), (src[2], (1, H))):
+        if not isinstance(p, FractalTensor):
             return None
-        dims = p._type._dims
-        if dims is None or dims != (len(xs), 4) or p.element_shape != shape:
+        typ, data = p._type, p._T
+        if typ._depth != 2 or typ._dims != widths or data is None or data.dtype != dtype or not _on_device(data) or p.element_shape != shape:
             return None
     return src
 
@@ -576,7 +598,8 @@ def _fold_verdict(func: Callable, xs, layers, H: int, dtype, seq_depth: int):
     indexed = layers is not None and layers[0][0] is not None
     L = len(xs)
     key = ('fold', _fingerprint(func), indexed, L if indexed else 0, H, dtype, seq_depth)
-    if key not in _verdicts:
+    verdict = _verdicts.get(key, _MISSING)
+    if verdict is _MISSING:
         stats['probes'] += 1
         verdict = None
         try:
@@ -593,7 +616,6 @@ def _fold_verdict(func: Callable, xs, layers, H: int, dtype, seq_depth: int):
         if verdict is None:
             stats['declined'] += 1
         _remember(key, verdict)
-    verdict = _verdicts[key]
     if verdict is None:
         return None
     dilations = verdict['dilations'] if verdict['dilations'] is not None else [verdict['dilation']] * L
@@ -602,11 +624,12 @@ def _fold_verdict(func: Callable, xs, layers, H: int, dtype, seq_depth: int):
 
 def _sequence_operand(seq, depths=(1, 2)):
     """(H, dtype) of a GPU FractalTensor of [1, H] rows that the LSTM kernels take, else None."""
-    if not isinstance(seq, FractalTensor) or seq.depth not in depths or seq.data is None or not _on_device(seq.data) or not seq.has_indices:
+    if not isinstance(seq, FractalTensor):
         return None
-    if len(seq.element_shape) != 2 or seq.element_shape[0] != 1:
+    data, shape = seq._T, seq.element_shape
+    if data is None or seq._type._depth not in depths or len(shape) != 2 or shape[0] != 1 or not _on_device(data) or not seq.has_indices:
         return None
-    H, dtype = seq.element_shape[1], seq.data.dtype
+    H, dtype = shape[1], data.dtype
     if H % 32 or dtype not in (torch.float32, torch.float16):
         return None
     return H, dtype
@@ -683,6 +706,17 @@ def try_fold(func: Callable, xs, initializer, kwargs):
     dilations = verdict['dilations']
     dilated = any(d != 1 for d in dilations)
     name = 'dilated_lstm' if dilated else 'stacked_lstm'
+    dims = seq._type._dims
+    if dims is not None and seq._type._depth == 2 and dtype == torch.float32 and verdict['layout'] == 'time':
+        # a regular batch: the result is made into a FractalTensor while the kernel runs
+        WU, bias = packed()
+        T = dims[0]
+        launched = _launch_lstm(seq._T.view(T, dims[1], H), WU, bias, [d if T > d else 1 for d in dilations] if dilated else None)
+        if launched is not None:
+            out = FractalTensor._regular(launched[0][-1].view(-1), dims, (1, H))
+            _finish_lstm(launched)
+            stats[name] += 1
+            return out
 
     from . import fused
     if seq.depth == 1:
@@ -949,21 +983,26 @@ def _try_map_of_sequences(func: Callable, xs):
 # ------------------------------------------------------------------ blockwise attention behind map
 
 def _attention_operands(xs):
-    """zip(qsss, ksss, vsss) -> dense q [B, Hd, nq, rq, D], k, v [B, Hd, nk, rk, D] as views, or None."""
+    """zip(qsss, ksss, vsss) -> the buffers of q, k, v and the shapes [B, Hd, nq, rq, D] of q, [B, Hd, nk, rk, D] of k and v, or
+    None."""
     src = getattr(xs, 'sources', None)
     if not isinstance(xs, Iterative) or src is None or len(src) != 3:
         return None
+    shapes = []
     for t in src:
-        if not isinstance(t, FractalTensor) or t.depth != 3 or t.data is None or not t.data.is_cuda or not t.is_regular():
+        if not isinstance(t, FractalTensor) or t._type._depth != 3 or t._T is None or not t._T.is_cuda:
             return None
-        if len(t.element_shape) != 2:
+        dims, element = t.dense_shape(), t.element_shape
+        if dims is None or len(element) != 2:
             return None
-    q, k, v = (t.as_dense() for t in src)
-    if k.shape != v.shape or q.shape[:2] != k.shape[:2] or q.shape[-1] != k.shape[-1] or q.dtype != k.dtype or q.dtype != v.dtype:
+        shapes.append(dims + element)
+    qs, ks, vs = shapes
+    q, k, v = (t._T for t in src)
+    if ks != vs or qs[:2] != ks[:2] or qs[-1] != ks[-1] or q.dtype != k.dtype or q.dtype != v.dtype:
         return None
-    if q.shape[-1] not in (32, 64, 96, 128):
+    if qs[-1] not in (32, 64, 96, 128):
         return None
-    return q, k, v
+    return q, k, v, qs, ks
 
 
 def _probe_attention(func: Callable, rq: int, rk: int, D: int, gen, dtype=torch.float16) -> Optional[float]:
@@ -1024,32 +1063,33 @@ def try_map(func: Callable, xs, kwargs):
     ops = _attention_operands(xs)
     if ops is None:
         return NotImplemented
-    q, k, v = ops
-    if q.dtype not in (torch.float16, torch.float32):
+    q, k, v, shape, (_, _, nk, rk, _) = ops
+    dtype = q.dtype
+    if dtype not in (torch.float16, torch.float32):
         return NotImplemented
-    B, Hd, nq, rq, D = q.shape
-    nk, rk = k.shape[2], k.shape[3]
-    key = ('map', _fingerprint(func), rq, rk, D, q.dtype)
-    if key not in _verdicts:
+    B, Hd, nq, rq, D = shape
+    key = ('map', _fingerprint(func), rq, rk, D, dtype)
+    verdict = _verdicts.get(key, _MISSING)
+    if verdict is _MISSING:
         stats['probes'] += 1
         try:
-            scale = _probe_attention(func, rq, rk, D, torch.Generator().manual_seed(20240301), q.dtype)
+            scale = _probe_attention(func, rq, rk, D, torch.Generator().manual_seed(20240301), dtype)
         except Exception:
             scale = None
         if scale is None:
             stats['declined'] += 1
-        _remember(key, None if scale is None else {'scale': scale})
-    verdict = _verdicts[key]
+        verdict = None if scale is None else {'scale': scale}
+        _remember(key, verdict)
     if verdict is None:
         return NotImplemented
     core = _core()
-    to4 = lambda t: t.reshape(B, Hd, t.shape[2] * t.shape[3], D)
-    if q.dtype == torch.float32 and not allow_half_attention:       # a program computes in its own precision
-        O = core.flash_attention_f32(to4(q).contiguous(), to4(k).contiguous(), to4(v).contiguous(), verdict['scale'])
+    q, k, v = q.view(B, Hd, nq * rq, D), k.view(B, Hd, nk * rk, D), v.view(B, Hd, nk * rk, D)
+    if dtype == torch.float32 and not allow_half_attention:       # a program computes in its own precision
+        O = core.flash_attention_f32(q.contiguous(), k.contiguous(), v.contiguous(), verdict['scale'])
     else:
-        O = core.flash_attention(to4(q).half().contiguous(), to4(k).half().contiguous(), to4(v).half().contiguous(), verdict['scale'])
+        O = core.flash_attention(q.half().contiguous(), k.half().contiguous(), v.half().contiguous(), verdict['scale']).to(dtype)
     stats['flash_attention'] += 1
-    return FractalTensor.from_dense(O.to(q.dtype).view(B, Hd, nq, rq, D), 3)
+    return FractalTensor._regular(O.view(-1), (B, Hd, nq), (rq, D))
 
 
 # ------------------------------------------------------------------ (a @ b) @ c behind Tensor.__matmul__

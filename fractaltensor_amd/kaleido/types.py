@@ -106,6 +106,8 @@ def str_to_internal_type(dtype: str) -> Number:
 
 def normalize_device(device: Optional[str]) -> str:
     """'cpu' or 'cuda' (the reference knows exactly these two, kaleido/frontend/types.py:195-197)."""
+    if device == 'cuda' or device == 'cpu':
+        return device
     if device is None:
         return 'cpu'
     d = str(device)
@@ -135,14 +137,7 @@ class TensorStorage(Storage):
         self._order = order or 'row'
         if self._order not in ('row', 'col'):
             raise ValueError("order should be 'row' or 'col'.")
-        if strides is not None:
-            self._strides = tuple(strides)
-        else:
-            st = list(row_major_strides(self._shape))
-            if self._order == 'col' and len(st) >= 2:
-                # column-major in the last two dimensions
-                st[-1], st[-2] = self._shape[-2], 1
-            self._strides = tuple(st)
+        self._strides = None if strides is None else tuple(strides)      # None: those of the order, worked out when asked for
 
     @property
     def shape(self) -> List[int]:
@@ -158,6 +153,12 @@ class TensorStorage(Storage):
 
     @property
     def strides(self) -> Tuple[int, ...]:
+        if self._strides is None:
+            st = list(row_major_strides(self._shape))
+            if self._order == 'col' and len(st) >= 2:
+                # column-major in the last two dimensions
+                st[-1], st[-2] = self._shape[-2], 1
+            self._strides = tuple(st)
         return self._strides
 
     @property
@@ -196,7 +197,9 @@ class FractalTensorStorage(Storage):
         self._indices = None
         self._dims = None     # (n1, ..., nk) while the index tree is the regular one of these widths (built when asked for)
         self._length = -1
-        self._depth = dtype._depth + 1 if isinstance(dtype, FractalTensorStorage) else 1
+        nested = isinstance(dtype, FractalTensorStorage)
+        self._depth = dtype._depth + 1 if nested else 1
+        self._leaf = dtype._leaf if nested else dtype
 
     @property
     def dtype(self):
@@ -258,10 +261,7 @@ class FractalTensorStorage(Storage):
             t = t._dtype
 
     def element_type(self):
-        t = self._dtype
-        while isinstance(t, FractalTensorStorage):
-            t = t._dtype
-        return t
+        return self._leaf
 
     def element_shape(self) -> Tuple[int, ...]:
         return tuple(self.element_type().element_shape())
