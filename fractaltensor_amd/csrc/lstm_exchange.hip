@@ -667,6 +667,10 @@ void lstm_exchange_kernel(ExchangeArgs a) {
   // are formed, the pieces of the next item's x are asked for one by one into the registers that have been used (a burst
   // of loads would hold up the wave: 64 bytes a cycle is what a compute unit gets), and while those of x are formed
   // (which is after this item's h has been published) the pieces of the next h.
+  // STORES_FIRST: a team too large for an XCD waits longest for its h, and what is asked for too early costs the whole way once
+  // more: its stores go in front (fp16 H 1024 L 4 T 64 B 16 238 -> 184 us).  With several row blocks h is there, and with a
+  // dilated recurrence sooner than the stores take (L 3 T 88 B 42 H 64 137 us with the stores in front, 121 behind).
+  constexpr bool STORES_FIRST = !MANY && W > 32 * exchange_per_cu(H, HALF, MANY);
   auto walk = [&](auto first_c, auto way_c) __attribute__((always_inline)) {
     constexpr bool FIRST = decltype(first_c)::value;
     constexpr std::integral_constant<int, decltype(way_c)::value == kAnyWay ? kAnyWay : kPlain> own_way{};
@@ -695,7 +699,7 @@ void lstm_exchange_kernel(ExchangeArgs a) {
     take_x(it);
     // nothing yet, but as many stores behind the loads of h as on the way round the loop: the compiler waits for the loads
     // by their number, and on the way round would wait for the stores of the item before with them
-    if constexpr (MANY) store_later(way_c);
+    if constexpr (!STORES_FIRST) store_later(way_c);
     while (true) {   // (a wave that has given up walks on without waiting, to every barrier the others wait at)
       const bool has_prev = it.t >= d;
       const Item next = after(it);
@@ -726,13 +730,11 @@ void lstm_exchange_kernel(ExchangeArgs a) {
       later_of(it, h, c);
       look_for_small(h);
       if (!more) break;
-      // With one row block the next h is what is waited for, and asking for it too early costs more than the stores in front
-      // (fp16 H 1024 L 4 T 64 B 16 238 -> 184 us); with several it is there, and the stores are in its way.
-      if constexpr (!MANY) store_later(way_c);
+      if constexpr (STORES_FIRST) store_later(way_c);
       asm volatile("" ::: "memory");
       take_x(next);
       asm volatile("" ::: "memory");
-      if constexpr (MANY) store_later(way_c);
+      if constexpr (!STORES_FIRST) store_later(way_c);
       asm volatile("" ::: "memory");
       it = next;
     }

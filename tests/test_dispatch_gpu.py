@@ -611,3 +611,19 @@ def test_a_pending_product_is_formed_by_any_other_use():
     c = torch.from_numpy((rng.standard_normal((96, 40)) / 8).astype(np.float16)).cuda()
     d = (Tensor.from_tensor(a) @ Tensor.from_tensor(b)) @ Tensor.from_tensor(c)
     assert dispatch.stats['b2b_gemm'] == 0 and torch.equal(d.data, (a @ b) @ c)
+
+
+def test_fading_stack_is_repeated_on_fp32_products_behind_the_result():
+    """The result object is made while the launch runs; one that meets states too small for split products is computed again
+    into the same buffer before it is handed out, and goes to fp32 products directly the next time."""
+    L, T, B, H = 8, 6, 16, 64
+    Wss, Uss, bss = programs.make_lstm_params(L, H, 1 / 64, seed=5, device='cuda', bias=False)
+    xss = programs.make_sequence_batch(T, B, H, seed=6, device='cuda')
+    core = _core()
+    W, U = Wss.as_dense(), Uss.as_dense()
+    WU = torch.cat([W.permute(0, 2, 1, 3).reshape(L, H, 4 * H), U.permute(0, 2, 1, 3).reshape(L, H, 4 * H)], dim=1).contiguous()
+    exact = core.stacked_lstm(xss.as_dense().view(T, B, H), WU, torch.zeros((L, 4 * H), device='cuda'), products='f32')[0][-1]
+    for _ in range(2):
+        out = programs.stacked_lstm(xss, Wss, Uss, bss)
+        assert torch.equal(out.as_dense().view(T, B, H), exact)
+    assert dispatch.stats['stacked_lstm'] == 2 and dispatch.stats['repeated_on_f32_products'] == 1
