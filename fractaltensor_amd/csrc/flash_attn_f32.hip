@@ -45,14 +45,11 @@ __device__ __forceinline__ void split_scale(unsigned max_bits, float* scale, flo
   *inv = __uint_as_float((unsigned)(eb - kF32Top) << 23);
 }
 
-__global__ void attn_f32_clear_kernel(unsigned* p, int n) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) p[i] = 0;
-}
-
-// largest |x| of every (batch, head) of K and V, as float bits (which order like the magnitudes): grid
-// (chunks, BH, 2), per_bh a multiple of 4
-__global__ __launch_bounds__(256) void attn_f32_absmax_kernel(const float* K, const float* V, unsigned* bits, size_t per_bh, int BH) {
+// The two launches of larger heads: largest |x| of every chunk of every (batch, head) of K and V, as float bits (which order like
+// the magnitudes), grid (chunks, BH, 2), per_bh a multiple of 4; then the planes, whose workgroups take the largest of a head's chunks.
+// (With one word a head, cleared by a launch and raised by atomics, the three took 24 us at 16 heads of 1280 keys of 128.)
+constexpr int kMaxChunks = 64;
+__global__ __launch_bounds__(256) void attn_f32_absmax_kernel(const float* K, const float* V, unsigned* chunk_bits, size_t per_bh, int BH) {
   __shared__ unsigned wave_max[4];
   const float* x = (blockIdx.z ? V : K) + (size_t)blockIdx.y * per_bh;
   unsigned m = 0;
@@ -65,11 +62,8 @@ __global__ __launch_bounds__(256) void attn_f32_absmax_kernel(const float* K, co
   for (int o = 32; o > 0; o >>= 1) m = max(m, (unsigned)__shfl_xor((int)m, o));
   if ((threadIdx.x & 63) == 0) wave_max[threadIdx.x >> 6] = m;
   __syncthreads();
-  // one atomic per workgroup: thousands of them on one word take longer than the reading
-  if (threadIdx.x == 0) {
-    m = max(max(wave_max[0], wave_max[1]), max(wave_max[2], wave_max[3]));
-    if (m) atomicMax(bits + blockIdx.z * BH + blockIdx.y, m);
-  }
+  if (threadIdx.x == 0)
+    chunk_bits[((size_t)blockIdx.z * BH + blockIdx.y) * gridDim.x + blockIdx.x] = max(max(wave_max[0], wave_max[1]), max(wave_max[2], wave_max[3]));
 }
 
 // Eight neighbouring floats of a row into its planes [top D | rest D].
@@ -92,15 +86,27 @@ __device__ __forceinline__ void split_eight(const float* X, _Float16* planes, lo
   *reinterpret_cast<v8h*>(dst + D) = rest;
 }
 
-// Planes of K (blockIdx.y 0) and V (1) under each (batch, head)'s scale, eight floats to a thread.
+// Planes under each head's scale, grid (workgroups of a head, BH, 2: K, V), eight floats to a thread; clears the counters.
 template <int D>
-__global__ __launch_bounds__(256) void attn_f32_split_kernel(const float* K, const float* V, _Float16* kplanes, _Float16* vplanes,
-                                                            const unsigned* group_bits, int rows_per_bh, long long rows, int BH) {
-  const long long chunk = (long long)blockIdx.x * 256 + threadIdx.x, row = chunk / (D / 8);
-  if (row >= rows) return;
+__global__ __launch_bounds__(256) void attn_f32_split_kernel(const float* K, const float* V, _Float16* kplanes, _Float16* vplanes, unsigned* bits,
+                                                            const unsigned* chunk_bits, int chunks, int Skv, int BH, int counters) {
+  const bool is_v = blockIdx.z != 0;
+  const int group = is_v * BH + blockIdx.y, lane = threadIdx.x & 63;
+  unsigned m = lane < chunks ? chunk_bits[(size_t)group * chunks + lane] : 0;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) m = max(m, (unsigned)__shfl_xor((int)m, o));
+  if (blockIdx.x == 0) {
+    if (threadIdx.x == 0) bits[group] = m;
+    if (group == 0)
+      for (int i = threadIdx.x; i < counters; i += 256) bits[2 * BH + i] = 0;
+  }
   float scale, inv;
-  split_scale(group_bits[blockIdx.y * BH + row / rows_per_bh], &scale, &inv);
-  split_eight<D>(blockIdx.y ? V : K, blockIdx.y ? vplanes : kplanes, chunk, scale);
+  split_scale(m, &scale, &inv);
+  const size_t head = (size_t)blockIdx.y * Skv * D;
+  const float* const X = (is_v ? V : K) + head;
+  _Float16* const planes = (is_v ? vplanes : kplanes) + 2 * head;
+  const int all = Skv * (D / 8);
+  for (int i = blockIdx.x * 256 + threadIdx.x; i < all; i += gridDim.x * 256) split_eight<D>(X, planes, i, scale);
 }
 
 // Largest magnitude and planes in one launch, for heads that a compute unit reads in a microsecond or two: each of a
@@ -110,8 +116,10 @@ __global__ __launch_bounds__(256) void attn_f32_split_kernel(const float* K, con
 constexpr int kPlanesThreads = 512;
 template <int D>
 __global__ __launch_bounds__(kPlanesThreads) void attn_f32_planes_kernel(const float* K, const float* V, _Float16* kplanes, _Float16* vplanes,
-                                                                         unsigned* bits, int Skv, int BH, int parts) {
+                                                                         unsigned* bits, int Skv, int BH, int parts, int counters) {
   __shared__ unsigned wave_max[kPlanesThreads / 64];
+  if (blockIdx.x == 0)   // the counters behind the magnitudes
+    for (int i = threadIdx.x; i < counters; i += kPlanesThreads) bits[2 * BH + i] = 0;
   const int id = xcd_consecutive(blockIdx.x, gridDim.x);
   const int group = id / parts, part = id - group * parts;   // group: (batch, head) of K, then of V
   const bool is_v = group >= BH;
@@ -138,6 +146,9 @@ __global__ __launch_bounds__(kPlanesThreads) void attn_f32_planes_kernel(const f
   for (int i = part * kPlanesThreads + threadIdx.x; i < chunks; i += parts * kPlanesThreads) split_eight<D>(X, planes, i, scale);
 }
 
+// Bytes a part of a block of 128 query rows leaves in the workspace.
+constexpr int f32_partial_bytes(int D) { return 128 * D * 4 + 4 * 64 * 8; }
+
 // 4 waves x 32 query rows per workgroup.  Two workgroups to a compute unit at head sizes up to 64 (B 4, 16 heads, 1024 keys of 64: 88
 // -> 77 us with a bound of 256 registers, of which the compiler had taken a few more), one above: the accumulators of O,
 // both planes of Q and the scores take some 400 registers at D = 128.  K and V tiles of 64 keys, both double buffered.  A wave
@@ -146,39 +157,59 @@ __global__ __launch_bounds__(kPlanesThreads) void attn_f32_planes_kernel(const f
 // under the score MFMAs of the half after (the comments in the kernel give the order).
 // KG == 2 (head sizes up to 64, whose registers allow two waves per SIMD): two groups of four waves share the query rows,
 // each walks half of the keys with tiles of its own in LDS, and the first takes in the second's result at the end.
-template <int D, int KG>
-__global__ __launch_bounds__(KG * 256, KG == 1 && D <= 64 ? 2 : 1) void flash_attn_f32_kernel(const float* __restrict__ Q, const _Float16* __restrict__ Kp,
+// PART: nparts workgroups share a block of query rows, each with its share of the tiles.  Each leaves its unnormalised
+// accumulators, reference and sum in the workspace (write-through: a block's workgroups may sit on several XCDs), and the one
+// that finds itself the last by the block's counter takes all of them in, in the order of their keys, so that the result does
+// not depend on who was last, and stores the block.
+// LDS layout of the tiles of four key groups at head size 32 (padded, they take 172 KB): V rows without padding, the planes of
+// every second pair of rows exchanged, so that four rows of a plane fall on different banks.
+struct FaFourGroups : FaLayout<64> {
+  static constexpr int VRS = 128, VTB = FA_KT * VRS;
+};
+template <int D, int KG> using F32Tiles = typename std::conditional<KG == 4, FaFourGroups, FaLayout<2 * D>>::type;
+
+template <int D, int KG, int WAVES, bool PART>
+__global__ __launch_bounds__(KG * WAVES * 64, KG == 1 && D <= 64 ? 2 : 1) void flash_attn_f32_kernel(const float* __restrict__ Q, const _Float16* __restrict__ Kp,
                                                                 const _Float16* __restrict__ Vp, float q_mul,
                                                                 const unsigned* __restrict__ kv_bits, float* __restrict__ O,
-                                                                int Sq, int Skv_all, int nqb, int BH) {
-  using L = FaLayout<2 * D>;          // a plane row is an fp16 row of 2 D elements
+                                                                int Sq, int Skv_whole, int nqb, int BH, int nparts,
+                                                                int* __restrict__ counters, unsigned char* __restrict__ partials) {
+  using L = F32Tiles<D, KG>;          // a plane row is an fp16 row of 2 D elements
+  constexpr bool SWZ = KG == 4;
+  static_assert(!SWZ || D == 32, "four key groups at head size 32");
   constexpr int DS = D / 16;          // k steps of S^T
   constexpr int DT = D / 32;          // d tiles of O^T
   constexpr int RB = 4 * D;           // bytes per plane row in global memory
   constexpr int KRS = L::KRS, VRS = L::VRS, KTB = L::KTB, VTB = L::VTB;
-  constexpr int WAVES = 4;
   constexpr int KCP = (KTB / 1024 + WAVES - 1) / WAVES, VCP = (VTB / 1024 + WAVES - 1) / WAVES;
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane((tid >> 6) & 3);   // within its key group
-  const int group = KG == 1 ? 0 : __builtin_amdgcn_readfirstlane(tid >> 8);
+  const int wave = __builtin_amdgcn_readfirstlane((tid >> 6) % WAVES);   // within its key group
+  const int group = KG == 1 ? 0 : __builtin_amdgcn_readfirstlane((tid >> 6) / WAVES);
   constexpr int GROUP_LDS = 2 * (KTB + VTB);
   unsigned char* const Kb = smem + group * GROUP_LDS;   // [2][KTB]
   unsigned char* const Vb = Kb + 2 * KTB;               // [2][VTB]
   const int j = lane & 31;
   const int hh = lane >> 5;
   const int id = xcd_consecutive(blockIdx.x, gridDim.x);   // a head's query blocks share an XCD
-  const int bh = id / nqb;
-  const int qb = id - bh * nqb;
+  const int block = PART ? id / nparts : id, part = PART ? id - block * nparts : 0;
+  const int bh = block / nqb;
+  const int qb = block - bh * nqb;
   const int q_base = qb * (WAVES * 32) + wave * 32;
 
-  // the first group has the first half of the tiles, one more than the second when they are odd (never fewer than two in all)
-  const int first_tiles = ((Skv_all + FA_KT - 1) / FA_KT + 1) / 2;
-  const int key_first = group * first_tiles * FA_KT;
-  const int Skv = KG == 1 ? Skv_all : group == 0 ? first_tiles * FA_KT : Skv_all - key_first;   // the keys this group sees
-  const _Float16* Kg = Kp + ((size_t)bh * Skv_all + key_first) * (2 * D);
-  const _Float16* Vg = Vp + ((size_t)bh * Skv_all + key_first) * (2 * D);
+  // the workgroup's tiles of keys: the first `long_parts` parts have one more than the others
+  const int all_tiles = (Skv_whole + FA_KT - 1) / FA_KT, each = PART ? all_tiles / nparts : all_tiles, long_parts = PART ? all_tiles - each * nparts : 0;
+  const int tile_first = part * each + min(part, long_parts);
+  const int key_part = tile_first * FA_KT;
+  const int Skv_all = PART && part + 1 < nparts ? (each + (part < long_parts ? 1 : 0)) * FA_KT : Skv_whole - key_part;   // its keys
+  // the groups have neighbouring shares of the tiles, the first ones one more where they do not divide (never fewer than one each)
+  const int part_tiles = (Skv_all + FA_KT - 1) / FA_KT, share = part_tiles / KG, long_groups = part_tiles - share * KG;
+  const int most_tiles = share + (long_groups > 0 ? 1 : 0);
+  const int key_first = (group * share + min(group, long_groups)) * FA_KT;
+  const int Skv = KG == 1 ? Skv_all : group + 1 < KG ? (share + (group < long_groups ? 1 : 0)) * FA_KT : Skv_all - key_first;   // the keys this group sees
+  const _Float16* Kg = Kp + ((size_t)bh * Skv_whole + key_part + key_first) * (2 * D);
+  const _Float16* Vg = Vp + ((size_t)bh * Skv_whole + key_part + key_first) * (2 * D);
   float* Og = O + (size_t)bh * Sq * D;
 
   // The lane's query row: the fp32 row is read, multiplied by q_mul (scale * log2 e: a score leaves the matrix unit in
@@ -244,7 +275,8 @@ __global__ __launch_bounds__(KG * 256, KG == 1 && D <= 64 ? 2 : 1) void flash_at
   for (int i = 0; i < VCP; ++i) {
     const int x = 1024 * (wave + WAVES * i) + 16 * lane;
     const int row = min(x / VRS, FA_KT - 1), col = x % VRS;
-    v_src[i] = row * RB + (col < RB ? col : 0);
+    if constexpr (SWZ) v_src[i] = row * RB + (col ^ (64 * ((row >> 1) & 1)));
+    else v_src[i] = row * RB + (col < RB ? col : 0);
   }
   // (a whole tile takes the copies' offsets as they are; the last tile of a ragged row of keys clamps each)
   auto copy_rows = [&](auto n_c, auto bytes_c, const unsigned (&src)[decltype(n_c)::value], const _Float16* rows, int key0,
@@ -280,11 +312,14 @@ __global__ __launch_bounds__(KG * 256, KG == 1 && D <= 64 ? 2 : 1) void flash_at
 
   const int k_lane = j * KRS + 16 * hh;
   const int v_lane = (4 * hh + ((lane & 15) >> 2)) * VRS + 32 * ((lane >> 4) & 1) + 8 * (lane & 3);
+  [[maybe_unused]] const int v_first = SWZ ? 64 * (((lane & 15) >> 3) & 1) : 0;   // where the rows this lane names (4 hh + its quarter) have their values
   using lds_v4s = __attribute__((address_space(3))) v4s;
   typedef short v8s __attribute__((ext_vector_type(8)));
   // A-operand of the P V product: step s (16 keys) and d tile dt of one half tile; plane 0 = values, 1 = remainders
   auto read_v = [&](const unsigned char* vbase, int s, int dt, int plane) __attribute__((always_inline)) {
-    const unsigned char* p0 = vbase + 16 * s * VRS + 64 * dt + plane * (2 * D);
+    const unsigned char* p0 = vbase + 16 * s * VRS + 64 * dt;
+    if constexpr (SWZ) p0 += plane ? 64 - v_first : v_first;
+    else p0 += plane * (2 * D);
     const v4s lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s*)(p0));
     const v4s hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s*)(p0 + 8 * VRS));
     const v8s both = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
@@ -537,40 +572,103 @@ __global__ __launch_bounds__(KG * 256, KG == 1 && D <= 64 ? 2 : 1) void flash_at
     const v16f none = zero16;
     pv_and_maxima(std::false_type{}, std::false_type{}, std::false_type{}, pend_v, nullptr, none, 0);
   }
-  if (KG == 2 && group == 1 && ntiles < first_tiles) {   // the first group's last tile
+  if (KG > 1 && ntiles < most_tiles) {   // the last tile of the groups that have one more
     __syncthreads();
     __syncthreads();
   }
   __syncthreads();   // LDS is reused below
   float l = l_run + __shfl_xor(l_run, 32);
-  if constexpr (KG == 2) {
-    // the second group leaves its accumulators, reference and sum in its part of LDS, by lane; the first takes them in by
+  if constexpr (KG > 1) {
+    // the other groups leave their accumulators, references and sums in their part of LDS, by lane; the first takes them in by
     // the rule of an online softmax
-    unsigned char* const other = smem + GROUP_LDS;
-    v4f* const oo = reinterpret_cast<v4f*>(other) + wave * (DT * 4 * 64) + lane;
-    float2* const oml = reinterpret_cast<float2*>(other + WAVES * (DT * 4 * 64 * 16)) + wave * 64 + lane;
-    static_assert(WAVES * (DT * 4 * 64 * 16 + 64 * 8) <= GROUP_LDS, "the second group's result fits its tiles' place");
-    if (group == 1) {
+    auto oo = [&](int g) __attribute__((always_inline)) { return reinterpret_cast<v4f*>(smem + g * GROUP_LDS) + wave * (DT * 4 * 64) + lane; };
+    auto oml = [&](int g) __attribute__((always_inline)) {
+      return reinterpret_cast<float2*>(smem + g * GROUP_LDS + WAVES * (DT * 4 * 64 * 16)) + wave * 64 + lane;
+    };
+    static_assert(WAVES * (DT * 4 * 64 * 16 + 64 * 8) <= GROUP_LDS, "a group's result fits its tiles' place");
+    if (group > 0) {
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-        for (int g = 0; g < 4; ++g) oo[(4 * dt + g) * 64] = v4f{om[dt][4 * g], om[dt][4 * g + 1], om[dt][4 * g + 2], om[dt][4 * g + 3]};
-      *oml = make_float2(m_ref, l);
+        for (int g = 0; g < 4; ++g) oo(group)[(4 * dt + g) * 64] = v4f{om[dt][4 * g], om[dt][4 * g + 1], om[dt][4 * g + 2], om[dt][4 * g + 3]};
+      *oml(group) = make_float2(m_ref, l);
     }
     __syncthreads();
-    if (group == 1) return;
-    const float2 ml = *oml;
-    const float m = fmaxf(m_ref, ml.x);
-    const float wm = __builtin_amdgcn_exp2f(m_ref - m), wo = __builtin_amdgcn_exp2f(ml.x - m);
-    l = wm * l + wo * ml.y;
+    if (!PART && group > 0) return;
+    if (group == 0) {
 #pragma unroll
-    for (int dt = 0; dt < DT; ++dt)
+      for (int other = 1; other < KG; ++other) {
+        const float2 ml = *oml(other);
+        const float m = fmaxf(m_ref, ml.x);
+        const float wm = __builtin_amdgcn_exp2f(m_ref - m), wo = __builtin_amdgcn_exp2f(ml.x - m);
+        l = wm * l + wo * ml.y;
+        m_ref = m;
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const v4f o = oo[(4 * dt + g) * 64];
+        for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-        for (int k = 0; k < 4; ++k) om[dt][4 * g + k] = wm * om[dt][4 * g + k] + wo * o[k];
+          for (int g = 0; g < 4; ++g) {
+            const v4f o = oo(other)[(4 * dt + g) * 64];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) om[dt][4 * g + k] = wm * om[dt][4 * g + k] + wo * o[k];
+          }
       }
+    }
+  }
+  if constexpr (PART) {
+    static_assert(WAVES == 4, "a partial result is that of 128 query rows");
+    __shared__ int arrived;
+    constexpr int PB = f32_partial_bytes(D), ML = PB - WAVES * 64 * 8;   // a part's accumulators, then its references and sums
+    const auto mine = __builtin_amdgcn_make_buffer_rsrc(partials + (size_t)block * nparts * PB, 0, (unsigned)(nparts * PB), 0x00020000);
+    constexpr int kAgent = 16;   // sc1
+    const unsigned o_at = (unsigned)(wave * (DT * 4 * 64) + lane) * 16, ml_at = (unsigned)(ML + (wave * 64 + lane) * 8);
+    if (group == 0) {
+#pragma unroll
+      for (int i = 0; i < 4 * DT; ++i) {
+        const v4f o = {om[i / 4][4 * (i % 4)], om[i / 4][4 * (i % 4) + 1], om[i / 4][4 * (i % 4) + 2], om[i / 4][4 * (i % 4) + 3]};
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4u, o), mine, o_at, part * PB + i * 1024, kAgent);
+      }
+      __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(v2u, make_float2(m_ref, l)), mine, ml_at, part * PB, kAgent);
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    }
+    __syncthreads();
+    if (tid == 0) arrived = __hip_atomic_fetch_add(counters + block, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    if (arrived != nparts - 1 || group > 0) return;
+    auto sum_of = [&](int p) __attribute__((always_inline)) {
+      return __builtin_bit_cast(v2f, __builtin_amdgcn_raw_buffer_load_b64(mine, ml_at, p * PB, kAgent));
+    };
+    auto piece = [&](int p, int i) __attribute__((always_inline)) {
+      return __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(mine, o_at, p * PB + i * 1024, kAgent));
+    };
+    // several parts' loads on their way at once: one after the other they take a microsecond each
+    constexpr int AT_ONCE = D == 32 ? 8 : D == 64 ? 4 : 2;
+    for (int p0 = 0; p0 < nparts; p0 += AT_ONCE) {
+      v2f ml[AT_ONCE];
+      v4f o[AT_ONCE][4 * DT];
+#pragma unroll
+      for (int a = 0; a < AT_ONCE; ++a) {
+        const int p = min(p0 + a, nparts - 1);
+        ml[a] = sum_of(p);
+#pragma unroll
+        for (int i = 0; i < 4 * DT; ++i) o[a][i] = piece(p, i);
+      }
+#pragma unroll
+      for (int a = 0; a < AT_ONCE; ++a) {
+        if (p0 + a >= nparts) break;
+        const bool first = p0 + a == 0;   // (the state so far is this part's own, and in the sum already)
+        const float m = first ? ml[a][0] : fmaxf(m_ref, ml[a][0]);
+        const float wm = first ? 0.0f : __builtin_amdgcn_exp2f(m_ref - m), wo = first ? 1.0f : __builtin_amdgcn_exp2f(ml[a][0] - m);
+        l = first ? ml[a][1] : wm * l + wo * ml[a][1];
+        m_ref = m;
+#pragma unroll
+        for (int i = 0; i < 4 * DT; ++i)
+#pragma unroll
+          for (int k = 0; k < 4; ++k) {
+            const float so_far = om[i / 4][4 * (i % 4) + k];
+            om[i / 4][4 * (i % 4) + k] = first ? o[a][i][k] : wm * so_far + wo * o[a][i][k];
+          }
+      }
+    }
   }
 
   // ---- normalise and store: the wave turns its 32 x D tile round through the LDS nobody reads any more (the
@@ -601,41 +699,83 @@ __global__ __launch_bounds__(KG * 256, KG == 1 && D <= 64 ? 2 : 1) void flash_at
 
 static size_t round256f(size_t v) { return (v + 255) / 256 * 256; }
 
-struct F32Layout {
-  size_t bits, kp, vp, total;
+// How the work is laid out: waves (of 32 query rows) and key groups of a workgroup, and workgroups that share a block's keys.
+struct F32Split {
+  int waves, groups, parts;
 };
-static F32Layout f32_layout(long long bh, int Skv, int D) {
+static F32Split f32_split(long long BH, int Sq, int Skv, int D, int cus) {
+  const int tiles = (Skv + FA_KT - 1) / FA_KT;
+  F32Split best = {4, 1, 1};
+  if ((long long)((Sq + 127) / 128) * BH > 2 * cus) return best;
+  // Time in tenths of what a wave that shares its SIMD needs for a tile (1.05, 2, 2.5, 3 us by head size).  Two waves of a SIMD hardly
+  // overlap, so what counts is the tiles that a SIMD works through; one that has only one wave takes a fifth longer.  What
+  // parts leave in the workspace and the last one takes in costs 4.5 us at head size 32 and 8 at 128.
+  const int merge = D == 32 ? 45 : 35;
+  auto workgroups = [&](const F32Split& f) { return (long long)((Sq + 32 * f.waves - 1) / (32 * f.waves)) * BH * f.parts; };
+  auto cost = [&](const F32Split& f) {
+    const long long per_simd = std::max(1LL, (workgroups(f) + cus - 1) / cus * f.groups * f.waves / 4);
+    const int chain = (tiles + f.groups * f.parts - 1) / (f.groups * f.parts);
+    return chain * (D > 64 ? 12 * per_simd : per_simd == 1 ? 12 : 10 * per_simd) + (f.parts > 1 ? merge : 0) + (f.groups > 1 ? 2 * f.groups : 0);
+  };
+  long long least = cost(best);
+  auto consider = [&](const F32Split& f) {
+    const int resident = D <= 64 && f.groups == 1 ? 2 : 1;   // workgroups of a compute unit, by registers and LDS
+    if (tiles < f.groups * f.parts || workgroups(f) > (long long)resident * cus || cost(f) >= least) return;
+    least = cost(f);
+    best = f;
+  };
+  if (D <= 64) {
+    consider({4, 2, 1});
+    consider({2, 2, 1});
+  }
+  if (D == 32) consider({2, 4, 1});
+  for (int parts = 2; parts <= 16; ++parts) {
+    consider({4, 1, parts});
+    if (D <= 64) consider({4, 2, parts});
+  }
+  return best;
+}
+
+struct F32Layout {
+  size_t bits, chunks, kp, vp, partials, total;
+  bool chunked;   // room for the largest magnitudes of chunks of a head
+};
+static F32Layout f32_layout(long long bh, int nqb, int parts, bool chunked, int Skv, int D) {
   F32Layout w;
-  w.bits = 0;
-  w.kp = round256f((size_t)2 * bh * sizeof(unsigned));
+  w.chunked = chunked;
+  const size_t counters = parts > 1 ? (size_t)bh * nqb : 0;
+  w.bits = 0;   // and the counters
+  w.chunks = round256f(((size_t)2 * bh + counters) * sizeof(unsigned));
+  w.kp = w.chunks + (chunked ? round256f((size_t)2 * bh * kMaxChunks * sizeof(unsigned)) : 0);
   w.vp = w.kp + round256f((size_t)bh * Skv * 2 * D * sizeof(_Float16));
-  w.total = w.vp + round256f((size_t)bh * Skv * 2 * D * sizeof(_Float16));
+  w.partials = w.vp + round256f((size_t)bh * Skv * 2 * D * sizeof(_Float16));
+  w.total = w.partials + (parts > 1 ? round256f((size_t)bh * nqb * parts * f32_partial_bytes(D)) : 0);
   return w;
 }
 
-template <int D, int KG>
-static int launch_fa_f32_blocks(const float* Q, const _Float16* kp, const _Float16* vp, const unsigned* bits, float* O, int BH, int Sq, int Skv,
-                                float scale, int lds_max, hipStream_t s) {
-  using L = FaLayout<2 * D>;
-  const size_t lds = std::max((size_t)KG * 2 * (L::KTB + L::VTB), (size_t)4 * 32 * (4 * D + 16));
+template <int D, int KG, int WAVES, bool PART>
+static int launch_fa_f32_blocks(const float* Q, const _Float16* kp, const _Float16* vp, unsigned* bits, float* O, int BH, int Sq, int Skv,
+                                float scale, int parts, char* partials, int lds_max, hipStream_t s) {
+  using L = F32Tiles<D, KG>;
+  const size_t lds = std::max((size_t)KG * 2 * (L::KTB + L::VTB), (size_t)WAVES * 32 * (4 * D + 16));
   if ((int)lds > lds_max) return fail(FTK_ERR_DEVICE, "ftk_flash_attn_f32: D=%d needs %zu bytes of LDS, the device offers %d", D, lds, lds_max);
-  const int nqb = (Sq + 127) / 128;
-  const long long blocks = (long long)nqb * BH;
+  const int nqb = (Sq + 32 * WAVES - 1) / (32 * WAVES);
+  const long long blocks = (long long)nqb * BH * parts;
   if (blocks > 0x7fffffffLL) return fail(FTK_ERR_UNSUPPORTED_SHAPE, "ftk_flash_attn_f32: grid too large");
   static DeviceOnce attr_once;
   unsigned attr_bit;
   if (attr_once.pending(&attr_bit)) {
-    FTK_HIP(hipFuncSetAttribute((const void*)flash_attn_f32_kernel<D, KG>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    FTK_HIP(hipFuncSetAttribute((const void*)flash_attn_f32_kernel<D, KG, WAVES, PART>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     attr_once.done(attr_bit);
   }
-  hipLaunchKernelGGL((flash_attn_f32_kernel<D, KG>), dim3((unsigned)blocks), dim3(KG * 256), lds, s, Q, kp, vp, scale * 1.4426950408889634f, bits, O, Sq,
-                     Skv, nqb, BH);
+  hipLaunchKernelGGL((flash_attn_f32_kernel<D, KG, WAVES, PART>), dim3((unsigned)blocks), dim3(KG * WAVES * 64), lds, s, Q, kp, vp, scale * 1.4426950408889634f,
+                     (const unsigned*)bits, O, Sq, Skv, nqb, BH, parts, reinterpret_cast<int*>(bits + 2 * BH), reinterpret_cast<unsigned char*>(partials));
   return check_launch("flash_attn_f32_kernel");
 }
 
 template <int D>
 static int launch_fa_f32(const float* Q, const float* K, const float* V, float* O, int BH, int Sq, int Skv, float scale, char* ws,
-                         const F32Layout& w, const DeviceProps& dp, hipStream_t s) {
+                         const F32Layout& w, const F32Split& split, const DeviceProps& dp, hipStream_t s) {
   unsigned* bits = reinterpret_cast<unsigned*>(ws + w.bits);
   _Float16* kp = reinterpret_cast<_Float16*>(ws + w.kp);
   _Float16* vp = reinterpret_cast<_Float16*>(ws + w.vp);
@@ -645,39 +785,51 @@ static int launch_fa_f32(const float* Q, const float* K, const float* V, float* 
   // than three launches).
   const size_t all_heads = 2 * (size_t)BH * head_bytes, most_read = (size_t)96 << 20;
   const int parts = (int)std::max<size_t>(1, std::min({512 / (2 * (size_t)BH), per_bh / (8 * kPlanesThreads), most_read / all_heads}));
+  const int counters = split.parts > 1 ? BH * ((Sq + 127) / 128) : 0;
   int rc;
-  if (head_bytes <= 512 * 1024 && all_heads * parts <= most_read) {
-    hipLaunchKernelGGL(attn_f32_planes_kernel<D>, dim3((unsigned)(2 * BH * parts)), dim3(kPlanesThreads), 0, s, K, V, kp, vp, bits, Skv, BH, parts);
+  if ((head_bytes <= 512 * 1024 && all_heads * parts <= most_read) || !w.chunked) {
+    hipLaunchKernelGGL(attn_f32_planes_kernel<D>, dim3((unsigned)(2 * BH * parts)), dim3(kPlanesThreads), 0, s, K, V, kp, vp, bits, Skv, BH, parts,
+                       counters);
     rc = check_launch("attn_f32_planes_kernel");
     if (rc) return rc;
   } else {
-    hipLaunchKernelGGL(attn_f32_clear_kernel, dim3((2 * BH + 255) / 256), dim3(256), 0, s, bits, 2 * BH);
-    rc = check_launch("attn_f32_clear_kernel");
-    if (rc) return rc;
-    const int chunks = (int)std::min<size_t>(std::max(1, 4096 / (2 * BH)), (per_bh + 4095) / 4096);   // some 4096 workgroups in all
-    hipLaunchKernelGGL(attn_f32_absmax_kernel, dim3(chunks, BH, 2), dim3(256), 0, s, K, V, bits, per_bh, BH);
+    const int chunks = (int)std::min<size_t>({(size_t)std::max(1, 2048 / (2 * BH)), (per_bh + 4095) / 4096, kMaxChunks});
+    unsigned* const chunk_bits = reinterpret_cast<unsigned*>(ws + w.chunks);
+    hipLaunchKernelGGL(attn_f32_absmax_kernel, dim3(chunks, BH, 2), dim3(256), 0, s, K, V, chunk_bits, per_bh, BH);
     rc = check_launch("attn_f32_absmax_kernel");
     if (rc) return rc;
-    const long long krows = (long long)BH * Skv;
-    hipLaunchKernelGGL(attn_f32_split_kernel<D>, dim3((unsigned)((krows * (D / 8) + 255) / 256), 2), dim3(256), 0, s, K, V, kp, vp, (const unsigned*)bits,
-                       Skv, krows, BH);
+    const int wgs = (int)std::min<size_t>(std::max(1, 4096 / (2 * BH)), (per_bh / 8 + 255) / 256);
+    hipLaunchKernelGGL(attn_f32_split_kernel<D>, dim3(wgs, BH, 2), dim3(256), 0, s, K, V, kp, vp, bits, (const unsigned*)chunk_bits, chunks, Skv, BH,
+                       counters);
     rc = check_launch("attn_f32_split_kernel");
     if (rc) return rc;
   }
-  // Two key groups while there is at most one block of query rows to a compute unit and more than two tiles of keys (us, the
-  // whole call without and with: B2 H8 S1024 D32 37.4, 25.9; B2 H12 S512 D64 32, 24; B1 H8 S2048 D64 80, 57; B1 H16 S2048 D32 67, 50).
-  if constexpr (D <= 64) {
-    if ((long long)((Sq + 127) / 128) * BH <= dp.cus && Skv > 2 * FA_KT)
-      return launch_fa_f32_blocks<D, 2>(Q, kp, vp, bits, O, BH, Sq, Skv, scale, dp.lds_optin, s);
+  char* const partials = ws + w.partials;
+  auto run = [&](auto groups_c, auto waves_c, auto part_c) {
+    return launch_fa_f32_blocks<D, decltype(groups_c)::value, decltype(waves_c)::value, decltype(part_c)::value>(
+        Q, kp, vp, bits, O, BH, Sq, Skv, scale, split.parts, partials, dp.lds_optin, s);
+  };
+  std::integral_constant<int, 1> one;
+  std::integral_constant<int, 2> two;
+  std::integral_constant<int, 4> four;
+  if constexpr (D == 32) {
+    if (split.groups == 4) return run(four, two, std::false_type{});
   }
-  return launch_fa_f32_blocks<D, 1>(Q, kp, vp, bits, O, BH, Sq, Skv, scale, dp.lds_optin, s);
+  if constexpr (D <= 64) {
+    if (split.groups == 2 && split.waves == 2) return run(two, two, std::false_type{});
+    if (split.groups == 2) return split.parts > 1 ? run(two, four, std::true_type{}) : run(two, four, std::false_type{});
+  }
+  return split.parts > 1 ? run(one, four, std::true_type{}) : run(one, four, std::false_type{});
 }
 
 }  // namespace ftk
 
 extern "C" size_t ftk_flash_attn_f32_workspace_bytes(int B, int Hd, int Sq, int Skv, int D) {
   if (B <= 0 || Hd <= 0 || Sq <= 0 || Skv <= 0 || D <= 0) return 0;
-  return ftk::f32_layout((long long)B * Hd, Skv, D).total;
+  const ftk::DeviceProps* dp = nullptr;   // (without a device no call follows)
+  const long long bh = (long long)B * Hd, nqb = (Sq + 127) / 128;
+  const int parts = ftk::device_props(&dp) == FTK_OK ? ftk::f32_split(bh, Sq, Skv, D, dp->cus).parts : 1;
+  return ftk::f32_layout(bh, (int)nqb, parts, true, Skv, D).total;
 }
 
 extern "C" int ftk_flash_attn_f32(const float* Q, const float* K, const float* V, float* O, int B, int Hd, int Sq, int Skv, int D,
@@ -693,19 +845,26 @@ extern "C" int ftk_flash_attn_f32(const float* Q, const float* K, const float* V
   const long long bh = (long long)B * Hd;
   if (bh > (1LL << 16)) return fail(FTK_ERR_UNSUPPORTED_SHAPE, "%s: B*Hd=%lld too large", who, bh);
   if ((long long)Skv * D >= (1LL << 31) || (long long)Sq * D >= (1LL << 31)) return fail(FTK_ERR_UNSUPPORTED_SHAPE, "%s: a head is too large", who);
-  const F32Layout w = f32_layout(bh, Skv, D);
+  const int nqb = (Sq + 127) / 128;
+  F32Layout w = f32_layout(bh, nqb, 1, false, Skv, D);
   if (!workspace || workspace_bytes < w.total)
     return fail(FTK_ERR_WORKSPACE, "%s: workspace of %zu bytes needed, %zu given", who, w.total, workspace ? workspace_bytes : (size_t)0);
   if (reinterpret_cast<uintptr_t>(workspace) % 256) return fail(FTK_ERR_INVALID_ARGUMENT, "%s: workspace must be 256-byte aligned", who);
   const DeviceProps* dp = nullptr;
   int rc = device_props(&dp);
   if (rc) return rc;
+  F32Split split = f32_split(bh, Sq, Skv, D, dp->cus);
+  // what a workspace smaller than the query asks for has no room for is done without
+  const F32Layout cut = f32_layout(bh, nqb, split.parts, true, Skv, D), whole = f32_layout(bh, nqb, 1, true, Skv, D);
+  if (workspace_bytes >= cut.total) w = cut;
+  else if (workspace_bytes >= whole.total) w = whole;
+  if (workspace_bytes < cut.total && split.parts > 1) split = {4, D <= 64 && bh * nqb <= dp->cus && Skv > 2 * FA_KT ? 2 : 1, 1};
   hipStream_t s = (hipStream_t)stream;
   char* ws = reinterpret_cast<char*>(workspace);
   switch (D) {
-    case 32: return launch_fa_f32<32>(Q, K, V, O, (int)bh, Sq, Skv, scale, ws, w, *dp, s);
-    case 64: return launch_fa_f32<64>(Q, K, V, O, (int)bh, Sq, Skv, scale, ws, w, *dp, s);
-    case 96: return launch_fa_f32<96>(Q, K, V, O, (int)bh, Sq, Skv, scale, ws, w, *dp, s);
-    default: return launch_fa_f32<128>(Q, K, V, O, (int)bh, Sq, Skv, scale, ws, w, *dp, s);
+    case 32: return launch_fa_f32<32>(Q, K, V, O, (int)bh, Sq, Skv, scale, ws, w, split, *dp, s);
+    case 64: return launch_fa_f32<64>(Q, K, V, O, (int)bh, Sq, Skv, scale, ws, w, split, *dp, s);
+    case 96: return launch_fa_f32<96>(Q, K, V, O, (int)bh, Sq, Skv, scale, ws, w, split, *dp, s);
+    default: return launch_fa_f32<128>(Q, K, V, O, (int)bh, Sq, Skv, scale, ws, w, split, *dp, s);
   }
 }

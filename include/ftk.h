@@ -498,8 +498,9 @@ int ftk_flash_attn_ws_f16(const void* Q, const void* K, const void* V, void* O,
  * results agree with a float64 evaluation to a few 1e-6 of the largest |O|.
  * Q, K, V, O 16-byte aligned.  Non-finite inputs give NaN.  The workspace (ftk_flash_attn_f32_workspace_bytes,
  * about the size of K and V together, 256-byte aligned) holds their split
- * planes (Q is split in the attention kernel's registers); three small
- * launches precede the attention kernel.  The reference has no device kernel
+ * planes (Q is split in the attention kernel's registers) and, where several
+ * workgroups share a query block's keys, what each of them found; one or two
+ * small launches precede the attention kernel.  The reference has no device kernel
  * for this program.
  */
 size_t ftk_flash_attn_f32_workspace_bytes(int B, int Hd, int Sq, int Skv, int D);

@@ -1584,3 +1584,34 @@ def test_b2b_gemm_wide_with_several_column_tiles(core, G, M, N, K, P):
     ref = np.matmul(np.matmul(A.astype(np.float64), B.astype(np.float64).transpose(0, 2, 1)).astype(np.float16).astype(np.float64),
                     C.astype(np.float64).transpose(0, 2, 1))
     assert ko.max_rel_err(D, ref) <= F16_TOL
+
+
+@pytest.mark.parametrize('B,Hd,Sq,Skv,D', [
+    (1, 1, 1, 1025, 32),         # seventeen tiles, the last of one key
+    (2, 8, 1024, 1024, 32),      # four key groups to 64 query rows
+    (1, 9, 70, 321, 32),         # the same, with six tiles for four groups, the last of one key
+    (1, 2, 130, 1000, 64),       # few query blocks, a ragged tile
+    (2, 8, 1000, 1024, 64),      # two key groups to 64 query rows
+    (1, 16, 1152, 1152, 64),     # more than half a block to a compute unit
+    (3, 16, 1300, 700, 64),      # heads that take two launches in front
+    (2, 3, 300, 1100, 96),
+    (1, 1, 128, 4097, 128),      # as many parts as there may be
+    (1, 5, 257, 640, 128),
+])
+def test_flash_attention_f32_shared_keys(core, B, Hd, Sq, Skv, D):
+    """Query blocks whose keys several groups of a workgroup, or several workgroups, share: the oracle's result within 1e-5 of its largest value (22 bits of
+    each factor, fp32 sums), the same bits in every launch and on a workspace that held something else, and without parts
+    where the workspace has no room for them."""
+    gen = torch.Generator(device='cuda').manual_seed(5)
+    Q, K, V = (torch.randn((B, Hd, s, D), generator=gen, device='cuda') for s in (Sq, Skv, Skv))
+    K[:, :, Skv // 2] *= 6.0                                            # the maximum moves in some part
+    need = int(core.lib.ftk_flash_attn_f32_workspace_bytes(B, Hd, Sq, Skv, D))
+    planes = 2 * B * Hd * Skv * 2 * D * 2
+    ref = ko.attention(Q.cpu().numpy(), K.cpu().numpy(), V.cpu().numpy(), D ** -0.5)
+    ws = torch.full((need,), 0x7f, dtype=torch.uint8, device='cuda')
+    first = core.flash_attention_f32(Q, K, V, workspace=ws)
+    assert ko.max_rel_err(first.cpu().numpy(), ref) <= 1e-5
+    for _ in range(3):
+        assert torch.equal(core.flash_attention_f32(Q, K, V, workspace=ws), first)
+    small = torch.empty(planes + 3 * 256 + 8 * B * Hd, dtype=torch.uint8, device='cuda')
+    assert ko.max_rel_err(core.flash_attention_f32(Q, K, V, workspace=small).cpu().numpy(), ref) <= 1e-5
