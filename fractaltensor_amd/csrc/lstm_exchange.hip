@@ -613,7 +613,7 @@ void lstm_exchange_kernel(ExchangeArgs a) {
       c[u] = __builtin_fmaf(gate(p[1]), c_prev[u], gate(p[0]) * tanh_f(p[3]));
       h[u] = gate(p[2]) * tanh_f(c[u]);
       // rounded to 32 bits before 16 in every loop: one instruction may do both, with another last bit now and then, and
-      // a ragged batch, which takes another loop than a dense one, gives the same bits
+      // a ragged batch, which takes another loop than a dense one, gives the same bits (with row blocks of the same kind)
       if constexpr (HALF) asm("" : "+v"(c[u]), "+v"(h[u]));
       unsigned word;
       if constexpr (HALF) {
@@ -1061,17 +1061,60 @@ int exchange_one_block_layers(int L, int B, int H, bool half) {
   return std::min({L, kXLayers, exchange_teams(H / exchange_units(H, half, false), exchange_slots(f.one)) / ((B + 15) / 16)});
 }
 
-// Layers of one launch (0: the device cannot hold one), and the kind of row block: 16 rows and one block per workgroup,
-// whose step is the shorter one, wherever that takes no more launches.  (L 23 T 67 B 10 fp32 H 512, three launches of
-// either kind: 831 us with blocks of 32, 540 with blocks of 16; at L 27 T 48 B 17, seven launches against four, they are level.)
-int exchange_layers(int L, int B, int H, bool half, bool* many) {
+// What the launches of a stack take, in microseconds, by measurement: a step of a row block where the launch has at most one, two,
+// ... workgroups per compute unit, what every further layer of the launch adds until the pipeline of layers is full, and
+// what a launch takes before its first step (weights, places; blocks of 16 rows: for each workgroup of a compute unit).
+struct ExchangeCost {
+  float one[4], one_layer, one_launch;     // blocks of 16 rows, one per workgroup
+  float many[2], many_layer, many_launch;  // blocks of 32 rows, each of those that a workgroup walks
+};
+
+ExchangeCost exchange_cost(int H, bool half) {
+  if (half) return H == 256   ? ExchangeCost{{1.2f, 1.4f, 1.4f, 1.6f}, 2.0f, 5.0f, {2.0f, 2.75f}, 2.7f, 14.0f}
+                   : H == 512 ? ExchangeCost{{1.3f, 1.75f, 1.75f, 1.75f}, 3.5f, 10.0f, {3.3f, 3.3f}, 5.0f, 20.0f}
+                              : ExchangeCost{{2.1f, 2.1f, 2.1f, 2.1f}, 6.0f, 30.0f, {3.75f, 3.75f}, 8.0f, 23.0f};
+  return H == 64    ? ExchangeCost{{1.15f, 1.35f, 1.6f, 1.85f}, 1.5f, 12.0f, {1.9f, 2.8f}, 1.0f, 13.0f}
+         : H == 128 ? ExchangeCost{{1.25f, 1.45f, 1.7f, 1.7f}, 1.6f, 14.0f, {1.95f, 2.9f}, 2.0f, 16.0f}
+         : H == 256 ? ExchangeCost{{1.35f, 1.8f, 1.8f, 1.8f}, 2.4f, 11.0f, {4.2f, 4.2f}, 5.0f, 28.0f}
+                    : ExchangeCost{{1.85f, 1.85f, 1.85f, 1.85f}, 4.0f, 40.0f, {3.5f, 3.5f}, 6.5f, 18.0f};
+}
+
+// Layers of one launch (0: the device cannot hold one), and the kind of row block.  16 rows and one block per workgroup, whose
+// step is the shorter one, wherever that takes no more launches (L 23 T 67 B 10 fp32 H 512, three launches of either kind: 831 us
+// with blocks of 32, 540 with blocks of 16), and where the launches it takes more cost less than the steps save: two 16-row workgroups
+// of H 256 on a compute unit do their steps in 1.8 us, one 32-row workgroup in 4.2.  us with blocks of 32 and of 16: fp32 L 6
+// T 128 B 256 H 256 1121, 786; L 31 T 40 B 20 H 256 332, 252; L 20 T 50 B 100 H 128 317, 246; fp16 L 7 T 43 B 142 H 256
+// 254, 127; the other way round at fp32 L 4 T 30 B 128 H 512 231, 334; fp16 L 15 T 25 B 107 H 512 422, 487.  `plain`: neither a
+// ragged batch nor a dilation; those take the general loop, which is no faster with blocks of 16 (ragged L 32 T 48 B 96 H 128 280, 374;
+// dilated L 6 T 100 B 256 H 128 230, 262).
+// The steps weigh against the launches, so T counts: fp32 L 12 B 250 H 128 at T 64 422, 309, at T 16 123, 157.
+int exchange_layers(int L, int T, int B, int H, bool half, bool plain, bool* many) {
   const ExchangeFlavour f = exchange_flavour_of(H, half);
   *many = false;
   if (!f.one) return 0;
+  const int nrb = (B + 31) / 32, W = H / exchange_units(H, half, true), slots = exchange_slots(f.many);
   const int one = exchange_one_block_layers(L, B, H, half);
-  const int more = one == L ? 0 : exchange_plan(L, H / exchange_units(H, half, true), (B + 31) / 32, exchange_slots(f.many)).layers;
-  *many = one == 0 || (one < L && more > 0 && (L + one - 1) / one > (L + more - 1) / more);
-  return *many ? more : one;
+  const int more = one == L ? 0 : exchange_plan(L, W, nrb, slots).layers;
+  if (more == 0 || (one > 0 && (L + one - 1) / one <= (L + more - 1) / more)) return one;
+  *many = true;
+  const DeviceProps* dp = nullptr;
+  if (!plain || one == 0 || device_props(&dp) != FTK_OK) return more;
+  const ExchangeCost cost = exchange_cost(H, half);
+  auto per_cu = [&](long long groups, int most) { return (int)std::min<long long>((groups + dp->cus - 1) / dp->cus, most); };
+  const int launches = (L + one - 1) / one, even = (L + launches - 1) / launches;
+  const int held = per_cu((long long)even * ((B + 15) / 16) * (H / exchange_units(H, half, false)), 4);
+  const float step_one = launches * cost.one[held - 1];
+  const float rest_one = launches * held * cost.one_launch + (L - launches) * cost.one_layer;
+  float step_many = 0, rest_many = 0;
+  for (int l0 = 0; l0 < L; l0 += more) {
+    const ExchangePlan p = exchange_plan(std::min(more, L - l0), W, nrb, slots);
+    const int blocks = (nrb + p.slices - 1) / p.slices;
+    step_many += blocks * cost.many[per_cu((long long)p.layers * p.slices * W, 2) - 1];
+    rest_many += cost.many_launch + (p.layers - 1) * cost.many_layer;
+  }
+  if (T * step_one + rest_one > 0.95f * (T * step_many + rest_many)) return more;
+  *many = false;
+  return even;
 }
 }  // namespace
 
@@ -1081,7 +1124,7 @@ bool exchange_one_block(int L, int B, int H, bool half) { return exchange_one_bl
 // Bytes of workspace that run_exchange uses on the current device; without a device, what it could at most.
 size_t exchange_need(int L, int T, int B, int H, bool half) {
   bool many;
-  const int most = exchange_layers(L, B, H, half, &many);
+  const int most = std::max(exchange_layers(L, T, B, H, half, true, &many), exchange_layers(L, T, B, H, half, false, &many));
   return exchange_workspace_bytes(most ? std::min(L, most) : L, T, B, H, half);
 }
 
@@ -1093,8 +1136,10 @@ int run_exchange(bool half, const void* xs, const void* WU, const float* bias, c
   *handled = false;
   const ExchangeFlavour f = exchange_flavour_of(H, half);
   if (!f.one) return FTK_OK;
+  bool plain = !active;
+  for (int l = 0; dil && l < L; ++l) plain = plain && dil[l] == 1;
   bool many;
-  const int most = exchange_layers(L, B, H, half, &many);
+  const int most = exchange_layers(L, T, B, H, half, plain, &many);
   if (most == 0) return FTK_OK;
   const int slots = exchange_slots(many ? f.many : f.one), block = many ? 32 : 16, nrb = (B + block - 1) / block;
   const int W = H / exchange_units(H, half, many);

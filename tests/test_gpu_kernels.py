@@ -1469,6 +1469,41 @@ def test_stacked_lstm_exchange_kernel(core, half, H, L, T, B, dil):
                 assert_lstm_close(torch.from_numpy(t), ref[:, ref_live], what)
 
 
+@pytest.mark.parametrize('half,H,L,T,B', [
+    (False, 128, 20, 48, 100),             # two launches of ten layers
+    (False, 256, 6, 33, 250),              # three launches of two layers, the last row block of ten rows
+    (False, 256, 13, 70, 101),             # the last launch of one layer
+    (False, 256, 31, 4, 17),               # sixteen and fifteen layers, a row block of one row
+    (True, 256, 7, 5, 142),                # four and three layers
+])
+def test_stack_in_more_launches_of_16_row_blocks(core, half, H, L, T, B):
+    """Dense stacks that a launch of 32-row blocks would hold more layers of: against the oracle, the same bits in every
+    launch and for dilations of one, and a ragged batch beside them on the same workspace."""
+    xs, WU, bs = lstm_inputs(78, L, T, B, H, 1.0 / np.sqrt(H))
+    rows = sorted({0, 15, 16, B // 2, B - 1})
+    if half:
+        xs, WU = xs.astype(np.float16), WU.astype(np.float16)
+        hr, cr = ko.stacked_lstm_f16(xs[:, rows], WU, bs, None)
+    else:
+        hr, cr = ko.stacked_lstm(xs[:, rows], WU, bs, dilations=None)
+    fn = core.stacked_lstm_f16 if half else core.stacked_lstm
+    nbytes = (core.lib.ftk_stacked_lstm_f16_workspace_bytes if half else core.stacked_lstm_workspace_bytes)(L, T, B, H)
+    ws = torch.full((nbytes,), 0x3c, dtype=torch.uint8, device='cuda')
+    first = fn(dev(xs), dev(WU), dev(bs), workspace=ws, check=True)
+    ragged = fn(dev(xs), dev(WU), dev(bs), workspace=ws, active_rows=[B] * T, check=True)
+    for kw in (dict(), dict(dilations=[1] * L)):
+        got = fn(dev(xs), dev(WU), dev(bs), workspace=ws, check=True, **kw)
+        assert all(torch.equal(a, b) for a, b in zip(got, first))
+    for out in (first, ragged):
+        for t, ref, what in ((out[0], hr, 'h'), (out[1], cr, 'c')):
+            t = t[:, :, rows].float().cpu()
+            if half:
+                # h and c carry an fp16 rounding, 2^-11 of themselves, through T steps and L layers that damp it
+                assert ko.max_rel_err(t.numpy(), ref.astype(np.float32)) <= 1e-2, what
+            else:
+                assert_lstm_close(t, ref, what)
+
+
 @pytest.mark.parametrize('H,L,T,B,dil', [
     (64, 2, 3, 1, None),                   # one pair of chunks without an h, two with one
     (64, 3, 4, 256, [1, 2, 3]),
