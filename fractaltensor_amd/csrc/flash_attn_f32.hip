@@ -14,7 +14,7 @@
 // 2^-17 of the largest.
 //
 // Launches: the largest |K| and |V| per (batch, head) and the split of K and V into planes [row][top D | rest D] in the
-// workspace, in one launch where heads are small, else in three; the attention kernel, which splits its rows of Q (times scale * log2 e)
+// workspace, in one launch where heads are small, else in two; the attention kernel, which splits its rows of Q (times scale * log2 e)
 // itself, in registers.  A plane row is an fp16 row of 2 D
 // elements, so tiles, copies and fragment reads are those of the fp16 kernel at twice the head dimension
 // (fa_common.h), and the contractions are its transposed ones: S^T = K Q^T, O^T += V^T P^T, a lane owns one query
@@ -111,8 +111,8 @@ __global__ __launch_bounds__(256) void attn_f32_split_kernel(const float* K, con
 
 // Largest magnitude and planes in one launch, for heads that a compute unit reads in a microsecond or two: each of a
 // head's `parts` workgroups finds the head's largest magnitude for itself (the others find the rows in their XCD's L2) and
-// writes its share of the planes.  The three launches of the other way (clear, largest, split) take 11 us whatever the size
-// (B 2, 8 heads, 1024 keys of 32).
+// writes its share of the planes.  (Three launches, with a clear in front, took 11 us whatever the size: B 2, 8 heads, 1024
+// keys of 32.)
 constexpr int kPlanesThreads = 512;
 template <int D>
 __global__ __launch_bounds__(kPlanesThreads) void attn_f32_planes_kernel(const float* K, const float* V, _Float16* kplanes, _Float16* vplanes,
@@ -155,8 +155,8 @@ constexpr int f32_partial_bytes(int D) { return 128 * D * 4 + 4 * 64 * 8; }
 // works through the tiles in halves of 32 keys, and with one wave per SIMD the softmax of a half has no other
 // wave's MFMAs to run beside: it is cut in two, the maxima under the P V MFMAs of the half before and the weights
 // under the score MFMAs of the half after (the comments in the kernel give the order).
-// KG == 2 (head sizes up to 64, whose registers allow two waves per SIMD): two groups of four waves share the query rows,
-// each walks half of the keys with tiles of its own in LDS, and the first takes in the second's result at the end.
+// KG > 1 (two groups at head sizes up to 64, whose registers allow two waves per SIMD; four at 32): the groups share the query rows,
+// each walks its part of the keys with tiles of its own in LDS, and the first takes in the others' results at the end.
 // PART: nparts workgroups share a block of query rows, each with its share of the tiles.  Each leaves its unnormalised
 // accumulators, reference and sum in the workspace (write-through: a block's workgroups may sit on several XCDs), and the one
 // that finds itself the last by the block's counter takes all of them in, in the order of their keys, so that the result does
@@ -782,7 +782,7 @@ static int launch_fa_f32(const float* Q, const float* K, const float* V, float* 
   const size_t per_bh = (size_t)Skv * D, head_bytes = per_bh * sizeof(float);
   // One launch while heads are small and what all its workgroups read for the largest magnitudes stays below 96 MB (a few
   // microseconds of L2); up to two workgroups to a compute unit (B 4, 16 heads, 1024 keys of 64: four parts each, 134 MB, were slower
-  // than three launches).
+  // than the launches below).
   const size_t all_heads = 2 * (size_t)BH * head_bytes, most_read = (size_t)96 << 20;
   const int parts = (int)std::max<size_t>(1, std::min({512 / (2 * (size_t)BH), per_bh / (8 * kPlanesThreads), most_read / all_heads}));
   const int counters = split.parts > 1 ? BH * ((Sq + 127) / 128) : 0;

@@ -5,7 +5,7 @@
 // about the length of one step.  A layer is spread over H / 16 workgroups of 4 waves (a team; with several row
 // slices a layer has several teams, each with batch rows of its own).  A workgroup owns 16 hidden units = 64 gate
 // columns and keeps its slice of [W;U] in registers for the whole launch.  An item is a block of 16 batch rows of one time
-// step (32 rows where a workgroup has several blocks to walk):
+// step (32 rows where a workgroup has several blocks to walk; exchange_layers chooses):
 //
 //   * Its four waves cut the CONTRACTION, not the columns: wave w multiplies quarter w of x_t and quarter w of h_{t-d}
 //     with all 64 columns.  A wave therefore loads exactly the activations it needs, from memory straight into the
@@ -23,8 +23,8 @@
 //     write-through stores, which is what a team that does not sit together uses.
 //
 // A step of a single layer takes 0.85 us at H = 64, 0.9 at 128, 1.2 at 256 and 1.9 at 512 (fp32), where a hand-over of the
-// persistent kernel's serial schedule took 5 to 6 and a launch per step 20 and more: L 20 T 30 B 32 H 128 1004 -> 82 us,
-// L 8 T 100 B 64 H 512 7.3 -> 0.76 .. 0.79 ms, L 1 T 16 B 64 H 256 100 -> 31 us for both kernels (27 and 4).
+// persistent kernel's serial schedule took 5 to 6 and a launch per step 20 and more: L 20 T 30 B 32 H 128 1004 -> 80 us,
+// L 8 T 100 B 64 H 512 7.3 -> 0.73 ms, L 1 T 16 B 64 H 256 100 -> 31 us for both kernels (27 and 4).
 //
 // The exchange buffers.  ring: the own layer's h for d = 1, four steps deep.  A workgroup that has all of h(t-1) knows
 // that every member of its team has read h(t-2) (it published h(t-1) behind a barrier that all its waves reached after
@@ -1120,6 +1120,15 @@ int exchange_layers(int L, int T, int B, int H, bool half, bool plain, bool* man
 
 // Whether the whole batch of every layer fits the chip with one block of 16 rows per workgroup.
 bool exchange_one_block(int L, int B, int H, bool half) { return exchange_one_block_layers(L, B, H, half) == L; }
+
+// Row blocks of 32 rows that a workgroup has to walk in a stack's first launch (0: the device holds none).
+int exchange_blocks(int L, int B, int H, bool half) {
+  const ExchangeFlavour f = exchange_flavour_of(H, half);
+  if (!f.many) return 0;
+  const int nrb = (B + 31) / 32;
+  const ExchangePlan p = exchange_plan(L, H / exchange_units(H, half, true), nrb, exchange_slots(f.many));
+  return p.layers ? (nrb + p.slices - 1) / p.slices : 0;
+}
 
 // Bytes of workspace that run_exchange uses on the current device; without a device, what it could at most.
 size_t exchange_need(int L, int T, int B, int H, bool half) {

@@ -68,6 +68,7 @@ int run_wavefront_split(const float* xs, const float* WU, const float* bias, con
 bool exchange_takes(int H, bool half);
 bool exchange_fits(int T, int B, int H, bool half);
 bool exchange_one_block(int L, int B, int H, bool half);
+int exchange_blocks(int L, int B, int H, bool half);
 size_t exchange_workspace_bytes(int L, int T, int B, int H, bool half);
 size_t exchange_need(int L, int T, int B, int H, bool half);
 int run_exchange(bool half, const void* xs, const void* WU, const float* bias, const int* dil, const int* active, void* hsss,
@@ -1819,9 +1820,15 @@ static bool f16_streams(int L, int B, int H, bool ragged) {
 // block per workgroup, because then the chain of dependent steps is the time (L 1 .. 8, T 32, B 64, H 256, fp32: 67 ..
 // 124 us against 198 .. 265; H 512, 8 layers, T 100: 0.76 .. 0.79 ms against 7.3).  With more rows than that it walks several blocks per
 // workgroup, and there
-//   H = 256 has the paired schedule of the persistent kernel, which feeds the matrix pipe better: ahead from 16 layers x
-//     256 rows on (L 16 B 192: 536 against 575 us, L 16 B 256: 660 against 585, L 32 B 192: 998 against 937; fp16 data: L 16
-//     B 192 370 / 382, L 32 B 192 769 / 597), and for dilated stacks, whose chains are short (L 6 T 128 B 256: 1.22 / 0.83 ms);
+//   H = 256 has the paired schedule of the persistent kernel, which feeds the matrix pipe better where it applies: to batches of
+//     whole 8 rows (without, T 64, us, exchange / persistent: fp32 L 32 B 250 2264 / 2658, L 31 B 99 1159 / 1598, dilated T 128
+//     L 6 B 100 590 / 1174; fp16 L 32 B 250 1150 / 2009), not to the odd one of an odd number of row blocks (fp32 L 20 B 200
+//     1561 / 1689, L 32 B 200 2005 / 1899; dilated L 6 B 224 584 / 730), and from some 112 layers x row blocks on (fp32 L 10 B 256
+//     744 / 1220, L 14 B 256 1128 / 926, L 28 T 48 B 128 904 / 858), with fp16 data, whose steps are the shorter ones in the exchange
+//     kernel, in stacks as deep as the chip holds (L 16 B 256 574 / 671, L 24 B 256 865 / 1038, L 32 B 128 568 / 760, B 192
+//     1036 / 909, B 256 1151 / 1122).  Dilated stacks, whose chains are short, are better there wherever the exchange kernel's workgroups have
+//     more than one row block to walk (fp32 L 6 T 128 B 128, one block: 587 / 731; L 4 B 256, one: 325 / 382; L 6 T 128 B 192, two:
+//     1105 / 771, B 256 1116 / 802; fp16 L 5 B 256 350 / 293);
 //   H = 1024 (fp16 data) holds four layers on the chip at a time, a pass over them takes some 3.6 us a step and block of 32 rows,
 //     and the streamed cells 5 us a step and layer per 256 rows, not below 12 layers' (T 64, ms, exchange and streamed: L 9
 //     B 256 4.21, 3.86; L 12 B 256 5.47, 4.49; L 16 B 192 5.58, 5.22, B 160 4.67, 5.09; L 20 B 192 7.01, 6.69, B 160 5.85,
@@ -1838,9 +1845,11 @@ static bool exchange_chosen(int L, int T, int B, int H, const int* dil, bool hal
   if (const char* e = getenv("FTK_LSTM_EXCHANGE")) return e[0] == '1';
   if (exchange_one_block(L, B, H, half)) return true;
   if (H == PH) {
+    const int nrb = (B + 31) / 32;
+    if (B % 8 != 0 || (nrb % 2 != 0 && L * nrb < 160)) return true;
     for (int l = 0; dil && l < L; ++l)
-      if (dil[l] != 1) return false;
-    return L * ((B + 31) / 32) < 112;
+      if (dil[l] != 1) return exchange_blocks(L, B, H, half) == 1;
+    return half ? L <= 28 || L * nrb < 192 || nrb % 2 != 0 : L * nrb < 112;
   }
   if (H == 1024) return ragged ? L < 12 || B <= 192 : 7ll * ((L + 3) / 4) * ((B + 31) / 32) <= 10ll * std::max(L, 12) * ((B + 255) / 256);
   if (half && f16_streams(L, B, H, ragged)) {   // H = 512

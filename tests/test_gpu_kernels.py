@@ -1469,6 +1469,42 @@ def test_stacked_lstm_exchange_kernel(core, half, H, L, T, B, dil):
                 assert_lstm_close(torch.from_numpy(t), ref[:, ref_live], what)
 
 
+@pytest.mark.parametrize('half,L,T,B,dil', [
+    (False, 32, 3, 250, None),             # no whole 8 rows: no pairs of row blocks
+    (False, 20, 3, 200, None),             # an odd number of row blocks
+    (False, 14, 3, 256, None),             # pairs
+    (False, 6, 9, 100, [1, 2, 4, 1, 2, 4]),
+    (False, 6, 9, 224, [1, 2, 4, 1, 2, 4]),
+    (False, 4, 9, 256, [1, 2, 4, 8]),      # one row block to walk
+    (False, 5, 9, 256, [1, 2, 4, 8, 1]),   # two, in pairs
+    (True, 32, 3, 255, None),              # an odd batch, which the pairs of batch rows do not take
+    (True, 24, 3, 256, None),
+    (True, 29, 3, 224, None),              # deep enough, but an odd number of row blocks
+    (True, 32, 3, 192, None),
+    (True, 6, 9, 100, [1, 2, 4, 1, 2, 4]),
+])
+def test_stacks_of_hidden_size_256_on_either_kernel(core, half, L, T, B, dil):
+    """Both sides of every line between the exchange kernel and the persistent one, dense and ragged, against the oracle."""
+    H = 256
+    xs, WU, bs = lstm_inputs(79, L, T, B, H, 1.0 / np.sqrt(H))
+    rows = sorted({0, 31, B // 2, B - 1})
+    if half:
+        xs, WU = xs.astype(np.float16), WU.astype(np.float16)
+        hr, cr = ko.stacked_lstm_f16(xs[:, rows], WU, bs, dil)
+    else:
+        hr, cr = ko.stacked_lstm(xs[:, rows], WU, bs, dilations=dil)
+    fn = core.stacked_lstm_f16 if half else core.stacked_lstm
+    for active in (None, [B] * T):
+        out = fn(dev(xs), dev(WU), dev(bs), dilations=dil, active_rows=active, check=True)
+        for t, ref, what in ((out[0], hr, 'h'), (out[1], cr, 'c')):
+            t = t[:, :, rows].float().cpu()
+            if half:
+                # h and c carry an fp16 rounding, 2^-11 of themselves, through T steps and L layers that damp it
+                assert ko.max_rel_err(t.numpy(), ref.astype(np.float32)) <= 1e-2, what
+            else:
+                assert_lstm_close(t, ref, what)
+
+
 @pytest.mark.parametrize('half,H,L,T,B', [
     (False, 128, 20, 48, 100),             # two launches of ten layers
     (False, 256, 6, 33, 250),              # three launches of two layers, the last row block of ten rows
