@@ -66,6 +66,16 @@ __global__ __launch_bounds__(256) void attn_f32_absmax_kernel(const float* K, co
     chunk_bits[((size_t)blockIdx.z * BH + blockIdx.y) * gridDim.x + blockIdx.x] = max(max(wave_max[0], wave_max[1]), max(wave_max[2], wave_max[3]));
 }
 
+// One word a head from the words of its chunks, a wave to each: where the workspace has no room for these beside the planes they
+// stand in the planes of V, which the launch behind this one writes.  A few microseconds; with a workgroup or a few to a head for
+// the whole preparation, as small heads have, the call took 3329 us in place of 2252 at 2 heads of 64 k keys of 128, 4079 in place of 2345 at 4.
+__global__ __launch_bounds__(64) void attn_f32_largest_kernel(const unsigned* chunk_bits, int chunks, unsigned* bits) {
+  unsigned m = (int)threadIdx.x < chunks ? chunk_bits[(size_t)blockIdx.x * chunks + threadIdx.x] : 0;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) m = max(m, (unsigned)__shfl_xor((int)m, o));
+  if (threadIdx.x == 0) bits[blockIdx.x] = m;
+}
+
 // Eight neighbouring floats of a row into its planes [top D | rest D].
 template <int D>
 __device__ __forceinline__ void split_eight(const float* X, _Float16* planes, long long chunk, float scale) {
@@ -86,7 +96,8 @@ __device__ __forceinline__ void split_eight(const float* X, _Float16* planes, lo
   *reinterpret_cast<v8h*>(dst + D) = rest;
 }
 
-// Planes under each head's scale, grid (workgroups of a head, BH, 2: K, V), eight floats to a thread; clears the counters.
+// Planes under each head's scale, grid (workgroups of a head, BH, 2: K, V), eight floats to a thread; clears the counters.  chunk_bits: the
+// words of each head's chunks, or bits itself, with one word a head (which then gets the value it has).
 template <int D>
 __global__ __launch_bounds__(256) void attn_f32_split_kernel(const float* K, const float* V, _Float16* kplanes, _Float16* vplanes, unsigned* bits,
                                                             const unsigned* chunk_bits, int chunks, int Skv, int BH, int counters) {
@@ -787,20 +798,25 @@ static int launch_fa_f32(const float* Q, const float* K, const float* V, float* 
   const int parts = (int)std::max<size_t>(1, std::min({512 / (2 * (size_t)BH), per_bh / (8 * kPlanesThreads), most_read / all_heads}));
   const int counters = split.parts > 1 ? BH * ((Sq + 127) / 128) : 0;
   int rc;
-  if ((head_bytes <= 512 * 1024 && all_heads * parts <= most_read) || !w.chunked) {
+  if (head_bytes <= 512 * 1024 && all_heads * parts <= most_read) {
     hipLaunchKernelGGL(attn_f32_planes_kernel<D>, dim3((unsigned)(2 * BH * parts)), dim3(kPlanesThreads), 0, s, K, V, kp, vp, bits, Skv, BH, parts,
                        counters);
     rc = check_launch("attn_f32_planes_kernel");
     if (rc) return rc;
   } else {
     const int chunks = (int)std::min<size_t>({(size_t)std::max(1, 2048 / (2 * BH)), (per_bh + 4095) / 4096, kMaxChunks});
-    unsigned* const chunk_bits = reinterpret_cast<unsigned*>(ws + w.chunks);
+    unsigned* const chunk_bits = reinterpret_cast<unsigned*>(ws + (w.chunked ? w.chunks : w.vp));   // (8 bytes a chunk, of 16 KB of V's planes or a whole head's)
     hipLaunchKernelGGL(attn_f32_absmax_kernel, dim3(chunks, BH, 2), dim3(256), 0, s, K, V, chunk_bits, per_bh, BH);
     rc = check_launch("attn_f32_absmax_kernel");
     if (rc) return rc;
+    if (!w.chunked) {
+      hipLaunchKernelGGL(attn_f32_largest_kernel, dim3(2 * BH), dim3(64), 0, s, (const unsigned*)chunk_bits, chunks, bits);
+      rc = check_launch("attn_f32_largest_kernel");
+      if (rc) return rc;
+    }
     const int wgs = (int)std::min<size_t>(std::max(1, 4096 / (2 * BH)), (per_bh / 8 + 255) / 256);
-    hipLaunchKernelGGL(attn_f32_split_kernel<D>, dim3(wgs, BH, 2), dim3(256), 0, s, K, V, kp, vp, bits, (const unsigned*)chunk_bits, chunks, Skv, BH,
-                       counters);
+    hipLaunchKernelGGL(attn_f32_split_kernel<D>, dim3(wgs, BH, 2), dim3(256), 0, s, K, V, kp, vp, bits, (const unsigned*)(w.chunked ? chunk_bits : bits),
+                       w.chunked ? chunks : 1, Skv, BH, counters);
     rc = check_launch("attn_f32_split_kernel");
     if (rc) return rc;
   }

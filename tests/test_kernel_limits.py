@@ -176,3 +176,45 @@ def test_deep_f16_stacks_at_512_units_take_the_faster_kernel(core, monkeypatch, 
             continue                                          # the persistent kernel
         h, _ = core.stacked_lstm_f16(xs, WU)
         assert torch.equal(h, default[0]) == (e == way)
+
+
+def _up(nbytes):
+    return (nbytes + 255) // 256 * 256
+
+
+@pytest.mark.parametrize('B,Hd,Sq,Skv,D,timed', [
+    (1, 1, 128, 65536, 128, True),
+    (1, 4, 128, 65536, 128, True),
+    (1, 2, 40, 16384, 32, False),
+    (3, 16, 130, 3001, 64, False),      # heads of 750 KB
+    (1, 1, 1, 4097, 32, False),         # a head of 512 KB and one key
+    (5, 60, 64, 1500, 32, False),       # small heads, together too much to be read by every workgroup
+    (2, 3, 70, 333, 96, False),         # small heads: one launch in front
+])
+def test_flash_attention_f32_on_a_workspace_of_planes_only(core, B, Hd, Sq, Skv, D, timed):
+    """A workspace without room for the words of the heads' chunks: the bits of the call that has it (without parts), and, since
+    the preparation is spread over as many workgroups, its time (1.5 to 1.8 times that, with a workgroup to each head)."""
+    gen = torch.Generator(device='cuda').manual_seed(7)
+    q, k, v = (torch.randn((B, Hd, s, D), generator=gen, device='cuda') for s in (Sq, Skv, Skv))
+    k[0, 0, Skv - 1, D - 1] = 37.0                                       # the largest of the first head is its last
+    v[-1, -1, Skv // 2, 3] = -99.0
+    planes_only = _up(8 * B * Hd) + 2 * _up(B * Hd * Skv * 2 * D * 2)
+    chunks = _up(2 * B * Hd * 64 * 4)
+    spaces = [torch.full((n,), 0x7f, dtype=torch.uint8, device='cuda') for n in (planes_only, planes_only + chunks)]
+    outs = [core.flash_attention_f32(q, k, v, workspace=w) for w in spaces]
+    assert torch.equal(outs[0], outs[1])
+    whole = core.flash_attention_f32(q, k, v)
+    assert float((outs[0] - whole).abs().max() / whole.abs().max()) <= 1e-5   # 22 bits of each factor, fp32 sums in another order
+    with pytest.raises(core.FtkError):
+        core.flash_attention_f32(q, k, v, workspace=spaces[0][:planes_only - 256])
+    if timed:
+        best = [1e9, 1e9]
+        for _ in range(5):
+            for i, w in enumerate(spaces):
+                start, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+                start.record()
+                core.flash_attention_f32(q, k, v, workspace=w)
+                end.record()
+                end.synchronize()
+                best[i] = min(best[i], start.elapsed_time(end))
+        assert best[0] <= 1.25 * best[1], best
