@@ -1061,33 +1061,45 @@ int exchange_one_block_layers(int L, int B, int H, bool half) {
   return std::min({L, kXLayers, exchange_teams(H / exchange_units(H, half, false), exchange_slots(f.one)) / ((B + 15) / 16)});
 }
 
-// What the launches of a stack take, in microseconds, by measurement: a step of a row block where the launch has at most one, two,
-// ... workgroups per compute unit, what every further layer of the launch adds until the pipeline of layers is full, and
-// what a launch takes before its first step (weights, places; blocks of 16 rows: for each workgroup of a compute unit).
+// What the launches of a stack take, in microseconds: `first` and, for each further one, `next` before the steps (weights, places, the
+// kernel in front, and what a deep stack's launches find less of in the caches), `layer` for every further layer of a launch until the
+// pipeline of layers is full, and for a step of each row block that a workgroup walks `step` and `fill` times the workgroups per compute
+// unit.  Fitted, for each hidden size, to the times of both kinds over 420 stacks of L up to 32, T 16 .. 128, B 8 .. 256 that blocks of 16
+// rows take more launches for; the times are met within 1.5 to 8 % (rms).
 struct ExchangeCost {
-  float one[4], one_layer, one_launch;     // blocks of 16 rows, one per workgroup
-  float many[2], many_layer, many_launch;  // blocks of 32 rows, each of those that a workgroup walks
+  float step, fill, layer, first, next;
 };
 
-ExchangeCost exchange_cost(int H, bool half) {
-  if (half) return H == 256   ? ExchangeCost{{1.2f, 1.4f, 1.4f, 1.6f}, 2.0f, 5.0f, {2.0f, 2.75f}, 2.7f, 14.0f}
-                   : H == 512 ? ExchangeCost{{1.3f, 1.75f, 1.75f, 1.75f}, 3.5f, 10.0f, {3.3f, 3.3f}, 5.0f, 20.0f}
-                              : ExchangeCost{{2.1f, 2.1f, 2.1f, 2.1f}, 6.0f, 30.0f, {3.75f, 3.75f}, 8.0f, 23.0f};
-  return H == 64    ? ExchangeCost{{1.15f, 1.35f, 1.6f, 1.85f}, 1.5f, 12.0f, {1.9f, 2.8f}, 1.0f, 13.0f}
-         : H == 128 ? ExchangeCost{{1.25f, 1.45f, 1.7f, 1.7f}, 1.6f, 14.0f, {1.95f, 2.9f}, 2.0f, 16.0f}
-         : H == 256 ? ExchangeCost{{1.35f, 1.8f, 1.8f, 1.8f}, 2.4f, 11.0f, {4.2f, 4.2f}, 5.0f, 28.0f}
-                    : ExchangeCost{{1.85f, 1.85f, 1.85f, 1.85f}, 4.0f, 40.0f, {3.5f, 3.5f}, 6.5f, 18.0f};
+ExchangeCost exchange_cost(int H, bool half, bool many) {
+  if (half) {
+    if (H == 256) return many ? ExchangeCost{2.63f, 0.04f, 3.0f, 6.0f, 6.0f} : ExchangeCost{0.82f, 0.32f, 1.55f, 16.0f, 21.5f};
+    if (H == 512) return many ? ExchangeCost{3.04f, 0.3f, 4.6f, 29.0f, 33.0f} : ExchangeCost{1.29f, 0.16f, 3.35f, 20.5f, 23.0f};
+    return many ? ExchangeCost{2.96f, 0.26f, 6.05f, 41.0f, 47.0f} : ExchangeCost{1.7f, 0.76f, 5.0f, 9.0f, 38.0f};
+  }
+  if (H == 64) return many ? ExchangeCost{1.44f, 0.64f, 1.75f, 0.0f, 0.0f} : ExchangeCost{0.35f, 0.48f, 0.0f, 51.5f, 51.5f};
+  if (H == 128) return many ? ExchangeCost{2.29f, 0.36f, 2.35f, 0.0f, 0.0f} : ExchangeCost{0.22f, 0.59f, 1.95f, 0.0f, 54.0f};
+  if (H == 256) return many ? ExchangeCost{3.77f, 0.48f, 4.25f, 38.0f, 38.0f} : ExchangeCost{1.01f, 0.42f, 3.15f, 0.0f, 37.0f};
+  return many ? ExchangeCost{2.86f, 0.35f, 4.1f, 35.0f, 36.0f} : ExchangeCost{1.73f, 0.24f, 4.35f, 11.5f, 34.0f};
 }
+
+// A launch is an ordinary one or, once a process uses a second stream or records graphs, a cooperative one, which takes 16 to 18 us more
+// (launch_resident).  Which it is depends on what the process did before, and what a call computes must not, so a launch more is
+// charged most of the difference always.  Loss against the better kind of each, mean over 2940 stacks near the line with ordinary launches
+// and 1900 with cooperative ones: 0.4 and 1.5 % with nothing charged, 0.8 and 0.5 % with 12 us, 1.2 and 0.4 % with 17.
+constexpr float kLaunchMore = 12.0f;
 
 // Layers of one launch (0: the device cannot hold one), and the kind of row block.  16 rows and one block per workgroup, whose
 // step is the shorter one, wherever that takes no more launches (L 23 T 67 B 10 fp32 H 512, three launches of either kind: 831 us
 // with blocks of 32, 540 with blocks of 16), and where the launches it takes more cost less than the steps save: two 16-row workgroups
 // of H 256 on a compute unit do their steps in 1.8 us, one 32-row workgroup in 4.2.  us with blocks of 32 and of 16: fp32 L 6
-// T 128 B 256 H 256 1121, 786; L 31 T 40 B 20 H 256 332, 252; L 20 T 50 B 100 H 128 317, 246; fp16 L 7 T 43 B 142 H 256
-// 254, 127; the other way round at fp32 L 4 T 30 B 128 H 512 231, 334; fp16 L 15 T 25 B 107 H 512 422, 487.  `plain`: neither a
-// ragged batch nor a dilation; those take the general loop, which is no faster with blocks of 16 (ragged L 32 T 48 B 96 H 128 280, 374;
-// dilated L 6 T 100 B 256 H 128 230, 262).
-// The steps weigh against the launches, so T counts: fp32 L 12 B 250 H 128 at T 64 422, 309, at T 16 123, 157.
+// T 128 B 256 H 256 1120, 782; L 31 T 40 B 20 H 256 333, 256; L 20 T 50 B 100 H 128 316, 261; fp16 L 12 T 30 B 142 H 256
+// 275, 190; the other way round at fp32 L 4 T 30 B 128 H 512 233, 336; L 23 T 17 B 253 H 256 (twelve launches) 699, 986; fp16 L 15 T 25 B 107
+// H 512 423, 484; L 3 T 74 B 41 H 1024 497, 607.  `plain`: neither a ragged batch nor a dilation; those take the general loop,
+// which is no faster with blocks of 16 (ragged L 32 T 48 B 96 H 128 280, 374; dilated L 6 T 100 B 256 H 128 230, 262).
+// The steps weigh against the launches, so T counts: fp32 L 12 B 250 H 128 at T 64 424, 310, at T 16 123, 156.  Near the line, with
+// ordinary launches and with cooperative ones: L 18 T 18 B 216 H 256 622, 704 and 643, 862; L 6 T 92 B 114 H 512 1257, 1236 and 1272, 1343.
+// Over 700 other stacks near the line, ordinary and cooperative: 8 and 4 % faster in the mean than 32-row blocks throughout, more than 2 %
+// slower in 7 and 37 (15 and 19 % at the most: H 128, where a stack that was run before finds its weights in L2).
 int exchange_layers(int L, int T, int B, int H, bool half, bool plain, bool* many) {
   const ExchangeFlavour f = exchange_flavour_of(H, half);
   *many = false;
@@ -1099,20 +1111,19 @@ int exchange_layers(int L, int T, int B, int H, bool half, bool plain, bool* man
   *many = true;
   const DeviceProps* dp = nullptr;
   if (!plain || one == 0 || device_props(&dp) != FTK_OK) return more;
-  const ExchangeCost cost = exchange_cost(H, half);
-  auto per_cu = [&](long long groups, int most) { return (int)std::min<long long>((groups + dp->cus - 1) / dp->cus, most); };
   const int launches = (L + one - 1) / one, even = (L + launches - 1) / launches;
-  const int held = per_cu((long long)even * ((B + 15) / 16) * (H / exchange_units(H, half, false)), 4);
-  const float step_one = launches * cost.one[held - 1];
-  const float rest_one = launches * held * cost.one_launch + (L - launches) * cost.one_layer;
-  float step_many = 0, rest_many = 0;
+  auto launch_us = [&](const ExchangeCost& c, bool first, int layers, int slices, int blocks, int team) {
+    return kLaunchMore + (first ? c.first : c.next) + (layers - 1) * c.layer + T * blocks * (c.step + c.fill * layers * slices * team / dp->cus);
+  };
+  const ExchangeCost c16 = exchange_cost(H, half, false), c32 = exchange_cost(H, half, true);
+  float us = 0;   // of 16-row blocks minus of 32-row blocks
+  for (int l0 = 0; l0 < L; l0 += even)
+    us += launch_us(c16, l0 == 0, std::min(even, L - l0), (B + 15) / 16, 1, H / exchange_units(H, half, false));
   for (int l0 = 0; l0 < L; l0 += more) {
     const ExchangePlan p = exchange_plan(std::min(more, L - l0), W, nrb, slots);
-    const int blocks = (nrb + p.slices - 1) / p.slices;
-    step_many += blocks * cost.many[per_cu((long long)p.layers * p.slices * W, 2) - 1];
-    rest_many += cost.many_launch + (p.layers - 1) * cost.many_layer;
+    us -= launch_us(c32, l0 == 0, p.layers, p.slices, (nrb + p.slices - 1) / p.slices, W);
   }
-  if (T * step_one + rest_one > 0.95f * (T * step_many + rest_many)) return more;
+  if (us >= 0) return more;
   *many = false;
   return even;
 }

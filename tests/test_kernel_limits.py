@@ -218,3 +218,23 @@ def test_flash_attention_f32_on_a_workspace_of_planes_only(core, B, Hd, Sq, Skv,
                 end.synchronize()
                 best[i] = min(best[i], start.elapsed_time(end))
         assert best[0] <= 1.25 * best[1], best
+
+
+@pytest.mark.parametrize('H,L,T,B,blocks', [
+    (256, 18, 18, 216, 32),      # 16 rows 704, 862; 32 rows 622, 643
+    (256, 23, 17, 253, 32),      # 986, 1197; 699, 717
+    (512, 6, 92, 114, 32),       # 1236, 1343; 1257, 1272
+    (256, 6, 128, 256, 16),      # 782, 834; 1120, 1137
+    (256, 31, 40, 20, 16),       # 256, 291; 333, 352
+    (512, 5, 119, 98, 16),       # 1293, 1384; 1481, 1501
+])
+def test_row_blocks_that_take_more_launches_pay_for_them(core, H, L, T, B, blocks):
+    """Both sides of the line between launches of 16-row blocks and fewer launches of 32-row blocks (beside the stacks: us of either
+    with ordinary launches and with cooperative ones).  A ragged call takes 32-row blocks for these stacks: a dense call has its
+    bits exactly if it takes them too."""
+    gen = torch.Generator(device='cuda').manual_seed(21)
+    xs = torch.randn((T, B, H), generator=gen, device='cuda')
+    WU = (torch.rand((L, 2 * H, 4 * H), generator=gen, device='cuda') * 2 - 1) * H ** -0.5
+    dense, ragged = core.stacked_lstm(xs, WU, check=True), core.stacked_lstm(xs, WU, active_rows=[B] * T, check=True)
+    same = all(torch.equal(a, b) for a, b in zip(dense, ragged))
+    assert same == (blocks == 32)
