@@ -496,12 +496,23 @@ int ftk_flash_attn_ws_f16(const void* Q, const void* K, const void* V, void* O,
  * split operands with fp32 accumulation (a row of Q, all of K and all of V of
  * a (batch, head) each share a power-of-two scale), the softmax state is fp32:
  * results agree with a float64 evaluation to a few 1e-6 of the largest |O|.
- * Q, K, V, O 16-byte aligned.  Non-finite inputs give NaN.  The workspace (ftk_flash_attn_f32_workspace_bytes,
- * about the size of K and V together, 256-byte aligned) holds their split
- * planes (Q is split in the attention kernel's registers) and, where several
- * workgroups share a query block's keys, what each of them found; one or two
- * small launches precede the attention kernel.  The reference has no device kernel
- * for this program.
+ * Q, K, V, O 16-byte aligned.  Non-finite inputs give NaN.  The workspace
+ * (256-byte aligned) holds the split planes of K and V, 4*D*Skv bytes each per
+ * (batch, head) and so as many as K and V themselves (Q is split in the
+ * attention kernel's registers), 520 bytes per (batch, head) for their scales
+ * and, where several workgroups share a query block's keys, what each of them
+ * found: 512*D + 2048 bytes for every workgroup, of which there are no more
+ * than the device holds at once.  For few and long queries that is most of it
+ * (256 compute units: up to 18 MB; one head of 4096 queries and 1024 keys of
+ * D 64: 17.8 MB beside 0.5 MB of planes).
+ * ftk_flash_attn_f32_workspace_bytes says how much on the current device.
+ * The call runs on any workspace with room for the planes and 8 bytes per
+ * (batch, head), each rounded up to 256 bytes (the planes of K and of V
+ * separately), else FTK_ERR_WORKSPACE.  On less than the query asks for, a
+ * query block's keys are not shared: grids of few query blocks are slower,
+ * and the last bits of O differ (the sums are taken in another order).  One to
+ * three small launches precede the attention kernel.  The reference has no
+ * device kernel for this program.
  */
 size_t ftk_flash_attn_f32_workspace_bytes(int B, int Hd, int Sq, int Skv, int D);
 int ftk_flash_attn_f32(const float* Q, const float* K, const float* V, float* O,

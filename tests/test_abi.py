@@ -135,3 +135,14 @@ def test_f16_stack_workspace_is_that_of_the_kernels_the_shape_goes_to():
     size = core.lib.ftk_stacked_lstm_f16_workspace_bytes
     assert size(32, 64, 256, 1024) == 256 + 32 * 2048 * 4096 * 2
     assert 0 < size(32, 64, 256, 256) < 4 << 20
+
+
+def test_f32_attention_workspace_is_what_the_header_says():
+    """Planes, 520 bytes a head and, on a device, what the workgroups that share keys leave: 512 D + 2048 bytes each, no more of them
+    than two to a compute unit."""
+    import fractaltensor_amd._core as core
+    up = lambda n: (n + 255) // 256 * 256
+    for B, Hd, Sq, Skv, D in [(1, 1, 4096, 1024, 64), (2, 8, 1024, 1024, 32), (1, 4, 128, 65536, 128), (4, 16, 640, 640, 96), (1, 1, 1, 1, 32)]:
+        n = int(core.lib.ftk_flash_attn_f32_workspace_bytes(B, Hd, Sq, Skv, D))
+        without = up(8 * B * Hd) + up(512 * B * Hd) + 2 * up(4 * D * Skv * B * Hd)
+        assert without <= n <= without + 512 * (512 * D + 2048) + 512 * 4 + 512

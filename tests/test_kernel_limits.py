@@ -238,3 +238,9 @@ def test_row_blocks_that_take_more_launches_pay_for_them(core, H, L, T, B, block
     dense, ragged = core.stacked_lstm(xs, WU, check=True), core.stacked_lstm(xs, WU, active_rows=[B] * T, check=True)
     same = all(torch.equal(a, b) for a, b in zip(dense, ragged))
     assert same == (blocks == 32)
+
+
+def test_f32_attention_workspace_of_few_query_blocks(core):
+    """The shape whose workspace the header names: sixteen workgroups to a query block, 34 KB from each."""
+    n = int(core.lib.ftk_flash_attn_f32_workspace_bytes(1, 1, 4096, 1024, 64))
+    assert 17.8e6 <= n - 2 * 4 * 64 * 1024 <= 17.9e6
