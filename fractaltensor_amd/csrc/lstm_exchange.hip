@@ -613,7 +613,8 @@ void lstm_exchange_kernel(ExchangeArgs a) {
       c[u] = __builtin_fmaf(gate(p[1]), c_prev[u], gate(p[0]) * tanh_f(p[3]));
       h[u] = gate(p[2]) * tanh_f(c[u]);
       // rounded to 32 bits before 16 in every loop: one instruction may do both, with another last bit now and then, and
-      // a ragged batch, which takes another loop than a dense one, gives the same bits (with row blocks of the same kind)
+      // a ragged batch, which takes another loop than a dense one, gives the same bits (with row blocks of either kind: the sums
+      // of the two matrix instructions are the same)
       if constexpr (HALF) asm("" : "+v"(c[u]), "+v"(h[u]));
       unsigned word;
       if constexpr (HALF) {

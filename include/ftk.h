@@ -137,6 +137,20 @@ size_t ftk_stacked_lstm_workspace_bytes(int L, int T, int B, int H);
  * plus those of hsss; ftk_stacked_lstm_workspace_bytes says how much); with a
  * smaller workspace or in the fp32-product mode through the fp32-MFMA cell
  * kernel of ftk_lstm_cell_f32, which needs none.
+ *
+ * Bits (all stacked-LSTM entry points).  A call gives the same bits every
+ * time, whatever the process did before it, on whatever stream and in a
+ * capture.  Which kernel forms the sums, and for how many batch rows at a time,
+ * goes by L, T, B and H, by whether the call has active_rows or a dilation other
+ * than 1, and by whether the workspace is as large as the query says; where two
+ * calls differ in these, their results agree to rounding (fp32: a few 1e-7 of the
+ * largest |h|; fp16: its last bit, at every step and layer) and not bit for
+ * bit.  So a sequence and its first half may differ in the last bits, and so
+ * may a dense batch and the same batch with active_rows.  A caller that needs
+ * the bits of a row not to depend on where the sequence ends passes
+ * active_rows in both calls: T does not count in the choice then, at H = 64
+ * (fp32), 128 (fp32), 256, 512 and 1024 (fp16), as long as a layer's h takes
+ * less than 2 GiB.  The order of the batch rows never counts.
  * Replaces StackedLstmRegion1/2/3
  * (kaleido/core/device/kernels/lstm/stacked_lstm/region1.h:11-43,
  * region2.h:15-70, region3.h:18-140) and the Python stacked_lstm

@@ -244,3 +244,37 @@ def test_f32_attention_workspace_of_few_query_blocks(core):
     """The shape whose workspace the header names: sixteen workgroups to a query block, 34 KB from each."""
     n = int(core.lib.ftk_flash_attn_f32_workspace_bytes(1, 1, 4096, 1024, 64))
     assert 17.8e6 <= n - 2 * 4 * 64 * 1024 <= 17.9e6
+
+
+@pytest.mark.parametrize('half,H,L,B', [
+    (False, 64, 19, 219), (False, 128, 12, 250), (False, 256, 18, 216), (False, 256, 6, 256), (False, 256, 14, 256), (False, 512, 5, 98),
+    (True, 256, 12, 142), (True, 256, 32, 256), (True, 512, 9, 109), (True, 512, 20, 224), (True, 1024, 3, 41),
+])
+def test_a_sequence_and_its_beginning_have_the_same_bits_with_active_rows(core, half, H, L, B):
+    """Shapes whose dense calls change the kernel, or the blocks of rows, with T (or are near that): with active_rows given, none
+    does."""
+    T, first = 72, 17
+    gen = torch.Generator(device='cuda').manual_seed(23)
+    dtype = torch.float16 if half else torch.float32
+    xs = torch.randn((T, B, H), generator=gen, device='cuda').to(dtype)
+    WU = ((torch.rand((L, 2 * H, 4 * H), generator=gen, device='cuda') * 2 - 1) * H ** -0.5).to(dtype)
+    call = core.stacked_lstm_f16 if half else core.stacked_lstm
+    whole = call(xs, WU, active_rows=[B] * T, check=True)
+    part = call(xs[:first].contiguous(), WU, active_rows=[B] * first, check=True)
+    for a, b in zip(whole, part):
+        assert torch.equal(a[:, :first], b)
+    # and the order of the rows: reversed, a dense call gives the rows reversed
+    dense = call(xs, WU, check=True)
+    turned = call(xs.flip(1).contiguous(), WU, check=True)
+    for a, b in zip(dense, turned):
+        assert torch.equal(a, b.flip(2))
+
+
+@pytest.mark.parametrize('H,L,T,B', [(256, 12, 30, 142), (512, 9, 40, 109), (1024, 3, 30, 64), (512, 5, 40, 142)])
+def test_f16_row_blocks_of_either_kind_give_the_same_bits(core, H, L, T, B):
+    """fp16 data, one fp16 product each: the 16-row and the 32-row matrix instructions add in the same order, so that a dense
+    call and a ragged one have the same bits whichever blocks they take (fp32 data: three products, with other sums)."""
+    xs, WU = _f16_stack(L, T, B, H, 24)
+    dense = core.stacked_lstm_f16(xs, WU, check=True)
+    ragged = core.stacked_lstm_f16(xs, WU, active_rows=[B] * T, check=True)
+    assert all(torch.equal(a, b) for a, b in zip(dense, ragged))
