@@ -407,7 +407,13 @@ void lstm_exchange_kernel(ExchangeArgs a) {
   // The sums.  fp32 data, blocks of 16 rows: the products with a remainder have sums of their own (cross), added at the end;
   // every addition rounds, and two thirds of them are of terms 2^-11 the size.  It also makes eight chains of the matrix
   // instructions, which with four wait for each other (19.9 instead of 16 cycles each).
+  // Blocks of 32 rows have no registers for that.  Up to H 256 all of a share's products with a remainder go in front of the others,
+  // while the sum is small (the x half) or half of what it will be (the h half): the error of h and c against float64 is 4 to 8 % less
+  // than in the order of the k steps (H 256 L 32 T 64 B 250 rms of c 1.66e-7, 1.77e-7; L 6 T 64 B 100 dilated 1.89e-7, 2.04e-7) and no
+  // larger than with the two chains of the persistent kernel's serial schedule; the time is the same (2259 us at L 32 T 64 B 250).  At H 512 it
+  // takes a tenth more (L 8 T 100 B 64 725 -> 796 us): there the products stay in the order of the k steps.
   constexpr bool TWO = !HALF && !MANY;
+  constexpr bool RESTS_FIRST = !HALF && MANY && H <= 256;
   accum acc[NT], cross[TWO ? NT : 1];
   auto multiply = [](v8h w, v8h x, accum c) __attribute__((always_inline)) -> accum {
     if constexpr (RT == 1) return __builtin_amdgcn_mfma_f32_16x16x32_f16(w, x, c, 0, 0, 0);
@@ -431,7 +437,7 @@ void lstm_exchange_kernel(ExchangeArgs a) {
     } else {
 #pragma unroll
       for (int tt = 0; tt < NT; ++tt) acc[tt] = multiply(wt[w][tt], top, first ? zero : acc[tt]);
-      if constexpr (!HALF) {
+      if constexpr (!HALF && !RESTS_FIRST) {
 #pragma unroll
         for (int tt = 0; tt < NT; ++tt) acc[tt] = multiply(wt[w][tt], rest, acc[tt]);
 #pragma unroll
@@ -439,32 +445,53 @@ void lstm_exchange_kernel(ExchangeArgs a) {
       }
     }
   };
+  // the two products with a remainder alone (RESTS_FIRST)
+  auto rest_products = [&](auto wc, v8h top, v8h rest, auto first_c) __attribute__((always_inline)) {
+    constexpr int w = decltype(wc)::value;
+    accum zero;
+#pragma unroll
+    for (int r = 0; r < AR; ++r) zero[r] = 0.0f;
+#pragma unroll
+    for (int tt = 0; tt < NT; ++tt) acc[tt] = multiply(wt[w][tt], rest, decltype(first_c)::value ? zero : acc[tt]);
+#pragma unroll
+    for (int tt = 0; tt < NT; ++tt) acc[tt] = multiply(wo[w][tt], top, acc[tt]);
+  };
   // all of a share of an exchange tile; base: the first resident k step.  each(i): called when v's part for k step i has
   // been used, for memory operations that are due then
   auto share_products = [&](share& v, auto base_c, auto first_c, auto each) __attribute__((always_inline)) {
     constexpr int base = decltype(base_c)::value;
     constexpr bool first = decltype(first_c)::value;
+    auto top_of = [&](int i) __attribute__((always_inline)) {
+      const v4u p = v[2 * i], q = v[2 * i + 1];
+      const v4u top = {__builtin_amdgcn_perm(p[1], p[0], 0x05040100), __builtin_amdgcn_perm(p[3], p[2], 0x05040100),
+                       __builtin_amdgcn_perm(q[1], q[0], 0x05040100), __builtin_amdgcn_perm(q[3], q[2], 0x05040100)};
+      return __builtin_bit_cast(v8h, top);
+    };
+    auto rest_of = [&](int i) __attribute__((always_inline)) {
+      const v4u p = v[2 * i], q = v[2 * i + 1];
+      const v4u rest = {__builtin_amdgcn_perm(p[1], p[0], 0x07060302), __builtin_amdgcn_perm(p[3], p[2], 0x07060302),
+                        __builtin_amdgcn_perm(q[1], q[0], 0x07060302), __builtin_amdgcn_perm(q[3], q[2], 0x07060302)};
+      return __builtin_bit_cast(v8h, rest);
+    };
+    if constexpr (RESTS_FIRST) {
+      static_for<XS>([&](auto ic) __attribute__((always_inline)) {
+        constexpr int i = decltype(ic)::value;
+        rest_products(std::integral_constant<int, base + i>{}, top_of(i), rest_of(i), std::integral_constant<bool, first && i == 0>{});
+        __builtin_amdgcn_sched_barrier(0x6);
+      });
+    }
     static_for<XS>([&](auto ic) __attribute__((always_inline)) {
       constexpr int i = decltype(ic)::value;
-      constexpr std::integral_constant<bool, first && i == 0> start{};
+      constexpr std::integral_constant<bool, first && i == 0 && !RESTS_FIRST> start{};
       if constexpr (HALF) {
         products(std::integral_constant<int, base + i>{}, __builtin_bit_cast(v8h, v[i]), v8h{}, start);
         each(ic);
         __builtin_amdgcn_sched_barrier(0x6);   // vector and scalar instructions may pass, the loads stay between the products
       } else {
-        const v4u p = v[2 * i], q = v[2 * i + 1];
-        v4u top, rest;
-        top[0] = __builtin_amdgcn_perm(p[1], p[0], 0x05040100);
-        top[1] = __builtin_amdgcn_perm(p[3], p[2], 0x05040100);
-        top[2] = __builtin_amdgcn_perm(q[1], q[0], 0x05040100);
-        top[3] = __builtin_amdgcn_perm(q[3], q[2], 0x05040100);
-        rest[0] = __builtin_amdgcn_perm(p[1], p[0], 0x07060302);
-        rest[1] = __builtin_amdgcn_perm(p[3], p[2], 0x07060302);
-        rest[2] = __builtin_amdgcn_perm(q[1], q[0], 0x07060302);
-        rest[3] = __builtin_amdgcn_perm(q[3], q[2], 0x07060302);
+        const v8h top = top_of(i), rest = rest_of(i);
         each(ic);
         __builtin_amdgcn_sched_barrier(0x6);   // vector and scalar instructions may pass, the loads stay between the products
-        products(std::integral_constant<int, base + i>{}, __builtin_bit_cast(v8h, top), __builtin_bit_cast(v8h, rest), start);
+        products(std::integral_constant<int, base + i>{}, top, rest, start);
       }
     });
   };
