@@ -718,10 +718,13 @@ static F32Split f32_split(long long BH, int Sq, int Skv, int D, int cus) {
   const int tiles = (Skv + FA_KT - 1) / FA_KT;
   F32Split best = {4, 1, 1};
   if ((long long)((Sq + 127) / 128) * BH > 2 * cus) return best;
-  // Time in tenths of what a wave that shares its SIMD needs for a tile (1.05, 2, 2.5, 3 us by head size).  Two waves of a SIMD hardly
-  // overlap, so what counts is the tiles that a SIMD works through; one that has only one wave takes a fifth longer.  What
-  // parts leave in the workspace and the last one takes in costs 4.5 us at head size 32 and 8 at 128.
-  const int merge = D == 32 ? 45 : 35;
+  // Time in tenths of what a wave that shares its SIMD needs for a tile (1.05, 1.35, 1.7, 1.9 us by head size).  Two waves of a SIMD
+  // hardly overlap, so what counts is the tiles that a SIMD works through; one that has only one wave takes a fifth longer.  What
+  // parts leave in the workspace and the last one takes in costs 1.4, 1.6, 2.2, 2.6 us and 0.55, 0.7, 0.85, 1.05 us a part: as much as
+  // 35 tenths with four to six parts, at every head size.  Over 580 grids of 1 to 64 heads, 32 to 4096 queries and 128 to 8192
+  // keys the split chosen takes 2.5, 3.3, 0.7 and 1.6 % longer in the mean than the best one of all for the grid, a quarter at the most; 25
+  // tenths serve as well, with 20 or 50 it is up to 1 % more.
+  const int merge = 35;
   auto workgroups = [&](const F32Split& f) { return (long long)((Sq + 32 * f.waves - 1) / (32 * f.waves)) * BH * f.parts; };
   auto cost = [&](const F32Split& f) {
     const long long per_simd = std::max(1LL, (workgroups(f) + cus - 1) / cus * f.groups * f.waves / 4);
