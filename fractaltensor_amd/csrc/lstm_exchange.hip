@@ -905,7 +905,7 @@ void lstm_exchange_kernel(ExchangeArgs a) {
     if (l == 0) walk(std::true_type{}, way_c);
     else walk(std::false_type{}, way_c);
   };
-  // One store instead of two wherever a team sits on one XCD (L 8 T 100 B 64 H 512 755 -> 730 us; fp32 at H 256 has no
+  // One store instead of two wherever a team sits on one XCD (L 8 T 100 B 64 H 512 747 -> 732 us; fp32 at H 256 has no
   // register left: with three copies of the loop it spills in the loop, 1070 -> 1190 us at L 16 T 114 B 104).
   if constexpr (MANY && (HALF || CT == 1)) {
     if (team_here && hand_plain) return walk_layer(std::integral_constant<int, kPlain>{});

@@ -1510,7 +1510,8 @@ def test_stacks_of_hidden_size_256_on_either_kernel(core, half, L, T, B, dil):
     (False, 256, 6, 33, 250),              # three launches of two layers, the last row block of ten rows
     (False, 256, 13, 70, 101),             # the last launch of one layer
     (False, 256, 31, 4, 17),               # sixteen and fifteen layers, a row block of one row
-    (True, 256, 7, 5, 142),                # four and three layers
+    (True, 256, 7, 5, 142),                # as many layers as one launch holds
+    (True, 256, 13, 12, 142),              # seven and six layers
 ])
 def test_stack_in_more_launches_of_16_row_blocks(core, half, H, L, T, B):
     """Dense stacks that a launch of 32-row blocks would hold more layers of: against the oracle, the same bits in every
