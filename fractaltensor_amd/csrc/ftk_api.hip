@@ -84,27 +84,44 @@ struct HipStreams {
     return FTK_OK;
   }
 };
-}  // namespace
 
-int launch_resident(const void* fn, dim3 grid, dim3 block, void** args, size_t lds, hipStream_t s) {
-  constexpr int kDev = 16;
-  static LaunchOrder<hipStream_t> devices[kDev];
-  static std::mutex mu;
-  static const bool always = [] {
+// The launch orders of all devices.
+struct Launches {
+  static constexpr int kDev = 16;
+  LaunchOrder<hipStream_t> devices[kDev];
+  std::mutex mu;
+  const bool always = [] {
     const char* e = getenv("FTK_COOPERATIVE_LAUNCH");
     return e && e[0] == '1';
   }();
+};
+Launches& launches() {
+  static Launches all;
+  return all;
+}
+}  // namespace
+
+int launch_resident(const void* fn, dim3 grid, dim3 block, void** args, size_t lds, hipStream_t s) {
+  Launches& all = launches();
   int dev = 0;
   FTK_HIP(hipGetDevice(&dev));
-  std::lock_guard<std::mutex> lock(mu);   // held over the launch: the streams have them in the order decided here
+  std::lock_guard<std::mutex> lock(all.mu);   // held over the launch: the streams have them in the order decided here
   bool cooperative = true;
-  if (!always && dev >= 0 && dev < kDev) {
-    const int rc = devices[dev].next(HipStreams(), s, s == hipStreamPerThread, &cooperative);
+  if (!all.always && dev >= 0 && dev < Launches::kDev) {
+    const int rc = all.devices[dev].next(HipStreams(), s, s == hipStreamPerThread, &cooperative);
     if (rc) return rc;
   }
   if (cooperative) FTK_HIP(hipLaunchCooperativeKernel(fn, grid, block, args, (unsigned)lds, s));
   else FTK_HIP(hipLaunchKernel(fn, grid, block, args, lds, s));
   return FTK_OK;
+}
+
+bool launch_is_cooperative(hipStream_t s) {
+  Launches& all = launches();
+  int dev = 0;
+  if (all.always || hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= Launches::kDev) return true;
+  std::lock_guard<std::mutex> lock(all.mu);
+  return all.devices[dev].cooperative(HipStreams(), s, s == hipStreamPerThread);
 }
 
 }  // namespace ftk

@@ -103,6 +103,8 @@ int device_props(const DeviceProps** out);
 // Launches a kernel whose workgroups wait for each other: `grid` is at most what the device holds at once.  As an
 // ordinary launch while that is enough, as a cooperative one otherwise (see ftk_api.hip).
 int launch_resident(const void* fn, dim3 grid, dim3 block, void** args, size_t lds, hipStream_t s);
+// Whether that is going to be a cooperative launch, as far as can be told before it is made.
+bool launch_is_cooperative(hipStream_t s);
 
 // ---- vector types for MFMA operands ----------------------------------------
 typedef float v4f __attribute__((ext_vector_type(4)));

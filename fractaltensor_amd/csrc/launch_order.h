@@ -52,6 +52,13 @@ class LaunchOrder {
     return 0;
   }
 
+  // Whether a launch on s is going to be cooperative, as far as can be told without making it: the first one on a second stream
+  // may still turn out to be.
+  template <typename Runtime>
+  bool cooperative(Runtime&& rt, Stream s, bool every_thread) const {
+    return cooperative_ || every_thread || rt.capturing(s);
+  }
+
  private:
   bool cooperative_ = false;   // from the second stream on
   bool pending_ = false;       // ordinary launches on last_ may still run, and no cooperative launch has been put behind them

@@ -1111,10 +1111,12 @@ ExchangeCost exchange_cost(int H, bool half, bool many) {
 }
 
 // A launch is an ordinary one or, once a process uses a second stream or records graphs, a cooperative one, which takes 16 to 18 us more
-// (launch_resident).  Which it is depends on what the process did before, and what a call computes must not, so a launch more is
-// charged most of the difference always.  Loss against the better kind of each, mean over 2940 stacks near the line with ordinary launches
-// and 1900 with cooperative ones: 0.4 and 1.5 % with nothing charged, 0.8 and 0.5 % with 12 us, 1.2 and 0.4 % with 17.
-constexpr float kLaunchMore = 12.0f;
+// (launch_resident).  Which it is depends on what the process did before.  With fp16 data both kinds of block give the same bits
+// (the sums of the two matrix instructions are the same), and a launch is charged what it is going to take.  With fp32 data they
+// do not, and what a call computes must not go by that: a launch more is charged most of the difference always.  Loss against the better
+// kind of each, mean over 2940 stacks near the line with ordinary launches and 1900 with cooperative ones: 0.4 and 1.5 % with nothing
+// charged, 0.8 and 0.5 % with 12 us, 1.2 and 0.4 % with 17.
+constexpr float kAnyLaunch = 12.0f, kCooperativeLaunch = 17.0f;
 
 // Layers of one launch (0: the device cannot hold one), and the kind of row block.  16 rows and one block per workgroup, whose
 // step is the shorter one, wherever that takes no more launches (L 23 T 67 B 10 fp32 H 512, three launches of either kind: 831 us
@@ -1127,8 +1129,9 @@ constexpr float kLaunchMore = 12.0f;
 // The steps weigh against the launches, so T counts: fp32 L 12 B 250 H 128 at T 64 424, 310, at T 16 123, 156.  Near the line, with
 // ordinary launches and with cooperative ones: L 18 T 18 B 216 H 256 622, 704 and 643, 862; L 6 T 92 B 114 H 512 1257, 1236 and 1272, 1343.
 // Over 700 other stacks near the line, ordinary and cooperative: 8 and 4 % faster in the mean than 32-row blocks throughout, more than 2 %
-// slower in 7 and 37 (15 and 19 % at the most: H 128, where a stack that was run before finds its weights in L2).
-int exchange_layers(int L, int T, int B, int H, bool half, bool plain, bool* many) {
+// slower in 9 and 36 (13 and 20 % at the most: H 64 and 128, where a stack that was run before finds its weights in L2).
+// each_launch: us that every launch is charged beyond its cost.
+int exchange_layers(int L, int T, int B, int H, bool half, bool plain, float each_launch, bool* many) {
   const ExchangeFlavour f = exchange_flavour_of(H, half);
   *many = false;
   if (!f.one) return 0;
@@ -1141,7 +1144,7 @@ int exchange_layers(int L, int T, int B, int H, bool half, bool plain, bool* man
   if (!plain || one == 0 || device_props(&dp) != FTK_OK) return more;
   const int launches = (L + one - 1) / one, even = (L + launches - 1) / launches;
   auto launch_us = [&](const ExchangeCost& c, bool first, int layers, int slices, int blocks, int team) {
-    return kLaunchMore + (first ? c.first : c.next) + (layers - 1) * c.layer + T * blocks * (c.step + c.fill * layers * slices * team / dp->cus);
+    return each_launch + (first ? c.first : c.next) + (layers - 1) * c.layer + T * blocks * (c.step + c.fill * layers * slices * team / dp->cus);
   };
   const ExchangeCost c16 = exchange_cost(H, half, false), c32 = exchange_cost(H, half, true);
   float us = 0;   // of 16-row blocks minus of 32-row blocks
@@ -1169,10 +1172,11 @@ int exchange_blocks(int L, int B, int H, bool half) {
   return p.layers ? (nrb + p.slices - 1) / p.slices : 0;
 }
 
-// Bytes of workspace that run_exchange uses on the current device; without a device, what it could at most.
+// Bytes of workspace that run_exchange uses on the current device, however it launches; without a device, what it could at most.
 size_t exchange_need(int L, int T, int B, int H, bool half) {
   bool many;
-  const int most = std::max(exchange_layers(L, T, B, H, half, true, &many), exchange_layers(L, T, B, H, half, false, &many));
+  int most = exchange_layers(L, T, B, H, half, false, kAnyLaunch, &many);
+  for (const float each_launch : {0.0f, kAnyLaunch, kCooperativeLaunch}) most = std::max(most, exchange_layers(L, T, B, H, half, true, each_launch, &many));
   return exchange_workspace_bytes(most ? std::min(L, most) : L, T, B, H, half);
 }
 
@@ -1187,7 +1191,7 @@ int run_exchange(bool half, const void* xs, const void* WU, const float* bias, c
   bool plain = !active;
   for (int l = 0; dil && l < L; ++l) plain = plain && dil[l] == 1;
   bool many;
-  const int most = exchange_layers(L, T, B, H, half, plain, &many);
+  const int most = exchange_layers(L, T, B, H, half, plain, !half ? kAnyLaunch : launch_is_cooperative(s) ? kCooperativeLaunch : 0.0f, &many);
   if (most == 0) return FTK_OK;
   const int slots = exchange_slots(many ? f.many : f.one), block = many ? 32 : 16, nrb = (B + block - 1) / block;
   const int W = H / exchange_units(H, half, many);

@@ -33,6 +33,12 @@ struct Device {
     if (order.next(rt, s, every_thread, &cooperative)) return "error";
     return rt.log + (cooperative ? "c" : "o");
   }
+  // what it says the next one will be, without asking for anything else
+  std::string ahead(int s, bool every_thread = false) {
+    rt.log.clear();
+    const bool cooperative = order.cooperative(rt, s, every_thread);
+    return rt.log + (cooperative ? "c" : "o");
+  }
 };
 
 static int failures = 0;
@@ -94,6 +100,18 @@ int main() {
     d.rt.streams[1] = StreamState::kBusy;
     expect("a handle per thread is put behind", d.launch(9, true), "9>1 c");
     expect("and leaves no ordinary launch after it", d.launch(1), "c");
+  }
+  {
+    Device d;
+    expect("told ahead: the first", d.ahead(1), "o");
+    d.launch(1);
+    d.rt.streams[2] = StreamState::kCapturing;
+    expect("told ahead: one stream", d.ahead(1), "o");
+    expect("told ahead: a handle per thread", d.ahead(9, true), "c");
+    expect("told ahead: a recording", d.ahead(2), "c");
+    expect("and none of it decides anything", d.launch(1), "o");
+    d.launch(2);
+    expect("told ahead: after a recording", d.ahead(1), "c");
   }
   return failures ? 1 : 0;
 }
