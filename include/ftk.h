@@ -127,20 +127,24 @@ size_t ftk_stacked_lstm_workspace_bytes(int L, int T, int B, int H);
  * L stacked LSTM layers over T steps; layer l reads layer l-1's hidden
  * sequence; zero initial state.  xs [T,B,H], WU [L,2H,4H], bias [L,4H] or
  * NULL, outputs hsss/csss [L,T,B,H] (every layer's h and c at every step).
- * H%32==0.  At H = 256 one persistent launch walks the (layer,time) wavefront
- * with each layer's weights held in registers.  Other hidden sizes do not fit
- * on chip and run as one fused-cell launch per wavefront diagonal with the
- * weights streamed: in the default product mode (see ftk_lstm_set_products)
- * through the fp16-MFMA kernel on operands split into two fp16 planes, for
- * which the workspace holds the planes of xs and of every h, the column
- * scales and a re-laid copy of the split weights (about 1.5x the bytes of WU
- * plus those of hsss; ftk_stacked_lstm_workspace_bytes says how much); with a
- * smaller workspace or in the fp32-product mode through the fp32-MFMA cell
- * kernel of ftk_lstm_cell_f32, which needs none.
+ * H%32==0.  In the default product mode (see ftk_lstm_set_products) and with
+ * the workspace the size query asks for, H = 64, 128, 256 and 512 keep the
+ * weights of as many layers on the chip as it holds, and deeper stacks run as
+ * consecutive launches, each reading the hidden sequence of the layer below.
+ * At H = 256 that is either of two kernels, and one of them also runs with
+ * fp32 products and with less workspace.  Every other call runs as one
+ * fused-cell launch per wavefront diagonal with the weights streamed: in the
+ * default product mode through the fp16-MFMA kernel on operands split into two
+ * fp16 planes, for which the workspace holds the planes of xs and of every h,
+ * the column scales and a re-laid copy of the split weights (about 1.5x the
+ * bytes of WU plus those of hsss); with a smaller workspace or in the
+ * fp32-product mode through the fp32-MFMA cell kernel of ftk_lstm_cell_f32,
+ * which needs none.  ftk_stacked_lstm_workspace_bytes says how much is enough
+ * for any of them.
  *
  * Bits (all stacked-LSTM entry points).  A call gives the same bits every
- * time, whatever the process did before it, on whatever stream and in a
- * capture.  Which kernel forms the sums, and for how many batch rows at a time,
+ * time, whatever the process did before it and on whatever stream.
+ * Which kernel forms the sums, and for how many batch rows at a time,
  * goes by L, T, B and H, by whether the call has active_rows or a dilation other
  * than 1, and by whether the workspace is as large as the query says; where two
  * calls differ in these, their results agree to rounding (fp32: a few 1e-7 of the
@@ -180,10 +184,9 @@ int ftk_dilated_lstm_f32(const float* xs, const float* WU, const float* bias,
  * each in [0,B]) = how many leading rows are still running at step t.  xs is
  * the dense [T,B,H] array with anything finite (zeros) in the dead places;
  * hsss/csss are written for the live (t, row) pairs, what the other places
- * hold afterwards is unspecified.  32-row blocks that have ended are skipped
- * by the persistent kernel; the streamed stacks of the other hidden sizes
- * compute the live rows of every step only; the fp32-MFMA fallback computes
- * everything.
+ * hold afterwards is unspecified.  Blocks of 16 or 32 rows that have ended are
+ * skipped where the weights are on the chip; the streamed stacks compute the
+ * live rows of every step only; the fp32-MFMA fallback computes everything.
  * dilations: host array or NULL (all 1).  Replaces the shrinking batch of
  * batched_cell (examples/stacked_rnn/stacked_rnn.py:45-51, hs_prev[0:xs.length])
  * over the layout of gen_dataset_time_major (examples/utils/data_utils.py:42-66).
