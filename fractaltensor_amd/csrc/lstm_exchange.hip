@@ -914,29 +914,38 @@ void lstm_exchange_kernel(ExchangeArgs a) {
   walk_layer(std::integral_constant<int, kAnyWay>{});
 }
 
-// In front of the kernel above: status block, places, the ring and the first two steps of `hand` (blockIdx.y < layers), and
-// the input rows as tiles (blockIdx.y == layers; one wave per row, rows past the batch are zeros).  fp32 rows are cut
-// under a power-of-two scale of their own.
+// In front of the kernel above, by workgroup: the input rows as tiles (the first row_groups of them; one wave per row, rows past
+// the batch are zeros; fp32 rows are cut under a power-of-two scale of their own), then the ring and the first two steps of
+// `hand`, kPrepareFill words of 16 bytes of a layer to a workgroup; the first of these has the status block and the places too.
+// Bound by its launch: with a grid of rows x (layers + 1) most of its workgroups had nothing to do, and dealing them out took
+// longer than the work (L 20 T 30 B 32 H 128, 5040 workgroups, 5.1 us; L 8 T 100 B 64 H 512, 9216, 14.7).
+constexpr int kPrepareFill = 1024;
 template <bool HALF>
 __global__ __launch_bounds__(256) void lstm_exchange_prepare_kernel(int* status, int first_word, int* place, int nplaces, v4u* ring,
-                                                                    size_t ring_per_layer, v4u* hand, size_t hand_per_layer,
-                                                                    size_t hand_first, const void* xs, float* xratio, int layers,
+                                                                    unsigned ring_per_layer, v4u* hand, size_t hand_per_layer,
+                                                                    unsigned hand_first, const void* xs, float* xratio, int row_groups,
                                                                     int T, int B, int nrb, int block, int H) {
-  const size_t at = (size_t)blockIdx.x * 256 + threadIdx.x, step = (size_t)gridDim.x * 256;
-  const int l = blockIdx.y;
-  if (l < layers) {
+  if ((int)blockIdx.x >= row_groups) {
+    const int g = (int)blockIdx.x - row_groups;
+    const unsigned of_layer = ring_per_layer + hand_first, groups = (of_layer + kPrepareFill - 1) / kPrepareFill;
+    const unsigned l = (unsigned)g / groups, first = ((unsigned)g - l * groups) * kPrepareFill + threadIdx.x;
     const v4u ones = {~0u, ~0u, ~0u, ~0u};
-    for (size_t i = at; i < ring_per_layer; i += step) ring[l * ring_per_layer + i] = ones;
-    for (size_t i = at; i < hand_first; i += step) hand[(l + 1) * hand_per_layer + i] = ones;
-    if (l == 0) {
-      for (size_t i = at; i < (size_t)nplaces; i += step) place[i] = 0;
-      if (at < kStatusBytes / sizeof(int) && (int)at >= first_word) status[at] = 0;
+    v4u* const ring_l = ring + (size_t)l * ring_per_layer;
+    v4u* const hand_l = hand + (size_t)(l + 1) * hand_per_layer;
+#pragma unroll
+    for (int n = 0; n < kPrepareFill / 256; ++n) {
+      const unsigned i = first + 256 * n;
+      if (i < of_layer) *(i < ring_per_layer ? ring_l + i : hand_l + (i - ring_per_layer)) = ones;
+    }
+    if (g == 0) {
+      for (int i = threadIdx.x; i < nplaces; i += 256) place[i] = 0;
+      if (threadIdx.x < kStatusBytes / sizeof(int) && (int)threadIdx.x >= first_word) status[threadIdx.x] = 0;
     }
     return;
   }
   const int lane = threadIdx.x & 63;
   const int per_step = nrb * block, rows = T * per_step;   // block: rows of a row block
-  for (int r = blockIdx.x * 4 + (threadIdx.x >> 6); r < rows; r += gridDim.x * 4) {
+  for (int r = blockIdx.x * 4 + (threadIdx.x >> 6); r < rows; r += row_groups * 4) {
     const int t = r / per_step, b = r - t * per_step;
     unsigned char* dst = reinterpret_cast<unsigned char*>(hand) + (size_t)(r / block) * exchange_tile_bytes(H, HALF, block) + (r % block) * 16;
     const size_t src = ((size_t)t * B + b) * H;
@@ -1227,16 +1236,13 @@ int run_exchange(bool half, const void* xs, const void* WU, const float* bias, c
     }
     const int groups = a.units * W;
     const unsigned grid = p.per_xcd ? 8u * p.per_xcd * W : (unsigned)((groups + 7) / 8 * 8);
-    const size_t ring_per_layer = (size_t)nrb * kXRing * tile / 16, hand_per_layer = (size_t)T * nrb * tile / 16;
-    const size_t hand_first = (size_t)std::min(T, 2) * nrb * tile / 16;
-    const size_t px = std::max({(ring_per_layer + 1023) / 1024, (hand_first + 1023) / 1024, ((size_t)T * nrb * block + 3) / 4});
-    const dim3 pgrid((unsigned)std::min<size_t>(px, 1024), lc + 1);
-    if (half)
-      hipLaunchKernelGGL(lstm_exchange_prepare_kernel<true>, pgrid, dim3(256), 0, s, a.status, l0 > 0 ? 2 : 0, a.place, groups,
-                         (v4u*)a.ring, ring_per_layer, (v4u*)a.hand, hand_per_layer, hand_first, x, xratio, lc, T, B, nrb, block, H);
-    else
-      hipLaunchKernelGGL(lstm_exchange_prepare_kernel<false>, pgrid, dim3(256), 0, s, a.status, l0 > 0 ? 2 : 0, a.place, groups,
-                         (v4u*)a.ring, ring_per_layer, (v4u*)a.hand, hand_per_layer, hand_first, x, xratio, lc, T, B, nrb, block, H);
+    const unsigned ring_per_layer = (unsigned)((size_t)nrb * kXRing * tile / 16), hand_first = (unsigned)((size_t)std::min(T, 2) * nrb * tile / 16);
+    const size_t hand_per_layer = (size_t)T * nrb * tile / 16;
+    const int row_groups = (int)std::min<size_t>(((size_t)T * nrb * block + 3) / 4, 2048);
+    const dim3 pgrid(row_groups + lc * ((ring_per_layer + hand_first + kPrepareFill - 1) / kPrepareFill));
+    auto prepare = half ? lstm_exchange_prepare_kernel<true> : lstm_exchange_prepare_kernel<false>;
+    hipLaunchKernelGGL(prepare, pgrid, dim3(256), 0, s, a.status, l0 > 0 ? 2 : 0, a.place, groups, (v4u*)a.ring, ring_per_layer, (v4u*)a.hand,
+                       hand_per_layer, hand_first, x, xratio, row_groups, T, B, nrb, block, H);
     int rc = check_launch("lstm_exchange_prepare_kernel");
     if (rc) return rc;
     void* kargs[] = {&a};
