@@ -13,7 +13,7 @@
 // what a sum of products is accurate to anyway: 22 significant bits of its own are kept by every element within
 // 2^-17 of the largest.
 //
-// Launches: the largest |K| and |V| per (batch, head) and the split of K and V into planes [row][top D | rest D] in the
+// Launches, where the attention kernel does not cut K and V itself (DIRECT): the largest |K| and |V| per (batch, head) and the split of K and V into planes [row][top D | rest D] in the
 // workspace, in one launch where heads are small, else in two; the attention kernel, which splits its rows of Q (times scale * log2 e)
 // itself, in registers.  A plane row is an fp16 row of 2 D
 // elements, so tiles, copies and fragment reads are those of the fp16 kernel at twice the head dimension
@@ -44,6 +44,8 @@ __device__ __forceinline__ void split_scale(unsigned max_bits, float* scale, flo
   *scale = __uint_as_float((unsigned)(127 + kF32Top + 127 - eb) << 23);
   *inv = __uint_as_float((unsigned)(eb - kF32Top) << 23);
 }
+
+__device__ __forceinline__ int clamped_eb(int eb) { return min(max(eb, 15), 254 - kF32Top); }   // the exponent field that split_scale goes by
 
 // The two launches of larger heads: largest |x| of every chunk of every (batch, head) of K and V, as float bits (which order like
 // the magnitudes), grid (chunks, BH, 2), per_bh a multiple of 4; then the planes, whose workgroups take the largest of a head's chunks.
@@ -160,6 +162,10 @@ __global__ __launch_bounds__(kPlanesThreads) void attn_f32_planes_kernel(const f
 // Bytes a part of a block of 128 query rows leaves in the workspace.
 constexpr int f32_partial_bytes(int D) { return 128 * D * 4 + 4 * 64 * 8; }
 
+// DIRECT: Kp and Vp are K and V themselves, no launch in front.  Each workgroup cuts a tile's fp32 rows into their planes on the way to LDS
+// (they are as long as the planes), K under a scale of the tile's own, V under that of the largest value of the group's tiles so
+// far: no magnitude of a whole head is needed first, and no element has fewer bits than under its head's scale.  Every query block pays for
+// it again: f32_split has the line.  The error against float64 is that of the other form, also with keys that differ by 2^20.
 // 4 waves x 32 query rows per workgroup.  Two workgroups to a compute unit at head sizes up to 64 (B 4, 16 heads, 1024 keys of 64: 88
 // -> 77 us with a bound of 256 registers, of which the compiler had taken a few more), one above: the accumulators of O,
 // both planes of Q and the scores take some 400 registers at D = 128.  K and V tiles of 64 keys, both double buffered.  A wave
@@ -179,9 +185,10 @@ struct FaFourGroups : FaLayout<64> {
 };
 template <int D, int KG> using F32Tiles = typename std::conditional<KG == 4, FaFourGroups, FaLayout<2 * D>>::type;
 
-template <int D, int KG, int WAVES, bool PART>
-__global__ __launch_bounds__(KG * WAVES * 64, KG == 1 && D <= 64 ? 2 : 1) void flash_attn_f32_kernel(const float* __restrict__ Q, const _Float16* __restrict__ Kp,
-                                                                const _Float16* __restrict__ Vp, float q_mul,
+template <int D, int KG, int WAVES, bool PART, bool DIRECT>
+__global__ __launch_bounds__(KG * WAVES * 64, KG == 1 && D <= 64 ? 2 : 1) void flash_attn_f32_kernel(const float* __restrict__ Q,
+                                                                const void* __restrict__ Kp,
+                                                                const void* __restrict__ Vp, float q_mul,
                                                                 const unsigned* __restrict__ kv_bits, float* __restrict__ O,
                                                                 int Sq, int Skv_whole, int nqb, int BH, int nparts,
                                                                 int* __restrict__ counters, unsigned char* __restrict__ partials) {
@@ -219,16 +226,116 @@ __global__ __launch_bounds__(KG * WAVES * 64, KG == 1 && D <= 64 ? 2 : 1) void f
   const int most_tiles = share + (long_groups > 0 ? 1 : 0);
   const int key_first = (group * share + min(group, long_groups)) * FA_KT;
   const int Skv = KG == 1 ? Skv_all : group + 1 < KG ? (share + (group < long_groups ? 1 : 0)) * FA_KT : Skv_all - key_first;   // the keys this group sees
-  const _Float16* Kg = Kp + ((size_t)bh * Skv_whole + key_part + key_first) * (2 * D);
-  const _Float16* Vg = Vp + ((size_t)bh * Skv_whole + key_part + key_first) * (2 * D);
+  // (a row of fp32 and its two planes are as long)
+  const _Float16* Kg = static_cast<const _Float16*>(Kp) + ((size_t)bh * Skv_whole + key_part + key_first) * (2 * D);
+  const _Float16* Vg = static_cast<const _Float16*>(Vp) + ((size_t)bh * Skv_whole + key_part + key_first) * (2 * D);
   float* Og = O + (size_t)bh * Sq * D;
+
+  // DIRECT: a tile's fp32 rows through registers, eight neighbouring floats of FN rows of K and of V to a lane.  Asked for a tile
+  // ahead; its largest magnitudes meet in LDS at the barrier in the middle of the tile before, behind which every wave cuts its
+  // rows into their planes in LDS.
+  constexpr int CPR8 = D / 8, FN = DIRECT ? D / (8 * WAVES) : 1;
+  __shared__ unsigned tile_max[DIRECT ? KG : 1][DIRECT ? WAVES : 1][2];
+  float4 fk[FN][2], fv[FN][2];
+  auto fetched = [&](auto i_c, int* row, int* c) __attribute__((always_inline)) {
+    const int x = 64 * (wave + WAVES * decltype(i_c)::value) + lane;
+    *row = x / CPR8;
+    *c = x - *row * CPR8;
+  };
+  [[maybe_unused]] auto fetch = [&](int kt) __attribute__((always_inline)) {
+    const int last = Skv - 1 - kt * FA_KT;   // rows past the end re-read the last key; their scores are masked
+    const float* const kb = reinterpret_cast<const float*>(Kg) + (size_t)kt * FA_KT * D;
+    const float* const vb = reinterpret_cast<const float*>(Vg) + (size_t)kt * FA_KT * D;
+    static_for<FN>([&](auto i_c) __attribute__((always_inline)) {
+      constexpr int i = decltype(i_c)::value;
+      int row, c;
+      fetched(i_c, &row, &c);
+      const unsigned at = (unsigned)(min(row, last) * D + 8 * c);
+      fk[i][0] = *reinterpret_cast<const float4*>(kb + at);
+      fk[i][1] = *reinterpret_cast<const float4*>(kb + at + 4);
+      fv[i][0] = *reinterpret_cast<const float4*>(vb + at);
+      fv[i][1] = *reinterpret_cast<const float4*>(vb + at + 4);
+    });
+  };
+  // the wave's largest magnitudes of the rows it fetched
+  [[maybe_unused]] auto publish_max = [&]() __attribute__((always_inline)) {
+    auto wave_max = [&](const float4 (&f)[FN][2]) __attribute__((always_inline)) -> unsigned {
+      float m = 0.0f;
+#pragma unroll
+      for (int i = 0; i < FN; ++i)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(m) : "v"(f[i][h].x), "v"(f[i][h].y));
+          asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(m) : "v"(f[i][h].z), "v"(f[i][h].w));
+        }
+      // within rows of 16 lanes, then over the four rows
+      unsigned b = __float_as_uint(m);
+      b = max(b, (unsigned)__builtin_amdgcn_mov_dpp((int)b, 0x128, 0xf, 0xf, true));
+      b = max(b, (unsigned)__builtin_amdgcn_mov_dpp((int)b, 0x124, 0xf, 0xf, true));
+      b = max(b, (unsigned)__builtin_amdgcn_mov_dpp((int)b, 0x122, 0xf, 0xf, true));
+      b = max(b, (unsigned)__builtin_amdgcn_mov_dpp((int)b, 0x121, 0xf, 0xf, true));
+      return max(max((unsigned)__builtin_amdgcn_readlane((int)b, 0), (unsigned)__builtin_amdgcn_readlane((int)b, 16)),
+                 max((unsigned)__builtin_amdgcn_readlane((int)b, 32), (unsigned)__builtin_amdgcn_readlane((int)b, 48)));
+    };
+    const unsigned mk = wave_max(fk), mv = wave_max(fv);
+    if (lane == 0) {
+      tile_max[group][wave][0] = mk;
+      tile_max[group][wave][1] = mv;
+    }
+  };
+  // Planes into buffer buf: K under the tile's own scale (k_undo: what undoes it), V under that of the largest magnitude of the
+  // group's tiles so far (v_eb: its exponent field), which O follows when it comes to the tile.
+  [[maybe_unused]] float k_undo = 0.0f;
+  [[maybe_unused]] int v_eb = 0;
+  [[maybe_unused]] auto put_planes = [&](int buf) __attribute__((always_inline)) {
+    unsigned mk = 0, mv = 0;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) {
+      mk = max(mk, tile_max[group][w][0]);
+      mv = max(mv, tile_max[group][w][1]);
+    }
+    mk = (unsigned)__builtin_amdgcn_readfirstlane((int)mk);
+    mv = (unsigned)__builtin_amdgcn_readfirstlane((int)mv);
+    v_eb = max(v_eb, (int)(mv >> 23));
+    float k_scale, v_scale_now, unused;
+    split_scale(mk, &k_scale, &k_undo);
+    split_scale((unsigned)v_eb << 23, &v_scale_now, &unused);
+    auto put = [&](const float4 (&f)[2], float scale, unsigned char* top_at, unsigned char* rest_at) __attribute__((always_inline)) {
+      const float v[8] = {f[0].x, f[0].y, f[0].z, f[0].w, f[1].x, f[1].y, f[1].z, f[1].w};
+      v4u top, rest;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const v2f x = {v[2 * e] * scale, v[2 * e + 1] * scale};
+        const unsigned tu = __builtin_bit_cast(unsigned, __builtin_convertvector(x, v2h));
+        unsigned ru;
+        asm("v_fma_mixlo_f16 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]\n\tv_fma_mixhi_f16 %0, %1, -1.0, %3 op_sel:[1,0,0] op_sel_hi:[1,0,0]"
+            : "=&v"(ru) : "v"(tu), "v"(x[0]), "v"(x[1]));
+        top[e] = tu;
+        rest[e] = ru;
+      }
+      *reinterpret_cast<v4u*>(top_at) = top;
+      *reinterpret_cast<v4u*>(rest_at) = rest;
+    };
+    static_for<FN>([&](auto i_c) __attribute__((always_inline)) {
+      constexpr int i = decltype(i_c)::value;
+      int row, c;
+      fetched(i_c, &row, &c);
+      unsigned char* const k_at = Kb + buf * KTB + row * KRS + 16 * c;
+      put(fk[i], k_scale, k_at, k_at + 2 * D);
+      unsigned char* const v_at = Vb + buf * VTB + row * VRS + 16 * c;
+      const int swapped = SWZ ? 64 * ((row >> 1) & 1) : 0;   // (SWZ: planes of 64 bytes)
+      put(fv[i], v_scale_now, v_at + swapped, v_at + (SWZ ? 64 - swapped : 2 * D));
+    });
+  };
+  if constexpr (DIRECT) fetch(0);
 
   // The lane's query row: the fp32 row is read, multiplied by q_mul (scale * log2 e: a score leaves the matrix unit in
   // exponent units), brought under the row's own power-of-two scale and split into the two planes here, in registers
   // (a lane and its partner 32 lanes on hold the row's two halves of every 16 columns).
   const int qrow = min(q_base + j, Sq - 1);
   v8h qt[DS], qr[DS];
-  float s_mul;
+  float s_mul;                     // what a score is multiplied by to undo the scales
+  [[maybe_unused]] float q_undo;   // the query row's part of it
   {
     const float* qsrc = Q + ((size_t)bh * Sq + qrow) * D + 8 * hh;
     float4 x[DS][2];
@@ -261,12 +368,16 @@ __global__ __launch_bounds__(KG * WAVES * 64, KG == 1 && D <= 64 ? 2 : 1) void f
           qr[s][4 * h + e] = (_Float16)(v[e] - (float)top);
         }
       }
-    float k_scale, k_inv;
-    split_scale(kv_bits[bh], &k_scale, &k_inv);
-    s_mul = q_inv * k_inv;   // what a score is multiplied by to undo the scales
+    q_undo = q_inv;
+    s_mul = 1.0f;
+    if constexpr (!DIRECT) {
+      float k_scale, k_inv;
+      split_scale(kv_bits[bh], &k_scale, &k_inv);
+      s_mul = q_inv * k_inv;
+    }
   }
-  float v_scale, v_inv;
-  split_scale(kv_bits[BH + bh], &v_scale, &v_inv);
+  [[maybe_unused]] float v_scale, v_inv;
+  if constexpr (!DIRECT) split_scale(kv_bits[BH + bh], &v_scale, &v_inv);
 
   v16f om[DT];
 #pragma unroll
@@ -462,8 +573,20 @@ __global__ __launch_bounds__(KG * WAVES * 64, KG == 1 && D <= 64 ? 2 : 1) void f
   // by more than kLazyBits, and O and the sum are brought to the new one.  Groups (key step, d tile: 3 MFMAs) are
   // taken two at a time, in an order in which no MFMA adds to the result of the one before it; a pair's V fragments are
   // requested under the pair before.
+  // (DIRECT: the V rows at pvbase are under the scale of exponent field pend_eb, O under that of o_eb)
+  [[maybe_unused]] int o_eb = 0, pend_eb = 0;
   auto pv_and_maxima = [&](auto maxima_c, auto next_k_c, auto mask_c, const unsigned char* pvbase, const unsigned char* next_kbase,
                            const v16f& am, int key0) __attribute__((always_inline)) {
+    if constexpr (DIRECT) {
+      if (pend_eb != o_eb) {
+        const float by = ldexpf(1.0f, clamped_eb(o_eb) - clamped_eb(pend_eb));
+        o_eb = pend_eb;
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) om[dt][r] *= by;
+      }
+    }
     // MAXIMA false: the product alone, behind the last half, all of whose weights are there; MASK: the half is ragged
     constexpr bool MAXIMA = decltype(maxima_c)::value, NEXT_K = decltype(next_k_c)::value, MASK = decltype(mask_c)::value;
     constexpr bool DEFER = kDefer && MAXIMA;
@@ -507,6 +630,7 @@ __global__ __launch_bounds__(KG * WAVES * 64, KG == 1 && D <= 64 ? 2 : 1) void f
       __builtin_amdgcn_sched_barrier(0);
     });
     if constexpr (MAXIMA) {
+      if constexpr (DIRECT) s_mul = q_undo * k_undo;   // (from here on `raw` is of the tile that `am` is of)
       mx = max_with_other_half(mx) * s_mul;   // finite: the half holds at least one key; s_mul > 0
       if (__builtin_amdgcn_ballot_w64(mx > m_ref + kLazyBits) != 0) {   // a row of the wave moves its reference
         const bool moves = mx > m_ref + kLazyBits;
@@ -527,23 +651,34 @@ __global__ __launch_bounds__(KG * WAVES * 64, KG == 1 && D <= 64 ? 2 : 1) void f
   // beside those of its second half, behind the barrier in the middle of the tile.  Copies complete in the order of their issue, so each of the two barriers waits for the
   // older of the two requests only.
   const int ntiles = (Skv + FA_KT - 1) / FA_KT;
-  copy_k(0, 0);
-  copy_v(0, 0);
-  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+  if constexpr (DIRECT) {
+    publish_max();
+    __syncthreads();
+    put_planes(0);
+    o_eb = pend_eb = v_eb;
+  } else {
+    copy_k(0, 0);
+    copy_v(0, 0);
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+  }
   __syncthreads();
 
   const unsigned char* pend_v = Vb + v_lane;   // the V rows of the half whose product is still to come (first: zero weights on tile 0)
   for (int kt = 0; kt < ntiles; ++kt) {
     const int buf = kt & 1;
     const bool more = kt + 1 < ntiles;
-    const bool whole_next = (kt + 2) * FA_KT <= Skv;   // a tile follows and all of its 64 keys exist
+    const bool whole_next = !DIRECT && (kt + 2) * FA_KT <= Skv;   // a tile follows and all of its 64 keys exist
+    [[maybe_unused]] const int tile_eb = v_eb;   // the scale of V of tile kt
+    if constexpr (DIRECT) {
+      if (more) fetch(kt + 1);
+    }
     {   // first half; beside its scores, K of tile kt + 1 is requested (K[buf ^ 1] was last read before the barrier that ended tile kt - 1)
       v16f am;
       const unsigned char* kbase = Kb + buf * KTB + k_lane;
       if (whole_next) {
         scores(std::false_type{}, std::integral_constant<int, 1>{}, kt + 1, buf ^ 1, kbase, pend_v, am);
       } else {
-        if (more) copy_k(kt + 1, buf ^ 1);   // the last, ragged tile: each copy clamps its rows
+        if (!DIRECT && more) copy_k(kt + 1, buf ^ 1);   // the last, ragged tile: each copy clamps its rows
         scores(std::false_type{}, std::integral_constant<int, 0>{}, 0, 0, kbase, pend_v, am);
       }
       if (kt * FA_KT + 32 <= Skv) pv_and_maxima(std::true_type{}, std::true_type{}, std::false_type{}, pend_v, kbase + 32 * KRS, am, kt * FA_KT);
@@ -551,16 +686,27 @@ __global__ __launch_bounds__(KG * WAVES * 64, KG == 1 && D <= 64 ? 2 : 1) void f
       pend_v = Vb + buf * VTB + v_lane;
     }
     // V of tile kt has landed in every wave (asked for half a tile ago or more); V[buf ^ 1] has been read for the last time
-    if (more) __builtin_amdgcn_s_waitcnt(vmcnt_at_most(KC_MIN));
-    else __builtin_amdgcn_s_waitcnt(0x0F70);
+    if constexpr (DIRECT) {
+      if (more) publish_max();
+    } else {
+      if (more) __builtin_amdgcn_s_waitcnt(vmcnt_at_most(KC_MIN));
+      else __builtin_amdgcn_s_waitcnt(0x0F70);
+    }
     __syncthreads();
+    const float k_undo_now = k_undo;
+    if constexpr (DIRECT) {
+      pend_eb = tile_eb;   // pend_v is now the tile's
+      if (more) put_planes(buf ^ 1);
+    }
+    const float k_undo_next = k_undo;
+    k_undo = k_undo_now;   // of the tile whose second half follows
     if (kt * FA_KT + 32 < Skv) {   // second half (a tile that is followed by another has one); beside its scores, V of tile kt + 1 is requested
       v16f am;
       const unsigned char* kbase = Kb + buf * KTB + k_lane + 32 * KRS;
       if (whole_next) {
         scores(std::true_type{}, std::integral_constant<int, 2>{}, kt + 1, buf ^ 1, kbase, pend_v, am);
       } else {
-        if (more) copy_v(kt + 1, buf ^ 1);
+        if (!DIRECT && more) copy_v(kt + 1, buf ^ 1);
         scores(std::true_type{}, std::integral_constant<int, 0>{}, 0, 0, kbase, pend_v, am);
       }
       if (kt * FA_KT + 64 <= Skv) pv_and_maxima(std::true_type{}, std::false_type{}, std::false_type{}, pend_v, nullptr, am, kt * FA_KT + 32);
@@ -568,7 +714,8 @@ __global__ __launch_bounds__(KG * WAVES * 64, KG == 1 && D <= 64 ? 2 : 1) void f
       pend_v = Vb + buf * VTB + v_lane + 32 * VRS;
     }
     // K of tile kt + 1 has landed; K[buf] has been read for the last time
-    if (more) __builtin_amdgcn_s_waitcnt(vmcnt_at_most(VC_MIN));
+    if (!DIRECT && more) __builtin_amdgcn_s_waitcnt(vmcnt_at_most(VC_MIN));
+    k_undo = k_undo_next;
     __syncthreads();
   }
   {   // the last half's weights, then its product
@@ -603,6 +750,7 @@ __global__ __launch_bounds__(KG * WAVES * 64, KG == 1 && D <= 64 ? 2 : 1) void f
 #pragma unroll
         for (int g = 0; g < 4; ++g) oo(group)[(4 * dt + g) * 64] = v4f{om[dt][4 * g], om[dt][4 * g + 1], om[dt][4 * g + 2], om[dt][4 * g + 3]};
       *oml(group) = make_float2(m_ref, l);
+      if (DIRECT && lane == 0) tile_max[group][wave][0] = (unsigned)o_eb;
     }
     __syncthreads();
     if (!PART && group > 0) return;
@@ -611,9 +759,15 @@ __global__ __launch_bounds__(KG * WAVES * 64, KG == 1 && D <= 64 ? 2 : 1) void f
       for (int other = 1; other < KG; ++other) {
         const float2 ml = *oml(other);
         const float m = fmaxf(m_ref, ml.x);
-        const float wm = __builtin_amdgcn_exp2f(m_ref - m), wo = __builtin_amdgcn_exp2f(ml.x - m);
+        float wm = __builtin_amdgcn_exp2f(m_ref - m), wo = __builtin_amdgcn_exp2f(ml.x - m);
         l = wm * l + wo * ml.y;
         m_ref = m;
+        if constexpr (DIRECT) {   // the two groups' O under the scale of the larger values
+          const int eb = __builtin_amdgcn_readfirstlane((int)tile_max[other][wave][0]), most = max(o_eb, eb);
+          wm = ldexpf(wm, clamped_eb(o_eb) - clamped_eb(most));
+          wo = ldexpf(wo, clamped_eb(eb) - clamped_eb(most));
+          o_eb = most;
+        }
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
@@ -687,6 +841,7 @@ __global__ __launch_bounds__(KG * WAVES * 64, KG == 1 && D <= 64 ? 2 : 1) void f
   constexpr int ORS = 4 * D + 16;
   constexpr int LPR = D / 4;   // 16-byte chunks per row
   unsigned char* const ot = smem + wave * (32 * ORS);
+  if constexpr (DIRECT) split_scale((unsigned)o_eb << 23, &v_scale, &v_inv);
   const float fin = v_inv / l;   // l in the scale of the weights' planes, as O's accumulators
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt)
@@ -713,41 +868,61 @@ static size_t round256f(size_t v) { return (v + 255) / 256 * 256; }
 // How the work is laid out: waves (of 32 query rows) and key groups of a workgroup, and workgroups that share a block's keys.
 struct F32Split {
   int waves, groups, parts;
+  bool direct;   // the attention kernel cuts K and V into planes itself
 };
 static F32Split f32_split(long long BH, int Sq, int Skv, int D, int cus) {
   const int tiles = (Skv + FA_KT - 1) / FA_KT;
-  F32Split best = {4, 1, 1};
-  if ((long long)((Sq + 127) / 128) * BH > 2 * cus) return best;
+  // What the planes in a launch or two of their own cost beyond the attention kernel's, and what cutting them itself costs that (us): for
+  // every tile of a wave more, for each query block again, and most where the wave is alone on its SIMD and has no registers left.
+  // Fitted to 137 grids of 2 to 96 heads, 64 to 2048 queries and keys.  us with planes and without: 16 heads S 1024 D 32 20.0, 17.9; 12 heads
+  // S 96 D 64 10.7, 7.9; 64 heads S 448 D 64 28.3, 20.4; 68 heads S 243 D 96 24.8, 19.1; 69 heads S 186 D 128 25.2, 19.9; the other
+  // way round 24 heads S 1728 D 64 85.8, 89.3; 12 heads S 1536 D 128 72, 105.
+  const float planes_us = 2.7f + 0.3e-6f * 8.0f * (float)BH * (float)Skv * (float)D;
+  // (chain: tiles of a wave; per_simd: waves that a SIMD gets in turn or at once)
+  auto direct_us = [&](int chain, long long per_simd) {
+    const float tile = D == 32 ? (per_simd == 1 ? 0.33f : 0.15f) : D == 64 ? (per_simd == 1 ? 0.6f : 0.23f) : D == 96 ? 0.7f : 1.45f;
+    return tile * (float)chain * (float)per_simd;
+  };
+  const long long blocks = (long long)((Sq + 127) / 128) * BH;
+  if (blocks > 2 * cus) return {4, 1, 1, direct_us(tiles, (blocks + cus - 1) / cus) < planes_us};
   // Time in tenths of what a wave that shares its SIMD needs for a tile (1.05, 1.35, 1.7, 1.9 us by head size).  Two waves of a SIMD
   // hardly overlap, so what counts is the tiles that a SIMD works through; one that has only one wave takes a fifth longer.  What
   // parts leave in the workspace and the last one takes in costs 1.4, 1.6, 2.2, 2.6 us and 0.55, 0.7, 0.85, 1.05 us a part: as much as
   // 35 tenths with four to six parts, at every head size.  Over 580 grids of 1 to 64 heads, 32 to 4096 queries and 128 to 8192
   // keys the split chosen takes 2.5, 3.3, 0.7 and 1.6 % longer in the mean than the best one of all for the grid, a quarter at the most; 25
   // tenths serve as well, with 20 or 50 it is up to 1 % more.
-  const int merge = 35;
-  auto workgroups = [&](const F32Split& f) { return (long long)((Sq + 32 * f.waves - 1) / (32 * f.waves)) * BH * f.parts; };
-  auto cost = [&](const F32Split& f) {
-    const long long per_simd = std::max(1LL, (workgroups(f) + cus - 1) / cus * f.groups * f.waves / 4);
-    const int chain = (tiles + f.groups * f.parts - 1) / (f.groups * f.parts);
-    return chain * (D > 64 ? 12 * per_simd : per_simd == 1 ? 12 : 10 * per_simd) + (f.parts > 1 ? merge : 0) + (f.groups > 1 ? 2 * f.groups : 0);
+  const int merge = 35, blocks128 = (int)blocks, blocks64 = (Sq + 63) / 64 * (int)BH;
+  const float tenths = 1.0f / (D == 32 ? 0.105f : D == 64 ? 0.135f : D == 96 ? 0.17f : 0.19f);
+  // What a split saves that cuts K and V itself counts for it (parts do not: their counters are cleared by the launch in front), but
+  // for longer chains of sums than the cheapest split has without that it is not taken.
+  struct Found {
+    F32Split split;
+    int cost, chain;
   };
-  long long least = cost(best);
-  auto consider = [&](const F32Split& f) {
-    const int resident = D <= 64 && f.groups == 1 ? 2 : 1;   // workgroups of a compute unit, by registers and LDS
-    if (tiles < f.groups * f.parts || workgroups(f) > (long long)resident * cus || cost(f) >= least) return;
-    least = cost(f);
-    best = f;
+  Found plain = {{4, 1, 1, false}, 1 << 30, 0}, best = plain;
+  auto consider = [&](int waves, int groups, int parts) {
+    const int workgroups = (waves == 4 ? blocks128 : blocks64) * parts, shares = groups * parts;
+    const int resident = D <= 64 && groups == 1 ? 2 : 1;   // workgroups of a compute unit, by registers and LDS
+    if (shares > 1 && (tiles < shares || workgroups > resident * cus)) return;
+    const int chain = (tiles + shares - 1) / shares, per_simd = std::max(1, (workgroups + cus - 1) / cus * groups * waves / 4);
+    const int cost = chain * (D > 64 ? 12 * per_simd : per_simd == 1 ? 12 : 10 * per_simd) + (parts > 1 ? merge : 0) + (groups > 1 ? 2 * groups : 0);
+    const float saved = parts > 1 ? 0.0f : planes_us - direct_us(chain, per_simd);
+    const bool direct = saved > 0.0f;
+    const int without = cost - (direct ? (int)(saved * tenths) : 0);
+    if (cost < plain.cost) plain = {{waves, groups, parts, direct}, cost, chain};
+    if (without < best.cost) best = {{waves, groups, parts, direct}, without, chain};
   };
+  consider(4, 1, 1);
   if (D <= 64) {
-    consider({4, 2, 1});
-    consider({2, 2, 1});
+    consider(4, 2, 1);
+    consider(2, 2, 1);
   }
-  if (D == 32) consider({2, 4, 1});
+  if (D == 32) consider(2, 4, 1);
   for (int parts = 2; parts <= 16; ++parts) {
-    consider({4, 1, parts});
-    if (D <= 64) consider({4, 2, parts});
+    consider(4, 1, parts);
+    if (D <= 64) consider(4, 2, parts);
   }
-  return best;
+  return best.chain <= plain.chain ? best.split : plain.split;
 }
 
 struct F32Layout {
@@ -767,8 +942,8 @@ static F32Layout f32_layout(long long bh, int nqb, int parts, bool chunked, int 
   return w;
 }
 
-template <int D, int KG, int WAVES, bool PART>
-static int launch_fa_f32_blocks(const float* Q, const _Float16* kp, const _Float16* vp, unsigned* bits, float* O, int BH, int Sq, int Skv,
+template <int D, int KG, int WAVES, bool PART, bool DIRECT = false>
+static int launch_fa_f32_blocks(const float* Q, const void* kp, const void* vp, unsigned* bits, float* O, int BH, int Sq, int Skv,
                                 float scale, int parts, char* partials, int lds_max, hipStream_t s) {
   using L = F32Tiles<D, KG>;
   const size_t lds = std::max((size_t)KG * 2 * (L::KTB + L::VTB), (size_t)WAVES * 32 * (4 * D + 16));
@@ -779,11 +954,11 @@ static int launch_fa_f32_blocks(const float* Q, const _Float16* kp, const _Float
   static DeviceOnce attr_once;
   unsigned attr_bit;
   if (attr_once.pending(&attr_bit)) {
-    FTK_HIP(hipFuncSetAttribute((const void*)flash_attn_f32_kernel<D, KG, WAVES, PART>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    FTK_HIP(hipFuncSetAttribute((const void*)flash_attn_f32_kernel<D, KG, WAVES, PART, DIRECT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     attr_once.done(attr_bit);
   }
-  hipLaunchKernelGGL((flash_attn_f32_kernel<D, KG, WAVES, PART>), dim3((unsigned)blocks), dim3(KG * WAVES * 64), lds, s, Q, kp, vp, scale * 1.4426950408889634f,
-                     (const unsigned*)bits, O, Sq, Skv, nqb, BH, parts, reinterpret_cast<int*>(bits + 2 * BH), reinterpret_cast<unsigned char*>(partials));
+  hipLaunchKernelGGL((flash_attn_f32_kernel<D, KG, WAVES, PART, DIRECT>), dim3((unsigned)blocks), dim3(KG * WAVES * 64), lds, s, Q, kp, vp, scale * 1.4426950408889634f,
+                     (const unsigned*)bits, O, Sq, Skv, nqb, BH, parts, bits ? reinterpret_cast<int*>(bits + 2 * BH) : nullptr, reinterpret_cast<unsigned char*>(partials));
   return check_launch("flash_attn_f32_kernel");
 }
 
@@ -800,8 +975,10 @@ static int launch_fa_f32(const float* Q, const float* K, const float* V, float* 
   const size_t all_heads = 2 * (size_t)BH * head_bytes, most_read = (size_t)96 << 20;
   const int parts = (int)std::max<size_t>(1, std::min({512 / (2 * (size_t)BH), per_bh / (8 * kPlanesThreads), most_read / all_heads}));
   const int counters = split.parts > 1 ? BH * ((Sq + 127) / 128) : 0;
-  int rc;
-  if (head_bytes <= 512 * 1024 && all_heads * parts <= most_read) {
+  int rc = FTK_OK;
+  if (split.direct) {
+    // no planes
+  } else if (head_bytes <= 512 * 1024 && all_heads * parts <= most_read) {
     hipLaunchKernelGGL(attn_f32_planes_kernel<D>, dim3((unsigned)(2 * BH * parts)), dim3(kPlanesThreads), 0, s, K, V, kp, vp, bits, Skv, BH, parts,
                        counters);
     rc = check_launch("attn_f32_planes_kernel");
@@ -825,6 +1002,11 @@ static int launch_fa_f32(const float* Q, const float* K, const float* V, float* 
   }
   char* const partials = ws + w.partials;
   auto run = [&](auto groups_c, auto waves_c, auto part_c) {
+    if constexpr (!decltype(part_c)::value) {
+      if (split.direct)
+        return launch_fa_f32_blocks<D, decltype(groups_c)::value, decltype(waves_c)::value, false, true>(Q, K, V, nullptr, O, BH, Sq, Skv, scale, 1, nullptr,
+                                                                                                         dp.lds_optin, s);
+    }
     return launch_fa_f32_blocks<D, decltype(groups_c)::value, decltype(waves_c)::value, decltype(part_c)::value>(
         Q, kp, vp, bits, O, BH, Sq, Skv, scale, split.parts, partials, dp.lds_optin, s);
   };
@@ -877,7 +1059,7 @@ extern "C" int ftk_flash_attn_f32(const float* Q, const float* K, const float* V
   const F32Layout cut = f32_layout(bh, nqb, split.parts, true, Skv, D), whole = f32_layout(bh, nqb, 1, true, Skv, D);
   if (workspace_bytes >= cut.total) w = cut;
   else if (workspace_bytes >= whole.total) w = whole;
-  if (workspace_bytes < cut.total && split.parts > 1) split = {4, D <= 64 && bh * nqb <= dp->cus && Skv > 2 * FA_KT ? 2 : 1, 1};
+  if (workspace_bytes < cut.total && split.parts > 1) split = {4, D <= 64 && bh * nqb <= dp->cus && Skv > 2 * FA_KT ? 2 : 1, 1, false};
   hipStream_t s = (hipStream_t)stream;
   char* ws = reinterpret_cast<char*>(workspace);
   switch (D) {

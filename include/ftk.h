@@ -511,7 +511,8 @@ int ftk_flash_attn_ws_f16(const void* Q, const void* K, const void* V, void* O,
  * blocks, flash_attention_utils.py:20-24; batch 2 x 8 heads x 1024 x 32 at
  * :96-110).  Products run on the fp16 matrix pipe as three fp16 products of
  * split operands with fp32 accumulation (a row of Q, all of K and all of V of
- * a (batch, head) each share a power-of-two scale), the softmax state is fp32:
+ * a (batch, head), or 64 keys of K and those of V so far, each share a
+ * power-of-two scale), the softmax state is fp32:
  * results agree with a float64 evaluation to a few 1e-6 of the largest |O|.
  * Q, K, V, O 16-byte aligned.  Non-finite inputs give NaN.  The workspace
  * (256-byte aligned) holds the split planes of K and V, 4*D*Skv bytes each per
@@ -527,8 +528,9 @@ int ftk_flash_attn_ws_f16(const void* Q, const void* K, const void* V, void* O,
  * (batch, head), each rounded up to 256 bytes (the planes of K and of V
  * separately), else FTK_ERR_WORKSPACE.  On less than the query asks for, a
  * query block's keys are not shared: grids of few query blocks are slower,
- * and the last bits of O differ (the sums are taken in another order).  One to
- * three small launches precede the attention kernel.  The reference has no
+ * and the last bits of O differ (the sums are taken in another order).  Up to
+ * three small launches precede the attention kernel, none on small grids, whose
+ * workgroups split K and V themselves and leave the workspace alone.  The reference has no
  * device kernel for this program.
  */
 size_t ftk_flash_attn_f32_workspace_bytes(int B, int Hd, int Sq, int Skv, int D);

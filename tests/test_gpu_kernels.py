@@ -1687,3 +1687,33 @@ def test_flash_attention_f32_shared_keys(core, B, Hd, Sq, Skv, D):
         assert torch.equal(core.flash_attention_f32(Q, K, V, workspace=ws), first)
     small = torch.empty(planes + 3 * 256 + 8 * B * Hd, dtype=torch.uint8, device='cuda')
     assert ko.max_rel_err(core.flash_attention_f32(Q, K, V, workspace=small).cpu().numpy(), ref) <= 1e-5
+
+
+@pytest.mark.parametrize('B,Hd,Sq,Skv,D', [
+    (1, 3, 70, 65, 32),          # two key groups to 64 query rows, a tile each, the last of one key
+    (2, 8, 468, 468, 32),        # four key groups
+    (2, 8, 1000, 961, 32),       # four tiles in a row to a group, the last of all of one key
+    (4, 9, 1014, 73, 32),        # one group, two workgroups to a compute unit
+    (1, 5, 100, 193, 64),
+    (6, 8, 590, 593, 64),        # two key groups to 128 query rows
+    (8, 8, 64, 64, 64),          # one tile
+    (4, 17, 243, 243, 96),
+    (2, 5, 90, 100, 128),
+    (3, 23, 186, 161, 128),      # more blocks than compute units
+])
+def test_flash_attention_f32_that_cuts_its_tiles_itself(core, B, Hd, Sq, Skv, D):
+    """Grids whose workgroups cut K and V into planes on their way to LDS, each tile of K under a scale of its own and V under that of
+    the tiles so far.  Values that grow, shrink and vanish from tile to tile against float64 within 1e-5 of a row's largest (22 bits of each
+    factor, fp32 sums), and exactly the same bits, moved, under another power of two."""
+    gen = torch.Generator(device='cuda').manual_seed(27)
+    Q, K, V = (torch.randn((B, Hd, s, D), generator=gen, device='cuda') for s in (Sq, Skv, Skv))
+    tile = torch.arange(Skv, device='cuda') // 64
+    K *= torch.exp2(-(tile * 5 % 7).float())[:, None]
+    shift = (tile * 7 % 20 - 6).float()
+    V *= torch.exp2(shift)[:, None] * (tile % 4 != 0 if Skv > 64 else tile + 1)[:, None]   # (the first tile of several is zeros)
+    O = core.flash_attention_f32(Q, K, V)
+    ref = torch.softmax(torch.matmul(Q.double().cpu(), K.double().cpu().transpose(2, 3)) * D ** -0.5, -1) @ V.double().cpu()
+    assert float(((O.double().cpu() - ref).abs().amax(-1) / ref.abs().amax(-1)).max()) <= 1e-5
+    for by in (2.0 ** 90, 2.0 ** -80):
+        assert torch.equal(core.flash_attention_f32(Q, K, V * by), O * by)
+    assert torch.equal(core.flash_attention_f32(Q * 2.0 ** 40, K * 2.0 ** -40, V), O)
