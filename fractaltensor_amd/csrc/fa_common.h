@@ -27,6 +27,19 @@ __device__ __forceinline__ void lds_dma16(const void* gbase, unsigned byte_off, 
       : "memory", "m0");
 }
 
+// The same for what is read once: `nt` keeps it from displacing other lines on its way through the caches.  512 MB by 256 workgroups of
+// four waves, 8 KB pieces: 6.2 TB/s without, 7.1 with.
+__device__ __forceinline__ void lds_dma16_once(const void* gbase, unsigned byte_off, void* lds_base) {
+  const unsigned lds_addr = (unsigned)reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) void*)lds_base);
+  asm volatile(
+      "s_mov_b32 m0, %0\n\t"
+      "s_nop 0\n\t"
+      "global_load_lds_dwordx4 %1, %2 nt"
+      :
+      : "s"(lds_addr), "v"(byte_off), "s"(gbase)
+      : "memory", "m0");
+}
+
 // max(x, x of lane^32) without a trip through LDS: v_permlane32_swap exchanges
 // the upper half of the first register with the lower half of the second, so
 // with both holding x, afterwards one holds the lower lanes' x in every lane

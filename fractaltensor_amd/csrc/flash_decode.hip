@@ -11,8 +11,9 @@
 // B: the resident queries), O^T = V^T P^T (A: V^T by the transposing LDS read, B: the weights as they come out of the
 // first product, the contraction taking the keys in the order a lane holds them).
 //
-// Measured (microseconds, with the 4-wave prompt kernel before): 1 query a head, 256 heads of 128, 4096 keys 116 -> 91
-// (5.9 TB/s; a copy reaches 4.9); 8 heads, 32768 keys 41 -> 29; 16 queries, 24 heads of 128, 1753 keys 34 -> 10.
+// Measured (microseconds, with the 4-wave prompt kernel before): 1 query a head, 256 heads of 128, 4096 keys 116 -> 91 -> 77
+// with copies that leave no lines in the caches (7.0 TB/s; nothing but such copies reaches 7.1); 8 heads, 32768 keys 41 -> 27; 16 queries,
+// 24 heads of 128, 1753 keys 34 -> 10.
 //
 // The keys of a head are cut over workgroups (parts) where heads alone do not fill the chip; attn_merge_kernel
 // (flash_attn.hip) merges what the parts leave.
@@ -46,7 +47,8 @@ struct DecodeShape {
   static constexpr size_t LDS = (size_t)kDecWaves * STAGES * 2 * TILE;
 };
 
-template <int D>
+// ONCE: what K and V hold together is more than the caches keep from call to call (launch_decode).
+template <int D, bool ONCE>
 __global__ __launch_bounds__(kDecWaves * 64) void flash_decode_kernel(const _Float16* __restrict__ Q, const _Float16* __restrict__ K,
                                                                       const _Float16* __restrict__ V, _Float16* __restrict__ O, int Sq,
                                                                       int Skv, float scale_log2e, int nparts, int part_keys,
@@ -81,8 +83,13 @@ __global__ __launch_bounds__(kDecWaves * 64) void flash_decode_kernel(const _Flo
     for (int i = 0; i < S::COPIES; ++i) {
       const int p = 64 * i + lane, row = p / CH, slot = p - row * CH;
       const unsigned off = (unsigned)(min(row, most) * (2 * D) + (slot ^ decode_swizzle<D>(row)) * 16);
-      lds_dma16(kb, off, dst + 1024 * i);
-      lds_dma16(vb, off, dst + S::TILE + 1024 * i);
+      if constexpr (ONCE) {
+        lds_dma16_once(kb, off, dst + 1024 * i);
+        lds_dma16_once(vb, off, dst + S::TILE + 1024 * i);
+      } else {
+        lds_dma16(kb, off, dst + 1024 * i);
+        lds_dma16(vb, off, dst + S::TILE + 1024 * i);
+      }
     }
   };
 
@@ -229,7 +236,7 @@ __global__ __launch_bounds__(kDecWaves * 64) void flash_decode_kernel(const _Flo
 
 // How the keys of bh heads are cut: the number of parts (1: not at all) and the keys of a part, a multiple of four tiles.
 // A compute unit holds one workgroup at a time (its LDS), so what is weighed is rounds of workgroups times the steps of a
-// workgroup, a tile for each of its four waves: 64 KB at D 128, 2.6 us at a compute unit's share of 6 TB/s, against
+// workgroup, a tile for each of its four waves: 64 KB at D 128, 2.6 us at a compute unit's share of 6 TB/s (2.3 at the 7 that copies which leave no lines behind reach), against
 // about 3 us that a workgroup and 4 us that the merge (a launch) cost beside that.
 int decode_parts(long long bh, int Skv, int D, int cus, int* part_keys) {
   const int groups = (Skv + kDecWaves * kDecKeys - 1) / (kDecWaves * kDecKeys);   // a tile for each wave
@@ -250,29 +257,41 @@ int decode_parts(long long bh, int Skv, int D, int cus, int* part_keys) {
   return best;
 }
 
-template <int D>
+template <int D, bool ONCE>
 static int launch(const void* Q, const void* K, const void* V, void* O, int BH, int Sq, int Skv, float scale, int nparts, int part_keys,
                   float* part_o, float* part_ml, hipStream_t s) {
   static DeviceOnce attr_once;
   unsigned attr_bit;
   if (attr_once.pending(&attr_bit)) {
-    FTK_HIP(hipFuncSetAttribute((const void*)flash_decode_kernel<D>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)DecodeShape<D>::LDS));
+    FTK_HIP(hipFuncSetAttribute((const void*)flash_decode_kernel<D, ONCE>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)DecodeShape<D>::LDS));
     attr_once.done(attr_bit);
   }
-  hipLaunchKernelGGL(flash_decode_kernel<D>, dim3((unsigned)(BH * nparts)), dim3(kDecWaves * 64), DecodeShape<D>::LDS, s, (const _Float16*)Q,
+  hipLaunchKernelGGL((flash_decode_kernel<D, ONCE>), dim3((unsigned)(BH * nparts)), dim3(kDecWaves * 64), DecodeShape<D>::LDS, s, (const _Float16*)Q,
                      (const _Float16*)K, (const _Float16*)V, (_Float16*)O, Sq, Skv, scale * 1.4426950408889634f, nparts, part_keys, part_o,
                      part_ml);
   return check_launch("flash_decode_kernel");
 }
 
+// A head's K and V are read by one XCD, whose L2 holds 4 MB: from 32 MB in all upwards they come from further away at every call, and
+// copies that leave no lines behind are faster (us, plain copies and these, on caches that were not just read: 16 x 16 heads, 4096 keys of
+// 128 90.9, 77.1; 10 x 8 heads, 3116 keys 26.8, 24.1; 16 x 16 heads, 465 keys 13.6, 12.2).  Below, a cache that was just read
+// is still there for plain copies (5 x 32 heads, 536 keys of 64, 22 MB 6.0, 6.4).
+constexpr long long kDecOnceBytes = 32LL << 20;
+
 // nparts workgroups per head, each leaving its part in part_o / part_ml when nparts > 1 (see attn_merge_kernel).
 int launch_decode(const void* Q, const void* K, const void* V, void* O, int BH, int Sq, int Skv, int D, float scale, int nparts,
                   int part_keys, float* part_o, float* part_ml, hipStream_t s) {
+  const bool once = 4LL * BH * Skv * D >= kDecOnceBytes;
+  auto with = [&](auto d_c) {
+    constexpr int d = decltype(d_c)::value;
+    return once ? launch<d, true>(Q, K, V, O, BH, Sq, Skv, scale, nparts, part_keys, part_o, part_ml, s)
+                : launch<d, false>(Q, K, V, O, BH, Sq, Skv, scale, nparts, part_keys, part_o, part_ml, s);
+  };
   switch (D) {
-    case 32: return launch<32>(Q, K, V, O, BH, Sq, Skv, scale, nparts, part_keys, part_o, part_ml, s);
-    case 64: return launch<64>(Q, K, V, O, BH, Sq, Skv, scale, nparts, part_keys, part_o, part_ml, s);
-    case 96: return launch<96>(Q, K, V, O, BH, Sq, Skv, scale, nparts, part_keys, part_o, part_ml, s);
-    default: return launch<128>(Q, K, V, O, BH, Sq, Skv, scale, nparts, part_keys, part_o, part_ml, s);
+    case 32: return with(std::integral_constant<int, 32>{});
+    case 64: return with(std::integral_constant<int, 64>{});
+    case 96: return with(std::integral_constant<int, 96>{});
+    default: return with(std::integral_constant<int, 128>{});
   }
 }
 
