@@ -9,6 +9,7 @@ namespace ftk {
 
 // Where the loop finds the operands of a tile of A [M, K] @ Bm [K, N].
 struct GemmSource {
+  static constexpr bool kOnce = false;
   unsigned a_voff[8], b_voff[4], a_back[2];
   const char *a_next, *b_next;
   size_t b_chunk;

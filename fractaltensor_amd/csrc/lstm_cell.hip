@@ -575,7 +575,9 @@ __global__ __launch_bounds__(WAVES * 64, 8 / WAVES) void lstm_cell_f16_kernel(Ce
 // ------------------------------------------------ packed fp16 cells, whole tiles
 // Where tile_product finds the operands of a cell: A's row is x_t, then h_{t-d}, each H long (whole pairs of chunks); Bm is
 // a unit block's packed weights, a chunk 16 KB in a row.
+template <bool ONCE>
 struct CellSource {
+  static constexpr bool kOnce = ONCE;
   unsigned a_voff[8], b_voff[4];
   unsigned a_back[2];                        // never used: the contraction has whole pairs
   const char *a_next, *b_next, *h_first;     // h_first: this wave's first row of h
@@ -603,16 +605,17 @@ struct CellSource {
 // it: with 128 x 64 outputs to a wave a k step read 12 KB of fragments for 16 MFMAs instead of 16 KB for 32, and two waves
 // per SIMD stood at the same barrier.  L 32 T 64 B 256 H 1024: 12.70 -> 11.63 ms for the stack.
 // A tile of a cell: rows 256 rb .. of the batch, units 64 ub .. .  SHARED: h and c are read by workgroups of this launch, on
-// any XCD, so they are written through to memory.
+// any XCD, so they are written through to memory.  ONCE: the weights of the cells of a stage are more than the last-level cache keeps
+// until the next (run_wavefront_f16).
 constexpr int kThrough = 16;   // sc1 in the cache-policy operand of a buffer store
-template <bool SHARED>
+template <bool SHARED, bool ONCE>
 __device__ __forceinline__ void cell_tile(const CellDescH& cd, int Bc, int H, int rb, int ub) {
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wr = wave >> 1, wc = wave & 1;
   const int j = lane & 31, hh = lane >> 5;
 
-  CellSource src;
+  CellSource<ONCE> src;
   src.nch = (cd.h_prev ? 2 * H : H) / GK;
   src.npairs = src.nch >> 1;
   src.x_pairs = H / (2 * GK);
@@ -706,7 +709,7 @@ __global__ __launch_bounds__(256, 1) void lstm_cell_tile_kernel(CellListH list, 
   const int Bc = cd.rows > 0 ? cd.rows : B;  // rows of this cell
   const int ub = slot % nub, rb = (slot / nub) % nrb;
   if (rb * GT >= Bc) return;  // a row block past the live rows of this step
-  cell_tile<false>(cd, Bc, H, rb, ub);
+  cell_tile<false, false>(cd, Bc, H, rb, ub);
 }
 
 // A whole dense stack in one launch.  With a launch per stage of independent cells, a stage whose tiles are no multiple of
@@ -762,6 +765,7 @@ __host__ __device__ inline void flow_cell(int k, int L, int T, int* l, int* t) {
   *l = low + pos;
   *t = stage - *l;
 }
+template <bool ONCE>
 __global__ __launch_bounds__(256, 1) void lstm_cell_flow_kernel(FlowArgs) {
   extern __shared__ __attribute__((aligned(1024))) unsigned char tile_smem[];
   int* const word = reinterpret_cast<int*>(tile_smem);   // the next tile: layer (-1: none), step, tile of the cell; the ticket kept
@@ -835,7 +839,7 @@ __global__ __launch_bounds__(256, 1) void lstm_cell_flow_kernel(FlowArgs) {
     cd.h = a.hsss + ((size_t)l * T + t) * cell;
     cd.c = a.csss + ((size_t)l * T + t) * cell;
     int* const done = a.done + l;
-    cell_tile<true>(cd, B, H, tile / nub, tile % nub);
+    cell_tile<true, ONCE>(cd, B, H, tile / nub, tile % nub);
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");   // h and c of this wave are in memory
     __syncthreads();
     if (threadIdx.x == 0) __hip_atomic_fetch_add(done, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -1044,32 +1048,36 @@ static int launch_cells(const CellList& list, int B, int I, int H, hipStream_t s
 
 // WU [n_layers, K2, 4H] -> per layer and block ub of UB hidden units the [K2][4*UB] tile the cell kernel keeps
 // in LDS: row k holds chunks of 8 columns, chunk 4*ug + q = gate q of units UB*ub + 8*ug .. +8, stored in slot
-// chunk ^ ((k & 3) << 2).  One thread per 16-byte chunk.
+// chunk ^ ((k & 3) << 2).  Threads go by the places written: a wave writes whole rows and reads whole lines of the four gates.
+// (By the places read, a wave wrote 16 bytes of 64 lines: 338 us in place of 162 for the 1.07 GB of L 32 H 1024.)
+constexpr int kPackEach = 4;   // chunks of a thread, all asked for at once
 __global__ __launch_bounds__(256) void lstm_pack_weights_f16_kernel(const _Float16* __restrict__ WU,
-                                                                    _Float16* __restrict__ packed, size_t chunks,
-                                                                    int K2, int H, int UB) {
-  const size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x;
-  if (idx >= chunks) return;
-  const int per_row = H / 2;  // 4H / 8
-  const int n8 = (int)(idx % per_row);
-  const size_t lk = idx / per_row;
-  const int k = (int)(lk % K2);
-  const size_t l = lk / K2;
-  const int col = 8 * n8;
-  const int q = col / H, u = col % H;
-  const int ub = u / UB, ug = (u % UB) >> 3;
-  const int slot = (4 * ug + q) ^ ((k & 3) << 2);
-  const v4u v = *reinterpret_cast<const v4u*>(WU + idx * 8);
-  *reinterpret_cast<v4u*>(packed + ((l * (H / UB) + ub) * K2 + k) * (4 * UB) + 8 * slot) = v;
+                                                                    _Float16* __restrict__ packed, unsigned chunks,
+                                                                    unsigned K2, unsigned H, unsigned UB) {
+  const unsigned groups = (chunks + 256 * kPackEach - 1) / (256 * kPackEach), l = blockIdx.x / groups;   // chunks: 16-byte ones of a layer
+  const size_t layer = (size_t)l * chunks;
+  const v4u* const src = reinterpret_cast<const v4u*>(WU) + layer;
+  v4u* const dst = reinterpret_cast<v4u*>(packed) + layer;
+  const unsigned first = (blockIdx.x - l * groups) * (256 * kPackEach) + threadIdx.x, slots = UB / 2;   // of a row
+  v4u v[kPackEach];
+#pragma unroll
+  for (int j = 0; j < kPackEach; ++j) {
+    const unsigned i = min(first + 256 * j, chunks - 1), row = i / slots, ub = row / K2, k = row - ub * K2;
+    const unsigned chunk = (i - row * slots) ^ ((k & 3) << 2);
+    v[j] = __builtin_nontemporal_load(src + ((size_t)k * (H / 2) + (chunk & 3) * (H / 8) + ub * (UB / 8) + (chunk >> 2)));
+  }
+#pragma unroll
+  for (int j = 0; j < kPackEach; ++j)
+    if (first + 256 * j < chunks) dst[first + 256 * j] = v[j];
 }
 
 // Hidden units per workgroup of the streaming kernel at hidden size H.
 static int cell_unit_block(int H) { return H % 64 == 0 ? 64 : 32; }
 
 static int pack_weights_f16(const void* WU, void* packed, int layers, int K2, int H, hipStream_t s) {
-  const size_t chunks = (size_t)layers * K2 * (H / 2);
-  hipLaunchKernelGGL(lstm_pack_weights_f16_kernel, dim3((unsigned)((chunks + 255) / 256)), dim3(256), 0, s,
-                     (const _Float16*)WU, (_Float16*)packed, chunks, K2, H, cell_unit_block(H));
+  const unsigned chunks = (unsigned)((size_t)K2 * (H / 2)), piece = 256 * kPackEach;
+  hipLaunchKernelGGL(lstm_pack_weights_f16_kernel, dim3((unsigned)((size_t)(chunks + piece - 1) / piece * layers)), dim3(256), 0, s, (const _Float16*)WU,
+                     (_Float16*)packed, chunks, (unsigned)K2, (unsigned)H, (unsigned)cell_unit_block(H));
   return check_launch("lstm_pack_weights_f16_kernel");
 }
 
@@ -1228,10 +1236,16 @@ int run_wavefront_f16(const void* xs, const void* WU, const float* bias, const i
   if (!one_launch)
     return run_wavefront_of<_Float16, CellListH>((const _Float16*)xs, (const _Float16*)packed, bias, dil, (_Float16*)hsss, (_Float16*)csss, L, T, B,
                                                  H, s, true, active);
+  // A stage reads the weights of min(L, T) layers, and the next stage reads them again.  What the last-level cache (256 MB) holds of
+  // them is worth having up to half as much again; beyond that, lines that are displaced before they are read again cost more
+  // (ms, T 64, copies of the weights that leave lines and that do not: 134 MB 3.82, 4.03; 335 MB 6.83, 6.83; 403 MB 8.20, 8.10; 537 MB
+  // 10.70, 10.49).
+  const bool once = (long long)std::min(L, T) * 16 * H * H > 384LL << 20;
   static DeviceOnce attr_once;
   unsigned attr_bit;
   if (attr_once.pending(&attr_bit)) {
-    FTK_HIP(hipFuncSetAttribute((const void*)lstm_cell_flow_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, G_LDS));
+    FTK_HIP(hipFuncSetAttribute((const void*)lstm_cell_flow_kernel<false>, hipFuncAttributeMaxDynamicSharedMemorySize, G_LDS));
+    FTK_HIP(hipFuncSetAttribute((const void*)lstm_cell_flow_kernel<true>, hipFuncAttributeMaxDynamicSharedMemorySize, G_LDS));
     attr_once.done(attr_bit);
   }
   FlowArgs a;
@@ -1252,7 +1266,7 @@ int run_wavefront_f16(const void* xs, const void* WU, const float* bias, const i
     const int polls = atoi(e);
     if (polls > 0 && polls <= (1 << 20) && (polls & (polls - 1)) == 0) a.patience = polls - 1;
   }
-  hipLaunchKernelGGL(lstm_cell_flow_kernel, dim3(dp->cus), dim3(256), G_LDS, s, a);
+  hipLaunchKernelGGL(once ? lstm_cell_flow_kernel<true> : lstm_cell_flow_kernel<false>, dim3(dp->cus), dim3(256), G_LDS, s, a);
   return check_launch("lstm_cell_flow_kernel");
 }
 

@@ -42,6 +42,12 @@ __device__ __forceinline__ void tile_dma16(const void* gbase, unsigned byte_off,
                :: "s"(lds_addr), "v"(byte_off), "s"(gbase) : "memory", "m0");
 }
 
+// (nt: leaving no line behind in the caches)
+__device__ __forceinline__ void tile_dma16_nt(const void* gbase, unsigned byte_off, unsigned lds_addr) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt"
+               :: "s"(lds_addr), "v"(byte_off), "s"(gbase) : "memory", "m0");
+}
+
 // LDS: three A buffers, then four Bm stages.  An A buffer holds the tile's 256 rows of a pair of chunks, 128 bytes
 // = 8 slots of 16 each: row r keeps k slot c in slot c ^ ((r >> 1) & 7) (16 rows in a row of one k slot fall on 16
 // different 16-byte bank groups).  A copy brings 8 rows' whole 128-byte lines; with 64-byte rows, a chunk at a time,
@@ -57,6 +63,7 @@ __device__ __forceinline__ void tile_dma16(const void* gbase, unsigned byte_off,
 // where the next one exists, (false_type) outside, where the bases have to stop at the last pair and chunk: what is
 // requested beyond the end is the last once more, into a buffer nothing reads any more, so that every wait below
 // counts the same number of copies whatever the length.  left_main_loop(ch): the unrolled loop ended in front of chunk ch.
+// kOnce: what is fetched of Bm is not fetched again soon, and its copies leave no lines in the caches.
 template <typename Src>
 __device__ __forceinline__ void tile_product(Src& src, int nch, v16f (&acc)[4][4]) {
   extern __shared__ __attribute__((aligned(1024))) unsigned char tile_smem[];
@@ -83,11 +90,16 @@ __device__ __forceinline__ void tile_product(Src& src, int nch, v16f (&acc)[4][4
   auto copy_b = [&](auto bs, auto i_c) __attribute__((always_inline)) {
     constexpr int i = decltype(i_c)::value;
     if constexpr (std::is_integral_v<decltype(bs)>) {
-      tile_dma16(src.b_next, src.b_voff[i], lds_wave_b + (unsigned)(bs * G_BST + i * 1024));
+      if constexpr (Src::kOnce) tile_dma16_nt(src.b_next, src.b_voff[i], lds_wave_b + (unsigned)(bs * G_BST + i * 1024));
+      else tile_dma16(src.b_next, src.b_voff[i], lds_wave_b + (unsigned)(bs * G_BST + i * 1024));
     } else {
       constexpr int BS = decltype(bs)::value;
-      asm volatile("s_add_u32 m0, %0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %3"
-                   :: "s"(lds_wave_b), "n"(BS * G_BST + i * 1024), "v"(src.b_voff[i]), "s"(src.b_next) : "memory", "m0", "scc");
+      if constexpr (Src::kOnce)
+        asm volatile("s_add_u32 m0, %0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %3 nt"
+                     :: "s"(lds_wave_b), "n"(BS * G_BST + i * 1024), "v"(src.b_voff[i]), "s"(src.b_next) : "memory", "m0", "scc");
+      else
+        asm volatile("s_add_u32 m0, %0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %3"
+                     :: "s"(lds_wave_b), "n"(BS * G_BST + i * 1024), "v"(src.b_voff[i]), "s"(src.b_next) : "memory", "m0", "scc");
     }
   };
   // fragment addresses: A within buffers 0 and 1 (a read's immediate offset reaches 64 KB) and within buffer 2, per k

@@ -1625,6 +1625,7 @@ def test_flash_attention_f32_key_groups_and_planes(core, B, Hd, Sq, Skv, D):
     (192, 3, 9, 70, [1, 3, 20]),           # dilated: the launches
     (320, 9, 9, 300, None),                # as many layers as steps
     (1024, 10, 4, 200, None),
+    (2048, 6, 6, 3, None),                 # more weights in a stage than the last-level cache is good for
 ])
 def test_streamed_f16_stack_in_one_launch(core, monkeypatch, H, L, T, B, dil):
     """The fp16 stack whose tiles wait for each other in one launch has the bits of a launch per stage of cells, three times on
