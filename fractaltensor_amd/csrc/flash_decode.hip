@@ -12,7 +12,7 @@
 // first product, the contraction taking the keys in the order a lane holds them).
 //
 // Measured (microseconds, with the 4-wave prompt kernel before): 1 query a head, 256 heads of 128, 4096 keys 116 -> 91 -> 77
-// with copies that leave no lines in the caches (7.0 TB/s; nothing but such copies reaches 7.1); 8 heads, 32768 keys 41 -> 27; 16 queries,
+// with copies that leave no lines in the caches (7.0 TB/s; nothing but such copies reaches 7.1); 8 heads, 32768 keys 41 -> 26; 16 queries,
 // 24 heads of 128, 1753 keys 34 -> 10.
 //
 // The keys of a head are cut over workgroups (parts) where heads alone do not fill the chip; attn_merge_kernel
@@ -47,7 +47,7 @@ struct DecodeShape {
   static constexpr size_t LDS = (size_t)kDecWaves * STAGES * 2 * TILE;
 };
 
-// ONCE: what K and V hold together is more than the caches keep from call to call (launch_decode).
+// ONCE: K and V are too large for the caches to keep from call to call (launch_decode).
 template <int D, bool ONCE>
 __global__ __launch_bounds__(kDecWaves * 64) void flash_decode_kernel(const _Float16* __restrict__ Q, const _Float16* __restrict__ K,
                                                                       const _Float16* __restrict__ V, _Float16* __restrict__ O, int Sq,
@@ -272,11 +272,13 @@ static int launch(const void* Q, const void* K, const void* V, void* O, int BH, 
   return check_launch("flash_decode_kernel");
 }
 
-// A head's K and V are read by one XCD, whose L2 holds 4 MB: from 32 MB in all upwards they come from further away at every call, and
-// copies that leave no lines behind are faster (us, plain copies and these, on caches that were not just read: 16 x 16 heads, 4096 keys of
-// 128 90.9, 77.1; 10 x 8 heads, 3116 keys 26.8, 24.1; 16 x 16 heads, 465 keys 13.6, 12.2).  Below, a cache that was just read
-// is still there for plain copies (5 x 32 heads, 536 keys of 64, 22 MB 6.0, 6.4).
-constexpr long long kDecOnceBytes = 32LL << 20;
+// From 128 MB of keys and values upwards, half of what the last-level cache holds, the copies leave no lines behind (ONCE): a program that
+// attends to several such caches in turn, a layer each, finds nothing of the next one there, and lines that displace others cost time.  us,
+// plain copies and these: 16 x 16 heads, 4096 keys of 128, 537 MB 90.9, 77.1; 10 x 8 heads, 3116 keys, 128 MB, three and more in turn 26.7,
+// 23.6, alone 22.8, 22.6.  The price is a single cache of almost the size of the last-level one that is read again and again (3 x 12 heads,
+// 13619 keys, 251 MB alone 40.5, 43.3, two and more in turn 49.2, 44.6); smaller ones would pay it as soon as a few fit together (6 x 32 heads, 1267
+// keys of 96, 93 MB, two in turn 15.7, 17.0, six 19.0, 17.6).
+constexpr long long kDecOnceBytes = 128LL << 20;
 
 // nparts workgroups per head, each leaving its part in part_o / part_ml when nparts > 1 (see attn_merge_kernel).
 int launch_decode(const void* Q, const void* K, const void* V, void* O, int BH, int Sq, int Skv, int D, float scale, int nparts,

@@ -1092,8 +1092,8 @@ def test_flash_attention_split_over_the_keys(core, B, Hd, Sq, Skv, D):
     (3, 90, 1, 300, 64),           # more heads than the chip takes at once, no parts
     (1, 1, 16, 9000, 128),         # as many parts as the merge takes
     (1, 5, 2, 4097, 32),
-    (4, 32, 1, 1025, 64),          # just above 32 MB of keys and values: copies that leave no lines in the caches
-    (2, 17, 2, 2500, 96),          # the same, in parts, the last tile ragged
+    (8, 64, 1, 1025, 64),          # just above 128 MB of keys and values: copies that leave no lines in the caches
+    (1, 24, 2, 14600, 96),         # the same, in parts, the last tile ragged
 ])
 def test_flash_attention_few_queries(core, B, Hd, Sq, Skv, D):
     """At most 16 queries a head: the waves of a workgroup cut the keys.  Against float64; the weights are rounded to
