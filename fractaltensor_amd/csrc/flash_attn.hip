@@ -56,13 +56,14 @@ int decode_parts(long long bh, int Skv, int D, int cus, int* part_keys);
 int launch_decode(const void* Q, const void* K, const void* V, void* O, int BH, int Sq, int Skv, int D, float scale, int nparts,
                   int part_keys, float* part_o, float* part_ml, hipStream_t s);
 
-// LDS layout of a tile without padding, for head size 128 with two key groups (padded, their ten tiles take 186 KB): K
-// row r keeps 16-byte chunk c in slot c ^ (r & 15), V row r its 64-byte group g in g ^ (r & 3).
+// LDS layout of a tile without padding, for head size 128 with two key groups and 64 with four (padded, their tiles take 186 and 204 KB).
+// D 128: K row r keeps 16-byte chunk c in slot c ^ (r & 15), V row r its 64-byte group g in g ^ (r & 3); D 64, whose rows are half of
+// the banks: c ^ (r / 2 & 7) and g ^ (r / 2 & 1).
 template <int D>
 struct FaSwizzled {
   static constexpr int KRS = 2 * D, VRS = 2 * D, KTB = FA_KT * KRS, VTB = FA_KT * VRS;
 };
-constexpr bool fa_swizzled(int D, int KG) { return D == 128 && KG == 2; }
+constexpr bool fa_swizzled(int D, int KG) { return (D == 128 && KG == 2) || (D == 64 && KG == 4); }
 
 constexpr float FA_TAU = 8.0f;     // slack (in powers of two) before the running maximum is moved
 // The reference of a key group that has met no finite score: so low that the first one moves it (a reference of 0 would
@@ -85,9 +86,9 @@ __device__ long long fa_trace_buf[FA_TRACE_TILES * 6];
 // PART: the workgroup takes one contiguous range of the keys (part_keys of them, a multiple of the tile) and leaves
 // its unnormalised accumulators, reference maximum and sum of exponentials in part_o / part_ml for attn_merge_kernel:
 // small grids with many keys are split over the keys so that they fill the chip.
-// KG == 2: the workgroup has two groups of WAVES waves for the same query rows.  Each walks half of the keys with tiles of
-// its own in LDS, and the first takes in the second's result at the end: two waves per SIMD where the grid of query
-// blocks does not fill the chip, each with half of the chain of tiles (see launch_fa's callers for where that pays).
+// KG > 1: the workgroup has KG groups of WAVES waves for the same query rows.  Each walks its share of the keys with tiles of
+// its own in LDS, and the first takes in the others' results at the end: two waves per SIMD where the grid of query
+// blocks does not fill the chip, each with a part of the chain of tiles (fa_four_groups, and launch_fa's callers, for where that pays).
 template <int D, int QT, int WAVES, int MINB, bool TRACE, bool RAG, bool PART = false, int KG = 1>
 __global__ __launch_bounds__(WAVES * KG * 64, MINB) void flash_attn_kernel(const _Float16* __restrict__ Q,
                                                          const _Float16* __restrict__ K,
@@ -100,7 +101,7 @@ __global__ __launch_bounds__(WAVES * KG * 64, MINB) void flash_attn_kernel(const
                                                          float* __restrict__ part_ml = nullptr) {
   constexpr bool SWZ = fa_swizzled(D, KG);
   using L = typename std::conditional<SWZ, FaSwizzled<D>, FaLayout<D>>::type;
-  static_assert(KG == 1 || (KG == 2 && QT == 1), "two key groups, one query tile a wave");
+  static_assert(KG == 1 || QT == 1, "key groups: one query tile a wave");
   constexpr int DS = D / 16;  // k steps of S^T
   constexpr int DT = D / 32;  // d tiles of O^T
   constexpr int RB = 2 * D;   // bytes per K or V row in global memory
@@ -133,10 +134,11 @@ __global__ __launch_bounds__(WAVES * KG * 64, MINB) void flash_attn_kernel(const
   const int q_base = qb * (WAVES * 32 * QT) + wave * (32 * QT);
   const int key_wg = PART ? part * part_keys : 0;
   const int Skv_wg = PART ? min(part_keys, Skv_all - key_wg) : Skv_all;   // the keys this workgroup sees
-  // the first group has the first half of the tiles, one more than the second when they are odd (never fewer than two in all)
-  const int first_tiles = ((Skv_wg + FA_KT - 1) / FA_KT + 1) / 2;
-  const int key_first = key_wg + group * first_tiles * FA_KT;
-  const int Skv = KG == 1 ? Skv_wg : group == 0 ? first_tiles * FA_KT : Skv_wg - first_tiles * FA_KT;   // the keys this group sees
+  // the groups have equal shares of the tiles in turn, the first ones a tile more where there is a remainder (never fewer tiles than groups)
+  const int tiles_wg = (Skv_wg + FA_KT - 1) / FA_KT, share = tiles_wg / KG, long_groups = tiles_wg - share * KG;
+  const int most_tiles = share + (long_groups > 0 ? 1 : 0);
+  const int key_group = (group * share + min(group, long_groups)) * FA_KT, key_first = key_wg + key_group;
+  const int Skv = KG == 1 ? Skv_wg : group + 1 < KG ? (share + (group < long_groups ? 1 : 0)) * FA_KT : Skv_wg - key_group;   // the keys this group sees
 
   const _Float16* Qg = Q + (size_t)bh * Sq * D;
   const _Float16* Kg = K + ((size_t)bh * Skv_all + key_first) * D;
@@ -179,14 +181,14 @@ __global__ __launch_bounds__(WAVES * KG * 64, MINB) void flash_attn_kernel(const
   for (int i = 0; i < KCP; ++i) {
     const int x = 1024 * (wave + WAVES * i) + 16 * lane;
     const int row = min(x / KRS, FA_KT - 1), col = x % KRS;
-    if constexpr (SWZ) k_src[i] = row * RB + (col ^ (16 * (row & 15)));
+    if constexpr (SWZ) k_src[i] = row * RB + (col ^ (16 * (D == 128 ? row & 15 : (row >> 1) & 7)));
     else k_src[i] = row * RB + (col < RB ? col : 0);
   }
 #pragma unroll
   for (int i = 0; i < VCP; ++i) {
     const int x = 1024 * (wave + WAVES * i) + 16 * lane;
     const int row = min(x / VRS, FA_KT - 1), col = x % VRS;
-    if constexpr (SWZ) v_src[i] = row * RB + (col ^ (64 * (row & 3)));
+    if constexpr (SWZ) v_src[i] = row * RB + (col ^ (64 * (D == 128 ? row & 3 : (row >> 1) & 1)));
     else v_src[i] = row * RB + (col < RB ? col : 0);
   }
   // copy i (of this wave's share) of K tile kt into the K buffer at dst; no-op past the wave's last copy
@@ -247,9 +249,9 @@ __global__ __launch_bounds__(WAVES * KG * 64, MINB) void flash_attn_kernel(const
   unsigned k_swz[SWZ ? DS : 1], v_swz[SWZ ? DT : 1];
   if constexpr (SWZ) {
 #pragma unroll
-    for (int s = 0; s < DS; ++s) k_swz[s] = (unsigned)(((2 * s + hh) ^ (j & 15)) * 16);
+    for (int s = 0; s < DS; ++s) k_swz[s] = (unsigned)(((2 * s + hh) ^ (D == 128 ? j & 15 : (j >> 1) & 7)) * 16);
 #pragma unroll
-    for (int dt = 0; dt < DT; ++dt) v_swz[dt] = (unsigned)((dt ^ ((lane & 15) >> 2)) * 64);
+    for (int dt = 0; dt < DT; ++dt) v_swz[dt] = (unsigned)((dt ^ (D == 128 ? (lane & 15) >> 2 : (lane & 15) >> 3)) * 64);
   }
 
   const int ntiles = (Skv + FA_KT - 1) / FA_KT;
@@ -468,7 +470,7 @@ __global__ __launch_bounds__(WAVES * KG * 64, MINB) void flash_attn_kernel(const
 #pragma unroll
       for (int r = 1; r < 16; ++r) m = fmaxf(m, sa[qt][r]);
       m = max_with_other_half(m);
-      if (KG == 2 && m == -INFINITY) m = FA_NO_REF;   // no score yet: the group's share must come out as nothing, not as a NaN
+      if (KG > 1 && m == -INFINITY) m = FA_NO_REF;   // no score yet: the group's share must come out as nothing, not as a NaN
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         sa[qt][r] -= m;
@@ -490,7 +492,7 @@ __global__ __launch_bounds__(WAVES * KG * 64, MINB) void flash_attn_kernel(const
     // A wave is held at issue while its copy instructions queue up in the memory pipeline.  With two waves
     // per SIMD the two take turns: the first issues its copies when the step begins, the second after the
     // first half tile, so that one of them always has MFMAs to issue.
-    const bool copy_first = KG == 2 ? group == 0 : WAVES < 8 || wave < WAVES / 2;
+    const bool copy_first = KG > 1 ? 2 * group < KG : WAVES < 8 || wave < WAVES / 2;
     if (copy_first) {
       if (kt + 2 < ntiles) copy_k_all(Kb + kfree, kt + 2);
       if (kt + 1 < ntiles) copy_v_all(Vb + vnext, kt + 1);
@@ -529,40 +531,46 @@ __global__ __launch_bounds__(WAVES * KG * 64, MINB) void flash_attn_kernel(const
     step(ntiles - 1, std::false_type{}, std::false_type{});
   }
 
-  if constexpr (KG == 2) {
-    if (group == 1 && ntiles < first_tiles) __syncthreads();   // the first group's last tile
-    // the second group leaves its accumulators, reference and sum in its part of LDS, by lane; the first takes them in
+  if constexpr (KG > 1) {
+    if (ntiles < most_tiles) __syncthreads();   // the longer groups' last tile
+    // the other groups leave their accumulators, reference and sum each in its part of LDS, by lane; the first takes them in, in turn,
     // by the rule of an online softmax
-    unsigned char* const other = smem + GROUP_LDS;
-    v4f* const oo = reinterpret_cast<v4f*>(other) + wave * (DT * 4 * 64) + lane;
-    float2* const oml = reinterpret_cast<float2*>(other + WAVES * (DT * 4 * 64 * 16)) + wave * 64 + lane;
-    static_assert(WAVES * (DT * 4 * 64 * 16 + 64 * 8) <= GROUP_LDS, "the second group's result fits its tiles' place");
-    if (group == 1) {
+    static_assert(WAVES * (DT * 4 * 64 * 16 + 64 * 8) <= GROUP_LDS, "a group's result fits its tiles' place");
+    auto oo = [&](int of) __attribute__((always_inline)) { return reinterpret_cast<v4f*>(smem + of * GROUP_LDS) + wave * (DT * 4 * 64) + lane; };
+    auto oml = [&](int of) __attribute__((always_inline)) {
+      return reinterpret_cast<float2*>(smem + of * GROUP_LDS + WAVES * (DT * 4 * 64 * 16)) + wave * 64 + lane;
+    };
+    if (group > 0) {
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
         for (int g = 0; g < 4; ++g)
-          oo[(4 * dt + g) * 64] = v4f{oacc[0][dt][4 * g], oacc[0][dt][4 * g + 1], oacc[0][dt][4 * g + 2], oacc[0][dt][4 * g + 3]};
-      *oml = make_float2(-nref[0][0], l_run[0] + __shfl_xor(l_run[0], 32));
+          oo(group)[(4 * dt + g) * 64] = v4f{oacc[0][dt][4 * g], oacc[0][dt][4 * g + 1], oacc[0][dt][4 * g + 2], oacc[0][dt][4 * g + 3]};
+      *oml(group) = make_float2(-nref[0][0], l_run[0] + __shfl_xor(l_run[0], 32));
     }
     __syncthreads();
-    if (group == 1) return;
-    const float2 ml = *oml;
-    const float l_mine = l_run[0] + __shfl_xor(l_run[0], 32), m_mine = -nref[0][0];
-    const float m = !(ml.y > 0.0f) ? m_mine : !(l_mine > 0.0f) ? ml.x : fmaxf(m_mine, ml.x);
-    const float wm = l_mine == 0.0f ? 0.0f : __builtin_amdgcn_exp2f(m_mine - m);
-    const float wo = ml.y == 0.0f ? 0.0f : __builtin_amdgcn_exp2f(ml.x - m);
-    l_run[0] = hh == 0 ? wm * l_mine + wo * ml.y : 0.0f;   // (the lanes' shares are added up below)
+    if (group > 0) return;
+    float l_mine = l_run[0] + __shfl_xor(l_run[0], 32), m_mine = -nref[0][0];
 #pragma unroll
-    for (int r = 0; r < 16; ++r) nref[0][r] = -m;
+    for (int of = 1; of < KG; ++of) {
+      const float2 ml = *oml(of);
+      const float m = !(ml.y > 0.0f) ? m_mine : !(l_mine > 0.0f) ? ml.x : fmaxf(m_mine, ml.x);
+      const float wm = l_mine == 0.0f ? 0.0f : __builtin_amdgcn_exp2f(m_mine - m);
+      const float wo = ml.y == 0.0f ? 0.0f : __builtin_amdgcn_exp2f(ml.x - m);
+      l_mine = wm * l_mine + wo * ml.y;
+      m_mine = m;
 #pragma unroll
-    for (int dt = 0; dt < DT; ++dt)
+      for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const v4f o = oo[(4 * dt + g) * 64];
+        for (int g = 0; g < 4; ++g) {
+          const v4f o = oo(of)[(4 * dt + g) * 64];
 #pragma unroll
-        for (int k = 0; k < 4; ++k) oacc[0][dt][4 * g + k] = wm * oacc[0][dt][4 * g + k] + wo * o[k];
-      }
+          for (int k = 0; k < 4; ++k) oacc[0][dt][4 * g + k] = wm * oacc[0][dt][4 * g + k] + wo * o[k];
+        }
+    }
+    l_run[0] = hh == 0 ? l_mine : 0.0f;   // (the lanes' shares are added up below)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) nref[0][r] = -m_mine;
   }
 
   // ---- normalise and store.  A lane holds d = 32dt + 8g + 4*half + r of its row: 8-byte pieces scattered over
@@ -1143,50 +1151,67 @@ static int launch_merge(const float* part_o, const float* part_ml, void* O, int 
   return check_launch("attn_merge_kernel");
 }
 
-// How many parts the keys are cut into (1: no split): the number that makes the sum of both costs least, in microseconds.
+// Blocks of 64 query rows in two waves, with four key groups, in place of 128 rows in four waves with two: as many waves, for half of the rows, each with
+// half of the tiles.  Where such blocks are at most one to a compute unit every chain is half as long and nothing has to wait for it; with more,
+// two rounds of half the length take as long as one, and longer than that for their prologues (336 blocks, 7 tiles of D 64: 14.4 us, 128 rows 9.6).  Up to
+// D 64: four groups' tiles of larger heads are more than LDS has.  us, 128 rows and 64: D 64, 24 blocks of 128, 4 tiles 6.9, 6.0; 56, 11 10.8, 9.1; 32,
+// 26 16.9, 12.2; 36, 61 33.7, 21.1; D 32, 120 blocks, 10 tiles 8.0, 6.7; 120, 63 29.8, 18.7; 77 grids of at most 256 such blocks 1.06 to 1.6
+// times as fast.  (Three groups to 128 rows at D 64, three waves a SIMD: 18.7 us for B3 H12 S777x1333, 19.7; a wave's vector instructions and
+// MFMAs fill a SIMD with two.  Tiles asked for two steps ahead: no different, so it is not their way that a step waits for.)
+static bool fa_four_groups(long long bh, int Sq, int Skv, int D, int cus) {
+  return D <= 64 && (long long)((Sq + 63) / 64) * bh <= cus && Skv > 3 * FA_KT;   // a key group walks at least one tile
+}
+
+// How many parts the keys are cut into (1: no split), in which blocks, and the keys of a part: what makes the sum of both costs least, in microseconds.
 // A workgroup's chain is half of its tiles (two key groups) of about 0.4 + 0.0095 D each (16 tiles of each group: 15 at
-// D = 64, 26 at 128).  Parts cost the merge's launch and its trip through memory, what every part writes and the merge
-// reads at about 2.5 TB/s (8 heads of 64, 2048 queries and keys: 2 parts take 23.2, one 19.3; 128 queries, 4096 keys: 12.5
-// and 30.5).  At most as many workgroups as compute units, at least four tiles to a part.
-static int fa_split_parts(long long bh, int Sq, int Skv, int D, int cus, int* part_keys) {
-  *part_keys = Skv;
-  if (Sq <= kDecodeQueries) return decode_parts(bh, Skv, D, cus, part_keys);
-  const long long blocks = (long long)((Sq + 127) / 128) * bh;
-  const long long most = std::min<long long>(std::min<long long>(cus / blocks, 64), Skv / (4 * FA_KT));
-  const float chain = (float)Skv / (2 * FA_KT) * (0.4f + 0.0095f * (float)D);
-  const float part = (float)(bh * Sq) * (float)(D + 2) * (8.0f / 2.5e6f);
-  float least = chain;
-  int want = 1;
-  for (int p = 2; p <= most; ++p) {
-    const float cost = chain / (float)p + 6.0f + part * (float)p;
-    if (cost < least) {
-      least = cost;
-      want = p;
-    }
+// D = 64, 26 at 128), or a quarter of 0.75 + 0.0045 D (11 of each of four groups: 11.3 at D 64; 12 at D 32 10.6).  Parts cost the merge's launch and its
+// trip through memory, 4.5 and what every part writes and the merge reads at about 2.5 TB/s (us: 4 heads of 32, 64 queries, 2048 keys: 8 parts 8.3, one
+// 9.8; 8 heads of 64, 300 queries, 2500 keys: 4 parts of four groups 12.0, 8 of two 13.5, one 15.5; 16 heads of 32, 64 queries, 1024 keys: 2 parts 9.5, one
+// 6.5; over 26 grids the choice is 1 % behind the best in the mean, with 6 in place of 4.5 it is 8 %).  At most as many workgroups as compute units, at least two tiles to a key group.
+struct FaSplit {
+  int parts, keys;
+  bool four_groups;
+};
+static FaSplit fa_split_parts(long long bh, int Sq, int Skv, int D, int cus) {
+  FaSplit split = {1, Skv, false};
+  if (Sq <= kDecodeQueries) {
+    split.parts = decode_parts(bh, Skv, D, cus, &split.keys);
+    return split;
   }
-  if (want < 2) return 1;
-  int keys = (int)(((Skv + want - 1) / want + FA_KT - 1) / FA_KT * FA_KT);
-  while ((Skv - 1) % keys < FA_KT) keys += FA_KT;   // the last part has more than a tile too: a key group walks at least one
-  *part_keys = keys;
-  return (Skv + keys - 1) / keys;
+  const float part = (float)(bh * Sq) * (float)(D + 2) * (8.0f / 2.5e6f);
+  const float chain2 = (float)Skv / (2 * FA_KT) * (0.4f + 0.0095f * (float)D), chain4 = (float)Skv / (4 * FA_KT) * (0.75f + 0.0045f * (float)D);
+  float least = fa_four_groups(bh, Sq, Skv, D, cus) ? chain4 : chain2;
+  int want = 1;
+  auto consider = [&](bool four_groups, float chain) {
+    const int rows = four_groups ? 64 : 128, groups = four_groups ? 4 : 2;
+    const long long blocks = (long long)((Sq + rows - 1) / rows) * bh;
+    const long long most = std::min<long long>(std::min<long long>(cus / blocks, 64), Skv / (2 * groups * FA_KT));
+    for (int p = 2; p <= most; ++p) {
+      const float cost = chain / (float)p + 4.5f + part * (float)p;
+      if (cost < least) {
+        least = cost;
+        want = p;
+        split.four_groups = four_groups;
+      }
+    }
+  };
+  consider(false, chain2);
+  if (D <= 64) consider(true, chain4);
+  if (want < 2) return split;
+  const int most_short = ((split.four_groups ? 4 : 2) - 1) * FA_KT;
+  split.keys = (int)(((Skv + want - 1) / want + FA_KT - 1) / FA_KT * FA_KT);
+  while ((Skv - 1) % split.keys < most_short) split.keys += FA_KT;   // the last part has a tile for every key group too
+  split.parts = (Skv + split.keys - 1) / split.keys;
+  return split;
 }
 
 static size_t fa_split_bytes(long long bh, int Sq, int D, int nparts) {
   return (size_t)nparts * bh * Sq * (D + 2) * sizeof(float);
 }
 
-template <int D>
-static int launch_fa_split(const void* Q, const void* K, const void* V, void* O, int BH, int Sq, int Skv, float scale, int nparts,
-                           int part_keys, float* ws, int lds_max, hipStream_t s) {
-  float* part_o = ws;
-  float* part_ml = ws + (size_t)nparts * BH * Sq * D;
-  const long long rows = (long long)BH * Sq;
-  if (Sq <= kDecodeQueries) {
-    const int rc = launch_decode(Q, K, V, O, BH, Sq, Skv, D, scale, nparts, part_keys, part_o, part_ml, s);
-    if (rc) return rc;
-    return launch_merge<D>(part_o, part_ml, O, nparts, Sq, rows, s);
-  }
-  constexpr int WAVES = 4, KG = 2;
+template <int D, int WAVES, int KG>
+static int launch_fa_parts(const void* Q, const void* K, const void* V, int BH, int Sq, int Skv, float scale, int nparts, int part_keys,
+                           float* part_o, float* part_ml, int lds_max, hipStream_t s) {
   using L = typename std::conditional<fa_swizzled(D, KG), FaSwizzled<D>, FaLayout<D>>::type;
   const size_t lds = (size_t)KG * (3 * L::KTB + 2 * L::VTB);
   if ((int)lds > lds_max) return fail(FTK_ERR_UNSUPPORTED_SHAPE, "ftk_flash_attn_ws_f16: needs %zu bytes of LDS", lds);
@@ -1201,20 +1226,37 @@ static int launch_fa_split(const void* Q, const void* K, const void* V, void* O,
   const long long total = (long long)nqb * BH * nparts;
   if (total > 0x7fffffffLL) return fail(FTK_ERR_UNSUPPORTED_SHAPE, "ftk_flash_attn_ws_f16: grid too large");
   hipLaunchKernelGGL((flash_attn_kernel<D, 1, WAVES, 1, false, true, true, KG>), dim3((unsigned)total), dim3(WAVES * KG * 64), lds, s,
-                     (const _Float16*)Q, (const _Float16*)K, (const _Float16*)V, (_Float16*)O, Sq, Skv, scale * 1.4426950408889634f, nqb,
+                     (const _Float16*)Q, (const _Float16*)K, (const _Float16*)V, (_Float16*)nullptr, Sq, Skv, scale * 1.4426950408889634f, nqb,
                      (long long*)nullptr, 0, nparts, part_keys, part_o, part_ml);
-  int rc = check_launch("flash_attn_kernel (key parts)");
-  if (rc) return rc;
-  return launch_merge<D>(part_o, part_ml, O, nparts, Sq, rows, s);
+  return check_launch("flash_attn_kernel (key parts)");
 }
 
-// Tuning hook: FTK_FA_VARIANT=1|2|3 pins the tiling variant (read once).
+template <int D>
+static int launch_fa_split(const void* Q, const void* K, const void* V, void* O, int BH, int Sq, int Skv, float scale, const FaSplit& split,
+                           float* ws, int lds_max, hipStream_t s) {
+  const int nparts = split.parts;
+  float* part_o = ws;
+  float* part_ml = ws + (size_t)nparts * BH * Sq * D;
+  int rc;
+  if (Sq <= kDecodeQueries) {
+    rc = launch_decode(Q, K, V, O, BH, Sq, Skv, D, scale, nparts, split.keys, part_o, part_ml, s);
+  } else if constexpr (D <= 64) {
+    rc = split.four_groups ? launch_fa_parts<D, 2, 4>(Q, K, V, BH, Sq, Skv, scale, nparts, split.keys, part_o, part_ml, lds_max, s)
+                           : launch_fa_parts<D, 4, 2>(Q, K, V, BH, Sq, Skv, scale, nparts, split.keys, part_o, part_ml, lds_max, s);
+  } else {
+    rc = launch_fa_parts<D, 4, 2>(Q, K, V, BH, Sq, Skv, scale, nparts, split.keys, part_o, part_ml, lds_max, s);
+  }
+  if (rc) return rc;
+  return launch_merge<D>(part_o, part_ml, O, nparts, Sq, (long long)BH * Sq, s);
+}
+
+// Tuning hook: FTK_FA_VARIANT=1|2|3|4 pins the tiling variant (read once).
 static int fa_variant_override() {
   static int v = -1;
   if (v < 0) {
     const char* e = getenv("FTK_FA_VARIANT");
     v = e ? atoi(e) : 0;
-    if (v < 1 || v > 3) v = 0;
+    if (v < 1 || v > 4) v = 0;
   }
   return v;
 }
@@ -1239,8 +1281,7 @@ extern "C" size_t ftk_flash_attn_f16_workspace_bytes(int B, int Hd, int Sq, int 
   if (B <= 0 || Hd <= 0 || Sq <= 0 || Skv <= 0 || D <= 0) return 0;
   const DeviceProps* dp = nullptr;
   const int cus = device_props(&dp) == FTK_OK ? dp->cus : 256;   // without a device: the part this library is written for
-  int keys = 0;
-  const int nparts = fa_split_parts((long long)B * Hd, Sq, Skv, D, cus, &keys);
+  const int nparts = fa_split_parts((long long)B * Hd, Sq, Skv, D, cus).parts;
   return nparts > 1 ? fa_split_bytes((long long)B * Hd, Sq, D, nparts) : 0;
 }
 
@@ -1252,17 +1293,16 @@ extern "C" int ftk_flash_attn_ws_f16(const void* Q, const void* K, const void* V
     const DeviceProps* dp = nullptr;
     int rc = device_props(&dp);
     if (rc) return rc;
-    int keys = 0;
     const long long bh = (long long)B * Hd;
-    const int nparts = fa_split_parts(bh, Sq, Skv, D, dp->cus, &keys);
-    if (nparts > 1 && workspace_bytes >= fa_split_bytes(bh, Sq, D, nparts) && reinterpret_cast<uintptr_t>(workspace) % 16 == 0) {
+    const FaSplit split = fa_split_parts(bh, Sq, Skv, D, dp->cus);
+    if (split.parts > 1 && workspace_bytes >= fa_split_bytes(bh, Sq, D, split.parts) && reinterpret_cast<uintptr_t>(workspace) % 16 == 0) {
       hipStream_t s = (hipStream_t)stream;
       float* ws = reinterpret_cast<float*>(workspace);
       switch (D) {
-        case 32: return launch_fa_split<32>(Q, K, V, O, (int)bh, Sq, Skv, scale, nparts, keys, ws, dp->lds_optin, s);
-        case 64: return launch_fa_split<64>(Q, K, V, O, (int)bh, Sq, Skv, scale, nparts, keys, ws, dp->lds_optin, s);
-        case 96: return launch_fa_split<96>(Q, K, V, O, (int)bh, Sq, Skv, scale, nparts, keys, ws, dp->lds_optin, s);
-        default: return launch_fa_split<128>(Q, K, V, O, (int)bh, Sq, Skv, scale, nparts, keys, ws, dp->lds_optin, s);
+        case 32: return launch_fa_split<32>(Q, K, V, O, (int)bh, Sq, Skv, scale, split, ws, dp->lds_optin, s);
+        case 64: return launch_fa_split<64>(Q, K, V, O, (int)bh, Sq, Skv, scale, split, ws, dp->lds_optin, s);
+        case 96: return launch_fa_split<96>(Q, K, V, O, (int)bh, Sq, Skv, scale, split, ws, dp->lds_optin, s);
+        default: return launch_fa_split<128>(Q, K, V, O, (int)bh, Sq, Skv, scale, split, ws, dp->lds_optin, s);
       }
     }
   }
@@ -1285,7 +1325,7 @@ extern "C" int ftk_flash_attn_f16(const void* Q, const void* K, const void* V, v
   hipStream_t s = (hipStream_t)stream;
   if (Sq <= kDecodeQueries) return launch_decode(Q, K, V, O, (int)bh, Sq, Skv, D, scale, 1, Skv, nullptr, nullptr, s);
   // Variant: 0 = choose by problem size, 1 = 4 waves x 32 query rows (interleaved kernel), 2 = the same with two key groups,
-  // 3 = 8 waves x 32 query rows.
+  // 3 = 8 waves x 32 query rows, 4 = 2 waves x 32 query rows with four key groups (fa_four_groups).
   // Two key groups where 128-row blocks are at most one to a compute unit: half of the chain of tiles to each wave, two
   // waves per SIMD, and half the padding of 256-row blocks (us, against 8 waves and 4 waves: B3 H12 S777x1333 D64 18.6,
   // 24.1, 27.0; B2 H12 S700 D96 12.4, 17.2, 16.6; B1 H12 S1536 D64 15.0, 21.3, 23.6; B1 H8 S512 D64 7.7, 9.7, 9.8; B1 H16 S2048
@@ -1294,7 +1334,9 @@ extern "C" int ftk_flash_attn_f16(const void* Q, const void* K, const void* V, v
   // the chip, and also on smaller grids once there are 512 keys or more (B2 H12 S2048 D64 33 against 49 us); with few
   // keys a launch is its own latency and the 128-row blocks spread a short problem over more compute units.
   int variant = fa_variant_override();
-  if (variant == 2 && Skv <= FA_KT) variant = 1;   // a key group walks at least one tile
+  if (variant == 4 && (D > 64 || Skv <= 3 * FA_KT)) variant = 2;   // a key group walks at least one tile
+  if (variant == 2 && Skv <= FA_KT) variant = 1;
+  if (variant == 0 && fa_four_groups(bh, Sq, Skv, D, dp->cus)) variant = 4;
   if (variant == 0 && (long long)((Sq + 127) / 128) * bh <= dp->cus && Skv > 2 * FA_KT) variant = 2;
   if (variant == 0) variant = ((long long)((Sq + 255) / 256) * bh >= dp->cus || Skv >= 512) ? 3 : 1;
   const int lds = dp->lds_optin;
@@ -1313,11 +1355,13 @@ extern "C" int ftk_flash_attn_f16(const void* Q, const void* K, const void* V, v
     return launch_fa_pp<96>(Q, K, V, O, (int)bh, Sq, Skv, scale, lds, s);
   }
   if (D == 64) {
+    if (variant == 4) return launch_fa<64, 1, 2, 1, 4>(Q, K, V, O, (int)bh, Sq, Skv, scale, lds, s);
     if (variant == 2) return launch_fa<64, 1, 4, 1, 2>(Q, K, V, O, (int)bh, Sq, Skv, scale, lds, s);
     if (variant == 1) return launch_fa<64, 1, 4, 1>(Q, K, V, O, (int)bh, Sq, Skv, scale, lds, s);
     return launch_fa_pp<64>(Q, K, V, O, (int)bh, Sq, Skv, scale, lds, s);
   }
   // D = 32: the head dimension of the reference's example program (examples/flash_attention/flash_attention.py:96-110)
+  if (variant == 4) return launch_fa<32, 1, 2, 1, 4>(Q, K, V, O, (int)bh, Sq, Skv, scale, lds, s);
   if (variant == 2) return launch_fa<32, 1, 4, 1, 2>(Q, K, V, O, (int)bh, Sq, Skv, scale, lds, s);
   if (variant == 1) return launch_fa<32, 1, 4, 1>(Q, K, V, O, (int)bh, Sq, Skv, scale, lds, s);
   return launch_fa_pp<32>(Q, K, V, O, (int)bh, Sq, Skv, scale, lds, s);

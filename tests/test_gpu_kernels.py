@@ -1592,6 +1592,30 @@ def test_flash_attention_two_key_groups(core, B, Hd, Sq, Skv, D):
 
 
 @pytest.mark.parametrize('B,Hd,Sq,Skv,D', [
+    (1, 3, 17, 193, 64),           # the fewest keys: a tile for each group, the last one a single key
+    (1, 3, 65, 256, 32),           # a second block of one row; whole tiles
+    (2, 5, 64, 257, 64),           # groups of two tiles, one, one and a single key
+    (2, 2, 200, 448, 64),          # two tiles, two, two and one
+    (4, 16, 256, 511, 64),         # as many blocks as compute units
+    (1, 7, 130, 1025, 32),         # groups of five tiles and four, the last ragged
+    (1, 2, 40, 4097, 64),          # parts of the keys as well, whose last would have fewer tiles than groups
+    (1, 3, 100, 8200, 32),
+])
+def test_flash_attention_four_key_groups(core, B, Hd, Sq, Skv, D):
+    """Small grids of smaller heads: four groups of waves share the keys of 64 query rows.  Against float64, weights and O rounded
+    to fp16; the largest scores in each quarter of the keys in turn."""
+    rng = np.random.default_rng(37)
+    Q, K, V = (rng.standard_normal((B, Hd, s, D)).astype(np.float16) for s in (Sq, Skv, Skv))
+    for quarter in range(4):
+        K2 = K.copy()
+        K2[..., quarter * Skv // 4:(quarter + 1) * Skv // 4, :] *= 3
+        ref = ko.attention(Q[:1, :3], K2[:1, :3], V[:1, :3], D ** -0.5)
+        for split in (True, False):
+            O = core.flash_attention(dev(Q), dev(K2), dev(V), D ** -0.5, split_keys=split)
+            assert ko.max_rel_err(O[:1, :3].float().cpu().numpy(), ref) <= F16_TOL
+
+
+@pytest.mark.parametrize('B,Hd,Sq,Skv,D', [
     (1, 2, 100, 129, 32),          # key groups of two tiles and a single key
     (2, 3, 129, 192, 64),          # two tiles and one
     (1, 5, 300, 321, 64),          # the second group a tile shorter, and ragged
