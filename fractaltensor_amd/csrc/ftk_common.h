@@ -145,14 +145,17 @@ __device__ __forceinline__ float sigmoid_f(float x) {
   return __builtin_amdgcn_rcpf(1.0f + fast_exp(-x));
 }
 
-// tanh(x) = 1 - 2/(1+e^{2x}) loses relative accuracy near 0 (the result is the
-// difference of two numbers close to 1), so small arguments use the odd Taylor
-// polynomial instead; the switch point keeps both branches below 2e-7 relative.
+// tanh(x) = 1 - 2/(1+e^{2x}) loses relative accuracy near 0 (the result is the difference of two numbers close to 1), so small
+// arguments use a polynomial instead; the switch point keeps both branches below 2e-7 relative.  x + x z q(z), z = x^2, with the
+// quadratic q whose largest relative error up to the switch is least (2.9e-9; found by weighted least squares): 6.2e-8 in fp32
+// arithmetic, where x (1 + z q) with the Taylor series to x^9, an instruction more, had 8.9e-8 (rms 2.3e-8, 2.8e-8).
+__device__ __forceinline__ float tanh_exp2x(float x) { return __builtin_amdgcn_exp2f(x * 2.8853900817779268f); }   // e^{2x}
+__device__ __forceinline__ float tanh_zq(float z) {
+  return z * __builtin_fmaf(z, __builtin_fmaf(z, -0.05143002858f, 0.13324236628f), -0.33333240088f);
+}
 __device__ __forceinline__ float tanh_f(float x) {
-  const float big = 1.0f - 2.0f * __builtin_amdgcn_rcpf(1.0f + fast_exp(2.0f * x));
-  const float x2 = x * x;
-  const float small =
-      x * (1.0f + x2 * (-0.33333333333f + x2 * (0.13333333333f + x2 * (-0.05396825397f + x2 * 0.02186948854f))));
+  const float big = 1.0f - 2.0f * __builtin_amdgcn_rcpf(1.0f + tanh_exp2x(x));
+  const float small = __builtin_fmaf(x, tanh_zq(x * x), x);
   return fabsf(x) < 0.25f ? small : big;
 }
 

@@ -1066,18 +1066,18 @@ void lstm_persistent_kernel(PersistArgs a) {
           if constexpr (g == 0) {
             eg_i = inv1p(v);
             tc_v = sb.z * em[12 + r] + sb.w;
-            tc_e = fast_exp(2.0f * tc_v);
+            tc_e = tanh_exp2x(tc_v);
             tc_x2 = tc_v * tc_v;
           }
           if constexpr (g == 1) {
             eg_f = inv1p(v);
-            tc_p = -0.33333333333f + tc_x2 * (0.13333333333f + tc_x2 * (-0.05396825397f + tc_x2 * 0.02186948854f));
+            tc_p = tanh_zq(tc_x2);
             tc_r = __builtin_amdgcn_rcpf(1.0f + tc_e);
           }
           if constexpr (g == 2) {
             eg_o = inv1p(v);
             const float big = 1.0f - 2.0f * tc_r;
-            const float small = tc_v * (1.0f + tc_x2 * tc_p);
+            const float small = __builtin_fmaf(tc_v, tc_p, tc_v);
             const float cand = fabsf(tc_v) < 0.25f ? small : big;   // tanh_f, in three parts
             cv[r] = eg_f * cpv[r] + eg_i * cand;
           }
