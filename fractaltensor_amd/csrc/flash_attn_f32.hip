@@ -7,14 +7,14 @@
 //   v * 2^e = top + rest,  top = fp16(v * 2^e),  rest = fp16(v * 2^e - top),
 // and top * top, top * rest and rest * top go into one fp32 accumulator; rest * rest, 2^-22 of a product, is
 // dropped.  What shares a power-of-two scale 2^e (its largest magnitude lands in [2^14, 2^15)): a row of Q, all
-// of K of one (batch, head), all of V of one (batch, head), and the fixed 2^7 for the softmax weights p in
-// [0, 2^8).  The two planes hold an element to within 2^-40 of its group's largest magnitude (2^-29 where the
+// of K of one (batch, head), all of V of one (batch, head) (DIRECT: a tile of K, V up to the tile), and the fixed
+// 2^7 for the softmax weights p in [0, 2^8).  The two planes hold an element to within 2^-40 of its group's largest magnitude (2^-29 where the
 // matrix unit flushes an fp16 subnormal: the remainder of an element below 2^-17 of the largest is one), which is
 // what a sum of products is accurate to anyway: 22 significant bits of its own are kept by every element within
 // 2^-17 of the largest.
 //
-// Launches, where the attention kernel does not cut K and V itself (DIRECT): the largest |K| and |V| per (batch, head) and the split of K and V into planes [row][top D | rest D] in the
-// workspace, in one launch where heads are small, else in two; the attention kernel, which splits its rows of Q (times scale * log2 e)
+// Launches, where the attention kernel does not cut K and V itself (DIRECT): the largest |K| and |V| per (batch, head)
+// and the split of K and V into planes [row][top D | rest D] in the workspace, in one launch where heads are small, else in two; the attention kernel, which splits its rows of Q (times scale * log2 e)
 // itself, in registers.  A plane row is an fp16 row of 2 D
 // elements, so tiles, copies and fragment reads are those of the fp16 kernel at twice the head dimension
 // (fa_common.h), and the contractions are its transposed ones: S^T = K Q^T, O^T += V^T P^T, a lane owns one query
