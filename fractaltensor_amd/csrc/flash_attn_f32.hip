@@ -1060,6 +1060,13 @@ extern "C" int ftk_flash_attn_f32(const float* Q, const float* K, const float* V
   if (workspace_bytes >= cut.total) w = cut;
   else if (workspace_bytes >= whole.total) w = whole;
   if (workspace_bytes < cut.total && split.parts > 1) split = {4, D <= 64 && bh * nqb <= dp->cus && Skv > 2 * FA_KT ? 2 : 1, 1, false};
+  // An O that takes the place of K or V (or of part of them) is written when every row of theirs has gone into the planes
+  auto over_o = [&](const float* kv) {
+    const uintptr_t o = reinterpret_cast<uintptr_t>(O), at = reinterpret_cast<uintptr_t>(kv);
+    const size_t row = (size_t)bh * D * sizeof(float);
+    return o < at + row * Skv && at < o + row * Sq;
+  };
+  if (over_o(K) || over_o(V)) split.direct = false;
   hipStream_t s = (hipStream_t)stream;
   char* ws = reinterpret_cast<char*>(workspace);
   switch (D) {

@@ -530,7 +530,8 @@ int ftk_flash_attn_ws_f16(const void* Q, const void* K, const void* V, void* O,
  * query block's keys are not shared: grids of few query blocks are slower,
  * and the last bits of O differ (the sums are taken in another order).  Up to
  * three small launches precede the attention kernel, none on small grids, whose
- * workgroups split K and V themselves and leave the workspace alone.  The reference has no
+ * workgroups split K and V themselves and leave the workspace alone (unless O
+ * overlaps K or V: an O in the place of Q, K or V is fine).  The reference has no
  * device kernel for this program.
  */
 size_t ftk_flash_attn_f32_workspace_bytes(int B, int Hd, int Sq, int Skv, int D);

@@ -1744,3 +1744,17 @@ def test_flash_attention_f32_that_cuts_its_tiles_itself(core, B, Hd, Sq, Skv, D)
     for by in (2.0 ** 90, 2.0 ** -80):
         assert torch.equal(core.flash_attention_f32(Q, K, V * by), O * by)
     assert torch.equal(core.flash_attention_f32(Q * 2.0 ** 40, K * 2.0 ** -40, V), O)
+
+
+@pytest.mark.parametrize('B,Hd,S,D', [(1, 3, 70, 32), (2, 8, 468, 32), (6, 8, 590, 64), (4, 17, 243, 96), (3, 23, 186, 128)])
+def test_flash_attention_f32_in_the_place_of_an_operand(core, B, Hd, S, D):
+    """`out` may be Q, K or V: sizes whose workgroups would cut K and V themselves while others write O.  Against float64 within 1e-5 of
+    a row's largest (22 bits of each factor, fp32 sums)."""
+    gen = torch.Generator(device='cuda').manual_seed(28)
+    Q, K, V = (torch.randn((B, Hd, S, D), generator=gen, device='cuda') for _ in range(3))
+    ref = torch.softmax(torch.matmul(Q.double().cpu(), K.double().cpu().transpose(2, 3)) * D ** -0.5, -1) @ V.double().cpu()
+    for place in range(3):
+        operands = [x.clone() for x in (Q, K, V)]
+        O = core.flash_attention_f32(*operands, out=operands[place])
+        assert O.data_ptr() == operands[place].data_ptr()
+        assert float(((O.double().cpu() - ref).abs().amax(-1) / ref.abs().amax(-1)).max()) <= 1e-5
