@@ -45,6 +45,11 @@ __device__ __forceinline__ void split_scale(unsigned max_bits, float* scale, flo
   *inv = __uint_as_float((unsigned)(eb - kF32Top) << 23);
 }
 
+// What undoes the scales of a row of Q and of K in a score.  Above zero also where both scales stand at their bound, as those of a row of zeros and
+// of keys of zeros do (a sample shorter than its batch): a masked key's score of -inf times zero would be a NaN.  A raw score is below 2^38, so what
+// is raised here was below 2^-88 and stays there.
+__device__ __forceinline__ float undo_scales(float q_undo, float k_undo) { return fmaxf(q_undo * k_undo, 0x1p-126f); }
+
 __device__ __forceinline__ int clamped_eb(int eb) { return min(max(eb, 15), 254 - kF32Top); }   // the exponent field that split_scale goes by
 
 // The two launches of larger heads: largest |x| of every chunk of every (batch, head) of K and V, as float bits (which order like
@@ -373,7 +378,7 @@ __global__ __launch_bounds__(KG * WAVES * 64, KG == 1 && D <= 64 ? 2 : 1) void f
     if constexpr (!DIRECT) {
       float k_scale, k_inv;
       split_scale(kv_bits[bh], &k_scale, &k_inv);
-      s_mul = q_inv * k_inv;
+      s_mul = undo_scales(q_inv, k_inv);
     }
   }
   [[maybe_unused]] float v_scale, v_inv;
@@ -630,7 +635,7 @@ __global__ __launch_bounds__(KG * WAVES * 64, KG == 1 && D <= 64 ? 2 : 1) void f
       __builtin_amdgcn_sched_barrier(0);
     });
     if constexpr (MAXIMA) {
-      if constexpr (DIRECT) s_mul = q_undo * k_undo;   // (from here on `raw` is of the tile that `am` is of)
+      if constexpr (DIRECT) s_mul = undo_scales(q_undo, k_undo);   // (from here on `raw` is of the tile that `am` is of)
       mx = max_with_other_half(mx) * s_mul;   // finite: the half holds at least one key; s_mul > 0
       if (__builtin_amdgcn_ballot_w64(mx > m_ref + kLazyBits) != 0) {   // a row of the wave moves its reference
         const bool moves = mx > m_ref + kLazyBits;

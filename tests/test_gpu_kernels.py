@@ -1758,3 +1758,34 @@ def test_flash_attention_f32_in_the_place_of_an_operand(core, B, Hd, S, D):
         O = core.flash_attention_f32(*operands, out=operands[place])
         assert O.data_ptr() == operands[place].data_ptr()
         assert float(((O.double().cpu() - ref).abs().amax(-1) / ref.abs().amax(-1)).max()) <= 1e-5
+
+
+@pytest.mark.parametrize('B,Hd,Sq,Skv,D', [
+    (1, 3, 70, 65, 32),          # two key groups, the last tile of one key
+    (2, 8, 1000, 961, 32),       # four key groups
+    (1, 7, 130, 1025, 32),       # parts
+    (1, 12, 100, 100, 64),       # a sample padded to its batch
+    (6, 8, 590, 593, 64),
+    (4, 17, 243, 243, 96),
+    (2, 3, 200, 333, 96),        # parts
+    (2, 5, 90, 100, 128),
+    (3, 23, 186, 161, 128),
+])
+def test_flash_attention_f32_of_rows_and_keys_of_zeros(core, B, Hd, Sq, Skv, D):
+    """Rows of Q and the last keys of K that are zeros, or so small that the scales of both stand at or near their bound, one head of all zeros, with masked
+    keys in the last tile; an output in the place of K takes the planes.  Against float64 within 1e-5 of a row's largest (22 bits of each
+    factor, fp32 sums)."""
+    gen = torch.Generator(device='cuda').manual_seed(29)
+    Q, K, V = (torch.randn((B, Hd, s, D), generator=gen, device='cuda') for s in (Sq, Skv, Skv))
+    for q_by, k_by in ((0.0, 0.0), (0.0, 2.0 ** -30), (2.0 ** -30, 0.0), (2.0 ** -60, 2.0 ** -70)):
+        Q2, K2 = Q.clone(), K.clone()
+        Q2[:, :, Sq // 3:] *= q_by
+        K2[:, :, (Skv - 1) // 64 * 64:] *= k_by
+        Q2[0, 0] *= q_by
+        K2[0, 0] *= k_by
+        ref = torch.softmax(torch.matmul(Q2.double().cpu(), K2.double().cpu().transpose(2, 3)) * D ** -0.5, -1) @ V.double().cpu()
+        flat = torch.empty(max(Q2.numel(), K2.numel()), device='cuda')
+        K_there = flat[:K2.numel()].view(K2.shape).copy_(K2)
+        for k, out in ((K2, None), (K_there, flat[:Q2.numel()].view(Q2.shape))):
+            O = core.flash_attention_f32(Q2, k, V, out=out)
+            assert float(((O.double().cpu() - ref).abs().amax(-1) / ref.abs().amax(-1)).max()) <= 1e-5   # (a NaN fails this too)
