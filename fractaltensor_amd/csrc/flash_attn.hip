@@ -134,11 +134,17 @@ __global__ __launch_bounds__(WAVES * KG * 64, MINB) void flash_attn_kernel(const
   const int q_base = qb * (WAVES * 32 * QT) + wave * (32 * QT);
   const int key_wg = PART ? part * part_keys : 0;
   const int Skv_wg = PART ? min(part_keys, Skv_all - key_wg) : Skv_all;   // the keys this workgroup sees
-  // the groups have equal shares of the tiles in turn, the first ones a tile more where there is a remainder (never fewer tiles than groups)
+  // Equal shares of the tiles in turn, the first groups a tile more where there is a remainder (never fewer tiles than groups).  PAIR: two groups
+  // have a form of their own of this and of the merge below, of which the compiler makes faster code from D 64 upwards (us, this form and the
+  // general one: B3 H12 S777x1333 D64 16.6, 16.8; B8 H8 S500x777 D64 12.1, 12.2; B2 H12 S700 D96 12.0, 12.1; B2 H12 S1200x900 D32 10.3, 10.2).
+  constexpr bool PAIR = KG == 2 && D > 32;
   const int tiles_wg = (Skv_wg + FA_KT - 1) / FA_KT, share = tiles_wg / KG, long_groups = tiles_wg - share * KG;
-  const int most_tiles = share + (long_groups > 0 ? 1 : 0);
-  const int key_group = (group * share + min(group, long_groups)) * FA_KT, key_first = key_wg + key_group;
-  const int Skv = KG == 1 ? Skv_wg : group + 1 < KG ? (share + (group < long_groups ? 1 : 0)) * FA_KT : Skv_wg - key_group;   // the keys this group sees
+  const int most_tiles = PAIR ? (tiles_wg + 1) / 2 : share + (long_groups > 0 ? 1 : 0);
+  const int key_group = (group * share + min(group, long_groups)) * FA_KT;
+  const int key_first = key_wg + (PAIR ? group * most_tiles * FA_KT : key_group);
+  const int Skv = KG == 1   ? Skv_wg   // the keys this group sees
+                  : PAIR    ? (group == 0 ? most_tiles * FA_KT : Skv_wg - most_tiles * FA_KT)
+                            : (group + 1 < KG ? (share + (group < long_groups ? 1 : 0)) * FA_KT : Skv_wg - key_group);
 
   const _Float16* Qg = Q + (size_t)bh * Sq * D;
   const _Float16* Kg = K + ((size_t)bh * Skv_all + key_first) * D;
@@ -531,10 +537,43 @@ __global__ __launch_bounds__(WAVES * KG * 64, MINB) void flash_attn_kernel(const
     step(ntiles - 1, std::false_type{}, std::false_type{});
   }
 
-  if constexpr (KG > 1) {
-    if (ntiles < most_tiles) __syncthreads();   // the longer groups' last tile
-    // the other groups leave their accumulators, reference and sum each in its part of LDS, by lane; the first takes them in, in turn,
+  if constexpr (PAIR) {
+    if (group == 1 && ntiles < most_tiles) __syncthreads();   // the first group's last tile
+    // the second group leaves its accumulators, reference and sum in its part of LDS, by lane; the first takes them in
     // by the rule of an online softmax
+    unsigned char* const other = smem + GROUP_LDS;
+    v4f* const oo = reinterpret_cast<v4f*>(other) + wave * (DT * 4 * 64) + lane;
+    float2* const oml = reinterpret_cast<float2*>(other + WAVES * (DT * 4 * 64 * 16)) + wave * 64 + lane;
+    static_assert(WAVES * (DT * 4 * 64 * 16 + 64 * 8) <= GROUP_LDS, "the second group's result fits its tiles' place");
+    if (group == 1) {
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+          oo[(4 * dt + g) * 64] = v4f{oacc[0][dt][4 * g], oacc[0][dt][4 * g + 1], oacc[0][dt][4 * g + 2], oacc[0][dt][4 * g + 3]};
+      *oml = make_float2(-nref[0][0], l_run[0] + __shfl_xor(l_run[0], 32));
+    }
+    __syncthreads();
+    if (group == 1) return;
+    const float2 ml = *oml;
+    const float l_mine = l_run[0] + __shfl_xor(l_run[0], 32), m_mine = -nref[0][0];
+    const float m = !(ml.y > 0.0f) ? m_mine : !(l_mine > 0.0f) ? ml.x : fmaxf(m_mine, ml.x);
+    const float wm = l_mine == 0.0f ? 0.0f : __builtin_amdgcn_exp2f(m_mine - m);
+    const float wo = ml.y == 0.0f ? 0.0f : __builtin_amdgcn_exp2f(ml.x - m);
+    l_run[0] = hh == 0 ? wm * l_mine + wo * ml.y : 0.0f;   // (the lanes' shares are added up below)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) nref[0][r] = -m;
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const v4f o = oo[(4 * dt + g) * 64];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) oacc[0][dt][4 * g + k] = wm * oacc[0][dt][4 * g + k] + wo * o[k];
+      }
+  } else if constexpr (KG > 1) {
+    if (ntiles < most_tiles) __syncthreads();   // the longer groups' last tile
+    // the same with any number of others, taken in one after the other
     static_assert(WAVES * (DT * 4 * 64 * 16 + 64 * 8) <= GROUP_LDS, "a group's result fits its tiles' place");
     auto oo = [&](int of) __attribute__((always_inline)) { return reinterpret_cast<v4f*>(smem + of * GROUP_LDS) + wave * (DT * 4 * 64) + lane; };
     auto oml = [&](int of) __attribute__((always_inline)) {
