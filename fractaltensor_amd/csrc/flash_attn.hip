@@ -1203,10 +1203,12 @@ static bool fa_four_groups(long long bh, int Sq, int Skv, int D, int cus) {
 
 // How many parts the keys are cut into (1: no split), in which blocks, and the keys of a part: what makes the sum of both costs least, in microseconds.
 // A workgroup's chain is half of its tiles (two key groups) of about 0.4 + 0.0095 D each (16 tiles of each group: 15 at
-// D = 64, 26 at 128), or a quarter of 0.75 + 0.0045 D (11 of each of four groups: 11.3 at D 64; 12 at D 32 10.6).  Parts cost the merge's launch and its
-// trip through memory, 4.5 and what every part writes and the merge reads at about 2.5 TB/s (us: 4 heads of 32, 64 queries, 2048 keys: 8 parts 8.3, one
-// 9.8; 8 heads of 64, 300 queries, 2500 keys: 4 parts of four groups 12.0, 8 of two 13.5, one 15.5; 16 heads of 32, 64 queries, 1024 keys: 2 parts 9.5, one
-// 6.5; over 26 grids the choice is 1 % behind the best in the mean, with 6 in place of 4.5 it is 8 %).  At most as many workgroups as compute units, at least two tiles to a key group.
+// D = 64, 26 at 128), or a quarter of 0.55 + 0.0109 D (5 and 6 of each of four groups: 9.8 and 10.9 at D 64).  Parts cost the merge's launch and its
+// trip through memory, 2.5 and what every part writes and the merge reads at about 2.5 TB/s, and 0.25 where four groups' blocks of at most 64
+// queries are no more than the others'.  Fitted to 220 grids of 1 to 64 heads, 17 to 4096 queries and 200 to 8192 keys with up to 14 splits each: the choice
+// is 0.3, 0.2, 0.2 and 0.5 % behind the best in the mean at D 32, 64, 96 and 128, 5 % at the most.  (With 4.5 for the merge and 0.75 + 0.0045 D, four groups
+// without parts were taken too often at D 64, 24 % behind at the most; us, that and this: 16 heads, 40 queries, 1795 keys 12.7, 10.2; 4 heads, 140, 1743
+// 12.2, 11.0; 3 heads, 3056, 7165 33.2, 30.4.)  At most as many workgroups as compute units, at least two tiles to a key group.
 struct FaSplit {
   int parts, keys;
   bool four_groups;
@@ -1218,15 +1220,16 @@ static FaSplit fa_split_parts(long long bh, int Sq, int Skv, int D, int cus) {
     return split;
   }
   const float part = (float)(bh * Sq) * (float)(D + 2) * (8.0f / 2.5e6f);
-  const float chain2 = (float)Skv / (2 * FA_KT) * (0.4f + 0.0095f * (float)D), chain4 = (float)Skv / (4 * FA_KT) * (0.75f + 0.0045f * (float)D);
+  const float chain2 = (float)Skv / (2 * FA_KT) * (0.4f + 0.0095f * (float)D), chain4 = (float)Skv / (4 * FA_KT) * (0.55f + 0.0109f * (float)D);
   float least = fa_four_groups(bh, Sq, Skv, D, cus) ? chain4 : chain2;
   int want = 1;
   auto consider = [&](bool four_groups, float chain) {
+    const float merge = four_groups && Sq <= 64 ? 2.75f : 2.5f;
     const int rows = four_groups ? 64 : 128, groups = four_groups ? 4 : 2;
     const long long blocks = (long long)((Sq + rows - 1) / rows) * bh;
     const long long most = std::min<long long>(std::min<long long>(cus / blocks, 64), Skv / (2 * groups * FA_KT));
     for (int p = 2; p <= most; ++p) {
-      const float cost = chain / (float)p + 4.5f + part * (float)p;
+      const float cost = chain / (float)p + merge + part * (float)p;
       if (cost < least) {
         least = cost;
         want = p;

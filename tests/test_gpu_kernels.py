@@ -1598,8 +1598,9 @@ def test_flash_attention_two_key_groups(core, B, Hd, Sq, Skv, D):
     (2, 2, 200, 448, 64),          # two tiles, two, two and one
     (4, 16, 256, 511, 64),         # as many blocks as compute units
     (1, 7, 130, 1025, 32),         # groups of five tiles and four, the last ragged
-    (1, 2, 40, 4097, 64),          # parts of the keys as well, whose last would have fewer tiles than groups
-    (1, 3, 100, 8200, 32),
+    (1, 2, 40, 4097, 64),          # parts of the keys, in blocks with two groups
+    (1, 3, 100, 8200, 32),         # parts of the keys as well
+    (1, 5, 70, 4708, 64),          # the same, whose last would have fewer tiles than groups
 ])
 def test_flash_attention_four_key_groups(core, B, Hd, Sq, Skv, D):
     """Small grids of smaller heads: four groups of waves share the keys of 64 query rows.  Against float64, weights and O rounded
