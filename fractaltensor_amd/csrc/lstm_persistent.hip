@@ -1956,6 +1956,8 @@ int ftk_stacked_lstm_f16(const void* xs, const void* WU, const float* bias, cons
   if (L <= 0 || T <= 0 || B <= 0 || H <= 0) return fail(FTK_ERR_INVALID_ARGUMENT, "%s: L, T, B, H must be positive", who);
   if (H % 32) return fail(FTK_ERR_UNSUPPORTED_SHAPE, "%s: H=%d must be a multiple of 32", who, H);
   if ((long long)B * H >= (1ll << 30)) return fail(FTK_ERR_UNSUPPORTED_SHAPE, "%s: B*H = %lld is too large", who, (long long)B * H);
+  // (the pieces of 16 bytes that a layer's weights are re-laid in, H * H of them, are counted in 32 bits)
+  if (H >= 1 << 16) return fail(FTK_ERR_UNSUPPORTED_SHAPE, "%s: H=%d is too large", who, H);
   // the persistent kernel holds the weights of H = 512, and of H = 256 with two batch rows per tile row (even B)
   const bool on_chip = !f16_streams(L, B, H, active_rows != nullptr);
   const int mode = H == PH ? kHalfData256 : kHalfData;

@@ -202,7 +202,7 @@ int ftk_stacked_lstm_ragged_f32(const float* xs, const float* WU,
  * The stack with fp16 storage, the numeric form of the reference's CuTe LSTM:
  * xs [T,B,H], WU [L,2H,4H], hsss, csss [L,T,B,H] all fp16 (h and c are rounded
  * to fp16 when written, and read back rounded), bias [L,4H] fp32 or NULL, gate
- * sums accumulated in fp32.  H%32==0.  H = 256, 512 and 1024, the hidden sizes
+ * sums accumulated in fp32.  H%32==0, H below 65536.  H = 256, 512 and 1024, the hidden sizes
  * of the reference's sweep, keep the fp16 weights of as many layers on the
  * chip as it holds and run deeper stacks as consecutive launches, where that
  * is the faster way.  Every other shape streams its weights through the fp16

@@ -69,6 +69,10 @@ def test_argument_errors_come_back_as_codes_not_crashes():
     assert lib.ftk_stacked_lstm_f16(one, one, nul, nul, nul, one, one, ci(1), ci(1), ci(4), ci(80), nul, ctypes.c_size_t(0), nul) == -2
     # a shape whose weights are streamed needs the workspace for their re-laid copy
     assert lib.ftk_stacked_lstm_f16(one, one, nul, nul, nul, one, one, ci(2), ci(3), ci(4), ci(1024), nul, ctypes.c_size_t(0), nul) == -3
+    # a layer of 2^32 16-byte pieces or more cannot be re-laid, with a workspace of any size
+    assert lib.ftk_stacked_lstm_f16(one, one, nul, nul, nul, one, one, ci(1), ci(1), ci(1), ci(65504), nul, ctypes.c_size_t(0), nul) == -3
+    for H in (65536, 65568, 131072):
+        assert lib.ftk_stacked_lstm_f16(one, one, nul, nul, nul, one, one, ci(1), ci(1), ci(1), ci(H), nul, ctypes.c_size_t(0), nul) == -2
     # the status block (256 bytes, its first int the status word) and the re-laid weights
     assert lib.ftk_stacked_lstm_f16_workspace_bytes(2, 3, 4, 1024) == 256 + 2 * 2048 * 4096 * 2
     # per-call options: an unknown products mode, a negative poll limit; the status query without a workspace
