@@ -1621,7 +1621,7 @@ def test_flash_attention_four_key_groups(core, B, Hd, Sq, Skv, D):
     (2, 3, 129, 192, 64),          # two tiles and one
     (1, 5, 300, 321, 64),          # the second group a tile shorter, and ragged
     (3, 2, 64, 1024, 32),          # equal groups
-    (1, 1, 16, 5, 32),             # planes of less than a workgroup's share
+    (1, 1, 16, 5, 32),             # a single tile of five keys
     (1, 1, 32, 4100, 32),          # a head just above what one launch makes the planes of
     (2, 2, 40, 1000, 128),         # head sizes without key groups
     (1, 3, 33, 77, 96),
@@ -1689,11 +1689,11 @@ def test_b2b_gemm_wide_with_several_column_tiles(core, G, M, N, K, P):
 @pytest.mark.parametrize('B,Hd,Sq,Skv,D', [
     (1, 1, 1, 1025, 32),         # seventeen tiles, the last of one key
     (2, 8, 1024, 1024, 32),      # four key groups to 64 query rows
-    (1, 9, 70, 321, 32),         # the same, with six tiles for four groups, the last of one key
+    (1, 9, 70, 321, 32),         # two key groups to 64 query rows, the last tile of one key
     (1, 2, 130, 1000, 64),       # few query blocks, a ragged tile
     (2, 8, 1000, 1024, 64),      # two key groups to 64 query rows
     (1, 16, 1152, 1152, 64),     # more than half a block to a compute unit
-    (3, 16, 1300, 700, 64),      # heads that take two launches in front
+    (3, 16, 1300, 700, 64),      # more blocks than compute units
     (2, 3, 300, 1100, 96),
     (1, 1, 128, 4097, 128),      # as many parts as there may be
     (1, 5, 257, 640, 128),
@@ -1745,6 +1745,32 @@ def test_flash_attention_f32_that_cuts_its_tiles_itself(core, B, Hd, Sq, Skv, D)
     for by in (2.0 ** 90, 2.0 ** -80):
         assert torch.equal(core.flash_attention_f32(Q, K, V * by), O * by)
     assert torch.equal(core.flash_attention_f32(Q * 2.0 ** 40, K * 2.0 ** -40, V), O)
+
+
+@pytest.mark.parametrize('B,Hd,Sq,Skv,D', [
+    (1, 9, 1000, 513, 32),       # four key groups: three tiles, two, two and two, the last of one key
+    (2, 8, 468, 1090, 32),       # five, five, four and four, the last of two keys
+    (1, 9, 700, 385, 32),        # two, two, two and a single key
+    (2, 8, 1000, 1024, 32),      # equal ones
+    (1, 1, 16, 5, 32),           # planes of less than a workgroup's share
+    (3, 16, 1300, 700, 64),      # planes that take two launches
+])
+def test_flash_attention_f32_uneven_key_groups_with_and_without_planes(core, B, Hd, Sq, Skv, D):
+    """Workgroups that cut K and V themselves and, with O in the place of K, the launches in front and their planes.  The largest scores and
+    values in each quarter of the keys in turn, against float64 within 1e-5 of a row's largest (22 bits of each factor, fp32 sums)."""
+    gen = torch.Generator(device='cuda').manual_seed(30)
+    Q, K, V = (torch.randn((B, Hd, s, D), generator=gen, device='cuda') for s in (Sq, Skv, Skv))
+    flat = torch.empty(max(Q.numel(), K.numel()), device='cuda')
+    for quarter in range(4):
+        at = slice(quarter * Skv // 4, (quarter + 1) * Skv // 4)
+        K2, V2 = K.clone(), V.clone()
+        K2[..., at, :] *= 3
+        V2[..., at, :] *= 2.0 ** 10
+        ref = torch.softmax(torch.matmul(Q.double().cpu(), K2.double().cpu().transpose(2, 3)) * D ** -0.5, -1) @ V2.double().cpu()
+        K_there = flat[:K2.numel()].view(K2.shape).copy_(K2)
+        for k, out in ((K2, None), (K_there, flat[:Q.numel()].view(Q.shape))):
+            O = core.flash_attention_f32(Q, k, V2, out=out)
+            assert float(((O.double().cpu() - ref).abs().amax(-1) / ref.abs().amax(-1)).max()) <= 1e-5
 
 
 @pytest.mark.parametrize('B,Hd,S,D', [(1, 3, 70, 32), (2, 8, 468, 32), (6, 8, 590, 64), (4, 17, 243, 96), (3, 23, 186, 128)])
