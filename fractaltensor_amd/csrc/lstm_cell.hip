@@ -1260,10 +1260,10 @@ int run_wavefront_f16(const void* xs, const void* WU, const float* bias, const i
     return run_wavefront_of<_Float16, CellListH>((const _Float16*)xs, (const _Float16*)packed, bias, dil, (_Float16*)hsss, (_Float16*)csss, L, T, B,
                                                  H, s, true, active);
   // A stage reads the weights of min(L, T) layers, and the next stage reads them again.  What the last-level cache (256 MB) holds of
-  // them is worth having up to half as much again; beyond that, lines that are displaced before they are read again cost more
-  // (ms, T 64, copies of the weights that leave lines and that do not: 134 MB 3.82, 4.03; 335 MB 6.83, 6.83; 403 MB 8.20, 8.10; 537 MB
-  // 10.70, 10.49).
-  const bool once = (long long)std::min(L, T) * 16 * H * H > 384LL << 20;
+  // them is worth having up to a quarter as much again; beyond that, lines that are displaced before they are read again cost more
+  // (ms, T 64, B 256, H 1024, copies of the weights that leave lines and that do not: 201 MB 4.27, 4.70; 268 MB 5.43, 5.62; 302 MB 6.12, 5.99, at
+  // T 18 3.35, 3.39, H 768 6.49, 6.57; 336 MB 6.73, 6.56, B 192 6.48, 6.28, H 2048 7.49, 7.28; 403 MB 7.96, 7.58, H 2048 8.02, 7.68, B 160 6.50, 6.50).
+  const bool once = (long long)std::min(L, T) * 16 * H * H >= 320LL << 20;
   static DeviceOnce attr_once;
   unsigned attr_bit;
   if (attr_once.pending(&attr_bit)) {

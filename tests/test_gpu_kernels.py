@@ -1651,6 +1651,7 @@ def test_flash_attention_f32_key_groups_and_planes(core, B, Hd, Sq, Skv, D):
     (320, 9, 9, 300, None),                # as many layers as steps
     (1024, 10, 4, 200, None),
     (2048, 6, 6, 3, None),                 # more weights in a stage than the last-level cache is good for
+    (1024, 20, 20, 270, None),             # the least that is: 320 MB, two row blocks
 ])
 def test_streamed_f16_stack_in_one_launch(core, monkeypatch, H, L, T, B, dil):
     """The fp16 stack whose tiles wait for each other in one launch has the bits of a launch per stage of cells, three times on
