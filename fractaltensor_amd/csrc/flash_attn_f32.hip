@@ -170,7 +170,8 @@ constexpr int f32_partial_bytes(int D) { return 128 * D * 4 + 4 * 64 * 8; }
 // DIRECT: Kp and Vp are K and V themselves, no launch in front.  Each workgroup cuts a tile's fp32 rows into their planes on the way to LDS
 // (they are as long as the planes), K under a scale of the tile's own, V under that of the largest value of the group's tiles so
 // far: no magnitude of a whole head is needed first, and no element has fewer bits than under its head's scale.  Every query block pays for
-// it again: f32_split has the line.  The error against float64 is that of the other form, also with keys that differ by 2^20.
+// it again: f32_split has the line.  The error against float64 is that of the other form, also with keys that differ by 2^20.  At D 128 it takes
+// all 512 registers and two spilled ones (12 bytes of scratch a lane); on the grids that f32_split gives it, it is the faster form as it is.
 // 4 waves x 32 query rows per workgroup.  Two workgroups to a compute unit at head sizes up to 64 (B 4, 16 heads, 1024 keys of 64: 88
 // -> 77 us with a bound of 256 registers, of which the compiler had taken a few more), one above: the accumulators of O,
 // both planes of Q and the scores take some 400 registers at D = 128.  K and V tiles of 64 keys, both double buffered.  A wave

@@ -274,10 +274,12 @@ static int launch(const void* Q, const void* K, const void* V, void* O, int BH, 
 
 // From 128 MB of keys and values upwards, half of what the last-level cache holds, the copies leave no lines behind (ONCE): a program that
 // attends to several such caches in turn, a layer each, finds nothing of the next one there, and lines that displace others cost time.  us,
-// plain copies and these: 16 x 16 heads, 4096 keys of 128, 537 MB 90.9, 77.1; 10 x 8 heads, 3116 keys, 128 MB, three and more in turn 26.7,
-// 23.6, alone 22.8, 22.6.  The price is a single cache of almost the size of the last-level one that is read again and again (3 x 12 heads,
-// 13619 keys, 251 MB alone 40.5, 43.3, two and more in turn 49.2, 44.6); smaller ones would pay it as soon as a few fit together (6 x 32 heads, 1267
-// keys of 96, 93 MB, two in turn 15.7, 17.0, six 19.0, 17.6).
+// plain copies and these: 16 x 16 heads, 4096 keys of 128, 537 MB 90.9, 77.1; 10 x 8 heads, 3116 keys, just below the line, three and more in turn
+// 26.7, 23.6, alone 22.8, 22.6.  The price is a single cache of up to the size of the last-level one that is read again and again, and two of half of it (3 x 12
+// heads, 13619 keys, 251 MB alone 40.4, 41.2 to 43.3, two in turn 48.0, 42.2, six 48.1, 43.5; 20 x 32, 1560 of 64, 256 MB 40.8, 43.6 and 49.3, 44.6; 5 x 12,
+// 9000 of 96, 207 MB 33.6, 34.8 and 40.5, 35.9; 6 x 12, 5000 of 96, 138 MB 23.9, 24.2 and 24.8, 25.3, six 28.4, 26.1); smaller ones would pay it as soon as a
+// few fit together (6 x 32 heads, 1267 keys of 96, 93 MB, two in turn 15.7, 17.0, six 19.0, 17.6).  (Only V's copies without lines from 128
+// to 256 MB: 40.4, 40.7, 44.3 for the 251 MB, 42.7, 42.6, 46.4 for the 256, 34.1, 34.0, 36.4 for 223 in place of 33.4, 34.5, 35.5: no better over all.)
 constexpr long long kDecOnceBytes = 128LL << 20;
 
 // nparts workgroups per head, each leaving its part in part_o / part_ml when nparts > 1 (see attn_merge_kernel).

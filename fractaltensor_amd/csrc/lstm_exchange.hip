@@ -917,8 +917,8 @@ void lstm_exchange_kernel(ExchangeArgs a) {
 // In front of the kernel above, by workgroup: the input rows as tiles (the first row_groups of them; one wave per row, rows past
 // the batch are zeros; fp32 rows are cut under a power-of-two scale of their own), then the ring and the first two steps of
 // `hand`, kPrepareFill words of 16 bytes of a layer to a workgroup; the first of these has the status block and the places too.
-// Bound by its launch: with a grid of rows x (layers + 1) most of its workgroups had nothing to do, and dealing them out took
-// longer than the work (L 20 T 30 B 32 H 128, 5040 workgroups, 5.1 us; L 8 T 100 B 64 H 512, 9216, 14.7).
+// (A grid of rows x (layers + 1), most of whose workgroups had nothing to do, took longer with many of them only: us under the tracer, that
+// grid and this, L 8 T 100 B 64 H 512, 9216 workgroups, 14.8, 12.3; L 20 T 30 B 32 H 128, 5040, 5.1, 5.1, the whole call 79.8, 78.7.)
 constexpr int kPrepareFill = 1024;
 template <bool HALF>
 __global__ __launch_bounds__(256) void lstm_exchange_prepare_kernel(int* status, int first_word, int* place, int nplaces, v4u* ring,
