@@ -116,6 +116,13 @@ int launch_resident(const void* fn, dim3 grid, dim3 block, void** args, size_t l
   return FTK_OK;
 }
 
+bool stream_records(hipStream_t s) {
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  const hipError_t e = hipStreamIsCapturing(s, &capture);
+  if (e != hipSuccess) (void)hipGetLastError();
+  return e != hipSuccess || capture != hipStreamCaptureStatusNone;
+}
+
 bool launch_is_cooperative(hipStream_t s) {
   Launches& all = launches();
   int dev = 0;

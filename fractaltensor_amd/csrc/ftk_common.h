@@ -105,6 +105,8 @@ int device_props(const DeviceProps** out);
 int launch_resident(const void* fn, dim3 grid, dim3 block, void** args, size_t lds, hipStream_t s);
 // Whether that is going to be a cooperative launch, as far as can be told before it is made.
 bool launch_is_cooperative(hipStream_t s);
+// whether s records a graph (or must not be asked because another stream does)
+bool stream_records(hipStream_t s);
 
 // ---- vector types for MFMA operands ----------------------------------------
 typedef float v4f __attribute__((ext_vector_type(4)));

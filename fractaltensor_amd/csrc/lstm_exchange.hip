@@ -31,7 +31,8 @@
 // they had h(t-2)), so it sets its words of slot t-2 back to all ones, which are used again at t+2.  hand: every h of
 // every layer, for the layer above and for dilated recurrences; the producer itself sets the words of step t+2 to
 // all ones before it publishes step t+1, and a consumer looks at step t+2 only after it has seen step t+1.  The first
-// two steps, the ring and the input rows (in the same form) are written by the small kernel in front.
+// two steps, the ring and the input rows (in the same form) are written at the start of the launch itself
+// (exchange_lay_out), or by a small kernel in front where that does not serve (run_exchange).
 //
 // Products.  fp32 data: an operand is an fp16 value and the fp16 of what that leaves, under a power-of-two scale of its
 // weight column or input row (h: 2^14); three fp16 matrix instructions per product, fp32 accumulation (see
@@ -42,6 +43,8 @@
 #include <stdlib.h>
 
 #include <algorithm>
+#include <atomic>
+#include <random>
 
 #include "ftk_common.h"
 
@@ -51,6 +54,7 @@ constexpr int kXLayers = 64;       // layers of one launch
 constexpr int kXBlocks = 128;      // row blocks a ragged batch may have
 constexpr int kXRing = 4;          // steps the own layer's ring holds
 constexpr int kXPlaces = 2048;     // workgroups of one launch
+constexpr int kXRowPlaces = 256;   // workgroups that lay out the input rows of a slice: what the layer that reads them looks at
 constexpr int kXHandTop = 14;      // the scale of h: 2^14 (|h| < 1)
 constexpr unsigned kXSmallBits = (127u - 12u - kXHandTop) << 23;   // h * 2^14 below 2^-12: see ftk_stacked_lstm_small_states
 
@@ -60,21 +64,26 @@ struct ExchangeArgs {
   void* hsss;
   void* csss;
   int* status;          // [0] error word, [1] small states
-  int* place;           // [groups]: 1 + the XCC id of every workgroup
+  unsigned long long* place;   // [groups]: launch << 8 | 1 + the XCC id, of every workgroup that is there and has laid out what it has to
+  unsigned long long launch;   // what tells this launch's words from any that were there before
+  const void* xs;       // not null: this launch lays out its own buffers (exchange_lay_out)
   unsigned char* ring;  // [L][nrb][kXRing] tiles
   unsigned char* hand;  // [L + 1][T][nrb] tiles: the input rows, then every layer's h
-  const float* xratio;  // [T][row of a block] what the products of an input row are multiplied by to match h's (fp32 data)
+  float* xratio;        // [row block][T, rounded up to even][row of it] what the products of an input row are multiplied by to match h's (fp32 data)
   int L, T, B, nrb;
   int slices;           // row slices = teams per layer; slice s walks row blocks s, s + slices, ...
   int units;            // L * slices teams
   int per_xcd;          // > 0: teams per XCD, unit u on XCD u / per_xcd; 0: workgroups in order
   int spin_limit;
   int ragged;
+  int row_layers;       // xs: layers whose workgroups lay out the input rows of their slice
+  int clear_status;     // xs: this launch clears the status words
   int dil[kXLayers];
   int steps_of[kXBlocks];   // ragged: steps row block rb takes part in (T reaches 262143 at H = 64)
 };
 
 typedef unsigned long long u64;
+typedef float v2f __attribute__((ext_vector_type(2)));
 
 // How words leave a workgroup that is not in a hurry: to `hand` as plain stores (the layer above, if any, on this XCD) or
 // write-through, to the ring as plain ones; or (teams over several XCDs) as either, by two stores of which one is out of bounds.
@@ -97,6 +106,113 @@ constexpr int exchange_units(int H, bool half, bool many) { return many && H * (
 constexpr int exchange_per_cu(int H, bool half, bool many) {
   const int weights = H * exchange_units(H, half, many) / (half ? 64 : 32);
   return weights >= 256 ? 1 : weights >= 128 || many ? 2 : 3;
+}
+
+// x times a power of two as an fp16 value and the fp16 of what that leaves: two instructions.
+__device__ __forceinline__ v2h value_and_rest(float x, float scale) {
+  const _Float16 top = (_Float16)__builtin_fmaf(x, scale, 0.0f);
+  return v2h{top, (_Float16)__builtin_fmaf(x, scale, -(float)top)};
+}
+
+// An input row in the form of the exchange buffers, by eight lanes, piece i of a lane's N being k group 8 i + lane / 8: put(i, w)
+// takes its 16 bytes, ratio(r) what the row's products are multiplied by.  fp32 rows are cut under a power-of-two scale of their own.
+template <bool HALF, int N, typename Put, typename Ratio>
+__device__ __forceinline__ void exchange_input_row(const v4u (&raw)[N], Put put, Ratio ratio) {
+  if constexpr (HALF) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) put(i, raw[i]);
+  } else {
+    float mx = 0.0f;
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) mx = fmaxf(mx, fabsf(__uint_as_float(raw[i][e])));
+#pragma unroll
+    for (int o = 32; o >= 8; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
+    const int eb = min(max((int)((__float_as_uint(mx) >> 23) & 0xff), 15), 254);
+    const float scale = __uint_as_float((unsigned)(127 + 14 + 127 - eb) << 23);   // the row's largest -> [2^14, 2^15)
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      v4u w;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) w[e] = __builtin_bit_cast(unsigned, value_and_rest(__uint_as_float(raw[i][e]), scale));
+      put(i, w);
+    }
+    ratio(__uint_as_float((unsigned)eb << 23));   // the products carry 2^(141 - eb), h's 2^14
+  }
+}
+
+// Before the first step of a launch that lays out its own buffers.  What others of this launch look at (see the top of the file) is written
+// here, in front of the weights; then the workgroup's place says that it is done.  Whoever reads waits for the places it depends on, and a
+// place is known as this launch's by the number in it, so nothing has to be cleared before the launch.  Words are written through, and no line of
+// them is written by two workgroups: no cache holds a part of one.
+//
+// Bound by latency: input rows that come from memory, stores that go there, places that come from there.  It takes 2 to 3 us where the kernel in
+// front took 3.4 to 12 and a launch (us a call with other inputs and weights each time, that kernel and this: L 2 T 36 B 155 H 64 50.1, 47.1; L 1 T 64
+// B 100 H 512 150.7, 141.4; L 8 T 100 B 64 H 512 726.5, 706; fp16 L 10 T 30 B 99 H 256 126.5, 121.2; over 47 drawn stacks 2 %).  With the places
+// behind the weights, and the rows between the loads of them, single layers began as early, but the places of a workgroup whose weights came late
+// held up the others (fp16 L 10 T 30 B 99 H 256 144.5), and all waves looking at them held up the weights.
+template <int H, bool HALF, bool MANY, typename Args>
+__device__ __forceinline__ void exchange_lay_out(const Args& a, int unit, int s, int l, int pc) {
+  constexpr int W = H / exchange_units(H, HALF, MANY), ROWS = MANY ? 32 : 16, TILE = exchange_tile_bytes(H, HALF, ROWS);
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int T = a.T, B = a.B, nrb = a.nrb;
+  // The input rows, 32 to a workgroup and 8 to a wave at a time: lane (row, k group) so that a store covers whole lines.
+  constexpr int PIECES = H / (HALF ? 64 : 32);
+  v4u raw[PIECES];
+  const int steps = (T + 1) & ~1, per_block = steps * ROWS / 32;
+  int group = l * W + pc;
+  const int groups = l < a.row_layers ? (MANY ? (nrb - s + a.slices - 1) / a.slices * per_block : per_block) : 0;
+  int t, rb, m;   // this lane's row: time step (the last may be past the end), row block, row of it
+  auto ask = [&]() __attribute__((always_inline)) {
+    const int block = MANY ? group / per_block : 0, r = (group - block * per_block) * 32 + wave * 8 + (lane & 7);
+    rb = s + block * a.slices;
+    t = r / ROWS;
+    m = r % ROWS;
+    const char* const from = reinterpret_cast<const char*>(a.xs) + ((size_t)min(t, T - 1) * B + min(rb * ROWS + m, B - 1)) * (H * (HALF ? 2 : 4));
+#pragma unroll
+    for (int i = 0; i < PIECES; ++i) raw[i] = reinterpret_cast<const v4u*>(from)[8 * i + (lane >> 3)];
+  };
+  if (group < groups) ask();
+  asm volatile("" ::: "memory");
+
+  // the words of this workgroup's units that stand for "not there yet": the ring, and the first two steps of `hand`
+  {
+    const auto ring = __builtin_amdgcn_make_buffer_rsrc(a.ring + (size_t)l * nrb * kXRing * TILE, 0, (unsigned)(nrb * kXRing * TILE), 0x00020000);
+    const auto hand = __builtin_amdgcn_make_buffer_rsrc(a.hand + (size_t)(l + 1) * T * nrb * TILE, 0, (unsigned)((size_t)T * nrb * TILE), 0x00020000);
+    constexpr int PART = TILE / W, STORES = PART / 16, AT_ONCE = 256 / STORES;   // bytes of a tile; tiles at a time
+    static_assert(256 % STORES == 0, "whole tiles at a time");
+    const v4u ones = {~0u, ~0u, ~0u, ~0u};
+    const int first = tid / STORES, at = pc * PART + tid % STORES * 16;
+    for (int rb = s; rb < (MANY ? nrb : s + 1); rb += a.slices) {
+#pragma unroll
+      for (int i = 0; i < kXRing; i += AT_ONCE)
+        if (i + first < kXRing) __builtin_amdgcn_raw_buffer_store_b128(ones, ring, (rb * kXRing + i + first) * TILE + at, 0, kAgentScope);
+#pragma unroll
+      for (int i = 0; i < 2; i += AT_ONCE)   // (a step past the last is out of the buffer)
+        if (i + first < 2) __builtin_amdgcn_raw_buffer_store_b128(ones, hand, ((i + first) * nrb + rb) * TILE + at, 0, kAgentScope);
+    }
+  }
+  if (a.clear_status && unit == 0 && pc == 0 && tid < (int)(kStatusBytes / sizeof(int)))
+    __hip_atomic_store(a.status + tid, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+
+  const auto rows = __builtin_amdgcn_make_buffer_rsrc(a.hand, 0, (unsigned)((size_t)T * nrb * TILE), 0x00020000);
+  const auto ratios = __builtin_amdgcn_make_buffer_rsrc(a.xratio, 0, (unsigned)((size_t)nrb * steps * ROWS * 4), 0x00020000);
+  while (group < groups) {
+    const unsigned live = rb * ROWS + m < B ? ~0u : 0u;   // rows past the batch are zeros
+#pragma unroll
+    for (int i = 0; i < PIECES; ++i) raw[i] &= live;
+    const unsigned at = t < T ? (unsigned)((t * nrb + rb) * TILE + m * 16 + (lane >> 3) * (ROWS * 16)) : 0x80000000u;
+    exchange_input_row<HALF>(raw, [&](int i, v4u w) __attribute__((always_inline)) {
+      __builtin_amdgcn_raw_buffer_store_b128(w, rows, at, i * (8 * ROWS * 16), kAgentScope);
+    }, [&](float ratio) __attribute__((always_inline)) {
+      if (lane < 8) __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(ratio), ratios, ((rb * steps + t) * ROWS + m) * 4, 0, kAgentScope);
+    });
+    group += a.row_layers * W;
+    if (group < groups) ask();
+  }
+  __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0): what this wave wrote is in memory
+  __syncthreads();
 }
 
 // MANY == false: one row block of 16 rows per workgroup, where an item waits for the one before it and the wait is what is
@@ -151,8 +267,13 @@ void lstm_exchange_kernel(ExchangeArgs a) {
 
   int xcc;
   asm volatile("s_getreg_b32 %0, hwreg(HW_REG_XCC_ID)" : "=s"(xcc));
-  xcc = (xcc & 0xff) + 1;
-  if (tid == 0) __hip_atomic_store(a.place + unit * W + pc, xcc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  xcc = (xcc & 0x7f) + 1;
+
+  // (the arguments are read again for it: what the loops need of them would be kept in registers otherwise, from here on)
+  auto* again = (const __attribute__((address_space(4))) ExchangeArgs*)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(again));
+  if (again->xs) exchange_lay_out<H, HALF, MANY>(*again, unit, s, l, pc);
+  if (tid == 0) __hip_atomic_store(a.place + unit * W + pc, a.launch << 8 | (unsigned)xcc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 
   // ---- resident weights: lane (m, kg) holds rows KW i + 8 kg .. +7 of column m of tile tt, for k step i.
   // A column is a gate of a unit, ordered so that a lane gets the four gates of a unit next to each other in its
@@ -200,7 +321,7 @@ void lstm_exchange_kernel(ExchangeArgs a) {
       const float* wl = reinterpret_cast<const float*>(a.WU) + base;
       float raw[KS][NT][8];
 #pragma unroll
-      for (int i = 0; i < KS; ++i)
+      for (int i = 0; i < KS; ++i) {
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
           const float* row = wl + (size_t)(w_row(i) + 8 * kg + e) * 4 * H;
@@ -213,6 +334,7 @@ void lstm_exchange_kernel(ExchangeArgs a) {
             for (int tt = 0; tt < NT; ++tt) raw[i][tt][e] = row[uo[tt]];
           }
         }
+      }
       // the largest magnitude of each of the workgroup's columns, over the four waves
       float* const cmaxs = reinterpret_cast<float*>(red);   // [4 waves][tile, column], then what undoes the scales
 #pragma unroll
@@ -238,11 +360,15 @@ void lstm_exchange_kernel(ExchangeArgs a) {
 #pragma unroll
         for (int i = 0; i < KS; ++i)
 #pragma unroll
-          for (int e = 0; e < 8; ++e) {
-            const float w = raw[i][tt][e] * scale;
-            const _Float16 top = (_Float16)w;
-            wt[i][tt][e] = top;
-            wo[i][tt][e] = (_Float16)(w - (float)top);
+          for (int e = 0; e < 8; e += 2) {   // six instructions for two
+            const v2f w = {raw[i][tt][e] * scale, raw[i][tt][e + 1] * scale};
+            const v2h top = __builtin_convertvector(w, v2h);
+            const v2f left = {__builtin_fmaf(raw[i][tt][e], scale, -(float)top[0]), __builtin_fmaf(raw[i][tt][e + 1], scale, -(float)top[1])};
+            const v2h rest = __builtin_convertvector(left, v2h);
+            wt[i][tt][e] = top[0];
+            wt[i][tt][e + 1] = top[1];
+            wo[i][tt][e] = rest[0];
+            wo[i][tt][e + 1] = rest[1];
           }
       }
       __syncthreads();
@@ -291,29 +417,42 @@ void lstm_exchange_kernel(ExchangeArgs a) {
       ebias[4 * u + g] = a.bias ? a.bias[(size_t)l * 4 * H + g * H + my_unit + u] * (g == 3 ? 1.0f : -kLog2e) : 0.0f;
 
   // ---- do the team, and the team above that reads from it, sit on this XCD?
-  bool alive = true;
-  auto look_at_places = [&](int u) -> bool {   // all of unit u's workgroups on this XCD
-    int v = xcc, n = 0;
-    for (int i0 = 0; i0 < W; i0 += 64) {
-      const int i = min(i0 + lane, W - 1);
-      int p = 0;
-      while (true) {
-        p = __hip_atomic_load(a.place + u * W + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (__builtin_amdgcn_ballot_w64(p == 0) == 0) break;
-        __builtin_amdgcn_s_sleep(2);
-        if (++n >= (1 << 20)) {
-          __hip_atomic_store(a.status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          alive = false;
-          return false;
-        }
-      }
-      if (p != xcc) v = 0;
-    }
-    return __builtin_amdgcn_ballot_w64(v != xcc) == 0;
-  };
-  const bool team_here = look_at_places(unit);
   const bool has_upper = l + 1 < a.L;
-  const bool upper_here = has_upper && alive ? look_at_places(unit + 1) : true;
+  // (looked at by one wave: all looking at all of them at once hold up the weights that other workgroups wait for)
+  __shared__ int places_seen;
+  if (wave == 0) {
+    static_assert(W <= 64, "a lane for each workgroup of a team");
+    const int i = min(lane, W - 1);
+    // xs: what is read of others' is there: the status words, and the layer below, or the input rows
+    const auto& b = *again;
+    const bool own_buffers = b.xs != nullptr;
+    const int from = l == 0 ? (unit - l) * W : (unit - 1) * W, count = !own_buffers ? 0 : l == 0 ? b.row_layers * W : W;
+    auto place = [&](int at) __attribute__((always_inline)) { return __hip_atomic_load(b.place + at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
+    auto missing_place = [&](u64 p) __attribute__((always_inline)) { return p >> 8 != b.launch; };
+    u64 own, up;
+    int seen = 4;
+    for (int n = 0;; ++n) {
+      own = place(unit * W + i);
+      up = place((has_upper ? unit + 1 : unit) * W + i);
+      const u64 first = place(own_buffers ? 0 : unit * W);
+      bool waits = missing_place(own) || missing_place(up) || missing_place(first);
+      for (int k = 0; k < count; k += 64) waits = missing_place(place(from + min(k + lane, count - 1))) || waits;
+      if (__builtin_amdgcn_ballot_w64(waits) == 0) break;
+      if (n >= (1 << 20)) {
+        __hip_atomic_store(b.status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        seen = 0;
+        break;
+      }
+      __builtin_amdgcn_s_sleep(4);
+    }
+    if (__builtin_amdgcn_ballot_w64((int)(own & 0xff) != xcc) == 0) seen |= 1;
+    if (!has_upper || __builtin_amdgcn_ballot_w64((int)(up & 0xff) != xcc) == 0) seen |= 2;
+    places_seen = seen;
+  }
+  __syncthreads();
+  const int seen = __builtin_amdgcn_readfirstlane(places_seen);
+  bool alive = (seen & 4) != 0;
+  const bool team_here = (seen & 1) != 0, upper_here = (seen & 2) != 0;
   const bool keep_c = d == 1 && s + a.slices >= nrb && !a.ragged;   // one row block: its c stays here
   // Teams that wait for one row block each have a loop with as few stores as their place allows (`lean`): every store
   // instruction of a wave is time on its way round.
@@ -343,7 +482,8 @@ void lstm_exchange_kernel(ExchangeArgs a) {
   const size_t hand_bytes = (size_t)T * tiles_t, out_bytes = (size_t)T * rows_t, ring_bytes = (size_t)nrb * kXRing * TILE;
   const auto hand_l = buffer(a.hand + (l + 1) * hand_bytes, hand_bytes);
   const auto below_l = buffer(a.hand + l * hand_bytes, hand_bytes);   // the layer below, or the input rows
-  const auto ratios = buffer(a.xratio, (size_t)T * nrb * ROWS * sizeof(float));
+  const int ratio_steps = (T + 1) & ~1;
+  const auto ratios = buffer(a.xratio, (size_t)ratio_steps * nrb * ROWS * sizeof(float));
   const auto own_l = own_by_ring ? buffer(a.ring + l * ring_bytes, ring_bytes) : hand_l;
   const auto h_out = buffer(reinterpret_cast<unsigned char*>(a.hsss) + l * out_bytes, out_bytes);
   const auto c_out = buffer(reinterpret_cast<unsigned char*>(a.csss) + l * out_bytes, out_bytes);
@@ -677,7 +817,7 @@ void lstm_exchange_kernel(ExchangeArgs a) {
   // line that was fetched too early holds all-ones words still; wait_share asks for it again past the caches.)
   auto x_at = [&](const Item& it) { return it.tile + it.rb * TILE; };
   auto ask_ratio = [&](const Item& it) __attribute__((always_inline)) {
-    xr = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(ratios, m * 4, (it.t * nrb + it.rb) * (ROWS * 4), 0));
+    xr = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(ratios, m * 4, (it.rb * ratio_steps + it.t) * (ROWS * 4), 0));
   };
   auto scale_input = [&](float ratio) __attribute__((always_inline)) {
 #pragma unroll
@@ -813,7 +953,7 @@ void lstm_exchange_kernel(ExchangeArgs a) {
       }
     };
     load_share(below_l, do_x ? get : 0x80000000u, x_at, v, cached);
-    if constexpr (FIRST && !HALF) xr = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(ratios, m * 4, s * (ROWS * 4), 0));
+    if constexpr (FIRST && !HALF) xr = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(ratios, m * 4, s * ratio_steps * (ROWS * 4), 0));
     // h is asked for in front of the products of x, where registers and its way leave time for it, and behind them: what comes
     // too early is not there yet, and to ask again only then costs the whole way once more.  (L 1 T 64 B 16: H 128
     // 69 us when asked for behind x only, 65 with both; L 20 T 30 B 32 H 128 83 and 81.6; fp16 H 512 88 and 78.)
@@ -864,7 +1004,7 @@ void lstm_exchange_kernel(ExchangeArgs a) {
         load_piece(ic, below_l, x_get, next_x, v, cached);
       });
       if constexpr (FIRST && !HALF)
-        xr = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(ratios, m * 4, ((more ? t + 1 : t) * nrb + s) * (ROWS * 4), 0));
+        xr = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(ratios, m * 4, (s * ratio_steps + (more ? t + 1 : t)) * (ROWS * 4), 0));
       give_sums(parity);
       // what was set back after the item before is complete before anything of this one is published
       asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(NL + (FIRST && !HALF ? 1 : 0)) : "memory");
@@ -914,14 +1054,14 @@ void lstm_exchange_kernel(ExchangeArgs a) {
   walk_layer(std::integral_constant<int, kAnyWay>{});
 }
 
-// In front of the kernel above, by workgroup: the input rows as tiles (the first row_groups of them; one wave per row, rows past
+// In front of the kernel above where it does not lay out its buffers itself (run_exchange), by workgroup: the input rows as tiles (the first row_groups of them; one wave per row, rows past
 // the batch are zeros; fp32 rows are cut under a power-of-two scale of their own), then the ring and the first two steps of
 // `hand`, kPrepareFill words of 16 bytes of a layer to a workgroup; the first of these has the status block and the places too.
 // (A grid of rows x (layers + 1), most of whose workgroups had nothing to do, took longer with many of them only: us under the tracer, that
 // grid and this, L 8 T 100 B 64 H 512, 9216 workgroups, 14.8, 12.3; L 20 T 30 B 32 H 128, 5040, 5.1, 5.1, the whole call 79.8, 78.7.)
 constexpr int kPrepareFill = 1024;
 template <bool HALF>
-__global__ __launch_bounds__(256) void lstm_exchange_prepare_kernel(int* status, int first_word, int* place, int nplaces, v4u* ring,
+__global__ __launch_bounds__(256) void lstm_exchange_prepare_kernel(int* status, int first_word, unsigned long long* place, int nplaces, v4u* ring,
                                                                     unsigned ring_per_layer, v4u* hand, size_t hand_per_layer,
                                                                     unsigned hand_first, const void* xs, float* xratio, int row_groups,
                                                                     int T, int B, int nrb, int block, int H) {
@@ -982,7 +1122,8 @@ __global__ __launch_bounds__(256) void lstm_exchange_prepare_kernel(int* status,
         }
         if (k < H) *reinterpret_cast<v4u*>(dst + (k >> 2) * (block * 16)) = w;
       }
-      if (lane == 0) xratio[r] = __uint_as_float((unsigned)eb << 23);   // the products carry 2^(141 - eb), h's 2^14
+      // the products carry 2^(141 - eb), h's 2^14
+      if (lane == 0) xratio[((size_t)(b / block) * ((T + 1) & ~1) + t) * block + b % block] = __uint_as_float((unsigned)eb << 23);
     }
   }
 }
@@ -1072,7 +1213,7 @@ ExchangePlan exchange_plan(int L, int W, int nrb, int slots) {   // W: workgroup
 }
 
 constexpr size_t align256(size_t v) { return (v + 255) / 256 * 256; }
-constexpr size_t exchange_xratio_at = align256(kStatusBytes + kXPlaces * sizeof(int));
+constexpr size_t exchange_xratio_at = align256(kStatusBytes + kXPlaces * sizeof(unsigned long long));
 
 }  // namespace
 
@@ -1082,7 +1223,7 @@ bool exchange_takes(int H, bool half) { return exchange_flavour_of(H, half).one 
 // Bytes of workspace for L layers: [status block][places][xratio][ring][hand], with either kind of row block.
 size_t exchange_workspace_bytes(int L, int T, int B, int H, bool half) {
   const size_t rows = (size_t)(B + 31) / 32 * 32;   // never less than with blocks of 16
-  return exchange_xratio_at + align256((size_t)T * rows * sizeof(float)) +
+  return exchange_xratio_at + align256((size_t)(T + 1) * rows * sizeof(float)) +
          rows * H * (half ? 2 : 4) * ((size_t)L * kXRing + (size_t)(L + 1) * T);
 }
 
@@ -1169,6 +1310,20 @@ int exchange_layers(int L, int T, int B, int H, bool half, bool plain, float eac
 }
 }  // namespace
 
+namespace {
+
+// A number that no launch of this process had, and that what a workspace holds by chance does not have: 56 bits, from a random start.
+unsigned long long exchange_launch_number() {
+  static std::atomic<unsigned long long> next{[] {
+    std::random_device r;
+    return (unsigned long long)r() << 32 | r();
+  }()};
+  while (true)
+    if (const unsigned long long v = next.fetch_add(1, std::memory_order_relaxed) & ((1ull << 56) - 1)) return v;
+}
+
+}  // namespace
+
 // Whether the whole batch of every layer fits the chip with one block of 16 rows per workgroup.
 bool exchange_one_block(int L, int B, int H, bool half) { return exchange_one_block_layers(L, B, H, half) == L; }
 
@@ -1206,6 +1361,7 @@ int run_exchange(bool half, const void* xs, const void* WU, const float* bias, c
   const int W = H / exchange_units(H, half, many);
   const size_t esize = half ? 2 : 4, slab = (size_t)T * B * H, wlayer = (size_t)8 * H * H, tile = exchange_tile_bytes(H, half, block);
   if (!ws || ws_bytes < exchange_workspace_bytes(std::min(L, most), T, B, H, half)) return FTK_OK;
+  const bool records = stream_records(s);
   for (int l0 = 0; l0 < L; l0 += most) {
     const int lc = std::min(most, L - l0);
     const ExchangePlan p = exchange_plan(lc, W, nrb, slots);
@@ -1216,10 +1372,10 @@ int run_exchange(bool half, const void* xs, const void* WU, const float* bias, c
     a.hsss = (char*)hsss + (size_t)l0 * slab * esize;
     a.csss = (char*)csss + (size_t)l0 * slab * esize;
     a.status = (int*)ws;
-    a.place = (int*)((char*)ws + kStatusBytes);
+    a.place = (unsigned long long*)((char*)ws + kStatusBytes);
     float* xratio = (float*)((char*)ws + exchange_xratio_at);
     a.xratio = xratio;
-    a.ring = (unsigned char*)ws + exchange_xratio_at + align256((size_t)T * nrb * block * sizeof(float));
+    a.ring = (unsigned char*)ws + exchange_xratio_at + align256((size_t)(T + 1) * nrb * block * sizeof(float));
     a.hand = a.ring + (size_t)lc * nrb * kXRing * tile;
     a.L = lc; a.T = T; a.B = B; a.nrb = nrb;
     a.slices = p.slices;
@@ -1236,17 +1392,33 @@ int run_exchange(bool half, const void* xs, const void* WU, const float* bias, c
     }
     const int groups = a.units * W;
     const unsigned grid = p.per_xcd ? 8u * p.per_xcd * W : (unsigned)((groups + 7) / 8 * 8);
-    const unsigned ring_per_layer = (unsigned)((size_t)nrb * kXRing * tile / 16), hand_first = (unsigned)((size_t)std::min(T, 2) * nrb * tile / 16);
-    const size_t hand_per_layer = (size_t)T * nrb * tile / 16;
-    const int row_groups = (int)std::min<size_t>(((size_t)T * nrb * block + 3) / 4, 2048);
-    const dim3 pgrid(row_groups + lc * ((ring_per_layer + hand_first + kPrepareFill - 1) / kPrepareFill));
-    auto prepare = half ? lstm_exchange_prepare_kernel<true> : lstm_exchange_prepare_kernel<false>;
-    hipLaunchKernelGGL(prepare, pgrid, dim3(256), 0, s, a.status, l0 > 0 ? 2 : 0, a.place, groups, (v4u*)a.ring, ring_per_layer, (v4u*)a.hand,
-                       hand_per_layer, hand_first, x, xratio, row_groups, T, B, nrb, block, H);
-    int rc = check_launch("lstm_exchange_prepare_kernel");
-    if (rc) return rc;
+    // The launch lays out its own buffers, unless it is recorded (a replay would find the places of the one before, with its number in them), or a
+    // workgroup had too many rows to lay out in front of its first step: a turn of 32 takes it 0.6 us once the first two are on their way
+    // beside the weights, the kernel in front takes 1 us for some 4000 rows more (us in a row, that kernel and without: L 1 H 64 T 24 B 8, 3 turns,
+    // 28.1, 27.5; T 128 B 8, 16 turns, 116.8, 123.4, B 250 129.2, 125.9; L 2 H 64 T 96 B 8, 6 turns, 113.2, 115.0, B 100 101.0, 98.8; L 1 H 256
+    // T 128 B 8, 4 turns, 159.5, 161.4, B 40 166.3, 163.6; 230 stacks in all).
+    a.launch = exchange_launch_number();
+    a.clear_status = l0 == 0;
+    const int row_groups = (nrb + p.slices - 1) / p.slices * ((T + 1) / 2 * 2) * block / 32;   // 32 rows each, of a slice
+    a.row_layers = std::max(1, std::min({lc, (row_groups + W - 1) / W, kXRowPlaces / W}));
+    const int turns = (row_groups + a.row_layers * W - 1) / (a.row_layers * W);
+    bool own = 0.6f * (turns - 2) <= 0.5f + (float)T * B / 4000;
+    if (const char* e = getenv("FTK_LSTM_EXCHANGE_FRONT")) own = e[0] != '1';   // =1 / =0: that kernel / none, where both can be
+    own = own && !records;
+    a.xs = own ? x : nullptr;
+    if (!own) {
+      const unsigned ring_per_layer = (unsigned)((size_t)nrb * kXRing * tile / 16), hand_first = (unsigned)((size_t)std::min(T, 2) * nrb * tile / 16);
+      const size_t hand_per_layer = (size_t)T * nrb * tile / 16;
+      const int prepare_groups = (int)std::min<size_t>(((size_t)T * nrb * block + 3) / 4, 2048);
+      const dim3 pgrid(prepare_groups + lc * ((ring_per_layer + hand_first + kPrepareFill - 1) / kPrepareFill));
+      auto prepare = half ? lstm_exchange_prepare_kernel<true> : lstm_exchange_prepare_kernel<false>;
+      hipLaunchKernelGGL(prepare, pgrid, dim3(256), 0, s, a.status, l0 > 0 ? 2 : 0, a.place, groups, (v4u*)a.ring, ring_per_layer, (v4u*)a.hand,
+                         hand_per_layer, hand_first, x, xratio, prepare_groups, T, B, nrb, block, H);
+      const int rc = check_launch("lstm_exchange_prepare_kernel");
+      if (rc) return rc;
+    }
     void* kargs[] = {&a};
-    rc = launch_resident(many ? f.many : f.one, dim3(grid), dim3(256), kargs, 0, s);
+    const int rc = launch_resident(many ? f.many : f.one, dim3(grid), dim3(256), kargs, 0, s);
     if (rc) return rc;
   }
   *handled = true;

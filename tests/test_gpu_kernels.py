@@ -1422,6 +1422,45 @@ def test_exchange_loops_give_the_same_bits(core, half, H, L, B, T):
 
 
 @pytest.mark.parametrize('half,H,L,T,B,dil', [
+    (False, 64, 1, 1, 1, None),            # one step, one row: the second row of a pair of steps is past the end
+    (False, 64, 1, 33, 17, None),          # workgroups with several turns of rows, an odd number of steps
+    (False, 64, 20, 2, 250, None),         # several 32-row blocks per workgroup
+    (False, 128, 3, 7, 40, [1, 2, 4]),
+    (False, 256, 2, 9, 33, None),
+    (False, 512, 9, 3, 20, None),          # two launches
+    (False, 512, 2, 5, 300, None),         # slices of one and of two row blocks
+    (True, 256, 40, 3, 31, None),          # more layers than there are rows to lay out
+    (True, 512, 2, 6, 70, None),
+    (True, 1024, 5, 4, 65, None),          # a layer larger than an XCD, two launches
+])
+def test_exchange_launches_lay_out_their_own_buffers(core, monkeypatch, half, H, L, T, B, dil):
+    """A launch that writes its own input rows and first words gives the bits of one behind the kernel that writes them, dense and ragged, on
+    a workspace that still holds what launches with other inputs, of another shape, and noise have left there."""
+    fn = core.stacked_lstm_f16 if half else core.stacked_lstm
+    size = core.lib.ftk_stacked_lstm_f16_workspace_bytes if half else core.stacked_lstm_workspace_bytes
+    other = (L + 1, T + 1, B + 3)
+    ws = torch.randint(0, 256, (max(size(L, T, B, H), size(*other, H)),), dtype=torch.uint8, device='cuda')
+    stacks = []
+    for seed, (l, t, b) in ((1, (L, T, B)), (2, (L, T, B)), (3, other)):
+        xs, WU, bs = lstm_inputs(seed, l, t, b, H, 1.0 / np.sqrt(H))
+        cast = (lambda a: dev(a.astype(np.float16))) if half else dev
+        lens = np.maximum(1, t - (np.arange(b) * t) // b)
+        d = None if dil is None else dil + [1] * (l - L)
+        for active in (None, [int((lens > i).sum()) for i in range(t)]):
+            live = torch.ones((t, b), dtype=torch.bool) if active is None else torch.from_numpy(np.arange(t)[:, None] < lens[None, :])
+            run = lambda ws, xs=cast(xs), WU=cast(WU), bs=dev(bs), d=d, active=active: fn(xs, WU, bs, dilations=d, workspace=ws, active_rows=active)
+            monkeypatch.setenv('FTK_LSTM_EXCHANGE_FRONT', '1')
+            ref = [r.cpu()[:, live] for r in run(torch.zeros_like(ws))]
+            stacks.append((run, live, ref))
+    monkeypatch.setenv('FTK_LSTM_EXCHANGE_FRONT', '0')
+    for turn in range(4):
+        for run, live, ref in stacks:
+            got = run(ws)
+            assert core.persistent_status(ws) == 0, 'a wait gave up'
+            assert all(torch.equal(g.cpu()[:, live], r) for g, r in zip(got, ref)), turn
+
+
+@pytest.mark.parametrize('half,H,L,T,B,dil', [
     (False, 64, 3, 5, 17, None),           # half a k step per wave: x and h waves; the second row block holds one row
     (False, 64, 32, 4, 130, None),         # several 32-row blocks per workgroup, the last of two rows
     (False, 128, 2, 1, 15, None),          # a single step
