@@ -956,7 +956,12 @@ void lstm_exchange_kernel(ExchangeArgs a) {
     if constexpr (FIRST && !HALF) xr = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(ratios, m * 4, s * ratio_steps * (ROWS * 4), 0));
     // h is asked for in front of the products of x, where registers and its way leave time for it, and behind them: what comes
     // too early is not there yet, and to ask again only then costs the whole way once more.  (L 1 T 64 B 16: H 128
-    // 69 us when asked for behind x only, 65 with both; L 20 T 30 B 32 H 128 83 and 81.6; fp16 H 512 88 and 78.)
+    // 69 us when asked for behind x only, 65 with both; L 20 T 30 B 32 H 128 83 and 81.6; fp16 H 512 88 and 78.)  The first time it is asked
+    // for when it is about to be there: in a stack of several layers, whose steps are the longer ones, some 320 cycles into the step (fp16 512), in a single
+    // layer at once, but for fp16 teams that share an XCD.  (us with 2, 4, 5, 6 and 8 times 64 cycles: L 6 T 80 B 16 H 128 106.1, 101.6, 100.5,
+    // 101.2, 104.5; L 5 T 60 B 60 H 64 79.7, 78.3, 78.0, 78.2, 79.5; fp16 L 4 T 60 B 32 H 256 81.9, 80.1, 79.1, 77.5, 74.9, with 10 and 15 75.5, 83.4;
+    // fp16 L 2 T 60 B 33 H 512 with 6, 8, 10 90.2, 88.9, 91.3; a single fp16 layer with 0, 1, 2: T 64 B 32 H 256 54.9, 55.9, 57.5, B 200 63.3, 63.2,
+    // 60.2.  At H 256 fp32, where it is asked for behind x only, any delay costs: L 4 T 60 B 16 93.2 without, 93.7 with 2, 95.7 with 4.)
     constexpr bool TWICE = HALF ? H <= 512 : H <= 128;
     share vh;
     float c[U] = {}, h[U];
@@ -975,7 +980,8 @@ void lstm_exchange_kernel(ExchangeArgs a) {
       const unsigned h_get_t = t > 0 ? h_get : 0x80000000u;
       __builtin_amdgcn_sched_barrier(0);
       if constexpr (TWICE) {
-        if (HALF || !FIRST || has_upper) __builtin_amdgcn_s_sleep(2);   // 128 cycles
+        if (!FIRST || has_upper) __builtin_amdgcn_s_sleep(HALF ? 8 : 5);   // 64 cycles each
+        else if (HALF && a.per_xcd > 1) __builtin_amdgcn_s_sleep(2);
         load_share(own_l, h_get_t, before, vh, fresh);
       }
       __builtin_amdgcn_sched_barrier(0);
