@@ -599,6 +599,15 @@ def flash_attention(Q, K, V, scale: Optional[float] = None, out: Optional[torch.
     return O
 
 
+def flash_attention_f32_flat(q, k, v, B: int, Hd: int, Sq: int, Skv: int, D: int, scale: float) -> torch.Tensor:
+    """flash_attention_f32 on the flat buffers of Q [B,Hd,Sq,D] and K, V [B,Hd,Skv,D]: the flat buffer of O."""
+    O = _fast.flash_attention_f32_flat(q, k, v, B, Hd, Sq, Skv, D, scale)
+    if O is not None:
+        return O
+    q, k, v = q.view(B, Hd, Sq, D), k.view(B, Hd, Skv, D), v.view(B, Hd, Skv, D)
+    return flash_attention_f32(q.contiguous(), k.contiguous(), v.contiguous(), scale).view(-1)
+
+
 def flash_attention_f32(Q, K, V, scale: Optional[float] = None, out: Optional[torch.Tensor] = None,
                         workspace: Optional[torch.Tensor] = None) -> torch.Tensor:
     """Non-causal attention with fp32 Q [B,Hd,Sq,D], K, V [B,Hd,Skv,D] -> O [B,Hd,Sq,D] fp32; D of 32, 64, 96 or 128.

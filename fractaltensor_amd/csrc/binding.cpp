@@ -12,6 +12,7 @@
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/python_variable.h>
 
+#include <climits>
 #include <cmath>
 #include <vector>
 
@@ -166,6 +167,38 @@ PyObject* flash_attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
   });
 }
 
+// flash_attention_f32_flat(q, k, v, B, Hd, Sq, Skv, D, scale) -> o: fp32 attention on the one-dimensional buffers of [B,Hd,Sq,D] and
+// [B,Hd,Skv,D].  (Three views of the operands and one of the result are 3 of the 17 us of host time of a short attention program.)
+PyObject* flash_attention_f32_flat(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  return guarded([&]() -> PyObject* {
+    if (n != 9 || !plain(a[0], at::kFloat) || !plain(a[1], at::kFloat) || !plain(a[2], at::kFloat) || !PyFloat_Check(a[8])) Py_RETURN_NONE;
+    int64_t size[5];
+    for (int i = 0; i < 5; ++i) {
+      if (!PyLong_Check(a[3 + i])) Py_RETURN_NONE;
+      size[i] = PyLong_AsLongLong(a[3 + i]);
+      if (size[i] <= 0 || size[i] > INT_MAX) {
+        PyErr_Clear();
+        Py_RETURN_NONE;
+      }
+    }
+    const int B = (int)size[0], Hd = (int)size[1], Sq = (int)size[2], Skv = (int)size[3], D = (int)size[4];
+    const at::Tensor &Q = tensor_of(a[0]), &K = tensor_of(a[1]), &V = tensor_of(a[2]);
+    __int128 of_q = (__int128)B * Hd * Sq * D, of_k = (__int128)B * Hd * Skv * D;
+    if (Q.dim() != 1 || K.dim() != 1 || V.dim() != 1 || Q.numel() != of_q || K.numel() != of_k || V.numel() != of_k) Py_RETURN_NONE;
+    at::Tensor O = empty(Q.sizes(), at::kFloat, Q), ws;
+    const size_t bytes = ftk_flash_attn_f32_workspace_bytes(B, Hd, Sq, Skv, D);
+    if (bytes) ws = empty({(int64_t)bytes}, at::kByte, Q);
+    if (!count("flash_attention_f32")) return nullptr;
+    void *const qp = Q.data_ptr(), *const kp = K.data_ptr(), *const vp = V.data_ptr(), *const op = O.data_ptr();
+    void *const wp = ws.defined() ? ws.data_ptr() : nullptr, *const s = stream();
+    const float scale = (float)PyFloat_AsDouble(a[8]);
+    const int rc = in_library([&] {
+      return ftk_flash_attn_f32((const float*)qp, (const float*)kp, (const float*)vp, (float*)op, B, Hd, Sq, Skv, D, scale, wp, bytes, s);
+    });
+    return rc ? raise(rc) : THPVariable_Wrap(std::move(O));
+  });
+}
+
 // stacked_lstm(half, xs [T,B,H], WU [L,2H,4H], bias [L,4H] or None, dilations or None, (h, c) or None, workspace or None,
 //              products, check or None, small) -> (h, c, small states met)
 // products: a code of ftk_lstm_options (-1: the process-wide mode).  check: wait for the stream and raise if the launch gave
@@ -284,6 +317,8 @@ PyMethodDef methods[] = {
     {"b2b_gemm", (PyCFunction)(void*)b2b_gemm, METH_FASTCALL, "b2b_gemm(A, B_nk, C_pn, out)"},
     {"flash_attention", (PyCFunction)(void*)flash_attention, METH_FASTCALL,
      "flash_attention(half, Q, K, V, scale, out, workspace, split_keys)"},
+    {"flash_attention_f32_flat", (PyCFunction)(void*)flash_attention_f32_flat, METH_FASTCALL,
+     "flash_attention_f32_flat(q, k, v, B, Hd, Sq, Skv, D, scale)"},
     {"stacked_lstm", (PyCFunction)(void*)stacked_lstm, METH_FASTCALL,
      "stacked_lstm(half, xs, WU, bias, dilations, out, workspace, products, check, small)"},
     {"stacked_lstm_result", (PyCFunction)(void*)stacked_lstm_result, METH_FASTCALL, "stacked_lstm_result(workspace)"},

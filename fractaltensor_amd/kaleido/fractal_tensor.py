@@ -185,6 +185,12 @@ class FractalTensor(Sequence):
     def _regular(flat: torch.Tensor, dims: Tuple[int, ...], element_shape: Tuple[int, ...]) -> 'FractalTensor':
         """A regular FractalTensor of these widths over a contiguous one-dimensional buffer."""
         typ = TensorStorage(element_shape, torch_type_to_internal_type(flat.dtype), device='cuda' if flat.is_cuda else flat.device.type)
+        if type(dims) is tuple and dims and 0 not in dims:
+            ft = FractalTensor.__new__(FractalTensor)
+            ft._type = FractalTensorStorage.regular(typ, dims)
+            ft._T = flat
+            ft._offsets = None
+            return ft
         for _ in range(len(dims) - 1):
             typ = FractalTensorStorage(typ)
         ft = FractalTensor(typ)

@@ -28,7 +28,7 @@ def require_same_shape(x, y):
 
 
 def require_iterative(xs):
-    if not isinstance(xs, (FractalTensor, Iterative)):
+    if type(xs) is not Iterative and not isinstance(xs, (FractalTensor, Iterative)):
         raise TypeError('Input should either a FractalTensor or a Iterative.')
     return xs
 

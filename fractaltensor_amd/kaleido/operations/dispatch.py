@@ -242,6 +242,44 @@ def _number_of(parts):
     return n
 
 
+_MODULE, _FUNCTION = type(os), type(_mark)
+_DATA = (Tensor, FractalTensor, Iterative, torch.Tensor)
+
+
+def _value_print(v, level: int, seen, looked):
+    """A default's or a closed-over value's part of a fingerprint (see there)."""
+    if isinstance(v, _SCALARS):
+        return v
+    if type(v) is _FUNCTION:                              # (in front: to ask whether it is a FractalTensor takes half a microsecond)
+        return _fingerprint(v, level + 1, seen, looked)
+    if isinstance(v, _DATA):
+        return type(v).__name__
+    if isinstance(v, (tuple, list)) and len(v) <= 16 and all(isinstance(e, _SCALARS) for e in v):
+        if looked is not None and isinstance(v, list):
+            looked.stable = False
+        return tuple(v)
+    if callable(v) and hasattr(v, '__code__'):
+        return _fingerprint(v, level + 1, seen, looked)
+    if isinstance(v, _MODULE):                            # a module: its name (ops, torch, math ...)
+        return ('module', v.__name__)
+    if isinstance(v, type):
+        return ('class', v.__module__, v.__qualname__)
+    if looked is not None:
+        looked.stable = False
+    return ('id', type(v).__name__, id(v))
+
+
+def _globals_print(code, g, level: int, record, seen, to):
+    """The scalars and functions that code reaches through the globals g; the names looked at are noted in `to`."""
+    names = []
+    for name in _code_names(code):
+        v = g.get(name, _MISSING)
+        to.add(name, v)
+        if v is not _MISSING and (isinstance(v, _SCALARS) or (callable(v) and hasattr(v, '__code__'))):
+            names.append((name, v if isinstance(v, _SCALARS) else _fingerprint(v, level + 1, seen, record)))
+    return (code, tuple(names))
+
+
 def _fingerprint(f, level: int = 0, seen=None, looked=None):
     """What identifies a user function between calls (a lambda is a new object at every call of the program, its
     code object is not): its code, its default arguments, the scalars and functions it closes over, and the scalars
@@ -251,7 +289,7 @@ def _fingerprint(f, level: int = 0, seen=None, looked=None):
     operand structure is checked on every call.
 
     seen: the functions met so far in this traversal, each with the place it was met at.  One met again stands as that
-    place.  What is kept between calls (of_globals) starts a traversal of its own: a place in a call's traversal may be
+    place.  What is kept between calls (_globals_print) starts a traversal of its own: a place in a call's traversal may be
     another function in the next call."""
     seen = {} if seen is None else seen
     code = getattr(f, '__code__', None)
@@ -268,54 +306,26 @@ def _fingerprint(f, level: int = 0, seen=None, looked=None):
             looked.function(f, code, getattr(f, '__defaults__', None), getattr(f, '__kwdefaults__', None), ())
         return ('deep', code)
     seen[id(f)] = len(seen)
-
-    def of_value(v):
-        if isinstance(v, _SCALARS):
-            return v
-        if isinstance(v, (Tensor, FractalTensor, Iterative, torch.Tensor)):
-            return type(v).__name__
-        if isinstance(v, (tuple, list)) and len(v) <= 16 and all(isinstance(e, _SCALARS) for e in v):
-            if looked is not None and isinstance(v, list):
-                looked.stable = False
-            return tuple(v)
-        if callable(v) and hasattr(v, '__code__'):
-            return _fingerprint(v, level + 1, seen, looked)
-        if isinstance(v, type(os)):                       # a module: its name (ops, torch, math ...)
-            return ('module', v.__name__)
-        if isinstance(v, type):
-            return ('class', v.__module__, v.__qualname__)
-        if looked is not None:
-            looked.stable = False
-        return ('id', type(v).__name__, id(v))
-
     parts = []
     defaults, kw, closure = getattr(f, '__defaults__', None), getattr(f, '__kwdefaults__', None), getattr(f, '__closure__', None)
-    for d in (defaults or ()):
-        parts.append(of_value(d))
-    for k, d in sorted(kw.items()) if kw else ():
-        parts.append((k, of_value(d)))
-    cells = [_content(cell) for cell in (closure or ())]
+    if defaults:
+        for d in defaults:
+            parts.append(_value_print(d, level, seen, looked))
+    if kw:
+        for k, d in sorted(kw.items()):
+            parts.append((k, _value_print(d, level, seen, looked)))
+    cells = [_content(cell) for cell in closure] if closure else []
     for v in cells:
         if v is not _MISSING:
-            parts.append(of_value(v))
+            parts.append(_value_print(v, level, seen, looked))
     g = getattr(f, '__globals__', None) or {}
-
-    def of_globals(record, seen, to):
-        names = []
-        for name in _code_names(code):
-            v = g.get(name, _MISSING)
-            to.add(name, v)
-            if v is not _MISSING and (isinstance(v, _SCALARS) or (callable(v) and hasattr(v, '__code__'))):
-                names.append((name, v if isinstance(v, _SCALARS) else _fingerprint(v, level + 1, seen, record)))
-        return (code, tuple(names))
-
     if looked is not None:               # reached from another function: part of that one's number
-        parts.append(of_globals(looked, seen, looked.function(f, code, defaults, kw, cells)))
+        parts.append(_globals_print(code, g, level, looked, seen, looked.function(f, code, defaults, kw, cells)))
         return tuple(parts)
     entry = _reached.get((id(code), id(g), level))
     if entry is None or not entry[0].unchanged(g):
         record = _Seen(g)
-        n = _number_of(of_globals(record, {}, record.names))
+        n = _number_of(_globals_print(code, g, level, record, {}, record.names))
         entry = (record, n, code)         # the code is kept alive: its id stays its own.  Other globals at the id of these
         if record.stable:                 # would be looked at name by name like these
             if len(_reached) >= _MAX_REACHED:
@@ -1058,7 +1068,7 @@ def try_map(func: Callable, xs, kwargs):
         return NotImplemented
     if _capturing() is not None:
         return NotImplemented
-    if isinstance(xs, FractalTensor):
+    if type(xs) is not Iterative and isinstance(xs, FractalTensor):
         return _try_map_of_sequences(func, xs)
     ops = _attention_operands(xs)
     if ops is None:
@@ -1083,13 +1093,13 @@ def try_map(func: Callable, xs, kwargs):
     if verdict is None:
         return NotImplemented
     core = _core()
-    q, k, v = q.view(B, Hd, nq * rq, D), k.view(B, Hd, nk * rk, D), v.view(B, Hd, nk * rk, D)
     if dtype == torch.float32 and not allow_half_attention:       # a program computes in its own precision
-        O = core.flash_attention_f32(q.contiguous(), k.contiguous(), v.contiguous(), verdict['scale'])
+        O = core.flash_attention_f32_flat(q, k, v, B, Hd, nq * rq, nk * rk, D, verdict['scale'])
     else:
-        O = core.flash_attention(q.half().contiguous(), k.half().contiguous(), v.half().contiguous(), verdict['scale']).to(dtype)
+        q, k, v = q.view(B, Hd, nq * rq, D), k.view(B, Hd, nk * rk, D), v.view(B, Hd, nk * rk, D)
+        O = core.flash_attention(q.half().contiguous(), k.half().contiguous(), v.half().contiguous(), verdict['scale']).to(dtype).view(-1)
     stats['flash_attention'] += 1
-    return FractalTensor._regular(O.view(-1), (B, Hd, nq), (rq, D))
+    return FractalTensor._regular(O, (B, Hd, nq), (rq, D))
 
 
 # ------------------------------------------------------------------ (a @ b) @ c behind Tensor.__matmul__

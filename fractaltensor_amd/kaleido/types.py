@@ -201,6 +201,24 @@ class FractalTensorStorage(Storage):
         self._depth = dtype._depth + 1 if nested else 1
         self._leaf = dtype._leaf if nested else dtype
 
+    @staticmethod
+    def regular(leaf: 'TensorStorage', dims) -> 'FractalTensorStorage':
+        """The type of a regular nesting of the widths dims, all above 0, over leaf: what the constructors and set_regular make, at once
+        (a result of three levels 5.5 -> 3 us; the attention kernel of a short call takes 6)."""
+        t = leaf
+        depth = 0
+        for n in reversed(dims):
+            of, t = t, FractalTensorStorage.__new__(FractalTensorStorage)
+            depth += 1
+            t._dtype = of
+            t._indices = None
+            t._dims = None
+            t._length = n
+            t._depth = depth
+            t._leaf = leaf
+        t._dims = dims
+        return t
+
     @property
     def dtype(self):
         return self._dtype

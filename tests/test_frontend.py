@@ -547,3 +547,19 @@ def test_fused_paths_refuse_cpu_inputs():
     q = programs.make_attention_input(1, 1, 64, 64, 64, seed=1)
     with pytest.raises(RuntimeError, match='GPU only'):
         ops.fused.flash_attention(q, q, q)
+
+
+@pytest.mark.parametrize('dims,element', [((3,), (2, 5)), ((2, 3), (4,)), ((1, 2, 3), (1, 1))])
+def test_a_regular_result_has_the_type_the_constructors_make(dims, element):
+    from fractaltensor_amd.kaleido.fractal_tensor import FractalTensor as FT
+    flat = torch.arange(float(np.prod(dims) * np.prod(element)))
+    at_once, built = FT._regular(flat, dims, element), FT._regular(flat, list(dims), element)
+    assert at_once.is_equal_type(built) and at_once.depth == built.depth == len(dims)
+    assert at_once.dense_shape() == built.dense_shape() == dims and at_once.element_shape == built.element_shape
+    a, b = at_once._type, built._type
+    while hasattr(a, '_length'):
+        assert (a._length, a._depth) == (b._length, b._depth) and a.is_equal_type(b) and vars(a).keys() == vars(b).keys()
+        a, b = a._dtype, b._dtype
+    assert vars(a) == vars(b) and at_once.indices == built.indices
+    assert torch.equal(at_once.as_dense(), built.as_dense()) and torch.equal(at_once.index(-1).data if len(dims) == 1 else at_once.index(-1).as_dense(),
+                                                                            built.index(-1).data if len(dims) == 1 else built.index(-1).as_dense())

@@ -1856,3 +1856,16 @@ def test_flash_attention_f32_of_rows_and_keys_of_zeros(core, B, Hd, Sq, Skv, D):
         for k, out in ((K2, None), (K_there, flat[:Q2.numel()].view(Q2.shape))):
             O = core.flash_attention_f32(Q2, k, V, out=out)
             assert float(((O.double().cpu() - ref).abs().amax(-1) / ref.abs().amax(-1)).max()) <= 1e-5   # (a NaN fails this too)
+
+
+@pytest.mark.parametrize('B,Hd,Sq,Skv,D', [(1, 1, 1, 1, 32), (2, 3, 65, 97, 64), (1, 4, 200, 33, 96), (1, 2, 16, 1024, 128)])
+def test_attention_on_flat_buffers_is_attention(core, B, Hd, Sq, Skv, D):
+    gen = torch.Generator(device='cuda').manual_seed(3)
+    q, k, v = (torch.randn((B, Hd, n, D), generator=gen, device='cuda') for n in (Sq, Skv, Skv))
+    ref = core.flash_attention_f32(q, k, v, 0.2)
+    assert torch.equal(core.flash_attention_f32_flat(q.view(-1), k.view(-1), v.view(-1), B, Hd, Sq, Skv, D, 0.2), ref.view(-1))
+    # operands the native call does not take go the long way: every other element of a buffer, and buffers of another size
+    strided = torch.stack([q.view(-1), q.view(-1)], dim=-1).view(-1)[::2]
+    assert torch.equal(core.flash_attention_f32_flat(strided, k.view(-1), v.view(-1), B, Hd, Sq, Skv, D, 0.2), ref.view(-1))
+    with pytest.raises(RuntimeError):
+        core.flash_attention_f32_flat(q.view(-1), k.view(-1), v.view(-1), B, Hd, Sq + 1, Skv, D, 0.2)
