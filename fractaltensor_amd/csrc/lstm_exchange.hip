@@ -1249,7 +1249,11 @@ int exchange_one_block_layers(int L, int B, int H, bool half) {
 // kernel in front, and what a deep stack's launches find less of in the caches), `layer` for every further layer of a launch until the
 // pipeline of layers is full, and for a step of each row block that a workgroup walks `step` and `fill` times the workgroups per compute
 // unit.  Fitted, for each hidden size, to the times of both kinds over 420 stacks of L up to 32, T 16 .. 128, B 8 .. 256 that blocks of 16
-// rows take more launches for; the times are met within 1.5 to 8 % (rms).
+// rows take more launches for; the times are met within 1.5 to 8 % (rms).  fp32 up to H 256 fitted again, to 280 stacks of L 3 .. 32, T 16 .. 128,
+// B 33 .. 256 whose weights and inputs change from call to call, when a launch had come to lay out its own buffers (the constants before
+// held a further launch for 37 to 54 us dearer): loss against the better kind in the mean, before and now, H 64 29.6 and 0.4 %, H 128 13.5 and 1.1,
+// H 256 3.7 and 2.1 (there a further launch is charged 8 us beyond the fit, half of what a cooperative one takes more); L 25 T 19 B 106 H 128
+// 194 -> 118 us, L 29 T 104 B 128 H 128 795 -> 572; over 30 other stacks 7.7 %.
 struct ExchangeCost {
   float step, fill, layer, first, next;
 };
@@ -1260,9 +1264,9 @@ ExchangeCost exchange_cost(int H, bool half, bool many) {
     if (H == 512) return many ? ExchangeCost{3.04f, 0.3f, 4.6f, 29.0f, 33.0f} : ExchangeCost{1.29f, 0.16f, 3.35f, 20.5f, 23.0f};
     return many ? ExchangeCost{2.96f, 0.26f, 6.05f, 41.0f, 47.0f} : ExchangeCost{1.7f, 0.76f, 5.0f, 9.0f, 38.0f};
   }
-  if (H == 64) return many ? ExchangeCost{1.44f, 0.64f, 1.75f, 0.0f, 0.0f} : ExchangeCost{0.35f, 0.48f, 0.0f, 51.5f, 51.5f};
-  if (H == 128) return many ? ExchangeCost{2.29f, 0.36f, 2.35f, 0.0f, 0.0f} : ExchangeCost{0.22f, 0.59f, 1.95f, 0.0f, 54.0f};
-  if (H == 256) return many ? ExchangeCost{3.77f, 0.48f, 4.25f, 38.0f, 38.0f} : ExchangeCost{1.01f, 0.42f, 3.15f, 0.0f, 37.0f};
+  if (H == 64) return many ? ExchangeCost{0.0f, 1.89f, 0.58f, 21.0f, 21.0f} : ExchangeCost{0.87f, 0.34f, 1.36f, 7.7f, 7.7f};
+  if (H == 128) return many ? ExchangeCost{2.58f, 0.27f, 2.15f, 0.0f, 0.0f} : ExchangeCost{0.77f, 0.39f, 1.76f, 6.8f, 8.4f};
+  if (H == 256) return many ? ExchangeCost{3.97f, 0.11f, 4.52f, 20.3f, 20.3f} : ExchangeCost{1.3f, 0.24f, 2.82f, 5.1f, 26.0f};
   return many ? ExchangeCost{2.86f, 0.35f, 4.1f, 35.0f, 36.0f} : ExchangeCost{1.73f, 0.24f, 4.35f, 11.5f, 34.0f};
 }
 
