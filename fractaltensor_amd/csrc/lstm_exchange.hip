@@ -23,8 +23,8 @@
 //     write-through stores, which is what a team that does not sit together uses.
 //
 // A step of a single layer takes 0.85 us at H = 64, 0.9 at 128, 1.2 at 256 and 1.9 at 512 (fp32), where a hand-over of the
-// persistent kernel's serial schedule took 5 to 6 and a launch per step 20 and more: L 20 T 30 B 32 H 128 1004 -> 80 us,
-// L 8 T 100 B 64 H 512 7.3 -> 0.73 ms, L 1 T 16 B 64 H 256 100 -> 31 us for both kernels (27 and 4).
+// persistent kernel's serial schedule took 5 to 6 and a launch per step 20 and more: L 20 T 30 B 32 H 128 1004 -> 78 us,
+// L 8 T 100 B 64 H 512 7.3 -> 0.72 ms, L 1 T 16 B 64 H 256 100 -> 29 us.
 //
 // The exchange buffers.  ring: the own layer's h for d = 1, four steps deep.  A workgroup that has all of h(t-1) knows
 // that every member of its team has read h(t-2) (it published h(t-1) behind a barrier that all its waves reached after
@@ -44,6 +44,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <chrono>
 #include <random>
 
 #include "ftk_common.h"
@@ -1325,8 +1326,12 @@ namespace {
 // A number that no launch of this process had, and that what a workspace holds by chance does not have: 56 bits, from a random start.
 unsigned long long exchange_launch_number() {
   static std::atomic<unsigned long long> next{[] {
-    std::random_device r;
-    return (unsigned long long)r() << 32 | r();
+    try {
+      std::random_device r;
+      return (unsigned long long)r() << 32 | r();
+    } catch (...) {   // no source of random numbers: the time, spread over the bits
+      return (unsigned long long)std::chrono::system_clock::now().time_since_epoch().count() * 0x9e3779b97f4a7c15ull;
+    }
   }()};
   while (true)
     if (const unsigned long long v = next.fetch_add(1, std::memory_order_relaxed) & ((1ull << 56) - 1)) return v;
