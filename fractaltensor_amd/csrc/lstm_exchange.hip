@@ -962,8 +962,14 @@ void lstm_exchange_kernel(ExchangeArgs a) {
     // layer at once, but for fp16 teams that share an XCD.  (us with 2, 4, 5, 6 and 8 times 64 cycles: L 6 T 80 B 16 H 128 106.1, 101.6, 100.5,
     // 101.2, 104.5; L 5 T 60 B 60 H 64 79.7, 78.3, 78.0, 78.2, 79.5; fp16 L 4 T 60 B 32 H 256 81.9, 80.1, 79.1, 77.5, 74.9, with 10 and 15 75.5, 83.4;
     // fp16 L 2 T 60 B 33 H 512 with 6, 8, 10 90.2, 88.9, 91.3; a single fp16 layer with 0, 1, 2: T 64 B 32 H 256 54.9, 55.9, 57.5, B 200 63.3, 63.2,
-    // 60.2.  At H 256 fp32, where it is asked for behind x only, any delay costs: L 4 T 60 B 16 93.2 without, 93.7 with 2, 95.7 with 4.)
+    // 60.2.  At H 64 with four teams or more to an XCD 192 cycles: L 20 T 60 B 20 96.6 with 3, 97.7, 99.4 and 101.4 with 4, 5, 6.  At H 256 fp32, where it is asked for behind x only, any delay costs: L 4 T 60 B 16 93.2 without, 93.7 with 2, 95.7 with 4.)
     constexpr bool TWICE = HALF ? H <= 512 : H <= 128;
+    int xcd_teams = 0;
+    if constexpr (TWICE) {
+      xcd_teams = __builtin_amdgcn_readfirstlane(a.per_xcd);
+      asm volatile("" : "+s"(xcd_teams));   // kept: left to itself the compiler reads the argument again in every step
+    }
+    const bool crowded = xcd_teams >= (HALF ? 2 : 4);
     share vh;
     float c[U] = {}, h[U];
     const unsigned x_get = do_x ? get : 0x80000000u, h_get = do_h ? get : 0x80000000u;   // out of bounds: zeros
@@ -981,8 +987,13 @@ void lstm_exchange_kernel(ExchangeArgs a) {
       const unsigned h_get_t = t > 0 ? h_get : 0x80000000u;
       __builtin_amdgcn_sched_barrier(0);
       if constexpr (TWICE) {
-        if (!FIRST || has_upper) __builtin_amdgcn_s_sleep(HALF ? 8 : 5);   // 64 cycles each
-        else if (HALF && a.per_xcd > 1) __builtin_amdgcn_s_sleep(2);
+        if (FIRST && !has_upper) {
+          if (HALF && crowded) __builtin_amdgcn_s_sleep(2);   // 64 cycles each
+        } else if (H == 64 && crowded) {
+          __builtin_amdgcn_s_sleep(3);
+        } else {
+          __builtin_amdgcn_s_sleep(HALF ? 8 : 5);
+        }
         load_share(own_l, h_get_t, before, vh, fresh);
       }
       __builtin_amdgcn_sched_barrier(0);
