@@ -54,7 +54,8 @@ namespace ftk {
 constexpr int kXLayers = 64;       // layers of one launch
 constexpr int kXBlocks = 128;      // row blocks a ragged batch may have
 constexpr int kXRing = 4;          // steps the own layer's ring holds
-constexpr int kXPlaces = 2048;     // workgroups of one launch
+constexpr int kXPlaces = 2047;     // workgroups of one launch
+constexpr int kXGaveUp = kXPlaces; // behind their places: the launch that a workgroup gave up in before all it waits for had come
 constexpr int kXRowPlaces = 256;   // workgroups that lay out the input rows of a slice: what the layer that reads them looks at
 constexpr int kXHandTop = 14;      // the scale of h: 2^14 (|h| < 1)
 constexpr unsigned kXSmallBits = (127u - 12u - kXHandTop) << 23;   // h * 2^14 below 2^-12: see ftk_stacked_lstm_small_states
@@ -65,7 +66,7 @@ struct ExchangeArgs {
   void* hsss;
   void* csss;
   int* status;          // [0] error word, [1] small states
-  unsigned long long* place;   // [groups]: launch << 8 | 1 + the XCC id, of every workgroup that is there and has laid out what it has to
+  unsigned long long* place;   // [groups]: launch << 8 | 1 + the XCC id, of every workgroup that is there and has laid out what it has to; [kXGaveUp]
   unsigned long long launch;   // what tells this launch's words from any that were there before
   const void* xs;       // not null: this launch lays out its own buffers (exchange_lay_out)
   unsigned char* ring;  // [L][nrb][kXRing] tiles
@@ -430,24 +431,35 @@ void lstm_exchange_kernel(ExchangeArgs a) {
     const int from = l == 0 ? (unit - l) * W : (unit - 1) * W, count = !own_buffers ? 0 : l == 0 ? b.row_layers * W : W;
     auto place = [&](int at) __attribute__((always_inline)) { return __hip_atomic_load(b.place + at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
     auto missing_place = [&](u64 p) __attribute__((always_inline)) { return p >> 8 != b.launch; };
+    // The workgroup that clears the status words may be the one that others have waited for in vain, and clear what they said.  So they note
+    // it behind the places first, and that workgroup looks there after it has cleared: of the two one is seen, whichever came first.
+    const bool clears = own_buffers && b.clear_status && unit == 0 && pc == 0;
+    const int first_at = !own_buffers ? unit * W : clears ? kXGaveUp : 0, looks = min(b.spin_limit, 1 << 20);
     u64 own, up;
-    int seen = 4;
-    for (int n = 0;; ++n) {
+    bool there = true;
+    for (int n = 1;; ++n) {
       own = place(unit * W + i);
       up = place((has_upper ? unit + 1 : unit) * W + i);
-      const u64 first = place(own_buffers ? 0 : unit * W);
-      bool waits = missing_place(own) || missing_place(up) || missing_place(first);
+      const u64 first = place(first_at);
+      bool waits = missing_place(own) || missing_place(up) || (!clears && missing_place(first));
       for (int k = 0; k < count; k += 64) waits = missing_place(place(from + min(k + lane, count - 1))) || waits;
-      if (__builtin_amdgcn_ballot_w64(waits) == 0) break;
-      if (n >= (1 << 20)) {
+      waits = __builtin_amdgcn_ballot_w64(waits) != 0;
+      if ((waits && n >= looks) || (clears && !missing_place(first))) {
+        __hip_atomic_store(b.place + kXGaveUp, b.launch << 8, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __hip_atomic_store(b.status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        seen = 0;
+        there = false;
         break;
       }
+      if (!waits) break;
       __builtin_amdgcn_s_sleep(4);
     }
-    if (__builtin_amdgcn_ballot_w64((int)(own & 0xff) != xcc) == 0) seen |= 1;
-    if (!has_upper || __builtin_amdgcn_ballot_w64((int)(up & 0xff) != xcc) == 0) seen |= 2;
+    int seen = 0;   // (a workgroup that has given up publishes and stores nothing: it takes the loop that asks whether it may)
+    if (there) {
+      seen = 4;
+      if (__builtin_amdgcn_ballot_w64((int)(own & 0xff) != xcc) == 0) seen |= 1;
+      if (!has_upper || __builtin_amdgcn_ballot_w64((int)(up & 0xff) != xcc) == 0) seen |= 2;
+    }
     places_seen = seen;
   }
   __syncthreads();
@@ -1231,7 +1243,7 @@ ExchangePlan exchange_plan(int L, int W, int nrb, int slots) {   // W: workgroup
 }
 
 constexpr size_t align256(size_t v) { return (v + 255) / 256 * 256; }
-constexpr size_t exchange_xratio_at = align256(kStatusBytes + kXPlaces * sizeof(unsigned long long));
+constexpr size_t exchange_xratio_at = align256(kStatusBytes + (kXPlaces + 1) * sizeof(unsigned long long));
 
 }  // namespace
 

@@ -254,8 +254,9 @@ int ftk_lstm_get_products(void);
  *               mode.  With F16X3 non-finite inputs give NaN where fp32
  *               arithmetic would give +-inf (the remainder plane of an infinite
  *               value is inf - inf);
- *   spin_limit: polls a bounded wait of the persistent kernel makes before it
- *               gives up, 0 = the default (2^22, seconds).
+ *   spin_limit: polls a bounded wait of the kernels whose workgroups wait for
+ *               each other makes before it gives up, 0 = the default (2^22,
+ *               seconds; 2^20 for a launch's workgroups to be there).
  * options == NULL means {DEFAULT, 0}.  No counterpart in the reference.
  */
 typedef struct ftk_lstm_options {

@@ -1460,6 +1460,38 @@ def test_exchange_launches_lay_out_their_own_buffers(core, monkeypatch, half, H,
             assert all(torch.equal(g.cpu()[:, live], r) for g, r in zip(got, ref)), turn
 
 
+def test_a_launch_whose_first_workgroup_came_too_late_says_so(core, monkeypatch):
+    """A workgroup that gives up waiting for the others may do so before the first one is there, which clears the status words: the word is set
+    when the launch ends all the same.  What such a workgroup leaves behind the places is written from the host, before the launch."""
+    monkeypatch.setenv('FTK_LSTM_EXCHANGE', '1')
+    monkeypatch.setenv('FTK_LSTM_EXCHANGE_FRONT', '0')
+    L, T, B, H = 2, 3, 20, 64
+    xs, WU, bs = (dev(a) for a in lstm_inputs(6, L, T, B, H, 1.0 / np.sqrt(H)))
+    ws = torch.zeros(core.stacked_lstm_workspace_bytes(L, T, B, H), dtype=torch.uint8, device='cuda')
+    ref = core.stacked_lstm(xs, WU, bs, workspace=ws, check=True)
+    places = ws[256:256 + 2048 * 8].view(torch.int64)                        # the launch's number, 56 bits, and 8 bits of each workgroup's own
+    places[2047] = ((int(places[0]) >> 8) + 1) << 8                          # of the launch that comes next
+    core.stacked_lstm(xs, WU, bs, workspace=ws)
+    assert core.persistent_status(ws) == 1
+    again = core.stacked_lstm(xs, WU, bs, workspace=ws, check=True)          # and the launch behind it is none of that
+    assert all(torch.equal(a, b) for a, b in zip(again, ref))
+
+
+@pytest.mark.parametrize('L,T,B,H', [(1, 1, 16, 64), (2, 1, 250, 256), (8, 1, 70, 128), (1, 4, 40, 512)])
+def test_a_start_that_gives_up_says_so(core, monkeypatch, L, T, B, H):
+    """One look at the other workgroups' places: where it is one too few the status word is set, also if no step waits for another; where
+    it is not set the results are there."""
+    monkeypatch.setenv('FTK_LSTM_EXCHANGE', '1')
+    monkeypatch.setenv('FTK_LSTM_EXCHANGE_FRONT', '0')
+    xs, WU, bs = (dev(a) for a in lstm_inputs(7, L, T, B, H, 1.0 / np.sqrt(H)))
+    ref = core.stacked_lstm(xs, WU, bs, check=True)
+    ws = torch.zeros(core.stacked_lstm_workspace_bytes(L, T, B, H), dtype=torch.uint8, device='cuda')
+    for _ in range(20):
+        out = tuple(torch.full_like(r, float('nan')) for r in ref)
+        core.stacked_lstm(xs, WU, bs, out=out, workspace=ws, spin_limit=1)
+        assert core.persistent_status(ws) == 1 or all(torch.equal(a, b) for a, b in zip(out, ref))
+
+
 @pytest.mark.parametrize('half,H,L,T,B,dil', [
     (False, 64, 3, 5, 17, None),           # half a k step per wave: x and h waves; the second row block holds one row
     (False, 64, 32, 4, 130, None),         # several 32-row blocks per workgroup, the last of two rows
