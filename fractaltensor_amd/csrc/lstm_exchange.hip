@@ -147,7 +147,7 @@ __device__ __forceinline__ void exchange_input_row(const v4u (&raw)[N], Put put,
 // Before the first step of a launch that lays out its own buffers.  What others of this launch look at (see the top of the file) is written
 // here, in front of the weights; then the workgroup's place says that it is done.  Whoever reads waits for the places it depends on, and a
 // place is known as this launch's by the number in it, so nothing has to be cleared before the launch.  Words are written through, and no line of
-// them is written by two workgroups: no cache holds a part of one.
+// them is written by two workgroups (they begin on a line of their own: exchange_places_at): no cache holds a part of one.
 //
 // Bound by latency: input rows that come from memory, stores that go there, places that come from there.  It takes 2 to 3 us where the kernel in
 // front took 3.4 to 12 and a launch (us a call with other inputs and weights each time, that kernel and this: L 2 T 36 B 155 H 64 50.1, 47.1; L 1 T 64
@@ -1243,18 +1243,29 @@ ExchangePlan exchange_plan(int L, int W, int nrb, int slots) {   // W: workgroup
 }
 
 constexpr size_t align256(size_t v) { return (v + 255) / 256 * 256; }
-constexpr size_t exchange_xratio_at = align256(kStatusBytes + (kXPlaces + 1) * sizeof(unsigned long long));
+constexpr size_t exchange_xratio_at = align256((kXPlaces + 1) * sizeof(unsigned long long));   // behind the places
+
+// What the workgroups write for each other begins on a line of its own, wherever a caller's workspace begins (the status block stays at its
+// start): no line is shared by workgroups that lay out different parts (exchange_lay_out), and a place is one access.
+size_t exchange_places_at(const void* ws) { return align256((size_t)ws + kStatusBytes) - (size_t)ws; }
 
 }  // namespace
 
 // Whether lstm_exchange runs this hidden size and type at all.
 bool exchange_takes(int H, bool half) { return exchange_flavour_of(H, half).one != nullptr; }
 
-// Bytes of workspace for L layers: [status block][places][xratio][ring][hand], with either kind of row block.
-size_t exchange_workspace_bytes(int L, int T, int B, int H, bool half) {
+namespace {
+// Bytes of [places][xratio][ring][hand] for L layers, with either kind of row block.
+size_t exchange_buffer_bytes(int L, int T, int B, int H, bool half) {
   const size_t rows = (size_t)(B + 31) / 32 * 32;   // never less than with blocks of 16
   return exchange_xratio_at + align256((size_t)(T + 1) * rows * sizeof(float)) +
          rows * H * (half ? 2 : 4) * ((size_t)L * kXRing + (size_t)(L + 1) * T);
+}
+}  // namespace
+
+// Bytes of workspace for L layers: the status block, up to 255 bytes to a line, and these.
+size_t exchange_workspace_bytes(int L, int T, int B, int H, bool half) {
+  return kStatusBytes + 256 + exchange_buffer_bytes(L, T, B, H, half);
 }
 
 // Whether a layer of a buffer stays below what a buffer descriptor and its offsets reach.
@@ -1382,8 +1393,8 @@ size_t exchange_need(int L, int T, int B, int H, bool half) {
   return exchange_workspace_bytes(most ? std::min(L, most) : L, T, B, H, half);
 }
 
-// Runs the stack; *handled is false when the device cannot hold a layer, or the workspace is smaller than exchange_need
-// says: other kernels may do with it.  Deeper stacks than a launch holds run as
+// Runs the stack; *handled is false when the device cannot hold a layer, or the workspace has less room than that:
+// other kernels may do with it.  Deeper stacks than a launch holds run as
 // consecutive launches, each reading the hidden sequence of the layer below it like the first reads xs.
 int run_exchange(bool half, const void* xs, const void* WU, const float* bias, const int* dil, const int* active, void* hsss,
                  void* csss, int L, int T, int B, int H, void* ws, size_t ws_bytes, hipStream_t s, bool* handled, int spin_limit) {
@@ -1398,7 +1409,9 @@ int run_exchange(bool half, const void* xs, const void* WU, const float* bias, c
   const int slots = exchange_slots(many ? f.many : f.one), block = many ? 32 : 16, nrb = (B + block - 1) / block;
   const int W = H / exchange_units(H, half, many);
   const size_t esize = half ? 2 : 4, slab = (size_t)T * B * H, wlayer = (size_t)8 * H * H, tile = exchange_tile_bytes(H, half, block);
-  if (!ws || ws_bytes < exchange_workspace_bytes(std::min(L, most), T, B, H, half)) return FTK_OK;
+  const size_t places_at = exchange_places_at(ws);
+  if (!ws || ws_bytes < places_at + exchange_buffer_bytes(std::min(L, most), T, B, H, half)) return FTK_OK;
+  char* const buffers = (char*)ws + places_at;
   const bool records = stream_records(s);
   for (int l0 = 0; l0 < L; l0 += most) {
     const int lc = std::min(most, L - l0);
@@ -1410,10 +1423,10 @@ int run_exchange(bool half, const void* xs, const void* WU, const float* bias, c
     a.hsss = (char*)hsss + (size_t)l0 * slab * esize;
     a.csss = (char*)csss + (size_t)l0 * slab * esize;
     a.status = (int*)ws;
-    a.place = (unsigned long long*)((char*)ws + kStatusBytes);
-    float* xratio = (float*)((char*)ws + exchange_xratio_at);
+    a.place = (unsigned long long*)buffers;
+    float* xratio = (float*)(buffers + exchange_xratio_at);
     a.xratio = xratio;
-    a.ring = (unsigned char*)ws + exchange_xratio_at + align256((size_t)(T + 1) * nrb * block * sizeof(float));
+    a.ring = (unsigned char*)buffers + exchange_xratio_at + align256((size_t)(T + 1) * nrb * block * sizeof(float));
     a.hand = a.ring + (size_t)lc * nrb * kXRing * tile;
     a.L = lc; a.T = T; a.B = B; a.nrb = nrb;
     a.slices = p.slices;

@@ -120,7 +120,11 @@ int ftk_lstm_elementwise_f32(const float* gates, const float* bias,
                              const float* c_prev, float* h, float* c, int B,
                              int H, ftk_stream_t stream);
 
-/* Bytes of workspace ftk_stacked_lstm_f32 / ftk_dilated_lstm_f32 need. */
+/* Bytes of workspace ftk_stacked_lstm_f32 / ftk_dilated_lstm_f32 need.  An LSTM
+ * workspace is best 256-byte aligned, as allocators give it, and at least 4-byte
+ * aligned (the status word is its first int).  What the workgroups of a launch
+ * write for each other begins at the next multiple of 256 behind the status
+ * block; the size queries count the bytes up to there. */
 size_t ftk_stacked_lstm_workspace_bytes(int L, int T, int B, int H);
 
 /*

@@ -1460,6 +1460,31 @@ def test_exchange_launches_lay_out_their_own_buffers(core, monkeypatch, half, H,
             assert all(torch.equal(g.cpu()[:, live], r) for g, r in zip(got, ref)), turn
 
 
+@pytest.mark.parametrize('half,H,L,T,B', [(False, 64, 3, 5, 70), (False, 256, 2, 4, 300), (True, 512, 2, 3, 33)])
+@pytest.mark.parametrize('offset', [0, 4, 64, 128, 200, 252])
+def test_exchange_buffers_begin_on_a_line(core, monkeypatch, half, H, L, T, B, offset):
+    """A workspace that begins anywhere: what the workgroups of a launch write for each other begins at the next 256 bytes behind the status
+    block, so that none of its lines is shared, inside what the size query asks for, and the bits are the same."""
+    monkeypatch.setenv('FTK_LSTM_EXCHANGE', '1')
+    fn = core.stacked_lstm_f16 if half else core.stacked_lstm
+    size = int((core.lib.ftk_stacked_lstm_f16_workspace_bytes if half else core.stacked_lstm_workspace_bytes)(L, T, B, H))
+    xs, WU, bs = lstm_inputs(8, L, T, B, H, 1.0 / np.sqrt(H))
+    xs, WU, bs = (dev(xs.astype(np.float16)), dev(WU.astype(np.float16)), dev(bs)) if half else (dev(xs), dev(WU), dev(bs))
+    ref = fn(xs, WU, bs, check=True)
+    memory = torch.randint(0, 256, (size + 512,), dtype=torch.uint8, device='cuda')
+    assert memory.data_ptr() % 256 == 0
+    ws, at, before = memory[offset:offset + size], (offset + 256 + 255) // 256 * 256, memory.clone()
+    numbers = []
+    for _ in range(3):
+        got = fn(xs, WU, bs, workspace=ws)
+        assert core.persistent_status(ws) == 0
+        assert all(torch.equal(a, b) for a, b in zip(got, ref))
+        numbers.append(int(memory[at:at + 8].view(torch.int64)) >> 8)        # of the launch, in the first workgroup's place
+        for first, last in ((0, offset), (offset + 256, at), (offset + size, size + 512)):
+            assert torch.equal(memory[first:last], before[first:last])
+    assert numbers[1] == numbers[0] + 1 and numbers[2] == numbers[1] + 1
+
+
 def test_a_launch_whose_first_workgroup_came_too_late_says_so(core, monkeypatch):
     """A workgroup that gives up waiting for the others may do so before the first one is there, which clears the status words: the word is set
     when the launch ends all the same.  What such a workgroup leaves behind the places is written from the host, before the launch."""
