@@ -1421,6 +1421,26 @@ def test_exchange_loops_give_the_same_bits(core, half, H, L, B, T):
         assert all(torch.equal(a, b) for a, b in zip(dense, general))
 
 
+def exchange_places(ws):
+    """Behind a workspace's status block, at a multiple of 256: a word for every workgroup of a launch of the exchange kernel, with the launch's
+    number above the lowest 8 bits, and as the last of them that number too where a workgroup gave up before all were there."""
+    at = (ws.data_ptr() + 256 + 255) // 256 * 256 - ws.data_ptr()
+    return ws[at:at + 2048 * 8].view(torch.int64)
+
+
+def lays_out_its_own_buffers(core, run, ws):
+    """Whether the stack that run(ws) launches writes its own input rows and first words: its first workgroup then sets the error word if the launch
+    that comes next is noted as one that was given up, which behind the kernel that writes them nobody looks at."""
+    run(ws)
+    places = exchange_places(ws)
+    places[-1] = ((int(places[0]) >> 8) + 1) << 8
+    run(ws)
+    own = core.persistent_status(ws) == 1
+    run(ws)
+    assert core.persistent_status(ws) == 0
+    return own
+
+
 @pytest.mark.parametrize('half,H,L,T,B,dil', [
     (False, 64, 1, 1, 1, None),            # one step, one row: the second row of a pair of steps is past the end
     (False, 64, 1, 33, 17, None),          # workgroups with several turns of rows, an odd number of steps
@@ -1435,7 +1455,9 @@ def test_exchange_loops_give_the_same_bits(core, half, H, L, B, T):
 ])
 def test_exchange_launches_lay_out_their_own_buffers(core, monkeypatch, half, H, L, T, B, dil):
     """A launch that writes its own input rows and first words gives the bits of one behind the kernel that writes them, dense and ragged, on
-    a workspace that still holds what launches with other inputs, of another shape, and noise have left there."""
+    a workspace that still holds what launches with other inputs, of another shape, and noise have left there.  The dense one is the oracle's
+    result too, and which of the two ran is looked at."""
+    monkeypatch.setenv('FTK_LSTM_EXCHANGE', '1')
     fn = core.stacked_lstm_f16 if half else core.stacked_lstm
     size = core.lib.ftk_stacked_lstm_f16_workspace_bytes if half else core.stacked_lstm_workspace_bytes
     other = (L + 1, T + 1, B + 3)
@@ -1451,13 +1473,38 @@ def test_exchange_launches_lay_out_their_own_buffers(core, monkeypatch, half, H,
             run = lambda ws, xs=cast(xs), WU=cast(WU), bs=dev(bs), d=d, active=active: fn(xs, WU, bs, dilations=d, workspace=ws, active_rows=active)
             monkeypatch.setenv('FTK_LSTM_EXCHANGE_FRONT', '1')
             ref = [r.cpu()[:, live] for r in run(torch.zeros_like(ws))]
+            assert not lays_out_its_own_buffers(core, run, torch.zeros_like(ws))
             stacks.append((run, live, ref))
+            if seed == 1 and active is None and half:
+                hr, cr = (r.astype(np.float32) for r in ko.stacked_lstm_f16(xs.astype(np.float16), WU.astype(np.float16), bs, d))
+                assert all(ko.max_rel_err(r.float().numpy().reshape(o.shape), o) <= F16_TOL for r, o in zip(ref, (hr, cr)))
+            elif seed == 1 and active is None:
+                for r, o in zip(ref, c_oracle.stacked_lstm(xs, WU, bs, d)):
+                    assert_lstm_close(r.view(l, t, b, H), o, 'behind the kernel in front')
     monkeypatch.setenv('FTK_LSTM_EXCHANGE_FRONT', '0')
+    assert all(lays_out_its_own_buffers(core, run, ws) for run, _, _ in stacks)
     for turn in range(4):
         for run, live, ref in stacks:
             got = run(ws)
             assert core.persistent_status(ws) == 0, 'a wait gave up'
             assert all(torch.equal(g.cpu()[:, live], r) for g, r in zip(got, ref)), turn
+
+
+@pytest.mark.parametrize('H,L,T,B,own', [
+    (64, 1, 16, 8, True),        # 2 turns of 32 rows to a workgroup (us in a row without and behind the kernel in front, beside the others)
+    (64, 1, 128, 8, False),      # 16 turns: 123.4, 116.8
+    (64, 1, 128, 250, True),     # the same, for a kernel in front with 32 times the rows: 125.9, 129.2
+    (64, 2, 96, 8, False),       # 6 turns: 115.0, 113.2
+    (64, 2, 96, 100, True),      # 98.8, 101.0
+    (256, 1, 128, 8, False),     # 4 turns: 161.4, 159.5
+    (256, 1, 128, 40, True),     # 163.6, 166.3
+])
+def test_stacks_with_many_rows_to_a_workgroup_keep_the_kernel_in_front(core, H, L, T, B, own):
+    """Both sides of the line between a launch that lays out its own buffers and one behind the kernel that does."""
+    xs, WU, bs = lstm_inputs(9, L, T, B, H, 1.0 / np.sqrt(H))
+    xs, WU, bs = dev(xs), dev(WU), dev(bs)
+    ws = torch.empty(core.stacked_lstm_workspace_bytes(L, T, B, H), dtype=torch.uint8, device='cuda')
+    assert lays_out_its_own_buffers(core, lambda ws: core.stacked_lstm(xs, WU, bs, workspace=ws), ws) == own
 
 
 @pytest.mark.parametrize('half,H,L,T,B', [(False, 64, 3, 5, 70), (False, 256, 2, 4, 300), (True, 512, 2, 3, 33)])
@@ -1494,8 +1541,8 @@ def test_a_launch_whose_first_workgroup_came_too_late_says_so(core, monkeypatch)
     xs, WU, bs = (dev(a) for a in lstm_inputs(6, L, T, B, H, 1.0 / np.sqrt(H)))
     ws = torch.zeros(core.stacked_lstm_workspace_bytes(L, T, B, H), dtype=torch.uint8, device='cuda')
     ref = core.stacked_lstm(xs, WU, bs, workspace=ws, check=True)
-    places = ws[256:256 + 2048 * 8].view(torch.int64)                        # the launch's number, 56 bits, and 8 bits of each workgroup's own
-    places[2047] = ((int(places[0]) >> 8) + 1) << 8                          # of the launch that comes next
+    places = exchange_places(ws)
+    places[-1] = ((int(places[0]) >> 8) + 1) << 8                          # of the launch that comes next
     core.stacked_lstm(xs, WU, bs, workspace=ws)
     assert core.persistent_status(ws) == 1
     again = core.stacked_lstm(xs, WU, bs, workspace=ws, check=True)          # and the launch behind it is none of that
