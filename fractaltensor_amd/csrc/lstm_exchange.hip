@@ -1249,13 +1249,30 @@ constexpr size_t exchange_xratio_at = align256((kXPlaces + 1) * sizeof(unsigned 
 // start): no line is shared by workgroups that lay out different parts (exchange_lay_out), and a place is one access.
 size_t exchange_places_at(const void* ws) { return align256((size_t)ws + kStatusBytes) - (size_t)ws; }
 
+// ring and hand begin at multiples of 16 KB: tiles are 4 to 128 KB, powers of two, and steps take longer where they lie across such bounds (us
+// with `hand` at 0, 256, 1024 bytes beyond one: H 64 L 5 T 94 B 31 117.8, 121.1, 118.6; H 128 L 7 T 80 B 14 108.3, 111.4, 108.7; H 256 L 4 T 105 B 44 148.2, 151.3,
+// 150.8, and 150.4 with `ring` at 256; fp16 L 3 T 77 B 78 H 256 90.5, 93.4, 91.8).  Right behind the words in front of them they began at
+// 256 bytes times what T and B make of it.
+constexpr size_t kXTilesAt = 16384;
+struct ExchangeTiles {
+  size_t ring, hand, end;   // bytes from the start of the workspace
+};
+ExchangeTiles exchange_tiles_at(const void* ws, size_t to, size_t ring_from, size_t ring_bytes, size_t hand_bytes) {
+  auto up = [&](size_t at) { return ((size_t)ws + at + to - 1) / to * to - (size_t)ws; };
+  ExchangeTiles t;
+  t.ring = up(ring_from);
+  t.hand = up(t.ring + ring_bytes);
+  t.end = t.hand + hand_bytes;
+  return t;
+}
+
 }  // namespace
 
 // Whether lstm_exchange runs this hidden size and type at all.
 bool exchange_takes(int H, bool half) { return exchange_flavour_of(H, half).one != nullptr; }
 
 namespace {
-// Bytes of [places][xratio][ring][hand] for L layers, with either kind of row block.
+// Bytes of [places][xratio][ring][hand] for L layers, with either kind of row block and nothing between them.
 size_t exchange_buffer_bytes(int L, int T, int B, int H, bool half) {
   const size_t rows = (size_t)(B + 31) / 32 * 32;   // never less than with blocks of 16
   return exchange_xratio_at + align256((size_t)(T + 1) * rows * sizeof(float)) +
@@ -1263,9 +1280,9 @@ size_t exchange_buffer_bytes(int L, int T, int B, int H, bool half) {
 }
 }  // namespace
 
-// Bytes of workspace for L layers: the status block, up to 255 bytes to a line, and these.
+// Bytes of workspace for L layers: the status block, up to 255 bytes to a line, these, and up to kXTilesAt in front of ring and hand each.
 size_t exchange_workspace_bytes(int L, int T, int B, int H, bool half) {
-  return kStatusBytes + 256 + exchange_buffer_bytes(L, T, B, H, half);
+  return kStatusBytes + 256 + 2 * kXTilesAt + exchange_buffer_bytes(L, T, B, H, half);
 }
 
 // Whether a layer of a buffer stays below what a buffer descriptor and its offsets reach.
@@ -1409,9 +1426,14 @@ int run_exchange(bool half, const void* xs, const void* WU, const float* bias, c
   const int slots = exchange_slots(many ? f.many : f.one), block = many ? 32 : 16, nrb = (B + block - 1) / block;
   const int W = H / exchange_units(H, half, many);
   const size_t esize = half ? 2 : 4, slab = (size_t)T * B * H, wlayer = (size_t)8 * H * H, tile = exchange_tile_bytes(H, half, block);
-  const size_t places_at = exchange_places_at(ws);
+  const size_t places_at = exchange_places_at(ws), xratio_at = places_at + exchange_xratio_at;
+  const size_t ring_from = xratio_at + align256((size_t)(T + 1) * nrb * block * sizeof(float));
   if (!ws || ws_bytes < places_at + exchange_buffer_bytes(std::min(L, most), T, B, H, half)) return FTK_OK;
-  char* const buffers = (char*)ws + places_at;
+  // (less room than the size query asks for, but enough with nothing between the buffers: so)
+  auto tiles_of = [&](int layers, size_t to) {
+    return exchange_tiles_at(ws, to, ring_from, (size_t)layers * nrb * kXRing * tile, (size_t)(layers + 1) * T * nrb * tile);
+  };
+  const size_t tiles_to = ws_bytes >= tiles_of(std::min(L, most), kXTilesAt).end ? kXTilesAt : 256;
   const bool records = stream_records(s);
   for (int l0 = 0; l0 < L; l0 += most) {
     const int lc = std::min(most, L - l0);
@@ -1423,11 +1445,12 @@ int run_exchange(bool half, const void* xs, const void* WU, const float* bias, c
     a.hsss = (char*)hsss + (size_t)l0 * slab * esize;
     a.csss = (char*)csss + (size_t)l0 * slab * esize;
     a.status = (int*)ws;
-    a.place = (unsigned long long*)buffers;
-    float* xratio = (float*)(buffers + exchange_xratio_at);
+    a.place = (unsigned long long*)((char*)ws + places_at);
+    float* xratio = (float*)((char*)ws + xratio_at);
     a.xratio = xratio;
-    a.ring = (unsigned char*)buffers + exchange_xratio_at + align256((size_t)(T + 1) * nrb * block * sizeof(float));
-    a.hand = a.ring + (size_t)lc * nrb * kXRing * tile;
+    const ExchangeTiles tiles = tiles_of(lc, tiles_to);
+    a.ring = (unsigned char*)ws + tiles.ring;
+    a.hand = (unsigned char*)ws + tiles.hand;
     a.L = lc; a.T = T; a.B = B; a.nrb = nrb;
     a.slices = p.slices;
     a.units = lc * p.slices;

@@ -124,7 +124,8 @@ int ftk_lstm_elementwise_f32(const float* gates, const float* bias,
  * workspace is best 256-byte aligned, as allocators give it, and at least 4-byte
  * aligned (the status word is its first int).  What the workgroups of a launch
  * write for each other begins at the next multiple of 256 behind the status
- * block; the size queries count the bytes up to there. */
+ * block, and their tiles of h, with the room that the size queries ask for, at
+ * multiples of 16 KB; the queries count the bytes up to there. */
 size_t ftk_stacked_lstm_workspace_bytes(int L, int T, int B, int H);
 
 /*

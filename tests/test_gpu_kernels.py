@@ -1532,6 +1532,33 @@ def test_exchange_buffers_begin_on_a_line(core, monkeypatch, half, H, L, T, B, o
     assert numbers[1] == numbers[0] + 1 and numbers[2] == numbers[1] + 1
 
 
+@pytest.mark.parametrize('L,T,B', [(2, 3, 32), (1, 1, 20), (3, 40, 64)])
+@pytest.mark.parametrize('offset', [0, 256, 1000, 16384 + 4096])
+def test_exchange_tiles_begin_at_16_kb(core, monkeypatch, L, T, B, offset):
+    """The tiles of h, and of the input rows in front of them, do not lie across multiples of 16 KB, wherever a workspace of the size asked for
+    begins; one that has no room for the bytes in front of them is taken all the same.  fp16 data: the input rows stand there as they are."""
+    monkeypatch.setenv('FTK_LSTM_EXCHANGE', '1')
+    H, tile, blocks = 512, 16384, (B + 15) // 16
+    up = lambda at, to: (at + to - 1) // to * to
+    size = int(core.lib.ftk_stacked_lstm_f16_workspace_bytes(L, T, B, H))
+    xs, WU, bs = lstm_inputs(8, L, T, B, H, 1.0 / np.sqrt(H))
+    xs, WU, bs = dev(xs.astype(np.float16)), dev(WU.astype(np.float16)), dev(bs)
+    ref = core.stacked_lstm_f16(xs, WU, bs, check=True)
+    for room in (size, size - 2 * 16384):
+        memory = torch.zeros(offset + room + 256, dtype=torch.uint8, device='cuda')
+        begins = memory.data_ptr()
+        assert begins % 256 == 0
+        got = core.stacked_lstm_f16(xs, WU, bs, workspace=memory[offset:offset + room])
+        assert core.persistent_status(memory[offset:offset + room]) == 0
+        assert all(torch.equal(a, b) for a, b in zip(got, ref))
+        to = 16384 if room == size else 256
+        ring = up(up(begins + offset + 256, 256) + 2048 * 8 + up((T + 1) * blocks * 16 * 4, 256), to)
+        at = up(ring + L * blocks * 4 * tile, to) - begins
+        rows = memory[at:at + T * blocks * tile].view(torch.float16).view(T, blocks, H // 8, 16, 8).permute(0, 1, 3, 2, 4).reshape(T, blocks * 16, H)
+        assert torch.equal(rows[:, :B], xs) and not bool(rows[:, B:].any())
+        assert not bool(memory[offset + room:].any())
+
+
 def test_a_launch_whose_first_workgroup_came_too_late_says_so(core, monkeypatch):
     """A workgroup that gives up waiting for the others may do so before the first one is there, which clears the status words: the word is set
     when the launch ends all the same.  What such a workgroup leaves behind the places is written from the host, before the launch."""
