@@ -80,6 +80,7 @@ struct ExchangeArgs {
   int ragged;
   int row_layers;       // xs: layers whose workgroups lay out the input rows of their slice
   int clear_status;     // xs: this launch clears the status words
+  int early;            // no h goes to another XCD: fp32 teams with one row block look for theirs at once (walk_lean)
   int dil[kXLayers];
   int steps_of[kXBlocks];   // ragged: steps row block rb takes part in (T reaches 262143 at H = 64)
 };
@@ -930,8 +931,8 @@ void lstm_exchange_kernel(ExchangeArgs a) {
   // T 64 B 16 in us, the loop above -> this one, one layer / eight: fp32 H 64 79 -> 62 / 107 -> 94, 128 83 -> 65 / 113 -> 99,
   // 256 103 -> 87 / 135 -> 116, 512 160 -> 142 / 196 -> 175; fp16 H 256 79 -> 58 / 105 -> 100, 512 106 -> 78 / 141 -> 118.
   // PLAIN: the layer above is on this XCD, or there is none.
-  auto walk_lean = [&](auto first_c, auto plain_c) __attribute__((always_inline)) {
-    constexpr bool FIRST = decltype(first_c)::value, PLAIN = decltype(plain_c)::value;
+  auto walk_lean = [&](auto first_c, auto plain_c, auto early_c) __attribute__((always_inline)) {
+    constexpr bool FIRST = decltype(first_c)::value, PLAIN = decltype(plain_c)::value, EARLY = decltype(early_c)::value;
     constexpr std::integral_constant<int, PLAIN ? 0 : kAgentScope> up_policy{};
     constexpr int step = TILE, wrap = kXRing * TILE - 1;
     const int words_at = s * kXRing * TILE;
@@ -970,11 +971,14 @@ void lstm_exchange_kernel(ExchangeArgs a) {
     // h is asked for in front of the products of x, where registers and its way leave time for it, and behind them: what comes
     // too early is not there yet, and to ask again only then costs the whole way once more.  (L 1 T 64 B 16: H 128
     // 69 us when asked for behind x only, 65 with both; L 20 T 30 B 32 H 128 83 and 81.6; fp16 H 512 88 and 78.)  The first time it is asked
-    // for when it is about to be there: in a stack of several layers, whose steps are the longer ones, some 320 cycles into the step (fp16 512), in a single
-    // layer at once, but for fp16 teams that share an XCD.  (us with 2, 4, 5, 6 and 8 times 64 cycles: L 6 T 80 B 16 H 128 106.1, 101.6, 100.5,
-    // 101.2, 104.5; L 5 T 60 B 60 H 64 79.7, 78.3, 78.0, 78.2, 79.5; fp16 L 4 T 60 B 32 H 256 81.9, 80.1, 79.1, 77.5, 74.9, with 10 and 15 75.5, 83.4;
-    // fp16 L 2 T 60 B 33 H 512 with 6, 8, 10 90.2, 88.9, 91.3; a single fp16 layer with 0, 1, 2: T 64 B 32 H 256 54.9, 55.9, 57.5, B 200 63.3, 63.2,
-    // 60.2.  At H 64 with four teams or more to an XCD 192 cycles: L 20 T 60 B 20 96.6 with 3, 97.7, 99.4 and 101.4 with 4, 5, 6.  At H 256 fp32, where it is asked for behind x only, any delay costs: L 4 T 60 B 16 93.2 without, 93.7 with 2, 95.7 with 4.)
+    // for when it is about to be there.  Where no h goes to another XCD (EARLY: a single layer, or fp32 stacks whose row slices have an XCD each or share
+    // one) steps are short and every cycle in front of it costs, but for fp16 teams that share an XCD; elsewhere the layer whose h comes from
+    // another XCD sets the pace, and it is some 320 cycles into the step (fp16 512), at H 64 with four teams or more to an XCD 192.
+    // (us with 0, 2, 4, 5, 6 and 8 times 64 cycles, EARLY: H 128 L 2 T 100 B 233 102.7, 106.5, 113.5, 113.5, 115.7, 120.9; H 64 L 5 T 86 B 108 90.1, 93.2, 97.9, 100.3,
+    // 102.2, 107.0; a single fp16 layer with 0, 1, 2: T 64 B 32 H 256 54.9, 55.9, 57.5, B 200 63.3, 63.2, 60.2.  Elsewhere with 2, 4, 5, 6, 8: L 6 T 80 B 16 H 128 106.1, 101.6,
+    // 100.5, 101.2, 104.5; L 5 T 60 B 60 H 64 79.7, 78.3, 78.0, 78.2, 79.5; fp16 L 4 T 60 B 32 H 256 81.9, 80.1, 79.1, 77.5, 74.9, with 10 and 15 75.5, 83.4;
+    // fp16 L 2 T 60 B 33 H 512 with 6, 8, 10 90.2, 88.9, 91.3; H 64 L 20 T 60 B 20 with 3, 4, 5, 6 96.6, 97.7, 99.4, 101.4.  At H 256 fp32, where it is
+    // asked for behind x only, any delay costs: L 4 T 60 B 16 93.2 without, 93.7 with 2, 95.7 with 4.)
     constexpr bool TWICE = HALF ? H <= 512 : H <= 128;
     int xcd_teams = 0;
     if constexpr (TWICE) {
@@ -999,12 +1003,14 @@ void lstm_exchange_kernel(ExchangeArgs a) {
       const unsigned h_get_t = t > 0 ? h_get : 0x80000000u;
       __builtin_amdgcn_sched_barrier(0);
       if constexpr (TWICE) {
-        if (FIRST && !has_upper) {
-          if (HALF && crowded) __builtin_amdgcn_s_sleep(2);   // 64 cycles each
-        } else if (H == 64 && crowded) {
-          __builtin_amdgcn_s_sleep(3);
-        } else {
-          __builtin_amdgcn_s_sleep(HALF ? 8 : 5);
+        if constexpr (!EARLY) {
+          if (HALF && FIRST && !has_upper) {
+            if (crowded) __builtin_amdgcn_s_sleep(2);   // 64 cycles each
+          } else if (H == 64 && crowded) {
+            __builtin_amdgcn_s_sleep(3);
+          } else {
+            __builtin_amdgcn_s_sleep(HALF ? 8 : 5);
+          }
         }
         load_share(own_l, h_get_t, before, vh, fresh);
       }
@@ -1064,10 +1070,19 @@ void lstm_exchange_kernel(ExchangeArgs a) {
   };
   if constexpr (!MANY) {
     if (lean) {
-      if (l == 0 && hand_plain) walk_lean(std::true_type{}, std::true_type{});
-      else if (l == 0) walk_lean(std::true_type{}, std::false_type{});
-      else if (hand_plain) walk_lean(std::false_type{}, std::true_type{});
-      else walk_lean(std::false_type{}, std::false_type{});
+      constexpr std::true_type yes{};
+      constexpr std::false_type no{};
+      if constexpr (!HALF && H <= 128) {
+        if (hand_plain && again->early) {
+          if (l == 0) walk_lean(yes, yes, yes);
+          else walk_lean(no, yes, yes);
+          return;
+        }
+      }
+      if (l == 0 && hand_plain) walk_lean(yes, yes, no);
+      else if (l == 0) walk_lean(yes, no, no);
+      else if (hand_plain) walk_lean(no, yes, no);
+      else walk_lean(no, no, no);
       return;
     }
   }
@@ -1473,6 +1488,8 @@ int run_exchange(bool half, const void* xs, const void* WU, const float* bias, c
     // T 128 B 8, 4 turns, 159.5, 161.4, B 40 166.3, 163.6; 230 stacks in all).
     a.launch = exchange_launch_number();
     a.clear_status = l0 == 0;
+    a.early = lc == 1 || (p.per_xcd > 0 && p.per_xcd % lc == 0);
+    if (const char* e = getenv("FTK_LSTM_EXCHANGE_EARLY")) a.early = e[0] == '1';   // =1 / =0: where no h of the team goes to another XCD / never
     const int row_groups = (nrb + p.slices - 1) / p.slices * ((T + 1) / 2 * 2) * block / 32;   // 32 rows each, of a slice
     a.row_layers = std::max(1, std::min({lc, (row_groups + W - 1) / W, kXRowPlaces / W}));
     const int turns = (row_groups + a.row_layers * W - 1) / (a.row_layers * W);

@@ -1421,6 +1421,40 @@ def test_exchange_loops_give_the_same_bits(core, half, H, L, B, T):
         assert all(torch.equal(a, b) for a, b in zip(dense, general))
 
 
+@pytest.mark.parametrize('H,L,T,B,early', [
+    (64, 3, 98, 121, True),      # eight slices of three layers, an XCD each (us when h is looked for at once and later: 98, 114; one layer 97)
+    (128, 2, 100, 233, True),    # fifteen of two, two slices to an XCD (102, 113; 101)
+    (64, 5, 7, 97, True),        # seven slices, the last XCD has none
+    (128, 2, 86, 32, False),     # slices over two XCDs (117, 106)
+    (64, 4, 9, 50, False),
+])
+def test_when_teams_look_for_their_h(core, monkeypatch, H, L, T, B, early):
+    """Stacks whose slices sit on one XCD each look for h at once, others later: the bits are those of the general loop with either, the call takes the
+    time of the better one, and the former's steps are as short as a single layer's."""
+    gen = torch.Generator(device='cuda').manual_seed(12)
+    xs = torch.randn((T, B, H), generator=gen, device='cuda')
+    WU = (torch.rand((L, 2 * H, 4 * H), generator=gen, device='cuda') * 2 - 1) * H ** -0.5
+    ref = core.stacked_lstm(xs, WU, active_rows=[B] * T, check=True)
+    out, alone = tuple(torch.empty_like(r) for r in ref), tuple(torch.empty_like(r[:1]) for r in ref)
+    best = {}
+    for _ in range(5):
+        for way in ('0', '1', None, 'one layer'):
+            monkeypatch.setenv('FTK_LSTM_EXCHANGE_EARLY', way) if way in ('0', '1') else monkeypatch.delenv('FTK_LSTM_EXCHANGE_EARLY', raising=False)
+            weights, results = (WU[:1], alone) if way == 'one layer' else (WU, out)
+            core.stacked_lstm(xs, weights, out=results, check=True)
+            assert all(torch.equal(a, b[:a.shape[0]]) for a, b in zip(results, ref))
+            start, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            start.record()
+            for _ in range(20):
+                core.stacked_lstm(xs, weights, out=results)
+            end.record()
+            end.synchronize()
+            best[way] = min(best.get(way, 1e9), start.elapsed_time(end))
+    if T > 50:      # (shorter ones differ by less than runs of one do)
+        assert best[None] <= 1.06 * min(best['0'], best['1']), best
+        assert not early or best[None] <= 1.08 * best['one layer'], best
+
+
 def exchange_places(ws):
     """Behind a workspace's status block, at a multiple of 256: a word for every workgroup of a launch of the exchange kernel, with the launch's
     number above the lowest 8 bits, and as the last of them that number too where a workgroup gave up before all were there."""
