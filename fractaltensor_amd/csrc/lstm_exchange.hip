@@ -973,11 +973,12 @@ void lstm_exchange_kernel(ExchangeArgs a) {
     // 69 us when asked for behind x only, 65 with both; L 20 T 30 B 32 H 128 83 and 81.6; fp16 H 512 88 and 78.)  The first time it is asked
     // for when it is about to be there.  Where no h goes to another XCD (EARLY: a single layer, or fp32 stacks whose row slices have an XCD each or share
     // one) steps are short and every cycle in front of it costs, but for fp16 teams that share an XCD; elsewhere the layer whose h comes from
-    // another XCD sets the pace, and it is some 320 cycles into the step (fp16 512), at H 64 with four teams or more to an XCD 192.
+    // another XCD sets the pace, and it is some 320 cycles into the step (fp16 512), at H 64 with three teams or more to an XCD 192.
     // (us with 0, 2, 4, 5, 6 and 8 times 64 cycles, EARLY: H 128 L 2 T 100 B 233 102.7, 106.5, 113.5, 113.5, 115.7, 120.9; H 64 L 5 T 86 B 108 90.1, 93.2, 97.9, 100.3,
     // 102.2, 107.0; a single fp16 layer with 0, 1, 2: T 64 B 32 H 256 54.9, 55.9, 57.5, B 200 63.3, 63.2, 60.2.  Elsewhere with 2, 4, 5, 6, 8: L 6 T 80 B 16 H 128 106.1, 101.6,
     // 100.5, 101.2, 104.5; L 5 T 60 B 60 H 64 79.7, 78.3, 78.0, 78.2, 79.5; fp16 L 4 T 60 B 32 H 256 81.9, 80.1, 79.1, 77.5, 74.9, with 10 and 15 75.5, 83.4;
-    // fp16 L 2 T 60 B 33 H 512 with 6, 8, 10 90.2, 88.9, 91.3; H 64 L 20 T 60 B 20 with 3, 4, 5, 6 96.6, 97.7, 99.4, 101.4.  At H 256 fp32, where it is
+    // fp16 L 2 T 60 B 33 H 512 with 6, 8, 10 90.2, 88.9, 91.3; H 64 with 3, 4, 5, 6 L 20 T 60 B 20 96.6, 97.7, 99.4,
+    // 101.4, L 9 T 77 B 18 98.6, 99.2, 100.4, 101.2, and with two teams to an XCD L 4 T 82 B 35 99.1, 98.4, 98.1, 98.5.  At H 256 fp32, where it is
     // asked for behind x only, any delay costs: L 4 T 60 B 16 93.2 without, 93.7 with 2, 95.7 with 4.)
     constexpr bool TWICE = HALF ? H <= 512 : H <= 128;
     int xcd_teams = 0;
@@ -985,7 +986,7 @@ void lstm_exchange_kernel(ExchangeArgs a) {
       xcd_teams = __builtin_amdgcn_readfirstlane(a.per_xcd);
       asm volatile("" : "+s"(xcd_teams));   // kept: left to itself the compiler reads the argument again in every step
     }
-    const bool crowded = xcd_teams >= (HALF ? 2 : 4);
+    const bool crowded = xcd_teams >= (HALF ? 2 : 3);
     share vh;
     float c[U] = {}, h[U];
     const unsigned x_get = do_x ? get : 0x80000000u, h_get = do_h ? get : 0x80000000u;   // out of bounds: zeros
