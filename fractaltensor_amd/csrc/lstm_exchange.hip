@@ -1313,15 +1313,15 @@ int exchange_one_block_layers(int L, int B, int H, bool half) {
   return std::min({L, kXLayers, exchange_teams(H / exchange_units(H, half, false), exchange_slots(f.one)) / ((B + 15) / 16)});
 }
 
-// What the launches of a stack take, in microseconds: `first` and, for each further one, `next` before the steps (weights, places, the
-// kernel in front, and what a deep stack's launches find less of in the caches), `layer` for every further layer of a launch until the
+// What the launches of a stack take, in microseconds: `first` and, for each further one, `next` before the steps (weights, places, what they lay
+// out, and what a deep stack's launches find less of in the caches), `layer` for every further layer of a launch until the
 // pipeline of layers is full, and for a step of each row block that a workgroup walks `step` and `fill` times the workgroups per compute
 // unit.  Fitted, for each hidden size, to the times of both kinds over 420 stacks of L up to 32, T 16 .. 128, B 8 .. 256 that blocks of 16
-// rows take more launches for; the times are met within 1.5 to 8 % (rms).  fp32 up to H 256 fitted again, to 280 stacks of L 3 .. 32, T 16 .. 128,
-// B 33 .. 256 whose weights and inputs change from call to call, when a launch had come to lay out its own buffers (the constants before
-// held a further launch for 37 to 54 us dearer): loss against the better kind in the mean, before and now, H 64 29.6 and 0.4 %, H 128 13.5 and 1.1,
-// H 256 3.7 and 2.1 (there a further launch is charged 8 us beyond the fit, half of what a cooperative one takes more); L 25 T 19 B 106 H 128
-// 194 -> 118 us, L 29 T 104 B 128 H 128 795 -> 572; over 30 other stacks 7.7 %.
+// rows take more launches for, when a kernel in front laid out their buffers; fp32 up to H 256 again, to 280 stacks of L 3 .. 32, T 16 .. 128, B 33 .. 256
+// whose weights and inputs change from call to call, since launches do that themselves (the constants before held a further launch for 37
+// to 54 us dearer).  Loss against the better kind, in the mean over stacks that were not fitted to, with ordinary and with cooperative launches: H 64 0 and
+// 0.2 % (9 stacks), H 128 0.2 and 1.0 (24), H 256 2.4 and 0.1 (62 near the line; with 8 us more charged for a further launch 6.7 and 0.3); with the
+// older constants fp32 H 512 0.1 % (27 stacks), fp16 H 256 0 (22), H 512 0 (29), H 1024 0 (6).
 struct ExchangeCost {
   float step, fill, layer, first, next;
 };
@@ -1334,7 +1334,7 @@ ExchangeCost exchange_cost(int H, bool half, bool many) {
   }
   if (H == 64) return many ? ExchangeCost{0.0f, 1.89f, 0.58f, 21.0f, 21.0f} : ExchangeCost{0.87f, 0.34f, 1.36f, 7.7f, 7.7f};
   if (H == 128) return many ? ExchangeCost{2.58f, 0.27f, 2.15f, 0.0f, 0.0f} : ExchangeCost{0.77f, 0.39f, 1.76f, 6.8f, 8.4f};
-  if (H == 256) return many ? ExchangeCost{3.97f, 0.11f, 4.52f, 20.3f, 20.3f} : ExchangeCost{1.3f, 0.24f, 2.82f, 5.1f, 26.0f};
+  if (H == 256) return many ? ExchangeCost{3.97f, 0.11f, 4.52f, 20.3f, 20.3f} : ExchangeCost{1.3f, 0.24f, 2.82f, 5.1f, 18.0f};
   return many ? ExchangeCost{2.86f, 0.35f, 4.1f, 35.0f, 36.0f} : ExchangeCost{1.73f, 0.24f, 4.35f, 11.5f, 34.0f};
 }
 
@@ -1343,21 +1343,20 @@ ExchangeCost exchange_cost(int H, bool half, bool many) {
 // (the sums of the two matrix instructions are the same), and a launch is charged what it is going to take.  With fp32 data they
 // do not, and what a call computes must not go by that: a launch more is charged most of the difference always.  Loss against the better
 // kind of each, mean over 2940 stacks near the line with ordinary launches and 1900 with cooperative ones: 0.4 and 1.5 % with nothing
-// charged, 0.8 and 0.5 % with 12 us, 1.2 and 0.4 % with 17.
+// charged, 0.8 and 0.5 % with 12 us, 1.2 and 0.4 % with 17 (with the constants of a kernel in front of every launch).
 constexpr float kAnyLaunch = 12.0f, kCooperativeLaunch = 17.0f;
 
 // Layers of one launch (0: the device cannot hold one), and the kind of row block.  16 rows and one block per workgroup, whose
-// step is the shorter one, wherever that takes no more launches (L 23 T 67 B 10 fp32 H 512, three launches of either kind: 831 us
-// with blocks of 32, 540 with blocks of 16), and where the launches it takes more cost less than the steps save: two 16-row workgroups
+// step is the shorter one, wherever that takes no more launches (L 23 T 67 B 10 fp32 H 512, three launches of either kind: 820 us
+// with blocks of 32, 527 with blocks of 16), and where the launches it takes more cost less than the steps save: two 16-row workgroups
 // of H 256 on a compute unit do their steps in 1.8 us, one 32-row workgroup in 4.2.  us with blocks of 32 and of 16: fp32 L 6
-// T 128 B 256 H 256 1120, 782; L 31 T 40 B 20 H 256 333, 256; L 20 T 50 B 100 H 128 316, 261; fp16 L 12 T 30 B 142 H 256
-// 275, 190; the other way round at fp32 L 4 T 30 B 128 H 512 233, 336; L 23 T 17 B 253 H 256 (twelve launches) 699, 986; fp16 L 15 T 25 B 107
-// H 512 423, 484; L 3 T 74 B 41 H 1024 497, 607.  `plain`: neither a ragged batch nor a dilation; those take the general loop,
-// which is no faster with blocks of 16 (ragged L 32 T 48 B 96 H 128 280, 374; dilated L 6 T 100 B 256 H 128 230, 262).
-// The steps weigh against the launches, so T counts: fp32 L 12 B 250 H 128 at T 64 424, 310, at T 16 123, 156.  Near the line, with
-// ordinary launches and with cooperative ones: L 18 T 18 B 216 H 256 622, 704 and 643, 862; L 6 T 92 B 114 H 512 1257, 1236 and 1272, 1343.
-// Over 700 other stacks near the line, ordinary and cooperative: 8 and 4 % faster in the mean than 32-row blocks throughout, more than 2 %
-// slower in 9 and 36 (13 and 20 % at the most: H 64 and 128, where a stack that was run before finds its weights in L2).
+// T 128 B 256 H 256 1091, 752; L 31 T 40 B 20 H 256 306, 243; L 20 T 50 B 100 H 128 303, 211; L 25 T 19 B 106 H 128 162, 119; fp16 L 12 T 30 B 142 H 256
+// 263, 170; the other way round at fp32 L 4 T 30 B 128 H 512 228, 315; L 8 T 42 B 215 H 128 126, 139; fp16 L 15 T 25 B 107
+// H 512 422, 487; L 3 T 74 B 41 H 1024 469, 562.  `plain`: neither a ragged batch nor a dilation; those take the general loop,
+// and ragged ones are slower with blocks of 16 (L 20 T 50 B 250 H 128 528, 639; L 16 T 64 B 220 H 256 1125, 1490; some dilated ones are
+// not: L 12 T 64 B 250 H 128 408, 374).
+// The steps weigh against the launches, so T counts: fp32 L 16 B 220 H 256 at T 18 375, 399, at T 64 1103, 1043.  Near the line, with
+// ordinary launches and with cooperative ones: L 18 T 18 B 216 H 256 603, 469 and 621, 624; L 6 T 92 B 114 H 512 1217, 1222 and 1236, 1316.
 // each_launch: us that every launch is charged beyond its cost.
 int exchange_layers(int L, int T, int B, int H, bool half, bool plain, float each_launch, bool* many) {
   const ExchangeFlavour f = exchange_flavour_of(H, half);

@@ -221,12 +221,16 @@ def test_flash_attention_f32_on_a_workspace_of_planes_only(core, B, Hd, Sq, Skv,
 
 
 @pytest.mark.parametrize('H,L,T,B,blocks', [
-    (256, 18, 18, 216, 32),      # 16 rows 704, 862; 32 rows 622, 643
-    (256, 23, 17, 253, 32),      # 986, 1197; 699, 717
-    (512, 6, 92, 114, 32),       # 1236, 1343; 1257, 1272
-    (256, 6, 128, 256, 16),      # 782, 834; 1120, 1137
-    (256, 31, 40, 20, 16),       # 256, 291; 333, 352
-    (512, 5, 119, 98, 16),       # 1293, 1384; 1481, 1501
+    (256, 16, 18, 220, 32),      # 16 rows 396, 534; 32 rows 373, 389
+    (256, 18, 18, 216, 16),      # 469, 624; 603, 621: of more launches, but 32-row blocks two to a workgroup
+    (256, 23, 17, 253, 32),      # 606, 804; 668, 682
+    (512, 6, 92, 114, 32),       # 1222, 1316; 1217, 1236
+    (256, 6, 128, 256, 16),      # 752, 784; 1091, 1094
+    (256, 31, 40, 20, 16),       # 243, 279; 306, 324
+    (512, 5, 119, 98, 16),       # 1257, 1324; 1478, 1494
+    (64, 29, 23, 137, 16),       # 117, 153; 148, 165
+    (128, 25, 19, 106, 16),      # 119, 154; 162, 180
+    (128, 8, 42, 215, 32),       # 139, 175; 126, 144
 ])
 def test_row_blocks_that_take_more_launches_pay_for_them(core, H, L, T, B, blocks):
     """Both sides of the line between launches of 16-row blocks and fewer launches of 32-row blocks (beside the stacks: us of either
