@@ -222,7 +222,7 @@ def test_flash_attention_f32_on_a_workspace_of_planes_only(core, B, Hd, Sq, Skv,
 
 @pytest.mark.parametrize('H,L,T,B,blocks', [
     (256, 16, 18, 220, 32),      # 16 rows 396, 534; 32 rows 373, 389
-    (256, 18, 18, 216, 16),      # 469, 624; 603, 621: of more launches, but 32-row blocks two to a workgroup
+    (256, 18, 18, 216, 16),      # 469, 624; 603, 621
     (256, 23, 17, 253, 32),      # 606, 804; 668, 682
     (512, 6, 92, 114, 32),       # 1222, 1316; 1217, 1236
     (256, 6, 128, 256, 16),      # 752, 784; 1091, 1094
