@@ -23,7 +23,7 @@
 //     write-through stores, which is what a team that does not sit together uses.
 //
 // A step of a single layer takes 0.85 us at H = 64, 0.9 at 128, 1.2 at 256 and 1.9 at 512 (fp32), where a hand-over of the
-// persistent kernel's serial schedule took 5 to 6 and a launch per step 20 and more: L 20 T 30 B 32 H 128 1004 -> 78 us,
+// persistent kernel's serial schedule took 5 to 6 and a launch per step 20 and more: L 20 T 30 B 32 H 128 1004 -> 76 us,
 // L 8 T 100 B 64 H 512 7.3 -> 0.72 ms, L 1 T 16 B 64 H 256 100 -> 29 us.
 //
 // The exchange buffers.  ring: the own layer's h for d = 1, four steps deep.  A workgroup that has all of h(t-1) knows
@@ -151,8 +151,8 @@ __device__ __forceinline__ void exchange_input_row(const v4u (&raw)[N], Put put,
 // them is written by two workgroups (they begin on a line of their own: exchange_places_at): no cache holds a part of one.
 //
 // Bound by latency: input rows that come from memory, stores that go there, places that come from there.  It takes 2 to 3 us where the kernel in
-// front took 3.4 to 12 and a launch (us a call with other inputs and weights each time, that kernel and this: L 2 T 36 B 155 H 64 50.1, 47.1; L 1 T 64
-// B 100 H 512 150.7, 141.4; L 8 T 100 B 64 H 512 726.5, 706; fp16 L 10 T 30 B 99 H 256 126.5, 121.2; over 47 drawn stacks 2 %).  With the places
+// front took 3.4 to 12 and a launch (us a call with other inputs and weights each time, that kernel and this: L 2 T 36 B 155 H 64 48.6, 46.6; L 1 T 64
+// B 100 H 512 145.2, 141.6; L 8 T 100 B 64 H 512 716, 714; fp16 L 10 T 30 B 99 H 256 125.2, 120.3).  With the places
 // behind the weights, and the rows between the loads of them, single layers began as early, but the places of a workgroup whose weights came late
 // held up the others (fp16 L 10 T 30 B 99 H 256 144.5), and all waves looking at them held up the weights.
 template <int H, bool HALF, bool MANY, typename Args>
@@ -1484,8 +1484,8 @@ int run_exchange(bool half, const void* xs, const void* WU, const float* bias, c
     // The launch lays out its own buffers, unless it is recorded (a replay would find the places of the one before, with its number in them), or a
     // workgroup had too many rows to lay out in front of its first step: a turn of 32 takes it 0.6 us once the first two are on their way
     // beside the weights, the kernel in front takes 1 us for some 4000 rows more (us in a row, that kernel and without: L 1 H 64 T 24 B 8, 3 turns,
-    // 28.1, 27.5; T 128 B 8, 16 turns, 116.8, 123.4, B 250 129.2, 125.9; L 2 H 64 T 96 B 8, 6 turns, 113.2, 115.0, B 100 101.0, 98.8; L 1 H 256
-    // T 128 B 8, 4 turns, 159.5, 161.4, B 40 166.3, 163.6; 230 stacks in all).
+    // 28.5, 28.2; T 128 B 8, 16 turns, 117.3, 124.4, B 250 129.5, 126.1; L 2 H 64 T 96 B 8, 6 turns, 111.5, 113.0, B 100 96.5, 94.5; L 1 H 256
+    // T 128 B 8, 4 turns, 161.4, 161.8, B 40 164.9, 162.4; 230 stacks in all).
     a.launch = exchange_launch_number();
     a.clear_status = l0 == 0;
     a.early = lc == 1 || (p.per_xcd > 0 && p.per_xcd % lc == 0);
